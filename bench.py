@@ -366,9 +366,11 @@ def main() -> int:
         # iteration
         ms3 = time_kernel(lambda: lib.dion_ns_line_3(Bm.data_ptr(), X.data_ptr(), C.data_ptr(), B, m, n, 0.0, st))
         # the vendor library's bf16 GEMM (hipBLASLt behind torch.bmm) on the same operands, same box, same
-        # run: the full product X X^T ("NT": both operands contiguous along the reduction index) and
-        # B X ("NN": X read as it lies, the form of the dominant launch)
-        ms_v_nt = time_kernel(lambda: torch.bmm(X, X.mT, out=A))
+        # run: the full product X X^T and B X ("NN": X read as it lies, the form of the dominant launch).  X^T is
+        # a contiguous copy: the library's batched bf16 product has faulted the GPU on a transposed right operand.
+        XT = X.mT.contiguous()
+        ms_v_nt = time_kernel(lambda: torch.bmm(X, XT, out=A))
+        del XT
         ms_v_nn = time_kernel(lambda: torch.bmm(Bm, X, out=C))
         result["vendor_bf16_gemm"] = {
             "X X^T, full product": {"ms": round(ms_v_nt, 4),
