@@ -545,6 +545,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
         s.g.Q = p.Q + b0 * p.strideQ;
         if (s.g.scale_vec) s.g.scale_vec += b0;
         s.g.batch = c * mpp;
+        s.g.rule_batch = batch;
         s.ptr0 = c0;
         s.n_ptr = c;
         s.x_code = dt(post->x_dtype);

@@ -184,6 +184,8 @@ struct GemmParams {
   int ldp, ldq, ldd, ldc, ldct;
   int M, N, K;
   int batch;
+  int rule_batch;    // batch the kernel is picked for, when this launch is one part of a larger product (0: batch): the
+                     // parts then add up in the same order, and give the same bits, as the whole
   int tri;           // 1: Q == P, only tiles with tile_row <= tile_col are computed, Ct mirrors
   int q_kmajor;      // 1: Q is stored [K][N] (reduction index along rows); not with tri
   int xcd_interleave;  // set by the launcher: tile list dealt to the XCDs in interleaved 32-tile chunks
@@ -206,7 +208,7 @@ __device__ __forceinline__ float gemm_alpha(const GemmParams& p, int b) {
 
 // Returns hipSuccess or the launch error; the tile configuration is picked by shape.
 hipError_t launch_gemm_nt(const GemmParams& p, hipStream_t stream);
-// Tile edge (128 or 256) launch_gemm_nt / launch_gemm_nt_post use for this problem: M and N must be
+// Tile edge (64, 128 or 256) launch_gemm_nt / launch_gemm_nt_post use for this problem: M and N must be
 // multiples of it, K of 128.
 int gemm_tile_edge(const GemmParams& p);
 // C = P * Q with Q K-major (p.q_kmajor, no tri, no D), the product consumed by the fused Muon update

@@ -32,7 +32,7 @@ namespace dion {
 template <int BM_, int BN_, int BK_, int WM_, int WN_, int NSTAGE_>
 struct TileCfg {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, NSTAGE = NSTAGE_;
-  static_assert(NSTAGE_ == 2, "the pipeline below is written for a two-slot ring");
+  static_assert(NSTAGE_ == 2 || NSTAGE_ == 4, "two-slot ring, or a four-slot one for launches that leave a CU one workgroup");
   static constexpr int NT = WM * WN * 64;
   static constexpr int CPR = BK / 8;            // 16-byte chunks per tile row
   static constexpr int ROWS_PER_LOAD = NT / CPR; // tile rows covered by one load instruction
@@ -191,6 +191,46 @@ __device__ __forceinline__ void tri_tile(int t, int T, int& ti, int& tj) {
   ti = tj = 0;  // unreachable for t < T(T+1)/2
 }
 
+// Tile number `pid` of a launch of `total` tiles -> (batch, tile row, tile column).  Hardware deals workgroups
+// round-robin over the 8 XCDs; each XCD (own L2) gets one contiguous run of the tile list, so that neighbours share
+// operands, or -- xcd_interleave -- 32 consecutive tiles of every 256: the 8 XCDs then work on neighbouring tile
+// groups (same matrix, same operand row panels) at the same time, and what one of them fetches from memory the
+// others find in the memory-side cache.  The latter pays when a matrix's operands are much larger than an XCD's L2.
+template <int BM, int BN>
+__device__ __forceinline__ void tile_of(const GemmParams& p, int pid, int total, int& b, int& ti, int& tj) {
+  const int tilesM = p.M / BM, tilesN = p.N / BN;
+  const int tiles_per_mat = p.tri ? (tilesM * (tilesM + 1)) / 2 : tilesM * tilesN;
+  int lt;
+  if (p.xcd_interleave && pid < (total & ~255)) {
+    const int j = pid & 255;
+    lt = (pid & ~255) + (j & 7) * 32 + (j >> 3);
+  } else if (p.xcd_interleave) {
+    lt = pid;
+  } else {
+    const int xcd = pid & 7, loc = pid >> 3;
+    const int q = total >> 3, r = total & 7;
+    lt = xcd * q + (xcd < r ? xcd : r) + loc;
+  }
+  b = lt / tiles_per_mat;
+  const int t = lt - b * tiles_per_mat;
+  if (p.tri) {
+    tri_tile(t, tilesM, ti, tj);
+  } else {
+    constexpr int GM = 8;
+    const int per_group = GM * tilesN;
+    const int g = t / per_group;
+    const int first = g * GM;
+    const int gsz = (tilesM - first) < GM ? (tilesM - first) : GM;
+    const int tg = t - g * per_group;
+    ti = first + tg % gsz;
+    tj = tg / gsz;
+  }
+  // (the same for every lane: say so, tile bases live in scalar registers)
+  b = __builtin_amdgcn_readfirstlane(b);
+  ti = __builtin_amdgcn_readfirstlane(ti);
+  tj = __builtin_amdgcn_readfirstlane(tj);
+}
+
 // Workgroup barrier preceded by the counter waits the software pipeline needs: every LDS read
 // this wave issued has returned (the ring slot they read is about to be refilled) and all but the
 // newest VM_LEFT direct-to-LDS loads of this wave have landed.  The "memory" clobber keeps the
@@ -307,45 +347,8 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
 
-  // ---- workgroup -> (batch, tile) map.  Hardware deals workgroups round-robin over the 8 XCDs;
-  // give each XCD (own L2) one contiguous run of the tile list so neighbours share operands.
-  const int tilesM = p.M / BM, tilesN = p.N / BN;
-  const int tiles_per_mat = p.tri ? (tilesM * (tilesM + 1)) / 2 : tilesM * tilesN;
-  const int total = gridDim.x;
-  int lt;
-  {
-    const int pid = blockIdx.x;
-    if (p.xcd_interleave && pid < (total & ~255)) {
-      // 256 consecutive workgroups = 32 per XCD: each XCD takes 32 consecutive tiles of the same 256-tile
-      // stretch, so the 8 XCDs work on neighbouring tile groups (same matrix, same operand row panels)
-      // at the same time, and what one of them fetches from memory the others find in the memory-side
-      // cache.  Pays when a matrix's operands are much larger than an XCD's L2.
-      const int j = pid & 255;
-      lt = (pid & ~255) + (j & 7) * 32 + (j >> 3);
-    } else if (p.xcd_interleave) {
-      lt = pid;
-    } else {
-      // one contiguous run of the tile list per XCD: a small matrix stays in one L2
-      const int xcd = pid & 7, loc = pid >> 3;
-      const int q = total >> 3, r = total & 7;
-      lt = xcd * q + (xcd < r ? xcd : r) + loc;
-    }
-  }
-  const int b = lt / tiles_per_mat;
-  const int t = lt - b * tiles_per_mat;
-  int ti, tj;
-  if (p.tri) {
-    tri_tile(t, tilesM, ti, tj);
-  } else {
-    constexpr int GM = 8;
-    const int per_group = GM * tilesN;
-    const int g = t / per_group;
-    const int first = g * GM;
-    const int gsz = (tilesM - first) < GM ? (tilesM - first) : GM;
-    const int tg = t - g * per_group;
-    ti = first + tg % gsz;
-    tj = tg / gsz;
-  }
+  int b, ti, tj;
+  tile_of<BM, BN>(p, blockIdx.x, gridDim.x, b, ti, tj);
 
   // ---- global -> LDS addressing.  Chunk q = j*NT + tid of a tile lands at LDS byte q*16; it holds
   // logical 16-byte chunk (q % CPR) ^ swz(row) of tile row q / CPR.
@@ -464,15 +467,71 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
 
   // ---- prologue: fill NSTAGE-1 ring slots, wait for slab 0, read its first fragments, start the
   // last free slot.
+  constexpr bool DEEP = NSTAGE > 2;
+  auto ring_barrier = [&](int newer) {
+    // slabs newer than the one waited for that may still be in flight
+    constexpr int PL = Cfg::P_LOADS;
+    if (newer >= 2) { if (one_operand) pipeline_barrier<2 * PL>(); else pipeline_barrier<2 * LPS>(); }
+    else if (newer == 1) { if (one_operand) pipeline_barrier<PL>(); else pipeline_barrier<LPS>(); }
+    else pipeline_barrier<0>();
+  };
 #pragma unroll
   for (int s = 0; s < NSTAGE - 1; ++s)
+    if (!DEEP || s < KT)
 #pragma unroll
-    for (int j = 0; j < LPS; ++j) issue_load(s, s, j);
-  pipeline_barrier<(NSTAGE - 2) * LPS>();
+      for (int j = 0; j < LPS; ++j) issue_load(s, s, j);
+  if constexpr (DEEP) ring_barrier((KT < NSTAGE - 1 ? KT : NSTAGE - 1) - 1);
+  else pipeline_barrier<(NSTAGE - 2) * LPS>();
   static_for<0, 8>([&](auto rc) { read_frag(ic0(), ic0(), rc); });
+  if (!DEEP || NSTAGE - 1 < KT)
 #pragma unroll
-  for (int j = 0; j < (SPREAD ? LPS / 2 : LPS); ++j) issue_load(NSTAGE - 1, NSTAGE - 1, j);
+    for (int j = 0; j < (SPREAD ? LPS / 2 : LPS); ++j) issue_load(NSTAGE - 1, NSTAGE - 1, j);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (DEEP) {
+    static_assert(!SPREAD, "");
+    int slot = 0;
+    auto slab = [&](int kt, auto refill) {
+      const int next = slot == NSTAGE - 1 ? 0 : slot + 1;
+      static_for<0, HP>([&](auto hc) {
+        constexpr int hp = decltype(hc)::value;
+        constexpr int st = hp / HALVES, part = hp % HALVES, fs = hp & 1, bs = st & 1;
+        constexpr bool last = (hp == HP - 1);
+        if constexpr (last) {
+          if constexpr (decltype(refill)::value) {
+            if (one_operand) pipeline_barrier<(NSTAGE - 2) * Cfg::P_LOADS>();
+            else pipeline_barrier<(NSTAGE - 2) * LPS>();
+          } else ring_barrier(KT - 2 - kt);
+          // every read of this slab has been issued and has returned: the address registers move to the next slot
+          const uint32_t d = (uint32_t)(next - slot) * (uint32_t)Cfg::P_BYTES;
+#pragma unroll
+          for (int t = 0; t < ST; ++t) { aoff[t] += d; if (!QK) boff[t] += d; }
+          if (QK)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) qoff[j] += d;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        static_for<0, NM>([&](auto qc) {
+          constexpr int q = decltype(qc)::value, i = q / 4, j = q % 4;
+          frag_wait<FS::allowed(hp, q)>(fa[fs][i], fb[bs][j]);
+          acc[part * 4 + i][j] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[fs][i], fb[bs][j], acc[part * 4 + i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (FS::read_behind(hp, q) >= 0) {
+            typedef std::integral_constant<int, FS::read_behind(hp, q)> rc;
+            if constexpr (last) read_frag(ic0(), ic0(), rc());
+            else read_frag(ic0(), std::integral_constant<int, hp + 1>(), rc());
+          }
+          if constexpr (decltype(refill)::value)
+            if constexpr (last && (q & 1) && q / 2 < LPS) issue_load(kt + NSTAGE, slot, q / 2);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      });
+      slot = next;
+    };
+    int kt = 0;
+    for (; kt + NSTAGE < KT; ++kt) slab(kt, std::true_type());
+    for (; kt < KT; ++kt) slab(kt, std::false_type());
+  } else
 
   // ---- main loop.  Halves run back to back across slab boundaries: while the MFMAs of one half issue, the
   // fragment reads of the next half (and, from the last half of a slab on, the refill of the slot that slab
@@ -752,35 +811,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
-  const int tilesM = p.M / BM, tilesN = p.N / BN;
-  const int tiles_per_mat = tilesM * tilesN;
   const int KT = p.K / BK;
-
-  // Tile number `pid` of the launch -> (batch, tile row, tile column): the same map as the kernel above
-  // uses for its workgroup index, so consecutive workgroups (= XCDs) share operand panels the same way.
-  auto tile_of = [&](int pid, int& b, int& ti, int& tj) {
-    int lt;
-    if (p.xcd_interleave && pid < (total_tiles & ~255)) {
-      const int j = pid & 255;
-      lt = (pid & ~255) + (j & 7) * 32 + (j >> 3);
-    } else if (p.xcd_interleave) {
-      lt = pid;
-    } else {
-      const int xcd = pid & 7, loc = pid >> 3;
-      const int q = total_tiles >> 3, r = total_tiles & 7;
-      lt = xcd * q + (xcd < r ? xcd : r) + loc;
-    }
-    b = lt / tiles_per_mat;
-    const int t = lt - b * tiles_per_mat;
-    constexpr int GM = 8;
-    const int per_group = GM * tilesN;
-    const int g = t / per_group;
-    const int first = g * GM;
-    const int gsz = (tilesM - first) < GM ? (tilesM - first) : GM;
-    const int tg = t - g * per_group;
-    ti = first + tg % gsz;
-    tj = tg / gsz;
-  };
 
   // ---- global -> LDS addressing (see the kernel above): per-lane offsets are the same for every tile,
   // the tile only moves the wave-uniform base pointers.
@@ -800,7 +831,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
 
   int b_c, ti_c, tj_c, b_n, ti_n, tj_n;
   int pid = blockIdx.x;
-  tile_of(pid, b_c, ti_c, tj_c);
+  tile_of<BM, BN>(p, pid, total_tiles, b_c, ti_c, tj_c);
   auto base_p = [&](int b, int ti) { return (const char*)(p.P + (int64_t)b * p.strideP + (int64_t)(ti * BM) * p.ldp); };
   auto base_q = [&](int b, int tj) { return (const char*)(p.Q + (int64_t)b * p.strideQ + tj * BN); };
   const char* gP_c = base_p(b_c, ti_c);
@@ -811,7 +842,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
     // fetched again and never read, which keeps the load count per slab fixed)
     const int np = pid + (int)gridDim.x;
     if (np < total_tiles) {
-      tile_of(np, b_n, ti_n, tj_n);
+      tile_of<BM, BN>(p, np, total_tiles, b_n, ti_n, tj_n);
       gP_n = base_p(b_n, ti_n);
       gQ_n = base_q(b_n, tj_n);
     } else {
@@ -983,7 +1014,274 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
 }
 
 // ---------------------------------------------------------------------------------------------
+// The same product for launches of few tiles: 64 x 64 tiles, the reduction of a tile split over the four
+// wavefronts of its workgroup.  With a handful of 128-wide tiles most CUs idle and each busy one walks the whole
+// reduction at the pace of its own operand stream (0.4-0.6 us per 64-deep slab, 64 slabs for 1024 x 4096); four times
+// as many tiles, each pulling a quarter of the bytes at once through four private rings, use the CUs that are
+// there.  A wavefront takes every fourth slab (64 x 64 of each operand) into a two-slot ring of its own and never
+// meets a barrier until its partial sums are added; the 64 x 64 wavefront tile keeps the fragment schedule of the
+// 128-wide kernel.  Per CU 64 KB of loads stay in flight.
+struct CfgK64 {
+  static constexpr int BM = 64, BN = 64, BK = 64, NT = 256, KW = 4;  // KW wavefronts share a reduction
+  static constexpr int OP_BYTES = 64 * 64 * 2;                       // one operand of one slab
+  static constexpr int WAVE_BYTES = 4 * OP_BYTES;                    // [P slot 0][P slot 1][Q slot 0][Q slot 1]
+  static constexpr int STG_PITCH = 64 * 2 + 16;
+  static constexpr int LDS_BYTES = KW * WAVE_BYTES;
+  // after the loop: partial sums [wavefront][row block][column block][lane] f32x4, then the staged transposed tile
+  static constexpr int PART_BYTES = KW * 16 * 64 * 16;
+  static_assert(PART_BYTES + 64 * STG_PITCH <= LDS_BYTES, "reduction and staging areas");
+};
+
+template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0>
+__global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
+  typedef CfgK64 Cfg;
+  typedef typename PostSel<POST>::xt XT;
+  constexpr int OPB = Cfg::OP_BYTES, KW = Cfg::KW, BK = Cfg::BK;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int b, ti, tj;
+  tile_of<64, 64>(p, blockIdx.x, gridDim.x, b, ti, tj);
+  const bool one_operand = !QK && p.tri && ti == tj && p.P == p.Q && p.ldp == p.ldq && p.strideP == p.strideQ;
+
+  // ---- global -> LDS: a load moves 8 tile rows of 128 bytes; lane l brings 16-byte chunk l % 8 of row l / 8.  The
+  // swizzles are those of the kernel above; a load's first row is a multiple of 8, and they differ between
+  // even and odd multiples, hence two offsets per operand.
+  const int lrow = lane >> 3, lchunk = lane & 7;
+  uint32_t offP[2], offQ[2];
+#pragma unroll
+  for (int o = 0; o < 2; ++o) {
+    const int pc = lchunk ^ ((o * 4 + (lrow >> 1)) & 7);
+    offP[o] = (uint32_t)(lrow * p.ldp + pc * 8) * 2u;
+    // K-major rows are 128 bytes: the four rows of a transposing read fall into the two halves of a 256-byte bank
+    // row twice; rows 2 and 3 swap their 64-byte groups, rows 8 apart their 32-byte halves
+    const int qc = QK ? ((((lchunk >> 2) ^ ((lrow >> 1) & 1)) << 2) | ((lchunk & 3) ^ (o << 1))) : pc;
+    offQ[o] = (uint32_t)(lrow * p.ldq + qc * 8) * 2u;
+  }
+  const char* gP = (const char*)(p.P + (int64_t)b * p.strideP + (int64_t)(ti * 64) * p.ldp);
+  const char* gQ = QK ? (const char*)(p.Q + (int64_t)b * p.strideQ + tj * 64)
+                      : (const char*)(p.Q + (int64_t)b * p.strideQ + (int64_t)(tj * 64) * p.ldq);
+  const uint32_t stepP = (uint32_t)(8 * p.ldp) * 2u, stepQ = (uint32_t)(8 * p.ldq) * 2u;
+  const int64_t slabQ = QK ? (int64_t)BK * p.ldq * 2 : (int64_t)BK * 2;
+  const int KT = p.K / BK;
+  const int nw = KT > wave ? (KT - wave + KW - 1) / KW : 0;  // slabs of this wavefront: wave, wave + KW, ...
+  char* const ring = lds + wave * Cfg::WAVE_BYTES;
+  constexpr int LPS = 16;
+  auto issue_load = [&](int t, int slot, int j) {
+    if (one_operand && j >= 8) return;
+    const int kt = wave + t * KW;
+    if (j < 8) {
+      const char* src = gP + (int64_t)kt * (BK * 2) + (uint64_t)j * stepP;
+      asm volatile("" : "+s"(src), "+v"(offP[j & 1]));
+      __builtin_amdgcn_global_load_lds(GLB_PTR(src + offP[j & 1]), LDS_PTR(ring + slot * OPB + j * 1024), 16, 0, 0);
+    } else {
+      const int jq = j - 8;
+      const char* src = gQ + kt * slabQ + (uint64_t)jq * stepQ;
+      asm volatile("" : "+s"(src), "+v"(offQ[jq & 1]));
+      __builtin_amdgcn_global_load_lds(GLB_PTR(src + offQ[jq & 1]), LDS_PTR(ring + (2 + slot) * OPB + jq * 1024), 16, 0, 0);
+    }
+  };
+
+  // ---- LDS -> register fragments (see the kernel above)
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)ring;
+  const int l16 = lane & 15, quad = lane >> 4;
+  uint32_t aoff[2], boff[2], qoff[4];
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    const int chunk = ((st * 4 + quad) ^ (l16 >> 1)) * 16;
+    aoff[st] = lds_base + (uint32_t)(l16 * 128 + chunk);
+    boff[st] = aoff[st] + (one_operand ? 0 : 2 * OPB);
+  }
+  if (QK) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      qoff[j] = lds_base + (uint32_t)(2 * OPB + (8 * quad + (l16 >> 2)) * 128 + (((j >> 1) ^ (l16 >> 3)) << 6) +
+                                      ((j ^ quad) & 1) * 32 + (l16 & 3) * 8);
+  }
+  typedef FragSched<1, 2, QK> FS;
+  bf16x8 fa[2][4], fb[2][4];
+  auto read_frag = [&](auto hnc, auto rc) {
+    constexpr int st = decltype(hnc)::value, r = decltype(rc)::value;
+    if constexpr (r == 0 || r > 4) {
+      constexpr int i = r == 0 ? 0 : r - 4;
+      lds_read16<i * 2048>(fa[st][i], aoff[st]);
+    } else if constexpr (QK) {
+      lds_read_tr<st * 4096, 512>(fb[st][r - 1], qoff[r - 1]);
+    } else {
+      lds_read16<(r - 1) * 2048>(fb[st][r - 1], boff[st]);
+    }
+  };
+  typedef std::integral_constant<int, 0> ic0;
+  typedef std::integral_constant<int, 1> ic1;
+
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- main loop over this wavefront's slabs: no other wavefront touches its ring, so its own load counter is all
+  // the synchronisation there is
+  if (nw > 0) {
+#pragma unroll
+    for (int j = 0; j < LPS; ++j) issue_load(0, 0, j);
+    if (nw > 1)
+#pragma unroll
+      for (int j = 0; j < LPS; ++j) issue_load(1, 1, j);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    if (nw > 1) {
+      if (one_operand) wait_vmcnt<LPS / 2>();
+      else wait_vmcnt<LPS>();
+    } else wait_vmcnt<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<0, 8>([&](auto rc) { read_frag(ic0(), rc); });
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t step = OPB;  // to the other slot: + OPB, then - OPB, ...
+    auto slab = [&](int t, auto refill) {
+      static_for<0, 2>([&](auto hc) {
+        constexpr int hp = decltype(hc)::value;
+        if constexpr (hp == 1) {
+          // the other slab has landed, and every read of this one has returned: its slot may be refilled
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt 0, lgkmcnt 0
+          asm volatile("" ::: "memory");
+#pragma unroll
+          for (int st = 0; st < 2; ++st) {
+            aoff[st] += step;
+            if (!QK) boff[st] += step;
+          }
+          if (QK)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) qoff[j] += step;
+          step = 0u - step;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        static_for<0, 16>([&](auto qc) {
+          constexpr int q = decltype(qc)::value, i = q / 4, j = q % 4;
+          frag_wait<FS::allowed(hp, q)>(fa[hp][i], fb[hp][j]);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[hp][i], fb[hp][j], acc[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (FS::read_behind(hp, q) >= 0) {
+            typedef std::integral_constant<int, FS::read_behind(hp, q)> rc;
+            if constexpr (hp == 1) read_frag(ic0(), rc());
+            else read_frag(ic1(), rc());
+          }
+          if constexpr (decltype(refill)::value && hp == 1) issue_load(t + 2, t & 1, q);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      });
+    };
+    int t = 0;
+    for (; t + 2 < nw; ++t) slab(t, std::true_type());
+    for (; t < nw; ++t) slab(t, std::false_type());
+  }
+  wait_vmcnt<0>();
+  // (see the kernel above: the read-ahead of the last half must land before its registers are let go)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      asm volatile("" ::"v"(fa[f][i]));
+      asm volatile("" ::"v"(fb[f][i]));
+    }
+
+  // ---- partial sums -> tile.  Wavefront w finishes row block w (16 rows): every other wavefront hands it its share
+  // through LDS, added in wavefront order.
+  const int row_base = ti * 64 + wave * 16, col_base = tj * 64;
+  float pa = 0.f, pcoeff = 0.f, pb = 0.f;
+  XT* xmat = nullptr;
+  if constexpr (POST != 0) {
+    const float wd = post.wd_dev ? *post.wd_dev : post.wd_host;
+    muon_post_coeffs(*post.lr_dev, wd, post.adj_ratio, pa, pcoeff, pb);
+    const int pi = b / post.mats_per_ptr;
+    xmat = (XT*)post.X.p[pi] + (int64_t)(b - pi * post.mats_per_ptr) * (HAS_C ? p.strideC : p.strideCt);
+  }
+  bf16_t dreg[4][4];
+  if (HAS_D) {
+    const bf16_t* Dp = p.D + (int64_t)b * p.strideD + (int64_t)(row_base + 4 * quad) * p.ldd + col_base + l16;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dreg[j][e] = Dp[(int64_t)e * p.ldd + j * 16];
+  }
+  __syncthreads();  // every wavefront is done with its ring
+  f32x4* part = (f32x4*)lds;  // [wavefront][row block][column block][lane]
+  static_for<0, 4>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part[((wave * 4 + i) * 4 + j) * 64 + lane] = acc[i][j];
+  });
+  __syncthreads();
+  const float alpha = gemm_alpha(p, b), beta = p.beta;
+  const bool on_diag = p.tri && ti == tj && p.diag != 0.0f;
+  char* stg = lds + Cfg::PART_BYTES;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f32x4 s = part[(wave * 4 + j) * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < KW; ++w) s += part[((w * 4 + wave) * 4 + j) * 64 + lane];
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = alpha * s[e];
+    if (HAS_D) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += beta * bf16_to_f32(dreg[j][e]);
+    }
+    if (on_diag) {
+      const int dcol = col_base + j * 16 + l16 - (row_base + 4 * quad);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (dcol == e) v[e] += p.diag;
+    }
+    if (HAS_C) {
+      const int64_t at = (int64_t)(row_base + 4 * quad) * p.ldc + col_base + l16 + j * 16;
+      if constexpr (POST != 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          st_store<XT>(xmat, at + (int64_t)e * p.ldc,
+                       muon_post_one(st_load<XT>(xmat, at + (int64_t)e * p.ldc), bf16_to_f32(f32_to_bf16(v[e])), pa,
+                                     pcoeff, pb, post.cautious));
+      } else {
+        bf16_t* Cp = p.C + (int64_t)b * p.strideC + at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Cp[(int64_t)e * p.ldc] = f32_to_bf16(v[e]);
+      }
+    }
+    if (HAS_CT) {
+      uint2 pk;
+      pk.x = pack_bf16x2(v[0], v[1]);
+      pk.y = pack_bf16x2(v[2], v[3]);
+      *(uint2*)(stg + (j * 16 + l16) * Cfg::STG_PITCH + (wave * 16 + 4 * quad) * 2) = pk;
+    }
+  }
+  if (HAS_CT) {
+    __syncthreads();
+    if constexpr (POST != 0) {
+      // the staged bf16 tile is the update of X[col][row]: a wavefront takes 16 of the 64 rows of X, lanes along a row
+      XT* xt = xmat + (int64_t)(col_base + wave * 16) * p.ldct + ti * 64 + lane;
+#pragma unroll 8
+      for (int c = 0; c < 16; ++c) {
+        const float u = bf16_to_f32(*(const bf16_t*)(stg + (wave * 16 + c) * Cfg::STG_PITCH + lane * 2));
+        const int64_t at = (int64_t)c * p.ldct;
+        st_store<XT>(xt, at, muon_post_one(st_load<XT>(xt, at), u, pa, pcoeff, pb, post.cautious));
+      }
+    } else if (!(p.tri && ti == tj)) {  // a diagonal tile is its own mirror
+      bf16_t* Ctp = p.Ct + (int64_t)b * p.strideCt + (int64_t)col_base * p.ldct + ti * 64;
+#pragma unroll
+      for (int it = 0; it < 2; ++it) {
+        const int c = (tid >> 3) + it * 32, ch = tid & 7;
+        *(uint4*)(Ctp + (int64_t)c * p.ldct + ch * 8) = *(const uint4*)(stg + c * Cfg::STG_PITCH + ch * 16);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 typedef TileCfg<128, 128, 64, 2, 2, 2> Cfg128;     // 4 wavefronts, 64x64 each; two workgroups per CU
+typedef TileCfg<128, 128, 64, 2, 2, 4> Cfg128d;    // the same on a four-slot ring: one workgroup per CU
 typedef TileCfg<256, 256, 64, 2, 4, 2> Cfg256w8;   // 8 wavefronts, 128x64 each: two per SIMD, one workgroup per CU
 constexpr int kWalkMaxK = 2048;                    // longest reduction the tile-walking kernel is used for
 
@@ -1005,6 +1303,23 @@ static hipError_t launch_epi(const GemmParams& p, hipStream_t stream,
   GemmParams pp = p;
   pp.xcd_interleave = xcd_interleave_pays(p) ? 1 : 0;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, pp, post);
+  return hipGetLastError();
+}
+
+template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0>
+static hipError_t launch_k64_epi(const GemmParams& p, hipStream_t stream,
+                                 const typename PostSel<POST>::arg& post = typename PostSel<POST>::arg()) {
+  static std::atomic<uint64_t> attr_done{0};
+  auto kern = gemm_k64_kernel<HAS_D, HAS_C, HAS_CT, QK, POST>;
+  if (hipError_t e = set_max_dynamic_lds_once((const void*)kern, CfgK64::LDS_BYTES, attr_done)) return e;
+  if (p.M % 64 || p.N % 64 || p.K % 64) return hipErrorInvalidValue;
+  const int64_t T = p.M / 64;
+  const int64_t total = (p.tri ? T * (T + 1) / 2 : T * (p.N / 64)) * p.batch;
+  if (total <= 0) return hipSuccess;
+  if (total > 0x7fffffff) return hipErrorInvalidValue;
+  GemmParams pp = p;
+  pp.xcd_interleave = xcd_interleave_pays(p) ? 1 : 0;
+  hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(CfgK64::NT), CfgK64::LDS_BYTES, stream, pp, post);
   return hipGetLastError();
 }
 
@@ -1039,7 +1354,7 @@ static hipError_t launch_walk(const GemmParams& p, hipStream_t stream) {
 // The operand / result combinations the Newton-Schulz drivers use.
 template <class Cfg>
 static hipError_t launch_cfg(const GemmParams& p, hipStream_t stream) {
-  if (p.M % Cfg::BM || p.N % Cfg::BN || p.K % (Cfg::BK * Cfg::NSTAGE)) return hipErrorInvalidValue;
+  if (p.M % Cfg::BM || p.N % Cfg::BN || p.K % 128) return hipErrorInvalidValue;
   const bool d = p.D != nullptr, c = p.C != nullptr, ct = p.Ct != nullptr;
   if (p.q_kmajor) {
     if (p.tri) return hipErrorInvalidValue;
@@ -1062,6 +1377,19 @@ static hipError_t launch_cfg(const GemmParams& p, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
+static hipError_t launch_k64(const GemmParams& p, hipStream_t stream) {
+  const bool d = p.D != nullptr, c = p.C != nullptr, ct = p.Ct != nullptr;
+  if (p.q_kmajor && !p.tri) {
+    if (!d && c && !ct) return launch_k64_epi<false, true, false, true>(p, stream);
+    if (!d && !c && ct) return launch_k64_epi<false, false, true, true>(p, stream);
+    return hipErrorInvalidValue;
+  }
+  if (p.tri && !d && c && ct) return launch_k64_epi<false, true, true, false>(p, stream);
+  if (p.tri && d && c && ct) return launch_k64_epi<true, true, true, false>(p, stream);
+  if (!p.tri && !d && c && !ct) return launch_k64_epi<false, true, false, false>(p, stream);
+  return hipErrorInvalidValue;
+}
+
 int gemm_pad_granule(int m, int n, int batch) {
   // 256-wide tiles need enough of them to fill 256 CUs; small problems use 128-wide tiles.
   const int64_t m256 = (m + 255) / 256;
@@ -1070,24 +1398,41 @@ int gemm_pad_granule(int m, int n, int batch) {
   return syrk_tiles >= 256 ? 256 : 128;
 }
 
-// 256-wide tiles when there are enough of them: a full product from 384 tiles (one and a half rounds of the
-// 256 CUs; 432 tiles of 12 x (768 x 3072) run 14 % faster than the 1728 128-wide ones, 108 tiles of
-// 12 x (768 x 768) 20 % slower), a symmetric one from 160 (16 x 1024-wide: 5 % faster; 72 tiles of
-// 12 x 768-wide: 70 % slower).  Rounds that are not full cost less than their geometry says: the part is
-// power-limited, and the CUs that are busy run faster while others idle.  Below the thresholds the 128-wide
-// tiles (two workgroups per CU) win.
-static bool wants_256_tiles(const GemmParams& p) {
-  const long T = p.M / 256;
-  const long t256 = (p.tri ? T * (T + 1) / 2 : T * (p.N / 256)) * p.batch;
-  return p.M % 256 == 0 && p.N % 256 == 0 && t256 >= (p.tri ? 160L : 384L);
+// Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box.
+//  * 256-wide tiles when there are enough of them: a full product from 384 (one and a half rounds of the 256 CUs;
+//    432 tiles of 12 x (768 x 3072) run 14 % faster than the 1728 128-wide ones, 108 tiles of 12 x (768 x 768) 20 %
+//    slower), a symmetric one from 160 (16 x 1024-wide: 5 % faster; 72 tiles of 12 x 768-wide: 70 % slower).  Rounds
+//    that are not full cost less than their geometry says: the part is power-limited, and the CUs that are busy run
+//    faster while others idle.
+//  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
+//    per CU, for symmetric products (whose 128-wide form has only a quarter as many) two per CU: X X^T of one
+//    768 x 3072 matrix 28.4 -> 10.0, of 1024 x 4096 42.9 -> 15.8; at two rounds 12 x (512 x 2048) 22.8 -> 16.8 (18.4
+//    with the form below), at three 4 x (1024 x 2816) 28.4 against 23.4; B X at 576 tiles (768 x 3072) 14.0 against 9.3.
+//  * 128-wide tiles, at most one per CU: the CU is one workgroup's alone, and a ring of four slots keeps three slabs
+//    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
+//    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
+//  * else 128-wide tiles on a two-slot ring, two workgroups per CU (288 tiles of 8 x (1024 x 4096): 50 against 62).
+enum TileKind { kTile64, kTile128Deep, kTile128, kTile256 };
+static TileKind pick_tile(const GemmParams& p) {
+  auto tiles = [&](int edge) -> int64_t {
+    const int64_t T = p.M / edge;
+    return (p.tri ? T * (T + 1) / 2 : T * (p.N / edge)) * (p.rule_batch > 0 ? p.rule_batch : p.batch);
+  };
+  if (p.M % 256 == 0 && p.N % 256 == 0 && tiles(256) >= (p.tri ? 160 : 384)) return kTile256;
+  if (tiles(64) <= (p.tri ? 512 : 256) && !(p.D && !p.tri)) return kTile64;
+  if (tiles(128) <= 256 && (p.tri || p.K > 1024)) return kTile128Deep;
+  return kTile128;
 }
 
-int gemm_tile_edge(const GemmParams& p) { return wants_256_tiles(p) ? 256 : 128; }
+int gemm_tile_edge(const GemmParams& p) {
+  const TileKind k = pick_tile(p);
+  return k == kTile256 ? 256 : k == kTile64 ? 64 : 128;
+}
 
 template <class Cfg>
 static hipError_t launch_post_cfg(const GemmParams& p, const FusedPost& post, int x_dtype, bool transposed,
                                   hipStream_t stream) {
-  if (p.M % Cfg::BM || p.N % Cfg::BN || p.K % (Cfg::BK * Cfg::NSTAGE)) return hipErrorInvalidValue;
+  if (p.M % Cfg::BM || p.N % Cfg::BN || p.K % 128) return hipErrorInvalidValue;
   if (x_dtype == 1) {
     return transposed ? launch_epi<Cfg, false, false, true, true, 1>(p, stream, post)
                       : launch_epi<Cfg, false, true, false, true, 1>(p, stream, post);
@@ -1104,14 +1449,28 @@ hipError_t launch_gemm_nt_post(const GemmParams& p, const FusedPost& post, int x
   if (!p.q_kmajor || p.tri || p.D || post.mats_per_ptr <= 0 || !post.lr_dev ||
       p.batch > (int64_t)kMaxPtrs * post.mats_per_ptr || (x_dtype != 0 && x_dtype != 1))
     return hipErrorInvalidValue;
-  return wants_256_tiles(p) ? launch_post_cfg<Cfg256w8>(p, post, x_dtype, transposed, stream)
-                            : launch_post_cfg<Cfg128>(p, post, x_dtype, transposed, stream);
+  switch (pick_tile(p)) {
+    case kTile256: return launch_post_cfg<Cfg256w8>(p, post, x_dtype, transposed, stream);
+    case kTile128Deep: return launch_post_cfg<Cfg128d>(p, post, x_dtype, transposed, stream);
+    case kTile64:
+      if (x_dtype == 1)
+        return transposed ? launch_k64_epi<false, false, true, true, 1>(p, stream, post)
+                          : launch_k64_epi<false, true, false, true, 1>(p, stream, post);
+      return transposed ? launch_k64_epi<false, false, true, true, 2>(p, stream, post)
+                        : launch_k64_epi<false, true, false, true, 2>(p, stream, post);
+    default: return launch_post_cfg<Cfg128>(p, post, x_dtype, transposed, stream);
+  }
 }
 
 hipError_t launch_gemm_nt(const GemmParams& p, hipStream_t stream) {
   if (p.M <= 0 || p.N <= 0 || p.K <= 0 || p.batch <= 0) return hipSuccess;
   if (p.tri && (p.M != p.N)) return hipErrorInvalidValue;
-  return wants_256_tiles(p) ? launch_cfg<Cfg256w8>(p, stream) : launch_cfg<Cfg128>(p, stream);
+  switch (pick_tile(p)) {
+    case kTile256: return launch_cfg<Cfg256w8>(p, stream);
+    case kTile128Deep: return launch_cfg<Cfg128d>(p, stream);
+    case kTile64: return launch_k64(p, stream);
+    default: return launch_cfg<Cfg128>(p, stream);
+  }
 }
 
 }  // namespace dion

@@ -1,0 +1,79 @@
+"""The GEMM forms for launches of few tiles (64-wide tiles with the reduction split over a workgroup's wavefronts;
+128-wide tiles on a four-slot ring) at the sizes where they can go wrong: fewer k slabs than wavefronts or ring
+slots, slab counts that are no multiple of either, one tile, tile counts on both sides of each rule.  References
+are float64 products of the same bf16 inputs; the bound on the mean error is that of one bf16 rounding of the result
+(2^-9 of its magnitude at most) plus fp32 accumulation."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _lib():
+    from dion_amd import _lib as L
+
+    return L.load(), L.check, torch.cuda.current_stream().cuda_stream
+
+
+def _close(res, ref):
+    """Every element within one bf16 rounding of the float64 value, with the fp32 sums (K terms, relative 2^-24
+    each, of the magnitude of the row's products) on top."""
+    err = (res.double() - ref).abs()
+    bound = ref.abs() * 2.0 ** -8 + ref.abs().mean() * 1e-4
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+# (batch, m, n, tile edge of the symmetric products, of B X)
+CASES = [
+    (1, 128, 128, 64, 64), (1, 128, 384, 64, 64), (3, 256, 640, 64, 64), (1, 896, 128, 64, 64),
+    (2, 384, 1664, 64, 128), (4, 512, 2048, 64, 128), (14, 512, 128, 64, 64), (15, 512, 128, 128, 64),
+    (1, 1408, 1408, 64, 128), (1, 2048, 2048, 128, 128), (1, 1920, 2176, 64, 128), (7, 1024, 1152, 128, 128),
+]
+
+
+@pytest.mark.parametrize("batch,m,n,sym_edge,full_edge", CASES)
+def test_products_of_few_tiles(batch, m, n, sym_edge, full_edge):
+    lib, check, st = _lib()
+    assert lib.dion_gemm_tile_edge(batch, m, m, 1) == sym_edge
+    assert lib.dion_gemm_tile_edge(batch, m, n, 0) == full_edge
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    X = torch.randn(batch, m, n, device=DEV, generator=g).to(torch.bfloat16)
+    A = torch.full((batch, m, m), float("nan"), device=DEV, dtype=torch.bfloat16)
+    B = torch.full_like(A, float("nan"))
+    Y = torch.full_like(X, float("nan"))
+    check(lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), batch, m, n, st), "line_1")
+    ref = X.double() @ X.double().mT.contiguous()
+    _close(A, ref)
+    assert torch.equal(A, A.mT)
+    S = (A.float() / n).to(torch.bfloat16)
+    check(lib.dion_ns_line_2(S.data_ptr(), B.data_ptr(), batch, m, ctypes.c_float(0.5), ctypes.c_float(2.0), st), "line_2")
+    Sd = S.double()
+    _close(B, 0.5 * (Sd @ Sd) + 2.0 * Sd)
+    assert torch.equal(B, B.mT)
+    check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, n, ctypes.c_float(0.0), st), "line_3")
+    _close(Y, B.double() @ X.double())
+    A2 = torch.empty_like(A)
+    check(lib.dion_ns_line_1(X.data_ptr(), A2.data_ptr(), batch, m, n, st), "line_1")
+    assert torch.equal(A, A2)
+
+
+@pytest.mark.parametrize("shape,cautious", [((1, 256, 512), False), ((1, 512, 256), True), ((1, 2048, 2048), False),
+                                            ((2, 384, 384), True)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_fused_update_of_few_tiles(shape, cautious, dtype):
+    """The update applied by these kernels equals the update pass on their stored result, bit for bit."""
+    from dion_amd import ops
+    from dion_amd.newton_schulz import NS5_COEFFS
+
+    torch.manual_seed(5)
+    batch = shape[0]
+    G = (torch.randn(*shape, device=DEV) * 0.02).to(torch.bfloat16)
+    X = [(torch.randn(*shape[1:], device=DEV) * 0.02).to(dtype) for _ in range(batch)]
+    X2 = [x.clone() for x in X]
+    lr = torch.tensor(0.02, device=DEV)
+    ops.ns_orthogonalize_update(G, X, NS5_COEFFS, 1.0, 1e-7, lr, 0.7, 0.01, cautious)
+    ops.muon_post(X2, ops.ns_orthogonalize(G, NS5_COEFFS, 1.0, 1e-7).view(batch, -1), lr, 0.7, 0.01, cautious)
+    assert all(torch.equal(a, b) for a, b in zip(X, X2))

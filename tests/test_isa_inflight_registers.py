@@ -149,3 +149,23 @@ def test_no_kernel_touches_a_register_a_transposing_read_is_in_flight_to(tmp_pat
     for kname, kbody in kernels.items():
         mfma = [i for i, l in enumerate(kbody) if "v_mfma" in l]
         assert not [l for l in kbody[mfma[0]:mfma[-1] + 1] if "scratch_" in l], kname
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not on PATH")
+def test_split_reduction_kernel_keeps_its_reads_apart(tmp_path):
+    """The same walk over the kernels for few tiles (gemm_k64_kernel) and the four-slot forms of gemm_nt_kernel."""
+    out = tmp_path / "gemm_nt.s"
+    subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-S", "--cuda-device-only", SRC, "-o",
+                    str(out)], check=True, capture_output=True, timeout=900)
+    text = out.read_text().split("\n")
+    starts = [i for i, l in enumerate(text)
+              if re.match(r"_ZN4dion\d+gemm_k64_kernel\S*:|_ZN4dion\d+gemm_nt_kernelINS_7TileCfgILi128ELi128ELi64ELi2ELi2ELi4E\S*:", l)]
+    assert len(starts) >= 19
+    for i in starts:
+        end = next(j for j in range(i, len(text)) if "s_endpgm" in text[j])
+        body = text[i + 1:end + 1]
+        n_reads, hazards = walk(body)
+        assert n_reads > 0 and not hazards, (text[i], hazards[:5])
+        mfma = [j for j, l in enumerate(body) if "v_mfma" in l]
+        assert not [l for l in body[mfma[0]:mfma[-1] + 1] if "scratch_" in l], text[i]
