@@ -663,8 +663,28 @@ static __device__ __forceinline__ float g_load(const GT* g, int64_t i) {
   return sizeof(GT) == 2 ? bf16_to_f32(((const bf16_t*)g)[i]) : ((const float*)g)[i];
 }
 
-// select rows: one wavefront per row, norms[mat][row] = sum_j |M+G| (of the values as stored).
-template <typename GT, typename MT>
+// select rows: one wavefront per row, norms[mat][row] = sum_j |M+G| (of the values as stored).  A lane adds the
+// columns lane, lane + 64, ... in that order, whatever the batch it loads them in.
+// Bound by HBM: sixteen columns' loads in flight per lane, non-temporal past the caches.  24 x (2048 x 8192), fp32 momentum,
+// bf16 gradients: 824 us (4.9 TB/s) one column at a time -> 730 us (5.5 TB/s); bf16 momentum 600 -> 420 us;
+// 12 x (768 x 3072) 52 -> 42 us.
+template <int B, typename GT, typename MT, bool NT>
+static __device__ __forceinline__ void acc_row_batch(const GT* __restrict__ g, MT* __restrict__ m, int c, float& s) {
+  float gv[B], mv[B];
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    mv[i] = st_load<MT, NT>(m, c + 64 * i);
+    gv[i] = st_load<GT, NT>(g, c + 64 * i);
+  }
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    const float v = st_round<MT>(__fadd_rn(mv[i], gv[i]));
+    st_store<MT, NT>(m, c + 64 * i, v);
+    s += fabsf(v);
+  }
+}
+
+template <typename GT, typename MT, bool NT>
 __global__ __launch_bounds__(256) void dion2_acc_rows_kernel(PtrTab G, PtrTab M, int mats_per_ptr,
                                                              int rows, int cols,
                                                              float* __restrict__ norms) {
@@ -673,14 +693,13 @@ __global__ __launch_bounds__(256) void dion2_acc_rows_kernel(PtrTab G, PtrTab M,
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
   const int64_t base = ((int64_t)(mat % mats_per_ptr) * rows + row) * cols;
-  const GT* g = (const GT*)G.p[mat / mats_per_ptr] + base;
-  MT* m = (MT*)M.p[mat / mats_per_ptr] + base;
+  const GT* __restrict__ g = (const GT*)G.p[mat / mats_per_ptr] + base;
+  MT* __restrict__ m = (MT*)M.p[mat / mats_per_ptr] + base;
   float s = 0.f;
-  for (int c = lane; c < cols; c += 64) {
-    const float v = st_round<MT>(__fadd_rn(st_load<MT>(m, c), g_load<GT>(g, c)));
-    st_store<MT>(m, c, v);
-    s += fabsf(v);
-  }
+  int c = 0;
+  for (; c + 64 * 16 <= cols; c += 64 * 16) acc_row_batch<16, GT, MT, NT>(g, m, c + lane, s);
+  for (; c + 64 * 4 <= cols; c += 64 * 4) acc_row_batch<4, GT, MT, NT>(g, m, c + lane, s);
+  for (c += lane; c < cols; c += 64) acc_row_batch<1, GT, MT, NT>(g, m, c, s);
   s = wave_sum(s);
   if (lane == 0) norms[(int64_t)mat * rows + row] = s;
 }
@@ -713,10 +732,33 @@ __global__ __launch_bounds__(256) void dion2_acc_cols_kernel(PtrTab G, PtrTab M,
                                      (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
+template <int B, typename GT, typename MT, bool NT>
+static __device__ __forceinline__ void acc_cols_batch(const GT* __restrict__ g, MT* __restrict__ m, int64_t i, int cols,
+                                                      float4& s) {
+  float gv[B][4], mv[B][4];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {  // cols % 4 == 0 on this path
+    st_load4<MT, NT>(m, (i >> 2) + (int64_t)b * cols, mv[b]);
+    st_load4<GT, NT>(g, (i >> 2) + (int64_t)b * cols, gv[b]);
+  }
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mv[b][e] = st_round<MT>(__fadd_rn(mv[b][e], gv[b][e]));
+    st_store4<MT, NT>(m, (i >> 2) + (int64_t)b * cols, mv[b]);
+    s.x += fabsf(mv[b][0]);
+    s.y += fabsf(mv[b][1]);
+    s.z += fabsf(mv[b][2]);
+    s.w += fabsf(mv[b][3]);
+  }
+}
+
 // 4 columns per thread (8- / 16-byte accesses): each block owns 256 columns, four row lanes.
+// Bound by HBM: eight rows' loads in flight per thread, non-temporal past the caches (24 x (8192 x 2048), fp32 momentum, bf16
+// gradients: 844 us (4.8 TB/s) with four -> 717 us (5.6 TB/s); 12 x (3072 x 768) 52 us either way).
 // With gridDim.z row slabs the block writes its slab's partial sums to out[(slab*n_mat + mat)*cols]
 // (n_mat = gridDim.y); dion2_sum_slabs_kernel adds the slabs in a fixed order.
-template <typename GT, typename MT>
+template <typename GT, typename MT, bool NT>
 __global__ __launch_bounds__(256) void dion2_acc_cols_vec_kernel(PtrTab G, PtrTab M, int mats_per_ptr,
                                                                  int rows, int cols, int slab_rows,
                                                                  float* __restrict__ norms) {
@@ -728,24 +770,14 @@ __global__ __launch_bounds__(256) void dion2_acc_cols_vec_kernel(PtrTab G, PtrTa
   const int c = (blockIdx.x * 64 + (threadIdx.x & 63)) * 4;
   const int ry = threadIdx.x >> 6;
   const int64_t base = (int64_t)(mat % mats_per_ptr) * rows * cols;
-  const GT* g = (const GT*)G.p[mat / mats_per_ptr] + base;
-  MT* m = (MT*)M.p[mat / mats_per_ptr] + base;
+  const GT* __restrict__ g = (const GT*)G.p[mat / mats_per_ptr] + base;
+  MT* __restrict__ m = (MT*)M.p[mat / mats_per_ptr] + base;
   float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
   if (c < cols) {
-#pragma unroll 4
-    for (int r = r0 + ry; r < r1; r += 4) {
-      const int64_t i4 = ((int64_t)r * cols + c) >> 2;  // cols % 4 == 0 on this path
-      float gv[4], mv[4];
-      st_load4<GT>(g, i4, gv);
-      st_load4<MT>(m, i4, mv);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) mv[e] = st_round<MT>(__fadd_rn(mv[e], gv[e]));
-      st_store4<MT>(m, i4, mv);
-      s.x += fabsf(mv[0]);
-      s.y += fabsf(mv[1]);
-      s.z += fabsf(mv[2]);
-      s.w += fabsf(mv[3]);
-    }
+    int r = r0 + ry;
+    // eight rows' loads in flight, added in row order
+    for (; r + 28 < r1; r += 32) acc_cols_batch<8, GT, MT, NT>(g, m, (int64_t)r * cols + c, cols, s);
+    for (; r < r1; r += 4) acc_cols_batch<1, GT, MT, NT>(g, m, (int64_t)r * cols + c, cols, s);
   }
   red[ry][threadIdx.x & 63] = s;
   __syncthreads();
@@ -783,17 +815,25 @@ hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M
                                    int mats_per_ptr, int rows, int cols, int select_rows,
                                    float* norms, bool vec4, float* slab_scratch, int slabs,
                                    hipStream_t st) {
-  // DISPATCH(kernel, grid, args...): the four (gradient, momentum) dtype pairs
-#define ACC_LAUNCH(K, GRID, ...)                                                                        \
+  const bool nt = exceeds_caches((int64_t)n_mat * rows * cols * ((m_dtype == 0 ? 4 : 8) + (g_dtype == 0 ? 2 : 4)));
+  // the four (gradient, momentum) dtype pairs; NTV... is empty for kernels without a non-temporal form
+#define ACC_LAUNCH_T(K, GRID, NTV, ...)                                                                 \
   do {                                                                                                  \
     if (g_dtype == 0 && m_dtype == 0)                                                                   \
-      hipLaunchKernelGGL((K<bf16_t, bf16_t>), GRID, dim3(256), 0, st, __VA_ARGS__);                      \
+      hipLaunchKernelGGL((K<bf16_t, bf16_t NTV>), GRID, dim3(256), 0, st, __VA_ARGS__);                  \
     else if (g_dtype == 0)                                                                              \
-      hipLaunchKernelGGL((K<bf16_t, float>), GRID, dim3(256), 0, st, __VA_ARGS__);                       \
+      hipLaunchKernelGGL((K<bf16_t, float NTV>), GRID, dim3(256), 0, st, __VA_ARGS__);                   \
     else if (m_dtype == 0)                                                                              \
-      hipLaunchKernelGGL((K<float, bf16_t>), GRID, dim3(256), 0, st, __VA_ARGS__);                       \
+      hipLaunchKernelGGL((K<float, bf16_t NTV>), GRID, dim3(256), 0, st, __VA_ARGS__);                   \
     else                                                                                                \
-      hipLaunchKernelGGL((K<float, float>), GRID, dim3(256), 0, st, __VA_ARGS__);                        \
+      hipLaunchKernelGGL((K<float, float NTV>), GRID, dim3(256), 0, st, __VA_ARGS__);                    \
+  } while (0)
+#define ACC_NT , true
+#define ACC_T , false
+#define ACC_LAUNCH(K, GRID, ...)                             \
+  do {                                                       \
+    if (nt) ACC_LAUNCH_T(K, GRID, ACC_NT, __VA_ARGS__);      \
+    else ACC_LAUNCH_T(K, GRID, ACC_T, __VA_ARGS__);          \
   } while (0)
   if (select_rows) {
     dim3 grid((rows + 3) / 4, n_mat);
@@ -812,8 +852,11 @@ hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M
     }
   } else {
     dim3 grid((cols + 63) / 64, n_mat);
-    ACC_LAUNCH(dion2_acc_cols_kernel, grid, G, M, mats_per_ptr, rows, cols, norms);
+    ACC_LAUNCH_T(dion2_acc_cols_kernel, grid, , G, M, mats_per_ptr, rows, cols, norms);
   }
+#undef ACC_NT
+#undef ACC_T
+#undef ACC_LAUNCH_T
 #undef ACC_LAUNCH
   return hipGetLastError();
 }
@@ -1098,95 +1141,180 @@ hipError_t launch_dion2_gather_prepared(const PtrTab& M, int m_dtype, int n_mat,
   return hipGetLastError();
 }
 
-// x = a*x - b*u[map] on selected slices, x = a*x elsewhere; one rounding of the sum.
-// Block (row group of 8, mat); 4 columns per thread on the vector path.  u is bf16 or fp32 (UT).
+// x = a*x - b*u[map] on selected slices, x = a*x elsewhere; one rounding of the sum.  u is bf16 or fp32 (UT).
 template <typename UT>
 static __device__ __forceinline__ float u_load(const UT* u, int64_t i) {
   return sizeof(UT) == 2 ? bf16_to_f32(((const bf16_t*)u)[i]) : ((const float*)u)[i];
 }
-template <typename UT>
-static __device__ __forceinline__ float4 u_load4(const UT* u, int64_t i) {
-  if (sizeof(UT) == 2) {
-    const uint2 raw = *(const uint2*)((const bf16_t*)u + i);
-    return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u),
-                       __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xffff0000u));
-  }
-  return *(const float4*)((const float*)u + i);
+struct Dion2PostArgs {
+  const int32_t* map;
+  const float *row_scale, *lr_dev, *adj_lr_dev, *wd_dev;
+  float adj_ratio, wd_host;
+};
+// x = a*x - b*u
+static __device__ __forceinline__ void dion2_post_coeffs(const Dion2PostArgs& p, float& a, float& b) {
+  const float lr = *p.lr_dev;
+  const float wd = p.wd_dev ? *p.wd_dev : p.wd_host;
+  a = __fsub_rn(1.0f, __fmul_rn(lr, wd));
+  b = __fmul_rn(p.adj_lr_dev ? *p.adj_lr_dev : lr, p.adj_ratio);
 }
 
-template <bool VEC, typename UT, typename XT>
-__global__ __launch_bounds__(256) void dion2_post_kernel(PtrTab X, int mats_per_ptr, int rows,
-                                                         int cols, int select_rows,
-                                                         const UT* __restrict__ U, int k,
-                                                         const int32_t* __restrict__ map,
-                                                         const float* __restrict__ row_scale,
-                                                         const float* __restrict__ lr_dev,
-                                                         const float* __restrict__ adj_lr_dev,
-                                                         float adj_ratio,
-                                                         const float* __restrict__ wd_dev,
-                                                         float wd_host) {
+// Any size and alignment, one element at a time; block (row group of 8, mat).
+template <typename UT, typename XT>
+__global__ __launch_bounds__(256) void dion2_post_kernel(PtrTab X, int mats_per_ptr, int rows, int cols, int select_rows,
+                                                         const UT* __restrict__ U, int k, Dion2PostArgs p) {
   const int mat = blockIdx.y;
   XT* x = (XT*)X.p[mat / mats_per_ptr] + (int64_t)(mat % mats_per_ptr) * rows * cols;
-  const float lr = *lr_dev;
-  const float wd = wd_dev ? *wd_dev : wd_host;
-  const float a = __fsub_rn(1.0f, __fmul_rn(lr, wd));
-  const float b0 = __fmul_rn(adj_lr_dev ? *adj_lr_dev : lr, adj_ratio);
-  float b = b0;
-  const int dim = select_rows ? rows : cols;
-  const int32_t* mp = map + (int64_t)mat * dim;
+  float a, b0;
+  dion2_post_coeffs(p, a, b0);
+  const int32_t* mp = p.map + (int64_t)mat * (select_rows ? rows : cols);
   const UT* u = U + (int64_t)mat * (select_rows ? (int64_t)k * cols : (int64_t)rows * k);
   const int r_end = (blockIdx.x * 8 + 8) < rows ? (blockIdx.x * 8 + 8) : rows;
   for (int r = blockIdx.x * 8; r < r_end; ++r) {
     XT* xr = x + (int64_t)r * cols;
-    if (select_rows) {
-      const int j = mp[r];
-      const UT* ur = u + (int64_t)(j < 0 ? 0 : j) * cols;
-      // per-row scale of the selected slice (rows selected only): u is multiplied by it first
-      if (row_scale && j >= 0) b = __fmul_rn(b0, row_scale[(int64_t)mat * k + j]);
-      if (VEC) {
-        for (int c4 = threadIdx.x; c4 < cols / 4; c4 += 256) {
-          float v[4];
-          st_load4<XT>(xr, c4, v);
-          float4 uv = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (j >= 0) uv = u_load4<UT>(ur, c4 * 4);
-          v[0] = fmaf(a, v[0], -(b * uv.x));
-          v[1] = fmaf(a, v[1], -(b * uv.y));
-          v[2] = fmaf(a, v[2], -(b * uv.z));
-          v[3] = fmaf(a, v[3], -(b * uv.w));
-          st_store4<XT>(xr, c4, v);
-        }
-      } else {
-        for (int c = threadIdx.x; c < cols; c += 256) {
-          const float uv = j >= 0 ? u_load<UT>(ur, c) : 0.f;
-          st_store<XT>(xr, c, fmaf(a, st_load<XT>(xr, c), -(b * uv)));
-        }
-      }
-    } else {
-      const UT* ur = u + (int64_t)r * k;
-      if (VEC) {
-        for (int c4 = threadIdx.x; c4 < cols / 4; c4 += 256) {
-          float v[4];
-          st_load4<XT>(xr, c4, v);
-          const int4 j4 = *(const int4*)(mp + c4 * 4);
-          const float u0 = j4.x >= 0 ? u_load<UT>(ur, j4.x) : 0.f;
-          const float u1 = j4.y >= 0 ? u_load<UT>(ur, j4.y) : 0.f;
-          const float u2 = j4.z >= 0 ? u_load<UT>(ur, j4.z) : 0.f;
-          const float u3 = j4.w >= 0 ? u_load<UT>(ur, j4.w) : 0.f;
-          v[0] = fmaf(a, v[0], -(b * u0));
-          v[1] = fmaf(a, v[1], -(b * u1));
-          v[2] = fmaf(a, v[2], -(b * u2));
-          v[3] = fmaf(a, v[3], -(b * u3));
-          st_store4<XT>(xr, c4, v);
-        }
-      } else {
-        for (int c = threadIdx.x; c < cols; c += 256) {
-          const int j = mp[c];
-          const float uv = j >= 0 ? u_load<UT>(ur, j) : 0.f;
-          st_store<XT>(xr, c, fmaf(a, st_load<XT>(xr, c), -(b * uv)));
-        }
-      }
+    const int jr = select_rows ? mp[r] : 0;
+    // per-row scale of the selected slice (rows selected only): u is multiplied by it first
+    const float b = p.row_scale && jr >= 0 ? __fmul_rn(b0, p.row_scale[(int64_t)mat * k + jr]) : b0;
+    const UT* ur = u + (select_rows ? (int64_t)(jr < 0 ? 0 : jr) * cols : (int64_t)r * k);
+    for (int c = threadIdx.x; c < cols; c += 256) {
+      const int j = select_rows ? (jr < 0 ? -1 : c) : mp[c];
+      const float uv = j >= 0 ? u_load<UT>(ur, j) : 0.f;
+      st_store<XT>(xr, c, fmaf(a, st_load<XT>(xr, c), -(b * uv)));
     }
   }
+}
+
+// Rows selected, groups of W consecutive elements (8 of bf16 X where rows allow it: 16-byte accesses, else 4): a
+// workgroup owns 8192 consecutive elements of a matrix whatever rows they lie in, a thread has sixteen elements of X (and,
+// in the selected rows, of U) in flight.
+// Bound by HBM (non-temporal past the caches).  24 x (2048 x 8192), k = 512, fp32 X: 682 us (5.0 TB/s) a row at a time ->
+// 570 us (6.0 TB/s); bf16 X 363 -> 276 us.
+constexpr int kPostRun = 8192;
+template <bool NT, int W, typename UT, typename XT>
+__global__ __launch_bounds__(256) void dion2_post_rows_kernel(PtrTab X, int mats_per_ptr, int rows, int cols,
+                                                              const UT* __restrict__ U, int k, Dion2PostArgs p) {
+  constexpr int N = 16 / W, kRound = 256 * N;  // groups per thread / per workgroup and round
+  const int mat = blockIdx.y;
+  const unsigned w = (unsigned)cols / W;
+  const int64_t n = (int64_t)rows * w;
+  XT* __restrict__ x = (XT*)X.p[mat / mats_per_ptr] + (int64_t)(mat % mats_per_ptr) * rows * cols;
+  const int32_t* __restrict__ mp = p.map + (int64_t)mat * rows;
+  const UT* __restrict__ u = U + (int64_t)mat * k * cols;
+  for (int round = 0; round < kPostRun / (kRound * W); ++round) {
+    const int64_t first = (int64_t)blockIdx.x * (kPostRun / W) + round * kRound;
+    if (first >= n) return;
+    const int row0 = (int)(first / w);
+    const unsigned rem0 = (unsigned)(first - (int64_t)row0 * w);
+    float v[N][W], uv[N][W], b[N];
+    int j[N];
+    unsigned c[N];
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+      const unsigned q = threadIdx.x + g * 256;
+      if (first + q < n) st_loadw<XT, W, NT>(x, first + q, v[g]);
+      const unsigned dr = (rem0 + q) / w;
+      c[g] = rem0 + q - dr * w;
+      j[g] = first + q < n ? mp[row0 + dr] : -1;
+    }
+    float a, b0;
+    dion2_post_coeffs(p, a, b0);
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+#pragma unroll
+      for (int e = 0; e < W; ++e) uv[g][e] = 0.f;
+      b[g] = b0;
+      if (j[g] >= 0) {
+        st_loadw<UT, W>(u, (int64_t)j[g] * w + c[g], uv[g]);
+        // per-row scale of the selected slice: u is multiplied by it first
+        if (p.row_scale) b[g] = __fmul_rn(b0, p.row_scale[(int64_t)mat * k + j[g]]);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+#pragma unroll
+      for (int e = 0; e < W; ++e) v[g][e] = fmaf(a, v[g][e], -(b[g] * uv[g][e]));
+      if (first + threadIdx.x + g * 256 < n) st_storew<XT, W, NT>(x, first + threadIdx.x + g * 256, v[g]);
+    }
+  }
+}
+
+// Columns selected, groups of four: a workgroup owns `rpb` rows; their selected values, rpb * k consecutive elements of U,
+// go through LDS (gathered from memory two bytes a lane they cost as much as X itself), a thread keeps its columns'
+// positions in registers and has four rows of X in flight.
+// Bound by HBM.  24 x (8192 x 2048), k = 512, fp32 X: 785 us (4.35 TB/s) with the gathers from memory -> 557 us (6.1 TB/s);
+// bf16 X 605 -> 271 us.
+template <bool NT, typename UT, typename XT>
+__global__ __launch_bounds__(256) void dion2_post_cols_kernel(PtrTab X, int mats_per_ptr, int rows, int cols, int rpb,
+                                                              const UT* __restrict__ U, int k, Dion2PostArgs p) {
+  extern __shared__ float4 post_lds[];
+  UT* lu = (UT*)post_lds;
+  const int mat = blockIdx.y;
+  const int r0 = blockIdx.x * rpb;
+  const int nr = rows - r0 < rpb ? rows - r0 : rpb;
+  XT* __restrict__ x = (XT*)X.p[mat / mats_per_ptr] + (int64_t)(mat % mats_per_ptr) * rows * cols + (int64_t)r0 * cols;
+  const int32_t* __restrict__ mp = p.map + (int64_t)mat * cols;
+  const UT* __restrict__ u = U + ((int64_t)mat * rows + r0) * k;
+  const int nu = nr * k;
+  const int nv = (((uintptr_t)u) & 15) == 0 ? nu * (int)sizeof(UT) / 16 : 0;  // whole 16-byte pieces
+  for (int i = threadIdx.x; i < nv; i += 256) post_lds[i] = ((const float4*)u)[i];
+  for (int i = nv * (16 / (int)sizeof(UT)) + threadIdx.x; i < nu; i += 256) lu[i] = u[i];
+  float a, b;
+  dion2_post_coeffs(p, a, b);
+  __syncthreads();
+  for (int c4 = threadIdx.x; c4 < cols / 4; c4 += 256) {
+    const int4 j4 = *(const int4*)(mp + c4 * 4);
+    const int j[4] = {j4.x, j4.y, j4.z, j4.w};
+    int jl[4];  // (an unselected column reads the row's first value and drops it)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) jl[e] = j[e] < 0 ? 0 : j[e];
+    auto rows_of = [&](int r, int n) {
+      float v[4][4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q < n) st_load4<XT, NT>(x, (((int64_t)(r + q) * cols) >> 2) + c4, v[q]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (q >= n) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float uv = u_load<UT>(lu, (r + q) * k + jl[e]);
+          v[q][e] = fmaf(a, v[q][e], -(b * (j[e] >= 0 ? uv : 0.f)));
+        }
+        st_store4<XT, NT>(x, (((int64_t)(r + q) * cols) >> 2) + c4, v[q]);
+      }
+    };
+    int r = 0;
+    for (; r + 4 <= nr; r += 4) rows_of(r, 4);
+    for (; r < nr; ++r) rows_of(r, 1);
+  }
+}
+
+constexpr int kPostLds = 32 * 1024;  // selected values of one workgroup's rows; five workgroups per CU
+
+template <typename UT, typename XT>
+static void dion2_post_dispatch(const PtrTab& X, int n_mat, int mats_per_ptr, int rows, int cols, int select_rows,
+                                const UT* U, int k, const Dion2PostArgs& p, bool vec4, hipStream_t st) {
+  const bool nt = exceeds_caches((int64_t)n_mat * rows * cols * 2 * (int)sizeof(XT));
+  const int64_t wg = ((int64_t)rows * cols + kPostRun - 1) / kPostRun;
+  if (vec4 && select_rows && wg <= (1 << 23)) {
+    const dim3 grid((unsigned)wg, n_mat);
+    const bool w8 = sizeof(XT) == 2 && cols % 8 == 0;
+    auto* kernel = w8 ? (nt ? dion2_post_rows_kernel<true, 8, UT, XT> : dion2_post_rows_kernel<false, 8, UT, XT>)
+                      : (nt ? dion2_post_rows_kernel<true, 4, UT, XT> : dion2_post_rows_kernel<false, 4, UT, XT>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, X, mats_per_ptr, rows, cols, U, k, p);
+    return;
+  }
+  const int64_t row_bytes = (int64_t)k * sizeof(UT);
+  if (vec4 && !select_rows && k > 0 && row_bytes <= kPostLds) {
+    const int rpb = row_bytes * 8 <= kPostLds ? 8 : (row_bytes * 4 <= kPostLds ? 4 : 1);
+    const dim3 grid((rows + rpb - 1) / rpb, n_mat);
+    const size_t lds = (size_t)(rpb * row_bytes + 15) / 16 * 16;
+    auto* kernel = nt ? dion2_post_cols_kernel<true, UT, XT> : dion2_post_cols_kernel<false, UT, XT>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, X, mats_per_ptr, rows, cols, rpb, U, k, p);
+    return;
+  }
+  hipLaunchKernelGGL((dion2_post_kernel<UT, XT>), dim3((rows + 7) / 8, n_mat), dim3(256), 0, st, X, mats_per_ptr, rows, cols,
+                     select_rows, U, k, p);
 }
 
 hipError_t launch_dion2_post(const PtrTab& X, int x_dtype, int n_mat, int mats_per_ptr, int rows, int cols,
@@ -1194,20 +1322,15 @@ hipError_t launch_dion2_post(const PtrTab& X, int x_dtype, int n_mat, int mats_p
                              const float* row_scale, const float* lr_dev, const float* adj_lr_dev,
                              float adj_ratio, const float* wd_dev, float wd_host, bool vec4,
                              hipStream_t st) {
-  dim3 grid((rows + 7) / 8, n_mat);
-#define D2POST_LAUNCH(V, UT, XT)                                                                          \
-  hipLaunchKernelGGL((dion2_post_kernel<V, UT, XT>), grid, dim3(256), 0, st, X, mats_per_ptr, rows, cols, \
-                     select_rows, (const UT*)U, k, map, row_scale, lr_dev, adj_lr_dev, adj_ratio,           \
-                     wd_dev, wd_host)
-#define D2POST_LAUNCH_X(V, UT) \
-  do { if (x_dtype == 0) D2POST_LAUNCH(V, UT, bf16_t); else D2POST_LAUNCH(V, UT, float); } while (0)
+  const Dion2PostArgs p{map, row_scale, lr_dev, adj_lr_dev, wd_dev, adj_ratio, wd_host};
+#define D2POST(UT, XT) \
+  dion2_post_dispatch<UT, XT>(X, n_mat, mats_per_ptr, rows, cols, select_rows, (const UT*)U, k, p, vec4, st)
   if (u_dtype == 0) {
-    if (vec4) D2POST_LAUNCH_X(true, bf16_t); else D2POST_LAUNCH_X(false, bf16_t);
+    if (x_dtype == 0) D2POST(bf16_t, bf16_t); else D2POST(bf16_t, float);
   } else {
-    if (vec4) D2POST_LAUNCH_X(true, float); else D2POST_LAUNCH_X(false, float);
+    if (x_dtype == 0) D2POST(float, bf16_t); else D2POST(float, float);
   }
-#undef D2POST_LAUNCH_X
-#undef D2POST_LAUNCH
+#undef D2POST
   return hipGetLastError();
 }
 

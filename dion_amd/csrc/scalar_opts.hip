@@ -20,38 +20,6 @@
 
 namespace dion {
 
-// Groups of four elements as in st_load4 / st_store4, with NT past the caches (non-temporal).
-typedef __attribute__((ext_vector_type(4))) unsigned mta_u32x4;
-typedef __attribute__((ext_vector_type(2))) unsigned mta_u32x2;
-template <typename T, bool NT>
-static __device__ __forceinline__ void mta_load4(const T* p, int64_t i4, float v[4]) {
-  if constexpr (!NT) {
-    st_load4<T>(p, i4, v);
-  } else if constexpr (sizeof(T) == 2) {
-    const mta_u32x2 raw = __builtin_nontemporal_load((const mta_u32x2*)p + i4);
-    v[0] = __uint_as_float(raw[0] << 16);
-    v[1] = __uint_as_float(raw[0] & 0xffff0000u);
-    v[2] = __uint_as_float(raw[1] << 16);
-    v[3] = __uint_as_float(raw[1] & 0xffff0000u);
-  } else {
-    const mta_u32x4 raw = __builtin_nontemporal_load((const mta_u32x4*)p + i4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(raw[e]);
-  }
-}
-template <typename T, bool NT>
-static __device__ __forceinline__ void mta_store4(T* p, int64_t i4, const float v[4]) {
-  if constexpr (!NT) {
-    st_store4<T>(p, i4, v);
-  } else if constexpr (sizeof(T) == 2) {
-    const mta_u32x2 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    __builtin_nontemporal_store(o, (mta_u32x2*)p + i4);
-  } else {
-    const mta_u32x4 o = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
-    __builtin_nontemporal_store(o, (mta_u32x4*)p + i4);
-  }
-}
-
 struct MtaTensors {
   uint64_t x[kMtaTensors], g[kMtaTensors], m[kMtaTensors], v[kMtaTensors], step[kMtaTensors];
   int64_t numel[kMtaTensors];
@@ -140,10 +108,10 @@ __global__ __launch_bounds__(256) void adamw_mt_kernel(MtaTensors a, int n, cons
       const int64_t q0 = (first + r * kMtaRound) / 4 + threadIdx.x;
 #pragma unroll
       for (int u = 0; u < kMtaGroups; ++u) {
-        mta_load4<ST, NT>(x, q0 + u * 256, xv[u]);
-        mta_load4<ST, NT>(m, q0 + u * 256, mv[u]);
-        mta_load4<ST, NT>(v, q0 + u * 256, vv[u]);
-        mta_load4<GT, NT>(g, q0 + u * 256, gv[u]);
+        st_load4<ST, NT>(x, q0 + u * 256, xv[u]);
+        st_load4<ST, NT>(m, q0 + u * 256, mv[u]);
+        st_load4<ST, NT>(v, q0 + u * 256, vv[u]);
+        st_load4<GT, NT>(g, q0 + u * 256, gv[u]);
       }
       if (r == 0) scalars();  // two powers: under the first loads
 #pragma unroll
@@ -152,9 +120,9 @@ __global__ __launch_bounds__(256) void adamw_mt_kernel(MtaTensors a, int n, cons
         for (int e = 0; e < 4; ++e)
           adamw_one<GT>(xv[u][e], gv[u][e], mv[u][e], vv[u][e], w1, sc.beta2, w2, inv_bc2_sqrt, sc.eps, adj_lr, aa,
                         coeff, sc.cautious);
-        mta_store4<ST, NT>(x, q0 + u * 256, xv[u]);
-        mta_store4<ST, NT>(m, q0 + u * 256, mv[u]);
-        mta_store4<ST, NT>(v, q0 + u * 256, vv[u]);
+        st_store4<ST, NT>(x, q0 + u * 256, xv[u]);
+        st_store4<ST, NT>(m, q0 + u * 256, mv[u]);
+        st_store4<ST, NT>(v, q0 + u * 256, vv[u]);
       }
     }
     return;
@@ -223,16 +191,16 @@ __global__ __launch_bounds__(256) void lion_mt_kernel(MtaTensors a, int n, const
       const int64_t q0 = (first + r * kMtaRound) / 4 + threadIdx.x;
 #pragma unroll
       for (int u = 0; u < kMtaGroups; ++u) {
-        mta_load4<ST, NT>(x, q0 + u * 256, xv[u]);
-        mta_load4<ST, NT>(m, q0 + u * 256, mv[u]);
-        mta_load4<GT, NT>(g, q0 + u * 256, gv[u]);
+        st_load4<ST, NT>(x, q0 + u * 256, xv[u]);
+        st_load4<ST, NT>(m, q0 + u * 256, mv[u]);
+        st_load4<GT, NT>(g, q0 + u * 256, gv[u]);
       }
 #pragma unroll
       for (int u = 0; u < kMtaGroups; ++u) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) lion_one(xv[u][e], gv[u][e], mv[u][e], w1, w2, lr, aa, coeff, cautious);
-        mta_store4<ST, NT>(x, q0 + u * 256, xv[u]);
-        mta_store4<ST, NT>(m, q0 + u * 256, mv[u]);
+        st_store4<ST, NT>(x, q0 + u * 256, xv[u]);
+        st_store4<ST, NT>(m, q0 + u * 256, mv[u]);
       }
     }
     return;
@@ -256,13 +224,10 @@ __global__ __launch_bounds__(256) void lion_mt_kernel(MtaTensors a, int n, const
   }
 }
 
-// What a launch touches is kept out of the caches (non-temporal loads and stores) once it is too large for the
-// 256 MB memory-side cache to hold until the next step: AdamW on 2 x (50304 x 768) fp32, 1.08 GB of tensors, 394 -> 356
-// us, 2 x (32000 x 1000) bf16, 0.51 GB, 181 -> 166; 2 x (32000 x 320) fp32, 0.29 GB, would go from 87 to 98.
 static bool past_caches(const int64_t* numel, int n, int bytes_per_element) {
   int64_t total = 0;
   for (int i = 0; i < n; ++i) total += numel[i];
-  return total * bytes_per_element >= (384LL << 20);
+  return exceeds_caches(total * bytes_per_element);
 }
 
 // false: more workgroups than one launch can have
