@@ -20,6 +20,7 @@ ABI_VERSION = 12  # dion_abi_version() of the library these signatures describe
 _u64p = ctypes.POINTER(ctypes.c_uint64)
 _i64p = ctypes.POINTER(ctypes.c_int64)
 _f32p = ctypes.POINTER(c_float)
+_i32p = ctypes.POINTER(c_int)
 
 # name -> (restype, argtypes); mirrors include/dion_hip.h one to one.
 SIGNATURES = {
@@ -46,12 +47,21 @@ SIGNATURES = {
                                                       c_int, _f32p, c_int, c_float, c_float, c_int, c_int, c_void_p,
                                                       c_float, c_void_p, c_float, c_int, c_void_p, c_size_t,
                                                       c_void_p]),
+    "dion_ns_padded_extents": (c_int, [c_int, c_int, c_int, c_int, c_int, _i32p, _i32p]),
+    "dion_ns_orthogonalize_padded": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, _f32p,
+                                             c_int, c_float, c_float, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "dion_ns_orthogonalize_update_padded": (c_int, [c_void_p, c_void_p, c_int, _u64p, c_int, c_int, c_int, c_int,
+                                                    c_int, _f32p, c_int, c_float, c_float, c_int, c_int, c_void_p,
+                                                    c_float, c_void_p, c_float, c_int, c_void_p, c_size_t,
+                                                    c_void_p]),
     "dion_ns_plan_audit_prepared": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                             c_size_t]),
     "dion_gemm_tile_edge": (c_int, [c_int, c_int, c_int, c_int]),
     "dion_muon_pre_sumsq_blocks": (c_int, [c_int, c_int]),
     "dion_muon_pre_prepared": (c_int, [_u64p, c_int, _u64p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                        c_float, c_int, c_void_p]),
+    "dion_muon_pre_padded": (c_int, [_u64p, c_int, _u64p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                     c_int, c_int, c_float, c_int, c_void_p]),
     "dion_muon_pre": (c_int, [_u64p, c_int, _u64p, c_int, c_void_p, c_int, c_int64, c_float, c_int, c_void_p]),
     "dion_scale_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_void_p]),
     "dion_muon_post": (c_int, [_u64p, c_int, c_void_p, c_int, c_int, c_int64, c_int, c_void_p, c_void_p, c_void_p,

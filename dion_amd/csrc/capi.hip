@@ -204,12 +204,23 @@ bool ns_small_path(int rows, int cols, int flags, int n_iters) {
   return n_iters <= kMaxSmallIters && ns_small_fits(rows, cols);
 }
 
-// The update rides on the last GEMM when that GEMM produces the caller's tensor directly: at least
-// one iteration, no padding between the matrices and the tiles, not the LDS-resident kernel.
+// The matrices do not fill whole tiles: they are iterated in zero-padded copies, mp x np each.
+bool ns_padded(int batch, int rows, int cols, int flags, int n_iters, int* mp = nullptr, int* np = nullptr) {
+  if (batch <= 0 || batch > 65535 || rows <= 0 || cols <= 0 || n_iters <= 0) return false;
+  if (ns_small_path(rows, cols, flags, n_iters)) return false;
+  const NsPlan pl = make_plan(batch, rows, cols, flags);
+  if (mp) *mp = pl.mp;
+  if (np) *np = pl.np;
+  return pl.mp != pl.m || pl.np != pl.n;
+}
+
+// The update rides on the last GEMM: at least one iteration, not the LDS-resident kernel.  (Padded matrices had a separate
+// update pass, without a limit to the number of parameters, before they fused: past what a launch list holds they
+// still take it.)
+constexpr int kMaxFusedPadded = 4096;
 bool ns_update_fuses(int batch, int rows, int cols, int flags, int n_iters) {
   if (n_iters <= 0 || ns_small_path(rows, cols, flags, n_iters)) return false;
-  const NsPlan pl = make_plan(batch, rows, cols, flags);
-  return pl.mp == pl.m && pl.np == pl.n;
+  return batch <= kMaxFusedPadded || !ns_padded(batch, rows, cols, flags, n_iters);
 }
 
 // A prepared input (short side along rows, unnormalised, with partial sums of squares) is taken when
@@ -225,7 +236,7 @@ bool ns_accepts_prepared(int batch, int rows, int cols, int flags, int n_iters) 
 
 // One kernel launch of a planned call.
 struct NsStep {
-  enum Kind { kNorm, kNormFinalize, kPrepare, kGemm, kGemmUpdate, kUnpad, kSmall } kind;
+  enum Kind { kNorm, kNormFinalize, kPrepare, kPadCopy, kGemm, kGemmUpdate, kUnpad, kSmall } kind;
   const char* what;
   GemmParams g;    // kGemm, kGemmUpdate
   // kGemmUpdate: the launch updates parameters ptr0 .. ptr0 + n_ptr - 1 of the call's table
@@ -287,11 +298,12 @@ NsStep blank_step(NsStep::Kind kind, const char* what) {
 // With `sumsq` the input is "prepared": bf16 [batch, m, n] with the short side along rows (the transpose
 // of a tall caller matrix), not normalised, and sumsq [batch, sumsq_blocks] holds partial sums of its
 // squares per matrix.  The normalisation is then folded into the first two GEMMs as a per-matrix factor
-// and neither the norm pass nor the prepare pass runs (only when ns_accepts_prepared).
+// and neither the norm pass nor the prepare pass runs (only when ns_accepts_prepared).  With `in_padded` it is
+// such an input in the padded layout instead: [batch, mp, np], zero outside m x n (only when ns_padded).
 int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int cols, const float* coeffs,
              int n_iters, float norm_scale, float eps, int flags, int gram_reset, void* workspace,
              size_t workspace_bytes, const PostSpec* post, NsCall& call, const float* sumsq = nullptr,
-             int sumsq_blocks = 0) {
+             int sumsq_blocks = 0, bool in_padded = false) {
   call.n_steps = 0;
   call.overflow = false;
   call.post = post;
@@ -319,8 +331,12 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     call.n_ptrs = post->n_ptrs;
     call.x_bytes = (size_t)post->mats_per_ptr * mat_elems * (post->x_dtype == DION_BF16 ? 2 : 4);
   }
+  int pad_m = 0, pad_n = 0;
+  const bool padded = ns_padded(batch, rows, cols, flags, n_iters, &pad_m, &pad_n);
   if (sumsq) {
-    if (!ns_accepts_prepared(batch, rows, cols, flags, n_iters) || in_dtype != DION_BF16 || sumsq_blocks <= 0)
+    if (in_padded) call.in_hi = call.in_lo + (size_t)batch * pad_m * pad_n * 2;
+    if (!(in_padded ? padded : ns_accepts_prepared(batch, rows, cols, flags, n_iters)) || in_dtype != DION_BF16 ||
+        sumsq_blocks <= 0)
       return fail(DION_E_INVALID,
                   "dion_ns_orthogonalize_prepared: %d x (%d x %d), %d iterations does not take a prepared input "
                   "(see dion_ns_accepts_prepared)", batch, rows, cols, n_iters);
@@ -386,14 +402,18 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
   const bool aliased = out && call.out_lo < call.in_hi && call.in_lo < call.out_hi;
   const bool in_place = self_prep && !pl.tall && in_dtype == DION_BF16 && !aliased;
   const bool copy_first = self_prep && pl.tall;
+  // A matrix that needs padding is copied, rounded to bf16 and unscaled, into its padded form; the copy delivers the
+  // partial sums of the norm, so it is the only pass over the input.  The partials (one per 64 x 64 tile) lie in the
+  // third X buffer, which only a call without iterations uses otherwise.
+  const bool pad_copy = padded && !sumsq;
   auto plan_norm = [&]() {
-    if (sumsq) {
-      NsStep s = blank_step(NsStep::kNormFinalize, "frobenius norm from the caller's partial sums");
+    if (sumsq || pad_copy) {
+      NsStep s = blank_step(NsStep::kNormFinalize, "frobenius norm");
       s.batch = batch;
       s.norm_scale = norm_scale;
       s.eps = eps;
-      s.partial = const_cast<float*>(sumsq);
-      s.nblk = sumsq_blocks;
+      s.partial = sumsq ? const_cast<float*>(sumsq) : (float*)Xt;
+      s.nblk = sumsq ? sumsq_blocks : (mp / 64) * (np / 64);
       s.inv = inv;
       call.push(s);
     } else {
@@ -414,7 +434,19 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     }
   };
   auto plan_prepare = [&]() {
-    if (!sumsq && !in_place) {
+    if (pad_copy) {
+      NsStep s = blank_step(NsStep::kPadCopy, "padded copy");
+      s.in = in;
+      s.in_dtype = in_dtype;
+      s.batch = batch;
+      s.R = rows;
+      s.C = cols;
+      s.same = X[0];
+      s.Rp = mp;
+      s.Cp = np;
+      s.partial = (float*)Xt;
+      call.push(s);
+    } else if (!sumsq && !in_place) {
       // Only X (short side along rows) is carried between iterations: X' = B X reads X with the
       // reduction index along rows.  With no iteration at all the result is the prepared input, and
       // the output copy of a tall input reads X^T: prepare that layout instead.
@@ -444,15 +476,13 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
       call.push(s);
     }
   };
-  if (copy_first) {
+  if (copy_first || pad_copy) {
     plan_prepare();
     plan_norm();
   } else {
     plan_norm();
     plan_prepare();
   }
-
-  const bool direct = (mp == pl.m && np == pl.n);
 
   // ---- the GEMM shapes of the iteration
   // sym(P, Q -> C): C = alpha P Q^T + beta D + diag I for symmetric m x m operands whose product
@@ -481,7 +511,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
   };
   // A prepared input is the unnormalised X_0: every GEMM that reads it carries the factor 1/(||X_0|| s + eps)
   // (squared for X_0 X_0^T); products of these GEMMs are normalised, and so is every later X.
-  const bf16_t* const x_raw = (sumsq || in_place) ? (const bf16_t*)in : self_prep ? X[0] : nullptr;
+  const bf16_t* const x_raw = (sumsq || in_place) ? (const bf16_t*)in : (self_prep || pad_copy) ? X[0] : nullptr;
   bool x_written = false;  // an X' has been written: from then on every X is normalised
   auto scaled = [&](GemmParams& p, const bf16_t* Xc, int pow) {
     if (x_raw && Xc == x_raw && !x_written) {
@@ -507,10 +537,10 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     p.alpha = 1.0f;
     call.push(s);
   };
-  // apply(S, Xc -> Xn | Xt | out | parameters): X' = S X (S symmetric m x m).  The last product of a
-  // tall input is written transposed (the caller's orientation); when no padding is in the way
-  // (`final_direct`) it goes straight into the caller's tensor, or into the update of the parameters.
-  auto apply = [&](const char* what, const bf16_t* S, const bf16_t* Xc, bf16_t* Xn, bool last, bool final_direct) {
+  // apply(S, Xc -> Xn | out | parameters): X' = S X (S symmetric m x m).  The last product goes straight into the
+  // caller's tensor, or into the update of the parameters, without its padding; that of a tall input is written
+  // transposed (the caller's orientation).
+  auto apply = [&](const char* what, const bf16_t* S, const bf16_t* Xc, bf16_t* Xn, bool last) {
     GemmParams p;
     memset(&p, 0, sizeof(p));
     p.P = S;
@@ -526,15 +556,20 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     p.batch = batch;
     p.alpha = 1.0f;
     scaled(p, Xc, 1);
-    if (final_direct && post) {
+    const int64_t sOut = (int64_t)rows * cols;
+    if (last && padded) {
+      p.out_rows = pl.m;
+      p.out_cols = pl.n;
+    }
+    if (last && post) {
       // the product is consumed by the update: one launch per kMaxPtrs parameters
       const int mpp = post->mats_per_ptr;
       if (pl.tall) {
-        p.strideCt = sX;
-        p.ldct = mp;
+        p.strideCt = sOut;
+        p.ldct = pl.m;
       } else {
-        p.strideC = sX;
-        p.ldc = np;
+        p.strideC = sOut;
+        p.ldc = pl.n;
       }
       for (int c0 = 0; c0 < post->n_ptrs; c0 += kMaxPtrs) {
         const int c = (post->n_ptrs - c0) < kMaxPtrs ? (post->n_ptrs - c0) : kMaxPtrs;
@@ -554,20 +589,16 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
       }
       return;
     }
-    if (final_direct) {
+    if (last) {
       if (pl.tall) {
         p.Ct = (bf16_t*)out;
-        p.strideCt = sX;
-        p.ldct = mp;
+        p.strideCt = sOut;
+        p.ldct = pl.m;
       } else {
         p.C = (bf16_t*)out;
-        p.strideC = sX;
-        p.ldc = np;
+        p.strideC = sOut;
+        p.ldc = pl.n;
       }
-    } else if (last && pl.tall) {
-      p.Ct = Xt;
-      p.strideCt = sX;
-      p.ldct = mp;
     } else {
       p.C = Xn;
       p.strideC = sX;
@@ -588,9 +619,8 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
       gram("A = X X^T", xc(), sq[0]);
       // a*I folded into B: the next GEMM needs no addend (one fewer pass over X)
       sym("B = c A A + b A + a I", sq[0], sq[0], sq[0], sq[1], c, b, a);
-      const bool fin = (it == n_iters - 1) && direct;
-      apply("X = B X", sq[1], xc(), X[cur ^ 1], it == n_iters - 1, fin);
-      wrote_out = fin;
+      apply("X = B X", sq[1], xc(), X[cur ^ 1], it == n_iters - 1);
+      wrote_out = it == n_iters - 1;
       cur ^= 1;
       x_written = true;
     }
@@ -613,7 +643,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     for (int it = 0; it < n_iters; ++it) {
       const float a = coeffs[3 * it], b = coeffs[3 * it + 1], c = coeffs[3 * it + 2];
       if (it == gram_reset && it > 0 && q >= 0) {
-        apply("X = Q X (restart)", sq[q], xc(), X[cur ^ 1], false, false);
+        apply("X = Q X (restart)", sq[q], xc(), X[cur ^ 1], false);
         cur ^= 1;
         x_written = true;
         used[q] = false;
@@ -643,17 +673,14 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
       }
     }
     if (q >= 0) {
-      apply("X = Q X", sq[q], xc(), X[cur ^ 1], true, direct);
-      wrote_out = direct;
-      cur ^= 1;
-      x_written = true;
+      apply("X = Q X", sq[q], xc(), X[cur ^ 1], true);
+      wrote_out = true;
     }
   }
   if (!wrote_out) {
     if (post) return fail(DION_E_INVALID, "dion_ns_orthogonalize_update: update not applied (internal)");
     NsStep s = blank_step(NsStep::kUnpad, "unpad");
-    // a tall result lies transposed-back in Xt: written there by the last product, or by the
-    // prepare step when there was no iteration
+    // no iteration: the prepared input, in Xt for a tall one
     s.src = pl.tall ? Xt : X[cur];
     s.src_stride = sX;
     s.ld = pl.tall ? mp : np;
@@ -695,7 +722,9 @@ int ns_audit(const NsCall& call) {
     const char* bad = nullptr;
     switch (s.kind) {
       case NsStep::kNormFinalize:
-        if (s.nblk <= 0 || !inside(s.partial, (size_t)s.batch * s.nblk * 4, call.sq_lo, call.sq_hi)) bad = "norm partials";
+        if (s.nblk <= 0 || !(call.sq_lo ? inside(s.partial, (size_t)s.batch * s.nblk * 4, call.sq_lo, call.sq_hi)
+                                        : rd(s.partial, (size_t)s.batch * s.nblk * 4)))
+          bad = "norm partials";
         else if (!wr(s.inv, (size_t)s.batch * 4)) bad = "reciprocal norms";
         break;
       case NsStep::kNorm: {
@@ -716,10 +745,21 @@ int ns_audit(const NsCall& call) {
         else if (!s.same && !s.trans) bad = "no destination";
         break;
       }
+      case NsStep::kPadCopy: {
+        // X-layout copy: short side along rows, Rp x Cp, and one partial sum per 64 x 64 tile of it
+        const size_t es = s.in_dtype == DION_BF16 ? 2 : 4;
+        const int m = s.R < s.C ? s.R : s.C, n = s.R < s.C ? s.C : s.R;
+        if (s.Rp % 64 || s.Cp % 64 || s.Rp < m || s.Cp < n) bad = "padded extents";
+        else if (!rd(s.in, (size_t)s.batch * s.R * s.C * es)) bad = "input";
+        else if (!wr(s.same, (size_t)s.batch * s.Rp * s.Cp * 2)) bad = "X";
+        else if (!wr(s.partial, (size_t)s.batch * (s.Rp / 64) * (s.Cp / 64) * 4)) bad = "norm partials";
+        break;
+      }
       case NsStep::kGemm:
       case NsStep::kGemmUpdate: {
         const GemmParams& p = s.g;
         const int tile = gemm_tile_edge(p);
+        const int om = p.out_rows > 0 ? p.out_rows : p.M, on = p.out_cols > 0 ? p.out_cols : p.N;  // stored extents
         if (p.M % tile || p.N % tile || p.K % 128 || (p.tri && p.M != p.N)) bad = "tile does not divide the extents";
         else if (!rd(p.P, span_bytes(p.batch, p.strideP, p.M, p.ldp, p.K, 2))) bad = "first operand";
         else if (!(p.q_kmajor ? rd(p.Q, span_bytes(p.batch, p.strideQ, p.K, p.ldq, p.N, 2))
@@ -729,14 +769,15 @@ int ns_audit(const NsCall& call) {
         else if (p.scale_vec && (!inside(p.scale_vec, (size_t)p.batch * 4, call.ws_lo, call.ws_hi) ||
                                  (p.scale_pow != 1 && p.scale_pow != 2)))
           bad = "per-matrix factors";
-        else if (p.C && !wr(p.C, span_bytes(p.batch, p.strideC, p.M, p.ldc, p.N, 2))) bad = "product";
-        else if (p.Ct && !wr(p.Ct, span_bytes(p.batch, p.strideCt, p.N, p.ldct, p.M, 2))) bad = "transposed product";
+        else if (om > p.M || on > p.N) bad = "stored extents";
+        else if (p.C && !wr(p.C, span_bytes(p.batch, p.strideC, om, p.ldc, on, 2))) bad = "product";
+        else if (p.Ct && !wr(p.Ct, span_bytes(p.batch, p.strideCt, on, p.ldct, om, 2))) bad = "transposed product";
         else if (s.kind == NsStep::kGemm && !p.C && !p.Ct) bad = "no destination";
         else if (s.kind == NsStep::kGemmUpdate) {
           // matrix b updates parameter b / mats_per_ptr at matrix offset b % mats_per_ptr
           const int es = s.x_code == 0 ? 2 : 4;
           const int mpp = call.post ? call.post->mats_per_ptr : 0;
-          const size_t one = s.transposed ? span_bytes(1, 0, p.N, p.ldct, p.M, es) : span_bytes(1, 0, p.M, p.ldc, p.N, es);
+          const size_t one = s.transposed ? span_bytes(1, 0, on, p.ldct, om, es) : span_bytes(1, 0, om, p.ldc, on, es);
           const size_t stride = (size_t)(s.transposed ? p.strideCt : p.strideC) * es;
           if (mpp <= 0 || s.n_ptr <= 0 || s.n_ptr > kMaxPtrs || p.batch != s.n_ptr * mpp || s.ptr0 < 0 ||
               s.ptr0 + s.n_ptr > call.n_ptrs || p.C || p.Ct)
@@ -782,6 +823,9 @@ int ns_execute(const NsCall& call, hipStream_t st) {
         e = launch_ns_prepare(s.in, s.in_dtype, s.batch, s.R, s.C, s.inv, s.same, s.Rp, s.Cp, s.ld_same,
                               s.stride_same, s.trans, s.ld_trans, s.stride_trans, st);
         break;
+      case NsStep::kPadCopy:
+        e = launch_ns_pad_copy(s.in, s.in_dtype, s.batch, s.R, s.C, s.same, s.Rp, s.Cp, s.partial, st);
+        break;
       case NsStep::kGemm:
         e = launch_gemm_nt(s.g, st);
         break;
@@ -815,10 +859,10 @@ int ns_execute(const NsCall& call, hipStream_t st) {
 int ns_run(const void* in, int in_dtype, void* out, int batch, int rows, int cols, const float* coeffs,
            int n_iters, float norm_scale, float eps, int flags, int gram_reset, void* workspace,
            size_t workspace_bytes, void* stream, const PostSpec* post, const float* sumsq = nullptr,
-           int sumsq_blocks = 0) {
+           int sumsq_blocks = 0, bool in_padded = false) {
   NsCall call;  // on the stack: planning allocates nothing
   if (int rc = ns_build(in, in_dtype, out, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset,
-                        workspace, workspace_bytes, post, call, sumsq, sumsq_blocks))
+                        workspace, workspace_bytes, post, call, sumsq, sumsq_blocks, in_padded))
     return rc;
   if (int rc = ns_audit(call)) return rc;
   return ns_execute(call, (hipStream_t)stream);
@@ -922,7 +966,7 @@ extern "C" int dion_ns_orthogonalize_update(const void* in, int in_dtype, const 
     return ns_run(in, in_dtype, nullptr, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset,
                   workspace, workspace_bytes, stream, &ps);
   }
-  // padded shapes and the LDS-resident kernel: orthogonalize into the tail of the workspace (the
+  // the LDS-resident kernel: orthogonalize into the tail of the workspace (the
   // last align256(batch * rows * cols * 2) bytes of what dion_ns_update_workspace_bytes reports),
   // then the plain update pass
   const size_t tail = align256((size_t)batch * rows * cols * 2);
@@ -953,6 +997,28 @@ extern "C" int dion_ns_orthogonalize_prepared(const void* in, const float* sumsq
                 workspace, workspace_bytes, stream, nullptr, sumsq, sumsq_blocks);
 }
 
+static int update_prepared(const char* who, bool in_padded, const void* in, const float* sumsq, int sumsq_blocks,
+                           const uint64_t* X_ptrs, int x_dtype, int n_ptrs, int mats_per_ptr, int rows, int cols,
+                           const float* coeffs, int n_iters, float norm_scale, float eps, int flags, int gram_reset,
+                           const float* lr_dev, float adj_ratio, const float* wd_dev, float wd_host, int cautious,
+                           void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = check_state_dtype(who, "x_dtype", x_dtype)) return rc;
+  if (n_ptrs < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0 || n_iters < 0)
+    return fail(DION_E_INVALID, "%s: bad size", who);
+  if ((int64_t)n_ptrs * mats_per_ptr > 0x7fffffff) return fail(DION_E_INVALID, "%s: too many matrices", who);
+  const int batch = n_ptrs * mats_per_ptr;
+  if (batch == 0 || rows == 0 || cols == 0) return DION_OK;
+  if (!X_ptrs || !lr_dev || !sumsq) return fail(DION_E_INVALID, "%s: null argument", who);
+  for (int i = 0; i < n_ptrs; ++i)
+    if (!X_ptrs[i]) return fail(DION_E_INVALID, "%s: parameter %d is null", who, i);
+  if (!(in_padded ? ns_padded(batch, rows, cols, flags, n_iters) : ns_accepts_prepared(batch, rows, cols, flags, n_iters)))
+    return fail(DION_E_INVALID, "%s: %d x (%d x %d) does not take a prepared input (see %s)", who, batch, rows, cols,
+                in_padded ? "dion_ns_padded_extents" : "dion_ns_accepts_prepared");
+  const PostSpec ps = {X_ptrs, x_dtype, n_ptrs, mats_per_ptr, lr_dev, adj_ratio, wd_dev, wd_host, cautious};
+  return ns_run(in, DION_BF16, nullptr, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset,
+                workspace, workspace_bytes, stream, &ps, sumsq, sumsq_blocks, in_padded);
+}
+
 extern "C" int dion_ns_orthogonalize_update_prepared(const void* in, const float* sumsq, int sumsq_blocks,
                                                      const uint64_t* X_ptrs, int x_dtype, int n_ptrs,
                                                      int mats_per_ptr, int rows, int cols, const float* coeffs,
@@ -960,23 +1026,36 @@ extern "C" int dion_ns_orthogonalize_update_prepared(const void* in, const float
                                                      int gram_reset, const float* lr_dev, float adj_ratio,
                                                      const float* wd_dev, float wd_host, int cautious,
                                                      void* workspace, size_t workspace_bytes, void* stream) {
-  if (int rc = check_state_dtype("dion_ns_orthogonalize_update_prepared", "x_dtype", x_dtype)) return rc;
-  if (n_ptrs < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0 || n_iters < 0)
-    return fail(DION_E_INVALID, "dion_ns_orthogonalize_update_prepared: bad size");
-  if ((int64_t)n_ptrs * mats_per_ptr > 0x7fffffff)
-    return fail(DION_E_INVALID, "dion_ns_orthogonalize_update_prepared: too many matrices");
-  const int batch = n_ptrs * mats_per_ptr;
+  return update_prepared("dion_ns_orthogonalize_update_prepared", false, in, sumsq, sumsq_blocks, X_ptrs, x_dtype, n_ptrs,
+                         mats_per_ptr, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset, lr_dev,
+                         adj_ratio, wd_dev, wd_host, cautious, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dion_ns_padded_extents(int batch, int rows, int cols, int flags, int n_iters, int* mp, int* np) {
+  if ((flags & ~DION_NS_GRAM) || batch > kMaxFusedPadded) return 0;
+  return ns_padded(batch, rows, cols, flags, n_iters, mp, np) ? 1 : 0;
+}
+
+extern "C" int dion_ns_orthogonalize_padded(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch,
+                                            int rows, int cols, const float* coeffs, int n_iters, float norm_scale,
+                                            float eps, int flags, int gram_reset, void* workspace,
+                                            size_t workspace_bytes, void* stream) {
   if (batch == 0 || rows == 0 || cols == 0) return DION_OK;
-  if (!X_ptrs || !lr_dev || !sumsq)
-    return fail(DION_E_INVALID, "dion_ns_orthogonalize_update_prepared: null argument");
-  for (int i = 0; i < n_ptrs; ++i)
-    if (!X_ptrs[i]) return fail(DION_E_INVALID, "dion_ns_orthogonalize_update_prepared: parameter %d is null", i);
-  if (!ns_update_fuses(batch, rows, cols, flags, n_iters))
-    return fail(DION_E_INVALID, "dion_ns_orthogonalize_update_prepared: %d x (%d x %d) does not take a prepared input "
-                "(see dion_ns_accepts_prepared)", batch, rows, cols);
-  const PostSpec ps = {X_ptrs, x_dtype, n_ptrs, mats_per_ptr, lr_dev, adj_ratio, wd_dev, wd_host, cautious};
-  return ns_run(in, DION_BF16, nullptr, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset,
-                workspace, workspace_bytes, stream, &ps, sumsq, sumsq_blocks);
+  if (!sumsq) return fail(DION_E_INVALID, "dion_ns_orthogonalize_padded: sumsq is null");
+  return ns_run(in, DION_BF16, out, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset, workspace,
+                workspace_bytes, stream, nullptr, sumsq, sumsq_blocks, true);
+}
+
+extern "C" int dion_ns_orthogonalize_update_padded(const void* in, const float* sumsq, int sumsq_blocks,
+                                                   const uint64_t* X_ptrs, int x_dtype, int n_ptrs, int mats_per_ptr,
+                                                   int rows, int cols, const float* coeffs, int n_iters,
+                                                   float norm_scale, float eps, int flags, int gram_reset,
+                                                   const float* lr_dev, float adj_ratio, const float* wd_dev,
+                                                   float wd_host, int cautious, void* workspace,
+                                                   size_t workspace_bytes, void* stream) {
+  return update_prepared("dion_ns_orthogonalize_update_padded", true, in, sumsq, sumsq_blocks, X_ptrs, x_dtype, n_ptrs,
+                         mats_per_ptr, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset, lr_dev,
+                         adj_ratio, wd_dev, wd_host, cautious, workspace, workspace_bytes, stream);
 }
 
 extern "C" int dion_gemm_tile_edge(int batch, int m, int n, int symmetric) {
@@ -1014,7 +1093,9 @@ static int plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters, 
   NsCall call;
   std::vector<uint64_t> xp;
   PostSpec ps;
-  const bool fused = with_update && ns_update_fuses(batch, rows, cols, flags, n_iters);
+  // (with_update == 1 asks about matrices that fill whole tiles; 2 about any)
+  const bool fused = with_update && ns_update_fuses(batch, rows, cols, flags, n_iters) &&
+                     (with_update == 2 || !ns_padded(batch, rows, cols, flags, n_iters));
   if (with_update && !fused)
     return fail(DION_E_INVALID, "dion_ns_plan_audit: this shape does not take the fused update");
   if (fused) {
@@ -1124,6 +1205,35 @@ extern "C" int dion_muon_pre_prepared(const uint64_t* G_ptrs, int g_dtype, const
                                      sumsq + first * blocks, c, mats_per_ptr, rows, cols, mu, nesterov,
                                      (hipStream_t)stream),
             "dion_muon_pre_prepared");
+  }
+  return DION_OK;
+}
+
+extern "C" int dion_muon_pre_padded(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, void* U,
+                                    float* sumsq, int n, int mats_per_ptr, int rows, int cols, int mp, int np, float mu,
+                                    int nesterov, void* stream) {
+  if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0) return fail(DION_E_INVALID, "dion_muon_pre_padded: bad size");
+  if (int rc = check_state_dtype("dion_muon_pre_padded", "m_dtype", m_dtype)) return rc;
+  if (g_dtype != DION_BF16 && g_dtype != DION_F32) return fail(DION_E_INVALID, "dion_muon_pre_padded: g_dtype");
+  if (n == 0 || rows == 0 || cols == 0) return DION_OK;
+  if (!G_ptrs || !M_ptrs || !U || !sumsq) return fail(DION_E_INVALID, "dion_muon_pre_padded: null argument");
+  const int m = rows < cols ? rows : cols, k = rows < cols ? cols : rows;
+  if (mp % 64 || np % 64 || mp < m || np < k || mp / 64 > 65535)
+    return fail(DION_E_INVALID, "dion_muon_pre_padded: %d x %d matrices padded to %d x %d", rows, cols, mp, np);
+  if (!aligned16((uint64_t)U)) return fail(DION_E_INVALID, "dion_muon_pre_padded: U is not 16-byte aligned");
+  const int chunk = ptr_chunk(mats_per_ptr);
+  if (chunk == 0) return fail(DION_E_INVALID, "dion_muon_pre_padded: mats_per_ptr %d > 65535", mats_per_ptr);
+  const bool aligned = table_aligned(G_ptrs, n) && table_aligned(M_ptrs, n);
+  const int64_t blocks = (int64_t)(mp / 64) * (np / 64);
+  for (int c0 = 0; c0 < n; c0 += chunk) {
+    const int c = (n - c0) < chunk ? (n - c0) : chunk;
+    PtrTab G, M;
+    fill_tab(G, G_ptrs + c0, c);
+    fill_tab(M, M_ptrs + c0, c);
+    const int64_t first = (int64_t)c0 * mats_per_ptr;
+    HIP_TRY(launch_muon_pre_padded(G, dt(g_dtype), M, dt(m_dtype), (bf16_t*)U + first * mp * np, sumsq + first * blocks,
+                                   c, mats_per_ptr, rows, cols, mp, np, mu, nesterov, aligned, (hipStream_t)stream),
+            "dion_muon_pre_padded");
   }
   return DION_OK;
 }

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 namespace dion {
 
@@ -117,6 +118,22 @@ __device__ __forceinline__ void st_store8(T* p, int64_t i8, const float v[8]) {
     st_store4<T, NT>(p, 2 * i8 + 1, v + 4);
   }
 }
+// A pair of elements as one access moves it.
+template <typename T>
+__device__ __forceinline__ void st_unpack2(std::conditional_t<sizeof(T) == 4, uint2, uint32_t> w, float v[2]) {
+  if constexpr (sizeof(T) == 4) {
+    v[0] = __uint_as_float(w.x);
+    v[1] = __uint_as_float(w.y);
+  } else {
+    v[0] = __uint_as_float(w << 16);
+    v[1] = __uint_as_float(w & 0xffff0000u);
+  }
+}
+template <typename T>
+__device__ __forceinline__ std::conditional_t<sizeof(T) == 4, uint2, uint32_t> st_pack2(const float v[2]) {
+  if constexpr (sizeof(T) == 4) return make_uint2(__float_as_uint(v[0]), __float_as_uint(v[1]));
+  else return pack_bf16x2(v[0], v[1]);
+}
 // W = 4 or 8 elements
 template <typename T, int W, bool NT = false>
 __device__ __forceinline__ void st_loadw(const T* p, int64_t i, float* v) {
@@ -207,6 +224,10 @@ struct GemmParams {
   int64_t strideP, strideQ, strideD, strideC, strideCt;  // batch strides in elements
   int ldp, ldq, ldd, ldc, ldct;
   int M, N, K;
+  // Valid extents of C (or of Ct's transpose) when they are smaller than M x N: the product of padded operands is then
+  // stored into a dense [out_rows][out_cols] tensor without its padding.  0: whole tiles are stored.  K-major Q, no D,
+  // one destination.
+  int out_rows, out_cols;
   int batch;
   int rule_batch;    // batch the kernel is picked for, when this launch is one part of a larger product (0: batch): the
                      // parts then add up in the same order, and give the same bits, as the whole

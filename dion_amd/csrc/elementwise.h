@@ -31,6 +31,10 @@ hipError_t launch_ns_prepare(const void* in, int in_dtype, int batch, int R, int
                              const float* inv_norm, bf16_t* same, int Rp, int Cp, int ld_same,
                              int64_t stride_same, bf16_t* trans, int ld_trans, int64_t stride_trans,
                              hipStream_t st);
+// in [batch, R, C] -> X [batch, Mp, Np], bf16, short side along rows (transposed when R > C), zero outside the matrix,
+// values unscaled; partial [batch][Mp / 64 * Np / 64]: sum of squares of every 64 x 64 tile of X.
+hipError_t launch_ns_pad_copy(const void* in, int in_dtype, int batch, int R, int C, bf16_t* X, int Mp, int Np,
+                              float* partial, hipStream_t st);
 hipError_t launch_unpad(const bf16_t* src, int64_t src_stride, int ld, bf16_t* dst, int batch, int R,
                         int C, hipStream_t st);
 // State tensors (parameters X, momentum M, second moments V) are fp32 or bf16: *_dtype 0 = bf16,
@@ -44,6 +48,11 @@ hipError_t launch_muon_pre(const PtrTab& G, int g_dtype, const PtrTab& M, int m_
 hipError_t launch_muon_pre_prepared(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, bf16_t* U,
                                     float* sumsq, int n, int mats, int rows, int cols, float mu,
                                     int nesterov, hipStream_t st);
+// muon_pre for matrices that need padding: X [n * mats][mp][np] (see launch_ns_pad_copy), sumsq [n * mats][mp / 64 *
+// np / 64].  mp, np multiples of 64; `aligned`: every pointer of G and M is 16-byte aligned; n * mats <= 65535.
+hipError_t launch_muon_pre_padded(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, bf16_t* X, float* sumsq,
+                                  int n, int mats, int rows, int cols, int mp, int np, float mu, int nesterov,
+                                  bool aligned, hipStream_t st);
 hipError_t launch_muon_post(const PtrTab& X, int x_dtype, const void* U, int u_dtype, int n, int64_t numel,
                             int cols, const float* row_scale, const float* lr_dev, const float* adj_lr_dev,
                             float adj_ratio, const float* wd_dev, float wd_host, int cautious, bool vec,

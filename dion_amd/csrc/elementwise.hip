@@ -388,6 +388,179 @@ __global__ __launch_bounds__(256) void muon_pre_transposed_kernel(PtrTab G, PtrT
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// Matrices that do not fill whole GEMM tiles, into the zero-padded form the iteration carries: X [mat][Mp][Np] bf16,
+// short side along rows, plus the sum of squares of every 64 x 64 tile of it.  One such tile per workgroup; a thread
+// brings sixteen elements, V side by side (V divides the row length, so a group never straddles a row's end; with
+// V = 8 a lane moves 16 or 32 bytes), all of them requested before the first is used, and the tile goes through LDS so
+// that X is written 16 bytes a lane whatever V and the orientation are.  The sums are taken there, in X order: a matrix
+// and its transpose give the same bits.
+// Bound: HBM.  12 x (2730 x 1000) fp32, momentum update included: 95 us beside another stream's GEMMs, where the update
+// (76), the norm's pass over its result (14) and the scaled copy (30) took 120; 4 x (2730 x 1000) fp32 copied: 15.0 us
+// where copy and norm took 23.4.
+// ------------------------------------------------------------------------------------------
+template <typename T, int V>
+static __device__ __forceinline__ void load_group(const T* p, int64_t i, float* v) {
+  if constexpr (V == 8) st_load8<T>(p, i >> 3, v);
+  else if constexpr (V == 2 && sizeof(T) == 2) {
+    const uint32_t w = *(const uint32_t*)(p + i);
+    v[0] = __uint_as_float(w << 16);
+    v[1] = __uint_as_float(w & 0xffff0000u);
+  } else if constexpr (V == 2) {
+    const float2 w = *(const float2*)(p + i);
+    v[0] = w.x;
+    v[1] = w.y;
+  } else v[0] = st_load<T>(p, i);
+}
+template <typename T, int V>
+static __device__ __forceinline__ void store_group(T* p, int64_t i, const float* v) {
+  if constexpr (V == 8) st_store8<T>(p, i >> 3, v);
+  else if constexpr (V == 2 && sizeof(T) == 2) *(uint32_t*)(p + i) = pack_bf16x2(v[0], v[1]);
+  else if constexpr (V == 2) *(float2*)(p + i) = make_float2(v[0], v[1]);
+  else st_store<T>(p, i, v[0]);
+}
+
+// Where the elements come from.  A plain tensor:
+template <typename T>
+struct PadCopyOp {
+  const T* in;
+  struct At { const T* p; };
+  __device__ __forceinline__ At at(int mat, int mats, int64_t mat_elems) const { return {in + (int64_t)mat * mat_elems}; }
+  struct Raw { float v[8]; };
+  template <int V>
+  static __device__ __forceinline__ void load(const At& a, int64_t i, Raw& r) { load_group<T, V>(a.p, i, r.v); }
+  template <int V>
+  __device__ __forceinline__ void finish(const At&, int64_t, Raw& r, float* u) const {
+#pragma unroll
+    for (int e = 0; e < V; ++e) u[e] = r.v[e];
+  }
+};
+// the momentum update of muon_pre_kernel:
+template <typename GT, typename MT>
+struct PadPreOp {
+  PtrTab G, M;
+  float mu;
+  int nesterov;
+  struct At { const GT* g; MT* m; };
+  __device__ __forceinline__ At at(int mat, int mats, int64_t mat_elems) const {
+    const int p = mat / mats;
+    const int64_t off = (int64_t)(mat - p * mats) * mat_elems;
+    return {(const GT*)G.p[p] + off, (MT*)M.p[p] + off};
+  }
+  struct Raw { float g[8], m[8]; };
+  template <int V>
+  static __device__ __forceinline__ void load(const At& a, int64_t i, Raw& r) {
+    load_group<GT, V>(a.g, i, r.g);
+    load_group<MT, V>(a.m, i, r.m);
+  }
+  template <int V>
+  __device__ __forceinline__ void finish(const At& a, int64_t i, Raw& r, float* u) const {
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      r.m[e] = __fadd_rn(__fmul_rn(r.m[e], mu), r.g[e]);
+      u[e] = nesterov ? __fadd_rn(__fmul_rn(r.m[e], mu), r.g[e]) : r.m[e];
+    }
+    store_group<MT, V>(a.m, i, r.m);
+  }
+};
+
+template <class Op, int V, bool TALL>
+__global__ __launch_bounds__(256) void pad_tile_kernel(const Op op, int mats, int R, int C, bf16_t* __restrict__ X,
+                                                       int Mp, int Np, float* __restrict__ partial) {
+  constexpr int CPR = 64 / V, RPP = 256 / CPR, NP = 64 / RPP;  // groups per tile row, rows per pass, passes
+  __shared__ __attribute__((aligned(16))) bf16_t tile[64][72];
+  __shared__ float red[16];
+  const int mat = blockIdx.z;
+  const int x0 = blockIdx.y * 64, y0 = blockIdx.x * 64;  // tile of X: first row, first column
+  const int r0 = TALL ? y0 : x0, c0 = TALL ? x0 : y0;    // and of the source
+  const auto at = op.at(mat, mats, (int64_t)R * C);
+  const int grp = threadIdx.x % CPR, rr = threadIdx.x / CPR;
+  const int c = c0 + grp * V;
+  typename Op::Raw raw[NP];
+#pragma unroll
+  for (int ps = 0; ps < NP; ++ps) {
+    const int r = r0 + rr + ps * RPP;
+    if (r < R && c < C) op.template load<V>(at, (int64_t)r * C + c, raw[ps]);
+  }
+#pragma unroll
+  for (int ps = 0; ps < NP; ++ps) {
+    const int i = rr + ps * RPP, r = r0 + i;
+    float u[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) u[e] = 0.f;
+    if (r < R && c < C) op.template finish<V>(at, (int64_t)r * C + c, raw[ps], u);
+    store_group<bf16_t, V>(&tile[i][0], grp * V, u);
+  }
+  __syncthreads();
+  bf16_t* x = X + ((int64_t)mat * Mp + x0) * Np + y0;
+  const int chunk = threadIdx.x & 7, row = threadIdx.x >> 3;
+  float ss = 0.f;
+#pragma unroll
+  for (int ps = 0; ps < 2; ++ps) {
+    const int i = row + ps * 32;  // row of X, eight columns from 8 * chunk on
+    u32x4_t w;
+    if (!TALL) w = *(const u32x4_t*)&tile[i][chunk * 8];
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        w[e] = (uint32_t)tile[chunk * 8 + 2 * e][i] | ((uint32_t)tile[chunk * 8 + 2 * e + 1][i] << 16);
+    *(u32x4_t*)(x + (int64_t)i * Np + chunk * 8) = w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = __uint_as_float(w[e] << 16), hi = __uint_as_float(w[e] & 0xffff0000u);
+      ss += lo * lo;
+      ss += hi * hi;
+    }
+  }
+  ss = block_sum(ss, red);
+  if (threadIdx.x == 0) partial[((int64_t)mat * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = ss;
+}
+
+template <class Op>
+static hipError_t launch_pad_tile(const Op& op, int n_mat, int mats, int R, int C, bool aligned, bf16_t* X, int Mp, int Np,
+                                  float* partial, hipStream_t st) {
+  const dim3 grid(Np / 64, Mp / 64, n_mat);
+  const int v = !aligned ? 1 : C % 8 == 0 ? 8 : C % 2 == 0 ? 2 : 1;
+#define PAD_LAUNCH(V, T) \
+  hipLaunchKernelGGL((pad_tile_kernel<Op, V, T>), grid, dim3(256), 0, st, op, mats, R, C, X, Mp, Np, partial)
+  if (R > C) {
+    if (v == 8) PAD_LAUNCH(8, true); else if (v == 2) PAD_LAUNCH(2, true); else PAD_LAUNCH(1, true);
+  } else {
+    if (v == 8) PAD_LAUNCH(8, false); else if (v == 2) PAD_LAUNCH(2, false); else PAD_LAUNCH(1, false);
+  }
+#undef PAD_LAUNCH
+  return hipGetLastError();
+}
+
+hipError_t launch_ns_pad_copy(const void* in, int in_dtype, int batch, int R, int C, bf16_t* X, int Mp, int Np,
+                              float* partial, hipStream_t st) {
+  const bool aligned = (((uintptr_t)in) & 15) == 0;
+  if (in_dtype == 0)
+    return launch_pad_tile(PadCopyOp<bf16_t>{(const bf16_t*)in}, batch, 1, R, C, aligned, X, Mp, Np, partial, st);
+  return launch_pad_tile(PadCopyOp<float>{(const float*)in}, batch, 1, R, C, aligned, X, Mp, Np, partial, st);
+}
+
+template <typename GT, typename MT>
+static hipError_t muon_pre_padded(const PtrTab& G, const PtrTab& M, bf16_t* X, float* sumsq, int n, int mats, int rows,
+                                  int cols, int mp, int np, float mu, int nesterov, bool aligned, hipStream_t st) {
+  PadPreOp<GT, MT> op;
+  op.G = G;
+  op.M = M;
+  op.mu = mu;
+  op.nesterov = nesterov;
+  return launch_pad_tile(op, n * mats, mats, rows, cols, aligned, X, mp, np, sumsq, st);
+}
+
+hipError_t launch_muon_pre_padded(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, bf16_t* X, float* sumsq,
+                                  int n, int mats, int rows, int cols, int mp, int np, float mu, int nesterov,
+                                  bool aligned, hipStream_t st) {
+  if (g_dtype == 0)
+    return m_dtype == 0 ? muon_pre_padded<bf16_t, bf16_t>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st)
+                        : muon_pre_padded<bf16_t, float>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st);
+  return m_dtype == 0 ? muon_pre_padded<float, bf16_t>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st)
+                      : muon_pre_padded<float, float>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st);
+}
+
 // Workgroups for the tile-per-workgroup kernels: one per 512 chunks, at most 2^20.
 static int ew_tiles(int64_t chunks) {
   int64_t b = (chunks + 511) / 512;

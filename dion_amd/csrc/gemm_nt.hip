@@ -327,7 +327,65 @@ struct PostSel<2> {
   typedef bf16_t xt;
 };
 
-template <class Cfg, bool HAS_D, bool HAS_C, bool HAS_CT, bool QK = false, int POST = 0>
+// Lines of a staged transposed tile to a bounded destination (GemmParams::out_rows): EPL consecutive elements per lane
+// (2 where every line starts on a pair), `stg` + line * pitch is line `line` of the tile, line < n_lines and element <
+// n_elems are stored.  POST 0 stores bf16 values to dst + line * ld, else the Muon update of X is applied there: sixteen
+// lines' parameters are requested before the first is updated (one at a time, every line cost a round trip to memory:
+// 12 x (2730 x 1000) fp32 222 us a launch).
+template <int EPL, int WIDTH, int LINES, int POST, typename XT>
+__device__ __forceinline__ void store_lines_bounded(const char* stg, int pitch, int lane, XT* dst, int ld, int n_lines,
+                                                    int n_elems, float pa, float pcoeff, float pb, int cautious) {
+  constexpr int PL = WIDTH / EPL < 64 ? WIDTH / EPL : 64;  // lanes per line
+  constexpr int LPP = 64 / PL;                             // lines per pass
+  constexpr int EP = WIDTH / EPL / PL;                     // passes per line
+  constexpr int NP = LINES / LPP, BI = NP < 16 ? NP : 16;  // passes, passes in flight
+  static_assert(NP % BI == 0, "");
+  const int l0 = lane / PL, e0 = (lane % PL) * EPL;
+  typedef std::conditional_t<EPL == 1, XT, std::conditional_t<sizeof(XT) == 4, uint2, uint32_t>> raw_t;
+#pragma unroll
+  for (int ep = 0; ep < EP; ++ep) {
+    const int el = e0 + ep * PL * EPL;
+    if (el >= n_elems) continue;
+    XT* const x = dst + (int64_t)l0 * ld + el;
+    const char* const q = stg + l0 * pitch + el * 2;
+#pragma unroll
+    for (int c0 = 0; c0 < NP; c0 += BI) {
+      raw_t xv[BI];
+      if constexpr (POST != 0) {
+#pragma unroll
+        for (int k = 0; k < BI; ++k) {
+          const int c = (c0 + k) * LPP;
+          if (l0 + c < n_lines) xv[k] = *(const raw_t*)(x + (int64_t)c * ld);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < BI; ++k) {
+        const int c = (c0 + k) * LPP;
+        if (l0 + c >= n_lines) continue;
+        raw_t* const o = (raw_t*)(x + (int64_t)c * ld);
+        if constexpr (POST == 0) {
+          *o = *(const raw_t*)(q + c * pitch);
+        } else if constexpr (EPL == 2) {
+          const uint32_t w = *(const uint32_t*)(q + c * pitch);
+          float v[2];
+          st_unpack2<XT>(xv[k], v);
+          v[0] = muon_post_one(v[0], __uint_as_float(w << 16), pa, pcoeff, pb, cautious);
+          v[1] = muon_post_one(v[1], __uint_as_float(w & 0xffff0000u), pa, pcoeff, pb, cautious);
+          *o = st_pack2<XT>(v);
+        } else {
+          const float u = bf16_to_f32(*(const bf16_t*)(q + c * pitch));
+          st_store<XT>((XT*)o, 0, muon_post_one(st_load<XT>(&xv[k], 0), u, pa, pcoeff, pb, cautious));
+        }
+      }
+      if constexpr (POST != 0) asm volatile("" ::: "memory");  // the next batch of loads stays behind these stores
+    }
+  }
+}
+
+// BND: the destination is dense, p.out_rows x p.out_cols, and smaller than the padded product (GemmParams): the last
+// product of a call then needs no pass that drops the padding (4 x (2730 x 1000): 22 us; 12 x: 100), and no separate
+// update pass (65 us more).  256-wide tiles take this kernel for it, not the tile-walking one.
+template <class Cfg, bool HAS_D, bool HAS_C, bool HAS_CT, bool QK = false, int POST = 0, bool BND = false>
 __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, ST = Cfg::ST, HALVES = Cfg::HALVES, NSTAGE = Cfg::NSTAGE;
@@ -335,6 +393,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
   constexpr int NM = 16;
   constexpr int LPS = Cfg::LOADS_PER_STAGE;
   static_assert(LPS <= NM / 2, "one refill load behind every second MFMA of a slab's last half");
+  static_assert(!BND || (QK && !HAS_D && HAS_C != HAS_CT), "bounded destinations: the last product of a call");
   // Refill of the slot a slab occupied: all of it during the slab's last half, or -- the plain product of two
   // K-contiguous operands on 256-wide tiles, i.e. X X^T -- half then and half during the next slab's first half.
   // Measured: X X^T 2-3 % faster that way; the polynomial GEMM (addend loads in the epilogue) 1 % slower, the
@@ -598,6 +657,9 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
                                            (int64_t)(row_base + 4 * quad) * p.ldc + col_base + l16
                                      : nullptr;
   const int ldd = p.ldd, ldc = p.ldc, ldct = p.ldct;
+  // BND: rows / columns of this wavefront's tile that exist; per lane, those left from its first row / column on
+  const int rows_in = BND ? p.out_rows - row_base : 0, cols_in = BND ? p.out_cols - col_base : 0;
+  const int lrows = rows_in - 4 * quad, lcols = cols_in - l16;
   typedef typename PostSel<POST>::xt XT;
   float pa = 0.f, pcoeff = 0.f, pb = 0.f;
   int pcautious = 0, pvec = 0;
@@ -630,7 +692,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
           pk[i][j][q] = pack_bf16x2(alpha * acc[i][j][2 * q], alpha * acc[i][j][2 * q + 1]);
     const __amdgpu_buffer_rsrc_t xr = bx_resource(uniform_ptr(xmat + (int64_t)row_base * ldc + col_base));
     const int xl = (4 * quad * ldc + l16) * (int)sizeof(XT);  // per lane
-    constexpr int HM = TM / 2;
+    constexpr int HM = BND ? 2 : TM / 2;
     auto run = [&](auto caut) {
       constexpr int CAUT = decltype(caut)::value;
 #pragma unroll
@@ -641,14 +703,21 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
 #pragma unroll
           for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < 4; ++e) {
+              if constexpr (BND) {
+                xv[ii][j][e] = 0.f;
+                if ((i0 + ii) * 16 + e >= lrows || j * 16 >= lcols) continue;
+              }
               xv[ii][j][e] = bx_load<XT>(xr, xl, (((i0 + ii) * 16 + e) * ldc + j * 16) * (int)sizeof(XT));
+            }
 #pragma unroll
         for (int ii = 0; ii < HM; ++ii)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+              if constexpr (BND)
+                if ((i0 + ii) * 16 + e >= lrows || j * 16 >= lcols) continue;
               const uint32_t w = pk[i0 + ii][j][e >> 1];
               const float u = __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
               bx_store<XT>(xr, xl, (((i0 + ii) * 16 + e) * ldc + j * 16) * (int)sizeof(XT),
@@ -695,7 +764,11 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
       }
       if (HAS_C && POST == 0) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) Cp[(int64_t)(i * 16 + e) * ldc + j * 16] = f32_to_bf16(v[e]);
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (BND)
+            if (i * 16 + e >= lrows || j * 16 >= lcols) continue;
+          Cp[(int64_t)(i * 16 + e) * ldc + j * 16] = f32_to_bf16(v[e]);
+        }
       }
       if (HAS_CT) {
         // four consecutive rows of column j * 16 + l16: 8 bytes of the staged [column][row] tile
@@ -706,7 +779,19 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
       }
     }
   }
-  if (HAS_CT) {
+  if constexpr (BND && HAS_CT) {
+    typedef std::conditional_t<POST == 0, bf16_t, XT> OT;
+    OT* dst;
+    bool pair = (ldct & 1) == 0;
+    if constexpr (POST != 0) {
+      dst = xmat + (int64_t)col_base * ldct + row_base;
+      pair = pair && pvec;
+    } else {
+      dst = p.Ct + (int64_t)b * p.strideCt + (int64_t)col_base * ldct + row_base;
+    }
+    if (pair) store_lines_bounded<2, Cfg::WTM, Cfg::WTN, POST>(stg, Cfg::STG_PITCH, lane, dst, ldct, cols_in, rows_in, pa, pcoeff, pb, pcautious);
+    else store_lines_bounded<1, Cfg::WTM, Cfg::WTN, POST>(stg, Cfg::STG_PITCH, lane, dst, ldct, cols_in, rows_in, pa, pcoeff, pb, pcautious);
+  } else if (HAS_CT) {
     if (mirror) {
       constexpr int CH = Cfg::WTM / 8;  // 16-byte chunks per staged row
       constexpr int RPI = 64 / CH;      // staged rows per store instruction
@@ -1032,7 +1117,7 @@ struct CfgK64 {
   static_assert(PART_BYTES + 64 * STG_PITCH <= LDS_BYTES, "reduction and staging areas");
 };
 
-template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0>
+template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0, bool BND = false>
 __global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
   typedef CfgK64 Cfg;
   typedef typename PostSel<POST>::xt XT;
@@ -1191,6 +1276,7 @@ __global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p
   // ---- partial sums -> tile.  Wavefront w finishes row block w (16 rows): every other wavefront hands it its share
   // through LDS, added in wavefront order.
   const int row_base = ti * 64 + wave * 16, col_base = tj * 64;
+  const int lrows = BND ? p.out_rows - row_base - 4 * quad : 0, lcols = BND ? p.out_cols - col_base - l16 : 0;
   float pa = 0.f, pcoeff = 0.f, pb = 0.f;
   XT* xmat = nullptr;
   if constexpr (POST != 0) {
@@ -1240,14 +1326,19 @@ __global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p
       const int64_t at = (int64_t)(row_base + 4 * quad) * p.ldc + col_base + l16 + j * 16;
       if constexpr (POST != 0) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < 4; ++e) {
+          if (BND && (e >= lrows || j * 16 >= lcols)) continue;
           st_store<XT>(xmat, at + (int64_t)e * p.ldc,
                        muon_post_one(st_load<XT>(xmat, at + (int64_t)e * p.ldc), bf16_to_f32(f32_to_bf16(v[e])), pa,
                                      pcoeff, pb, post.cautious));
+        }
       } else {
         bf16_t* Cp = p.C + (int64_t)b * p.strideC + at;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) Cp[(int64_t)e * p.ldc] = f32_to_bf16(v[e]);
+        for (int e = 0; e < 4; ++e) {
+          if (BND && (e >= lrows || j * 16 >= lcols)) continue;
+          Cp[(int64_t)e * p.ldc] = f32_to_bf16(v[e]);
+        }
       }
     }
     if (HAS_CT) {
@@ -1259,7 +1350,24 @@ __global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p
   }
   if (HAS_CT) {
     __syncthreads();
-    if constexpr (POST != 0) {
+    if constexpr (BND) {
+      // (a wavefront takes 16 of the 64 lines)
+      typedef std::conditional_t<POST == 0, bf16_t, XT> OT;
+      OT* dst;
+      int cautious = 0;
+      bool pair = (p.ldct & 1) == 0;
+      if constexpr (POST != 0) {
+        dst = xmat + (int64_t)(col_base + wave * 16) * p.ldct + ti * 64;
+        pair = pair && post.vec_ok;
+        cautious = post.cautious;
+      } else {
+        dst = p.Ct + (int64_t)b * p.strideCt + (int64_t)(col_base + wave * 16) * p.ldct + ti * 64;
+      }
+      const char* sp = stg + wave * 16 * Cfg::STG_PITCH;
+      const int nl = p.out_cols - (col_base + wave * 16), ne = p.out_rows - ti * 64;
+      if (pair) store_lines_bounded<2, 64, 16, POST>(sp, Cfg::STG_PITCH, lane, dst, p.ldct, nl, ne, pa, pcoeff, pb, cautious);
+      else store_lines_bounded<1, 64, 16, POST>(sp, Cfg::STG_PITCH, lane, dst, p.ldct, nl, ne, pa, pcoeff, pb, cautious);
+    } else if constexpr (POST != 0) {
       // the staged bf16 tile is the update of X[col][row]: a wavefront takes 16 of the 64 rows of X, lanes along a row
       XT* xt = xmat + (int64_t)(col_base + wave * 16) * p.ldct + ti * 64 + lane;
 #pragma unroll 8
@@ -1289,11 +1397,11 @@ constexpr int kWalkMaxK = 2048;                    // longest reduction the tile
 // one matrix is at least 16 MB; below that a contiguous run per XCD keeps whole matrices in one L2.
 static bool xcd_interleave_pays(const GemmParams& p) { return (int64_t)p.M * p.K * 2 >= (16L << 20); }
 
-template <class Cfg, bool HAS_D, bool HAS_C, bool HAS_CT, bool QK = false, int POST = 0>
+template <class Cfg, bool HAS_D, bool HAS_C, bool HAS_CT, bool QK = false, int POST = 0, bool BND = false>
 static hipError_t launch_epi(const GemmParams& p, hipStream_t stream,
                              const typename PostSel<POST>::arg& post = typename PostSel<POST>::arg()) {
   static std::atomic<uint64_t> attr_done{0};
-  auto kern = gemm_nt_kernel<Cfg, HAS_D, HAS_C, HAS_CT, QK, POST>;
+  auto kern = gemm_nt_kernel<Cfg, HAS_D, HAS_C, HAS_CT, QK, POST, BND>;
   if (hipError_t e = set_max_dynamic_lds_once((const void*)kern, Cfg::LDS_BYTES, attr_done)) return e;
   const int tilesM = p.M / Cfg::BM, tilesN = p.N / Cfg::BN;
   const int64_t per_mat = p.tri ? (int64_t)tilesM * (tilesM + 1) / 2 : (int64_t)tilesM * tilesN;
@@ -1306,11 +1414,11 @@ static hipError_t launch_epi(const GemmParams& p, hipStream_t stream,
   return hipGetLastError();
 }
 
-template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0>
+template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0, bool BND = false>
 static hipError_t launch_k64_epi(const GemmParams& p, hipStream_t stream,
                                  const typename PostSel<POST>::arg& post = typename PostSel<POST>::arg()) {
   static std::atomic<uint64_t> attr_done{0};
-  auto kern = gemm_k64_kernel<HAS_D, HAS_C, HAS_CT, QK, POST>;
+  auto kern = gemm_k64_kernel<HAS_D, HAS_C, HAS_CT, QK, POST, BND>;
   if (hipError_t e = set_max_dynamic_lds_once((const void*)kern, CfgK64::LDS_BYTES, attr_done)) return e;
   if (p.M % 64 || p.N % 64 || p.K % 64) return hipErrorInvalidValue;
   const int64_t T = p.M / 64;
@@ -1351,11 +1459,21 @@ static hipError_t launch_walk(const GemmParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+static bool bounded(const GemmParams& p) { return p.out_rows > 0; }
+static bool bounds_ok(const GemmParams& p) {
+  return p.out_rows > 0 && p.out_rows <= p.M && p.out_cols > 0 && p.out_cols <= p.N && p.q_kmajor && !p.tri && !p.D;
+}
+
 // The operand / result combinations the Newton-Schulz drivers use.
 template <class Cfg>
 static hipError_t launch_cfg(const GemmParams& p, hipStream_t stream) {
   if (p.M % Cfg::BM || p.N % Cfg::BN || p.K % 128) return hipErrorInvalidValue;
   const bool d = p.D != nullptr, c = p.C != nullptr, ct = p.Ct != nullptr;
+  if (bounded(p)) {
+    if (!bounds_ok(p) || c == ct) return hipErrorInvalidValue;
+    return c ? launch_epi<Cfg, false, true, false, true, 0, true>(p, stream)
+             : launch_epi<Cfg, false, false, true, true, 0, true>(p, stream);
+  }
   if (p.q_kmajor) {
     if (p.tri) return hipErrorInvalidValue;
     if constexpr (Cfg::BM == 256) {
@@ -1379,6 +1497,11 @@ static hipError_t launch_cfg(const GemmParams& p, hipStream_t stream) {
 
 static hipError_t launch_k64(const GemmParams& p, hipStream_t stream) {
   const bool d = p.D != nullptr, c = p.C != nullptr, ct = p.Ct != nullptr;
+  if (bounded(p)) {
+    if (!bounds_ok(p) || c == ct) return hipErrorInvalidValue;
+    return c ? launch_k64_epi<false, true, false, true, 0, true>(p, stream)
+             : launch_k64_epi<false, false, true, true, 0, true>(p, stream);
+  }
   if (p.q_kmajor && !p.tri) {
     if (!d && c && !ct) return launch_k64_epi<false, true, false, true>(p, stream);
     if (!d && !c && ct) return launch_k64_epi<false, false, true, true>(p, stream);
@@ -1429,16 +1552,23 @@ int gemm_tile_edge(const GemmParams& p) {
   return k == kTile256 ? 256 : k == kTile64 ? 64 : 128;
 }
 
-template <class Cfg>
-static hipError_t launch_post_cfg(const GemmParams& p, const FusedPost& post, int x_dtype, bool transposed,
-                                  hipStream_t stream) {
+template <class Cfg, int POST, bool BND>
+static hipError_t launch_post_cfg(const GemmParams& p, const FusedPost& post, bool transposed, hipStream_t stream) {
   if (p.M % Cfg::BM || p.N % Cfg::BN || p.K % 128) return hipErrorInvalidValue;
-  if (x_dtype == 1) {
-    return transposed ? launch_epi<Cfg, false, false, true, true, 1>(p, stream, post)
-                      : launch_epi<Cfg, false, true, false, true, 1>(p, stream, post);
+  return transposed ? launch_epi<Cfg, false, false, true, true, POST, BND>(p, stream, post)
+                    : launch_epi<Cfg, false, true, false, true, POST, BND>(p, stream, post);
+}
+
+template <int POST, bool BND>
+static hipError_t launch_post(const GemmParams& p, const FusedPost& post, bool transposed, hipStream_t stream) {
+  switch (pick_tile(p)) {
+    case kTile256: return launch_post_cfg<Cfg256w8, POST, BND>(p, post, transposed, stream);
+    case kTile128Deep: return launch_post_cfg<Cfg128d, POST, BND>(p, post, transposed, stream);
+    case kTile64:
+      return transposed ? launch_k64_epi<false, false, true, true, POST, BND>(p, stream, post)
+                        : launch_k64_epi<false, true, false, true, POST, BND>(p, stream, post);
+    default: return launch_post_cfg<Cfg128, POST, BND>(p, post, transposed, stream);
   }
-  return transposed ? launch_epi<Cfg, false, false, true, true, 2>(p, stream, post)
-                    : launch_epi<Cfg, false, true, false, true, 2>(p, stream, post);
 }
 
 hipError_t launch_gemm_nt_post(const GemmParams& p, const FusedPost& post, int x_dtype, bool transposed,
@@ -1449,17 +1579,13 @@ hipError_t launch_gemm_nt_post(const GemmParams& p, const FusedPost& post, int x
   if (!p.q_kmajor || p.tri || p.D || post.mats_per_ptr <= 0 || !post.lr_dev ||
       p.batch > (int64_t)kMaxPtrs * post.mats_per_ptr || (x_dtype != 0 && x_dtype != 1))
     return hipErrorInvalidValue;
-  switch (pick_tile(p)) {
-    case kTile256: return launch_post_cfg<Cfg256w8>(p, post, x_dtype, transposed, stream);
-    case kTile128Deep: return launch_post_cfg<Cfg128d>(p, post, x_dtype, transposed, stream);
-    case kTile64:
-      if (x_dtype == 1)
-        return transposed ? launch_k64_epi<false, false, true, true, 1>(p, stream, post)
-                          : launch_k64_epi<false, true, false, true, 1>(p, stream, post);
-      return transposed ? launch_k64_epi<false, false, true, true, 2>(p, stream, post)
-                        : launch_k64_epi<false, true, false, true, 2>(p, stream, post);
-    default: return launch_post_cfg<Cfg128>(p, post, x_dtype, transposed, stream);
+  if (bounded(p)) {
+    if (!bounds_ok(p)) return hipErrorInvalidValue;
+    return x_dtype == 1 ? launch_post<1, true>(p, post, transposed, stream)
+                        : launch_post<2, true>(p, post, transposed, stream);
   }
+  return x_dtype == 1 ? launch_post<1, false>(p, post, transposed, stream)
+                      : launch_post<2, false>(p, post, transposed, stream);
 }
 
 hipError_t launch_gemm_nt(const GemmParams& p, hipStream_t stream) {

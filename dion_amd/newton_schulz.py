@@ -106,20 +106,31 @@ def accepts_prepared(func, batch: int, rows: int, cols: int) -> bool:
     return ops.ns_accepts_prepared(batch, rows, cols, len(coeffs), gram)
 
 
+def padded_extents(func, batch: int, rows: int, cols: int):
+    """Extents of the padded form (``ops.muon_pre_padded``) in which the built-in operator ``func`` takes ``batch``
+    matrices of ``rows x cols``, or None."""
+    if func not in SCHEDULES:
+        return None
+    coeffs, _s, _e, gram, _r = SCHEDULES[func]
+    return ops.ns_padded_extents(batch, rows, cols, len(coeffs), gram)
+
+
 @torch.no_grad()
-def orthogonalize_prepared(func, U: Tensor, sumsq: Tensor, rows: int, cols: int, epsilon) -> Tensor:
+def orthogonalize_prepared(func, U: Tensor, sumsq: Tensor, rows: int, cols: int, epsilon, padded: bool = False) -> Tensor:
     """``func(G, epsilon)`` for a built-in ``func`` on the prepared form of ``G``."""
     coeffs, norm_scale, eps, gram, reset = _schedule_args(func, epsilon)
-    return ops.ns_orthogonalize_prepared(U, sumsq, rows, cols, coeffs, norm_scale, eps, gram=gram, gram_reset=reset)
+    return ops.ns_orthogonalize_prepared(U, sumsq, rows, cols, coeffs, norm_scale, eps, gram=gram, gram_reset=reset,
+                                         padded=padded)
 
 
 @torch.no_grad()
 def orthogonalize_update_prepared(func, U: Tensor, sumsq: Tensor, rows: int, cols: int, epsilon, X, lr: Tensor,
-                                  adj_ratio: float, weight_decay, cautious_wd: bool = False) -> None:
+                                  adj_ratio: float, weight_decay, cautious_wd: bool = False,
+                                  padded: bool = False) -> None:
     """``orthogonalize_update`` on the prepared form of ``G``."""
     coeffs, norm_scale, eps, gram, reset = _schedule_args(func, epsilon)
     ops.ns_orthogonalize_update_prepared(U, sumsq, rows, cols, X, coeffs, norm_scale, eps, lr, adj_ratio,
-                                         weight_decay, cautious_wd, gram=gram, gram_reset=reset)
+                                         weight_decay, cautious_wd, gram=gram, gram_reset=reset, padded=padded)
 
 
 # The reference exposes Triton-backed twins of the two schedules; here there is one

@@ -256,9 +256,23 @@ def ns_accepts_prepared(batch: int, rows: int, cols: int, n_iters: int, gram: bo
                                              int(n_iters)))
 
 
-def _check_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: int) -> Tuple[int, int]:
+def ns_padded_extents(batch: int, rows: int, cols: int, n_iters: int, gram: bool = False) -> Optional[Tuple[int, int]]:
+    """``(m, n)`` of the zero-padded form in which ``batch`` matrices of ``rows x cols`` are iterated, for matrices that
+    ``muon_pre_padded`` can hand over in it; None when they fill whole GEMM tiles or take the small-matrix kernel."""
+    mp, np_ = _lib.c_int(0), _lib.c_int(0)
+    takes = _lib.load().dion_ns_padded_extents(int(batch), int(rows), int(cols), DION_NS_GRAM if gram else 0,
+                                               int(n_iters), mp, np_)
+    return (mp.value, np_.value) if takes else None
+
+
+def _check_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: int, n_iters: int, gram: bool, padded: bool) -> Tuple[int, int]:
     _check_bf16(U, "U")
     m, n = min(rows, cols), max(rows, cols)
+    if padded:
+        extents = ns_padded_extents(U.shape[0], rows, cols, n_iters, gram)
+        if extents is None:
+            raise ValueError(f"{U.shape[0]} matrices of {rows} x {cols} have no padded form")
+        m, n = extents
     if U.ndim != 3 or U.shape[1] != m or U.shape[2] != n or not U.is_contiguous():
         raise ValueError(f"a prepared input of {rows} x {cols} matrices is a contiguous [batch, {m}, {n}] tensor, "
                          f"got {tuple(U.shape)}")
@@ -270,44 +284,45 @@ def _check_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: int) -> Tuple[int
 
 
 def ns_orthogonalize_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: int, coeffs, norm_scale: float,
-                              epsilon: float, gram: bool = False, gram_reset: int = 0) -> Tensor:
+                              epsilon: float, gram: bool = False, gram_reset: int = 0, padded: bool = False) -> Tensor:
     """``ns_orthogonalize`` of the matrices ``muon_pre_prepared`` wrote: ``U [batch, min, max]`` holds them
     with the short side along rows and unnormalised, ``sumsq [batch, blocks]`` partial sums of their squares.
-    Returns ``[batch, rows, cols]`` bf16.  The Frobenius normalisation rides on the first two GEMMs."""
-    batch, blocks = _check_prepared(U, sumsq, rows, cols)
-    out = torch.empty(batch, rows, cols, dtype=torch.bfloat16, device=U.device)
+    Returns ``[batch, rows, cols]`` bf16.  The Frobenius normalisation rides on the first two GEMMs.
+    ``padded``: ``U`` is in the padded form that ``muon_pre_padded`` writes."""
     carr, n_iters = _flat_coeffs(coeffs)
+    batch, blocks = _check_prepared(U, sumsq, rows, cols, n_iters, gram, padded)
+    out = torch.empty(batch, rows, cols, dtype=torch.bfloat16, device=U.device)
     flags = DION_NS_GRAM if gram else 0
     lib = _lib.load()
     ws = _workspace(U.device, lib.dion_ns_workspace_bytes(batch, rows, cols, flags))
-    check(lib.dion_ns_orthogonalize_prepared(U.data_ptr(), sumsq.data_ptr(), blocks, out.data_ptr(), batch, rows,
-                                             cols, carr, n_iters, float(norm_scale), float(epsilon), flags,
-                                             int(gram_reset), ws.data_ptr(), ws.numel(), _stream_handle(U.device)),
-          "ns_orthogonalize_prepared")
+    entry = lib.dion_ns_orthogonalize_padded if padded else lib.dion_ns_orthogonalize_prepared
+    check(entry(U.data_ptr(), sumsq.data_ptr(), blocks, out.data_ptr(), batch, rows, cols, carr, n_iters,
+                float(norm_scale), float(epsilon), flags, int(gram_reset), ws.data_ptr(), ws.numel(),
+                _stream_handle(U.device)), "ns_orthogonalize_prepared")
     return out
 
 
 def ns_orthogonalize_update_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: int, X: List[Tensor], coeffs,
                                      norm_scale: float, epsilon: float, lr: Tensor, adj_ratio: float, weight_decay,
-                                     cautious_wd: bool = False, gram: bool = False, gram_reset: int = 0) -> None:
+                                     cautious_wd: bool = False, gram: bool = False, gram_reset: int = 0,
+                                     padded: bool = False) -> None:
     """``ns_orthogonalize_update`` on a prepared input (see ``ns_orthogonalize_prepared``): the update of
     every ``X[i]`` (``[mats, rows, cols]``) rides on the last GEMM."""
-    batch, blocks = _check_prepared(U, sumsq, rows, cols)
+    carr, n_iters = _flat_coeffs(coeffs)
+    batch, blocks = _check_prepared(U, sumsq, rows, cols, n_iters, gram, padded)
     n = len(X)
     if n == 0 or batch % n:
         raise ValueError(f"{batch} matrices do not divide over {n} parameters")
     mats_per_ptr = batch // n
     xp, xcode = _state_ptrs(X, "X", mats_per_ptr * rows * cols)
     lr_p, wd_p, wd_h = _scalar_args(lr, weight_decay, U.device)
-    carr, n_iters = _flat_coeffs(coeffs)
     flags = DION_NS_GRAM if gram else 0
     lib = _lib.load()
     ws = _workspace(U.device, lib.dion_ns_update_workspace_bytes(batch, rows, cols, flags, n_iters))
-    check(lib.dion_ns_orthogonalize_update_prepared(U.data_ptr(), sumsq.data_ptr(), blocks, xp, xcode, n,
-                                                    mats_per_ptr, rows, cols, carr, n_iters, float(norm_scale),
-                                                    float(epsilon), flags, int(gram_reset), lr_p,
-                                                    float(adj_ratio), wd_p, wd_h, int(bool(cautious_wd)),
-                                                    ws.data_ptr(), ws.numel(), _stream_handle(U.device)),
+    entry = lib.dion_ns_orthogonalize_update_padded if padded else lib.dion_ns_orthogonalize_update_prepared
+    check(entry(U.data_ptr(), sumsq.data_ptr(), blocks, xp, xcode, n, mats_per_ptr, rows, cols, carr, n_iters,
+                float(norm_scale), float(epsilon), flags, int(gram_reset), lr_p, float(adj_ratio), wd_p, wd_h,
+                int(bool(cautious_wd)), ws.data_ptr(), ws.numel(), _stream_handle(U.device)),
           "ns_orthogonalize_update_prepared")
 
 
@@ -383,6 +398,26 @@ def muon_pre_prepared(G: List[Tensor], M: List[Tensor], momentum: float, nestero
     check(lib.dion_muon_pre_prepared(gp, _dtype_code(G[0], "G"), mp, mcode, U.data_ptr(), sumsq.data_ptr(), n, mats,
                                      rows, cols, float(momentum), int(bool(nesterov)), _stream_handle(dev)),
           "muon_pre_prepared")
+    return U, sumsq
+
+
+def muon_pre_padded(G: List[Tensor], M: List[Tensor], momentum: float, nesterov: bool, mats: int, rows: int, cols: int,
+                    extents: Tuple[int, int]) -> Tuple[Tensor, Tensor]:
+    """``muon_pre_prepared`` for matrices that do not fill whole tiles: ``U [N * mats, *extents]`` in the zero-padded
+    form of ``ns_padded_extents``."""
+    n = len(G)
+    assert n == len(M) and n > 0
+    numel = M[0].numel()
+    if numel != mats * rows * cols:
+        raise ValueError(f"parameters of {numel} elements are not {mats} matrices of {rows} x {cols}")
+    gp = _list_ptrs(G, "G", G[0].dtype, numel)
+    mp, mcode = _state_ptrs(M, "M", numel)
+    dev = M[0].device
+    U = torch.empty((n * mats, *extents), dtype=torch.bfloat16, device=dev)
+    sumsq = torch.empty((n * mats, extents[0] // 64 * (extents[1] // 64)), dtype=torch.float32, device=dev)
+    check(_lib.load().dion_muon_pre_padded(gp, _dtype_code(G[0], "G"), mp, mcode, U.data_ptr(), sumsq.data_ptr(), n, mats,
+                                           rows, cols, extents[0], extents[1], float(momentum), int(bool(nesterov)),
+                                           _stream_handle(dev)), "muon_pre_padded")
     return U, sumsq
 
 

@@ -87,20 +87,26 @@ class _MomentumOrtho(OrthoOptimizer):
         # short side along rows, unnormalised, with the partial sums of the Frobenius norm from the same pass
         # (no separate norm / scale / transpose pass over the arena; the factor rides on the first two GEMMs).
         flat3d = flatten and len(shape) >= 3
-        prepared = (self.prepared_input and split_sizes is None and not flat3d and not self._custom_ns
-                    and ns.accepts_prepared(self._newton_schulz_func, n * mats, rows, cols)
+        # The others are written into the zero-padded form the iteration carries, by the same pass.
+        handed_over = self.prepared_input and split_sizes is None and not flat3d and not self._custom_ns
+        prepared = (handed_over and ns.accepts_prepared(self._newton_schulz_func, n * mats, rows, cols)
                     and all(t.data_ptr() % 16 == 0 for t in G + M))
-        if prepared:
-            U, sumsq = ops.muon_pre_prepared(G, M, group["mu"], group["nesterov"], mats, rows, cols)
+        extents = ns.padded_extents(self._newton_schulz_func, n * mats, rows, cols) if handed_over else None
+        if prepared or extents is not None:
+            padded = extents is not None
+            if padded:
+                U, sumsq = ops.muon_pre_padded(G, M, group["mu"], group["nesterov"], mats, rows, cols, extents)
+            else:
+                U, sumsq = ops.muon_pre_prepared(G, M, group["mu"], group["nesterov"], mats, rows, cols)
             yield
             _note_stream(U)
             _note_stream(sumsq)
             func = self._newton_schulz_func
             if not self._normalize and self.fused_update:
                 ns.orthogonalize_update_prepared(func, U, sumsq, rows, cols, eps, X, group["lr"], ratio,
-                                                 group["weight_decay"], group["cautious_wd"])
+                                                 group["weight_decay"], group["cautious_wd"], padded=padded)
                 return
-            O = ns.orthogonalize_prepared(func, U, sumsq, rows, cols, eps)
+            O = ns.orthogonalize_prepared(func, U, sumsq, rows, cols, eps, padded=padded)
             del U, sumsq
             yield
             _note_stream(O)

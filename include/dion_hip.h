@@ -105,7 +105,7 @@ int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* out, int ba
 
 /* Host-only self-check of the planning code (no device work, usable without a GPU): builds the launch
  * list of dion_ns_orthogonalize (with_update == 0) or of the fused form of
- * dion_ns_orthogonalize_update (with_update != 0; DION_E_INVALID if the shape does not fuse) over
+ * dion_ns_orthogonalize_update (with_update 1: matrices that fill whole tiles, 2: any; DION_E_INVALID if the shape does not fuse) over
  * synthetic, never dereferenced addresses and runs the bounds check every real call runs before
  * its first launch: each launch's reads inside the input or the workspace, its writes inside the
  * workspace, the output or one parameter, tile shapes dividing the padded extents.  Returns the
@@ -121,9 +121,8 @@ int dion_ns_plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters,
  * `muon_update_newton_schulz` + `muon_update_post_orthogonalize`, dion/muon.py:249-277.
  * in: [n_ptrs * mats_per_ptr, rows, cols] as for dion_ns_orthogonalize; X_ptrs: host array of n_ptrs
  * device pointers, each to mats_per_ptr contiguous [rows, cols] matrices of x_dtype, updated in place.
- * When the matrices fill whole tiles (rows, cols multiples of 128; more than 64 rows or
- * columns on the short side) the last GEMM applies the update in its epilogue; otherwise the library
- * runs the two passes itself, through the tail of the workspace.  Workspace size from
+ * With more than 64 rows or columns on the short side the last GEMM applies the update in its epilogue;
+ * otherwise the library runs the two passes itself, through the tail of the workspace.  Workspace size from
  * dion_ns_update_workspace_bytes (same flags and n_iters).  lr / weight decay as for dion_muon_post. */
 size_t dion_ns_update_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters);
 int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X_ptrs, int x_dtype, int n_ptrs,
@@ -163,6 +162,22 @@ int dion_ns_orthogonalize_update_prepared(const void* in, const float* sumsq, in
                                           const float* lr_dev, float adj_ratio, const float* wd_dev,
                                           float wd_host, int cautious, void* workspace,
                                           size_t workspace_bytes, void* stream);
+/* The same for matrices that do not fill whole tiles: the producer (dion_muon_pre_padded) writes them into the
+ * zero-padded form they are iterated in -- bf16 [batch, mp, np], short side along rows, zero outside
+ * min(rows, cols) x max(rows, cols), 16-byte aligned -- with partial sums of squares as above.
+ * dion_ns_padded_extents returns 1 and the extents when such a call pads its matrices (at least one iteration, more
+ * than 64 rows or columns on the short side, at most 4096 matrices), 0 otherwise.  Results differ from
+ * dion_ns_orthogonalize on the same matrices by nothing: it makes the same copy itself. */
+int dion_ns_padded_extents(int batch, int rows, int cols, int flags, int n_iters, int* mp, int* np);
+int dion_ns_orthogonalize_padded(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch, int rows,
+                                 int cols, const float* coeffs, int n_iters, float norm_scale, float eps, int flags,
+                                 int gram_reset, void* workspace, size_t workspace_bytes, void* stream);
+int dion_ns_orthogonalize_update_padded(const void* in, const float* sumsq, int sumsq_blocks, const uint64_t* X_ptrs,
+                                        int x_dtype, int n_ptrs, int mats_per_ptr, int rows, int cols,
+                                        const float* coeffs, int n_iters, float norm_scale, float eps, int flags,
+                                        int gram_reset, const float* lr_dev, float adj_ratio, const float* wd_dev,
+                                        float wd_host, int cautious, void* workspace, size_t workspace_bytes,
+                                        void* stream);
 /* dion_ns_plan_audit for the prepared form (host only, no device work). */
 int dion_ns_plan_audit_prepared(int batch, int rows, int cols, int n_iters, int flags, int gram_reset,
                                 int with_update, int x_dtype, int mats_per_ptr, size_t audit_ws_bytes);
@@ -206,6 +221,12 @@ int dion_muon_pre_sumsq_blocks(int rows, int cols);
 int dion_muon_pre_prepared(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, void* U,
                            float* sumsq, int n, int mats_per_ptr, int rows, int cols, float mu, int nesterov,
                            void* stream);
+/* The same into the padded form (see dion_ns_padded_extents): U bf16 [n * mats_per_ptr, mp, np], every element written,
+ * sumsq fp32 [n * mats_per_ptr, mp / 64 * np / 64].  Any rows, cols and alignment of G and M. */
+int dion_muon_pre_padded(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, void* U, float* sumsq,
+                         int n, int mats_per_ptr, int rows, int cols, int mp, int np, float mu, int nesterov,
+                         void* stream);
+
 
 /* Weight decay + update for one shape group.
  *   X_i = (1 - lr wd) X_i - lr adj_ratio U[i]            (cautious == 0)

@@ -148,3 +148,17 @@ def test_prepared_input_plans(shape):
                 (shape, lib.dion_last_error().decode())
         # a workspace cut short is caught for this form too
         assert _audit_prepared(lib, shape, 5, flags, ws=4096) == -1
+
+
+@pytest.mark.parametrize("shape", [s for s in RAGGED_SHAPES if min(s[1:]) > 64 and (s[1] % 128 or s[2] % 128)])
+def test_padded_plans_with_the_update(shape):
+    """Matrices with padding: one copy in, the update in the last product, stored extents without the padding."""
+    lib = _lib.load()
+    b = shape[0]
+    for flags in (0, GRAM):
+        for x_dtype in (F32, BF16):
+            for in_dtype in (F32, BF16):
+                n = _audit(lib, shape, 5, flags, in_dtype, with_update=2, x_dtype=x_dtype)
+                assert n > 0, lib.dion_last_error().decode()
+                if not flags or max(shape[1:]) < 3 * min(shape[1:]):
+                    assert n == 2 + 3 * 4 + 2 + (b + 63) // 64
