@@ -5,6 +5,7 @@ hands raw device pointers and the current stream to the library, and returns tor
 torch is used for device memory and streams only; all arithmetic happens in the HIP kernels.
 There is no CPU implementation behind these functions: CPU tensors raise.
 """
+import functools
 import math
 from typing import List, Optional, Sequence, Tuple
 
@@ -17,7 +18,9 @@ from ._lib import DION_BF16, DION_F32, DION_NS_GRAM, check, ptr_table
 
 
 def _stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    # (the handle alone: a Stream object per launch was 2 us of host time)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def _require_gpu(t: Tensor, name: str) -> None:
@@ -201,10 +204,18 @@ def ns_orthogonalize(G: Tensor, coeffs: Sequence[Sequence[float]], norm_scale: f
 
 
 def _flat_coeffs(coeffs):
+    return _tuple_coeffs(coeffs) if type(coeffs) is tuple else _list_coeffs(coeffs)
+
+
+def _list_coeffs(coeffs):
     flat = [float(v) for abc in coeffs for v in abc]
     if len(flat) % 3:
         raise ValueError("coeffs must be (a, b, c) triples")
     return (_lib.ctypes.c_float * max(1, len(flat)))(*flat), len(flat) // 3
+
+
+# the built-in schedules, as the library takes them (which only reads them)
+_tuple_coeffs = functools.lru_cache(maxsize=16)(_list_coeffs)
 
 
 def ns_orthogonalize_update(G: Tensor, X: List[Tensor], coeffs: Sequence[Sequence[float]], norm_scale: float,
@@ -330,15 +341,19 @@ def ns_orthogonalize_update_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: 
 # optimizer-step kernels on lists of same-shape parameters
 # ---------------------------------------------------------------------------------------------
 def _list_ptrs(ts: List[Tensor], name: str, dtype=None, numel=None):
+    # A step passes a few hundred tensors through here: the checks are spelled out instead of called.
+    ptrs = []
     for t in ts:
-        _require_gpu(t, name)
+        if type(t) is not Tensor or not t.is_cuda:
+            _require_gpu(t, name)
         if not t.is_contiguous():
             raise ValueError(f"{name}: tensors must be contiguous")
         if dtype is not None and t.dtype != dtype:
             raise TypeError(f"{name}: expected {dtype}, got {t.dtype}")
         if numel is not None and t.numel() != numel:
             raise ValueError(f"{name}: all tensors of a shape group must have {numel} elements")
-    return ptr_table([t.data_ptr() for t in ts])
+        ptrs.append(t.data_ptr())
+    return ptr_table(ptrs)
 
 
 def _state_ptrs(ts: List[Tensor], name: str, numel=None):

@@ -40,6 +40,13 @@ def _note_stream(t: Tensor) -> None:
         t.record_stream(torch.cuda.current_stream(t.device))
 
 
+def _as_matrices(tensors: List[Tensor], mats: int, rows: int, cols: int) -> List[Tensor]:
+    """Every tensor as ``[mats, rows, cols]``; one matrix per tensor stays as it is."""
+    if tensors[0].shape == (rows, cols):
+        return tensors
+    return [t.view(mats, rows, cols) for t in tensors]
+
+
 def _require_state_dtype(params: List[Tensor], who: str) -> None:
     """Parameters (and with them momentum / second moments, dion/megabatch_base.py:198-203) are kept in
     float32 or bfloat16; the kernels compute in fp32 and round a bf16 value once, on store."""
@@ -283,10 +290,10 @@ class Dion2(OrthoOptimizer):
                 print(f"[Dion2] Shape {tuple(shape)}: single GPU, shorter dim ({dim}) -> "
                       f"select top-{k} {what} by L1 norm")
 
-        X = [p.data.view(mats, rows, cols) for p in params]
-        G = [p.grad.contiguous().view(mats, rows, cols) for p in params]
-        M = [self._get_or_initialize_state(p, self._algo_name)["momentum"].view(mats, rows, cols)
-             for p in params]
+        X = _as_matrices([p.data for p in params], mats, rows, cols)
+        G = _as_matrices([p.grad.contiguous() for p in params], mats, rows, cols)
+        M = _as_matrices([self._get_or_initialize_state(p, self._algo_name)["momentum"] for p in params],
+                         mats, rows, cols)
 
         if self.assembled_selection and group["selection_scope"] == "global":
             if flatten and len(shape) >= 3:
@@ -408,11 +415,11 @@ class NorDion2(OrthoOptimizer):
         n = len(params)
         select_dim = -2  # whole rows, so the per-neuron normalisation sees complete neurons
         k = min(max(1, int(math.ceil(group["fraction"] * rows))), rows)
-        X = [p.data.view(mats, rows, cols) for p in params]
-        G = [p.grad.contiguous().view(mats, rows, cols) for p in params]
+        X = _as_matrices([p.data for p in params], mats, rows, cols)
+        G = _as_matrices([p.grad.contiguous() for p in params], mats, rows, cols)
         states = [self._get_or_initialize_state(p, self._algo_name) for p in params]
-        M = [s["momentum"].view(mats, rows, cols) for s in states]
-        V = [s["variance_neuron"].view(mats, rows, 1) for s in states]
+        M = _as_matrices([s["momentum"] for s in states], mats, rows, cols)
+        V = _as_matrices([s["variance_neuron"] for s in states], mats, rows, 1)
 
         if self.assembled_selection and group["selection_scope"] == "global":
             if flatten and len(shape) >= 3:
