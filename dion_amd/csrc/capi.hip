@@ -199,15 +199,15 @@ struct PostSpec {
 // per-head regime: whole iteration resident in LDS, one workgroup per matrix, no workspace.  The Gram
 // flag changes nothing here: the recurrence saves memory traffic of rectangular GEMMs, and a matrix
 // that never leaves LDS has none; the standard iteration applies the same polynomial.
-bool ns_small_path(int rows, int cols, int flags, int n_iters) {
+bool ns_small_path(int batch, int rows, int cols, int flags, int n_iters) {
   (void)flags;
-  return n_iters <= kMaxSmallIters && ns_small_fits(rows, cols);
+  return n_iters <= kMaxSmallIters && ns_small_fits(batch, rows, cols);
 }
 
 // The matrices do not fill whole tiles: they are iterated in zero-padded copies, mp x np each.
 bool ns_padded(int batch, int rows, int cols, int flags, int n_iters, int* mp = nullptr, int* np = nullptr) {
   if (batch <= 0 || batch > 65535 || rows <= 0 || cols <= 0 || n_iters <= 0) return false;
-  if (ns_small_path(rows, cols, flags, n_iters)) return false;
+  if (ns_small_path(batch, rows, cols, flags, n_iters)) return false;
   const NsPlan pl = make_plan(batch, rows, cols, flags);
   if (mp) *mp = pl.mp;
   if (np) *np = pl.np;
@@ -219,7 +219,7 @@ bool ns_padded(int batch, int rows, int cols, int flags, int n_iters, int* mp = 
 // still take it.)
 constexpr int kMaxFusedPadded = 4096;
 bool ns_update_fuses(int batch, int rows, int cols, int flags, int n_iters) {
-  if (n_iters <= 0 || ns_small_path(rows, cols, flags, n_iters)) return false;
+  if (n_iters <= 0 || ns_small_path(batch, rows, cols, flags, n_iters)) return false;
   return batch <= kMaxFusedPadded || !ns_padded(batch, rows, cols, flags, n_iters);
 }
 
@@ -228,7 +228,7 @@ bool ns_update_fuses(int batch, int rows, int cols, int flags, int n_iters) {
 // outside the LDS-resident kernel and with at least one iteration to carry the normalisation.
 bool ns_accepts_prepared(int batch, int rows, int cols, int flags, int n_iters) {
   if (batch <= 0 || batch > 65535 || rows <= 0 || cols <= 0 || n_iters <= 0) return false;
-  if (ns_small_path(rows, cols, flags, n_iters)) return false;
+  if (ns_small_path(batch, rows, cols, flags, n_iters)) return false;
   if (((int64_t)rows * cols) % 4096) return false;
   const NsPlan pl = make_plan(batch, rows, cols, flags);
   return pl.mp == pl.m && pl.np == pl.n;
@@ -345,7 +345,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     call.sq_lo = (const char*)sumsq;
     call.sq_hi = call.sq_lo + (size_t)batch * sumsq_blocks * 4;
   }
-  if (ns_small_path(rows, cols, flags, n_iters)) {
+  if (ns_small_path(batch, rows, cols, flags, n_iters)) {
     NsStep s = blank_step(NsStep::kSmall, "small-matrix Newton-Schulz");
     s.in = in;
     s.in_dtype = in_dtype;
@@ -919,7 +919,7 @@ extern "C" int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* 
                                             float eps, int flags, int gram_reset, void* stream) {
   size_t need = 0;
   if (batch > 0 && rows > 0 && cols > 0 && !(flags & ~DION_NS_GRAM) && n_iters >= 0 &&
-      !ns_small_path(rows, cols, flags, n_iters))
+      !ns_small_path(batch, rows, cols, flags, n_iters))
     need = make_plan(batch, rows, cols, flags).total;
   if (need > (size_t)DION_NS_STATIC_SCRATCH_BYTES)
     return fail(DION_E_WORKSPACE,
@@ -937,7 +937,7 @@ extern "C" int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* 
 
 extern "C" size_t dion_ns_update_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  const size_t ns = ns_small_path(rows, cols, flags, n_iters) ? 0 : align256(make_plan(batch, rows, cols, flags).total);
+  const size_t ns = ns_small_path(batch, rows, cols, flags, n_iters) ? 0 : align256(make_plan(batch, rows, cols, flags).total);
   if (ns_update_fuses(batch, rows, cols, flags, n_iters)) return ns;
   return ns + align256((size_t)batch * rows * cols * 2);
 }
@@ -1080,7 +1080,7 @@ static int plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters, 
   if (int rc = check_state_dtype("dion_ns_plan_audit", "x_dtype", x_dtype)) return rc;
   float coeffs[48];
   for (int i = 0; i < 48; ++i) coeffs[i] = 1.0f;
-  const bool small = ns_small_path(rows, cols, flags, n_iters);
+  const bool small = ns_small_path(batch, rows, cols, flags, n_iters);
   const size_t ws_bytes = small ? 0 : make_plan(batch, rows, cols, flags).total;
   // disjoint synthetic regions, 1 TiB apart
   char* const base = (char*)(uintptr_t)0x100000000000ull;

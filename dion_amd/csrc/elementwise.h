@@ -16,8 +16,8 @@ struct NsCoeffs {
   int n;
   float c[kMaxSmallIters][3];
 };
-// True when a rows x cols matrix (short side <= 64) fits the one-workgroup-per-matrix kernel.
-bool ns_small_fits(int rows, int cols);
+// True when `batch` matrices of rows x cols go to the one-workgroup-per-matrix kernel.
+bool ns_small_fits(int batch, int rows, int cols);
 hipError_t launch_ns_small(const void* in, int in_dtype, bf16_t* out, int batch, int rows, int cols,
                            const NsCoeffs& co, float norm_scale, float eps, hipStream_t st);
 

@@ -1,462 +1,378 @@
-// Whole Newton-Schulz / Polar-Express orthogonalization of one small matrix per workgroup, resident
-// in LDS from the Frobenius normalisation to the last iteration: the per-head regime (e.g. 64 x 768
-// attention heads), where the general path is 15 launches of GEMMs too small to fill a CU.
+// Whole Newton-Schulz / Polar-Express orthogonalization of one small matrix per workgroup, in registers
+// from the Frobenius normalisation to the last iteration: the per-head regime (e.g. 64 x 768 attention
+// heads), where the general path is 15 launches of GEMMs too small to fill a CU.
 //
 // Follows the same arithmetic as the batched driver (dion/newton_schulz_triton.py:508-522,
 // dion/polar_express.py:30-50): X = bf16(G) / (||.||_F * s + eps); A = X X^T; B = c A A + b A + a I;
 // X = B X, with A, B and X rounded to bf16 once per iteration and fp32 MFMA accumulation.
 //
-// Layout: X [64][n_pad] bf16 in LDS (row pitch + 16 B so that 16 consecutive rows hit 16 distinct
-// 16-byte bank slots), A and B [64][64].  X' = B X needs X with the reduction index along rows:
-// those fragments come from ds_read_b64_tr_b16 (a 4 x 16 block of 16-bit elements transposed
-// across a 16-lane group), so no transposed copy of X is kept.
 #include "elementwise.h"
 
 namespace dion {
 
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-constexpr int kThreads = 512;    // eight wavefronts: two per SIMD, so LDS and MFMA latencies of one hide behind the other
-constexpr int kMaxChunks = 18;  // 16-byte chunks a thread may hold while loading (n_pad <= 1152)
-constexpr int kPartialBytes = 4 * 3 * 64 * 16;  // A = X X^T: f32x4 per lane, three tiles, four wavefront groups
-constexpr int kMaxLds = 160 * 1024 - 1024;      // dynamic LDS of one workgroup: the static part (reduction scratch) takes the first KB
-#define LDS3(p) ((__attribute__((address_space(3))) s16x4*)(p))
+constexpr int kMaxLds = 160 * 1024 - 1024;  // dynamic LDS of one workgroup; the static part takes the rest
 
-static __device__ __forceinline__ bf16x8 join_tr(s16x4 lo, s16x4 hi) {
-  typedef __attribute__((ext_vector_type(8))) short s16x8;
-  s16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  return __builtin_bit_cast(bf16x8, v);
+// ------------------------------------------------------------------------------------------
+// A wavefront owns groups of 32 columns of X and keeps them as MFMA fragments: lane l of fragment x[g][t] holds row
+// l % 16 of row tile t and eight columns of group g.  That is an operand of A = X X^T as it is (the reduction runs over
+// columns, in any order both operands share), so the Gram product reads nothing.  X' = B X reduces over rows, which lie
+// across lanes: a product with the identity (exact: one term of each sum is not zero) turns a fragment so that lanes
+// run along columns, and X'^T = X^T B, with B symmetric, comes out in the layout x started in.  What crosses
+// wavefronts is only A's partial sums, A and B (16 MT square), through LDS; X crosses memory once in and once out.
+// Rows and columns are numbered so that the four consecutive indices a lane receives of each of two neighbouring 16-wide
+// tiles are eight consecutive ones: 16 bytes a lane from and to memory, and 16-byte reads of B.
+//
+// MT row tiles (rows padded to 16 MT), at most KC column groups per wavefront (of which the first KF exist in every
+// wavefront), NW wavefronts.  NW = 4 leaves room for two workgroups per CU: one's reduction and load phases run under the
+// other's MFMAs.
+//
+// What bounds it, 432 x (64 x 768), 43 us: 17 us are the 84 MB in and out (5 TB/s, no iteration), 4.7 us an iteration of
+// two matrices on one CU, of which 2.8 are MFMA time (the turning products are a quarter of it); the rest is the latency
+// of three barriers and A's partial sums through LDS.  The form with X in LDS and one workgroup per CU took 60.
+// 256 x (64 x 2048) 76 us, 300 x (128 x 768) 135, 200 x (80 x 1000) 54, 1000 x (128 x 1024) 453, where the GEMM chain on
+// matrices padded to 128 rows took 1074, 724, 296 and 2626; 16 x (128 x 256) 42 against 90.
+// ------------------------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(4))) unsigned rx4;
+static __device__ __forceinline__ f32x4 mfma_rx(rx4 a, rx4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <typename T>
+static __device__ __forceinline__ rx4 load8_bf16(const T* p) {
+  if constexpr (sizeof(T) == 2) return *(const rx4*)p;
+  else {
+    const float4 a = ((const float4*)p)[0], b = ((const float4*)p)[1];
+    return rx4{pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w)};
+  }
 }
 
-// One workgroup per CU walks matrices blockIdx.x, blockIdx.x + gridDim.x, ...: while the iterations of one
-// matrix run out of LDS, the next matrix is already on its way into registers (it is read from memory once,
-// the registers hold it until the norm is known), and the stores of the last iteration are left in flight.
-// CH: 16-byte chunks of a matrix a thread holds (12 for n_pad <= 768, else kMaxChunks).  Only the small form
-// has the registers to keep the next matrix next to the live values of an iteration; the large one fetches
-// each matrix when its turn comes.
-template <typename T, int CH>
-__global__ __launch_bounds__(kThreads) void ns_small_kernel(const T* __restrict__ in, bf16_t* __restrict__ out,
-                                                       int batch, int rows, int cols, int n_pad, NsCoeffs co,
-                                                       float norm_scale, float eps) {
-  constexpr bool kPrefetch = CH <= 12;
+template <int MT, int NW>
+struct RegCfg {
+  static constexpr int MR = MT * 16, AP = MR * 2 + 16;
+  static constexpr int NTILE = MT * (MT + 1) / 2;   // tiles of the symmetric A
+  static constexpr int PASSES = NTILE <= 10 ? 1 : NTILE <= 21 ? 3 : 4;
+  static constexpr int GT = (NTILE + PASSES - 1) / PASSES;  // tiles of A summed across wavefronts at a time
+  static constexpr int LDS = 2 * MR * AP + NW * GT * 1024;
+};
+
+template <int MT, int KC, int NW, int KF, typename T>
+__global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict__ in, bf16_t* __restrict__ out, int rows,
+                                                            int cols, NsCoeffs co, float norm_scale, float eps) {
+  typedef RegCfg<MT, NW> C;
+  constexpr int MR = C::MR, AP = C::AP, GT = C::GT, ST = MT / 2;
+  // x takes 4 MT KC registers: past 96 there is no room for a second turned group (256 x (64 x 2048) 76 -> 130 us)
+  constexpr bool PIPE = MT * KC <= 24;
+  constexpr bool BREG = MT <= 4;  // B's fragments stay in registers over the column groups
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  __shared__ float red[16];
-  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ float red[NW];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  char* const As = lds;
+  char* const Bs = As + MR * AP;
+  f32x4* const Ps = (f32x4*)(Bs + MR * AP);  // [wavefront][tile][lane]
   const bool tall = rows > cols;
-  const int m = tall ? cols : rows, n = tall ? rows : cols;  // m <= 64
-  const int xp = n_pad * 2 + 16;                              // X row pitch in bytes
-  constexpr int ap = 64 * 2 + 16;                             // A / B row pitch in bytes
-  char* Xs = lds;
-  char* As = lds + 64 * xp;
-  char* Bs = As + 64 * ap;
-  const int64_t mat_elems = (int64_t)rows * cols;
-  // Each thread keeps its 16-byte chunks of a matrix in registers between the load, the reduction and the
-  // scaled store to LDS, so a matrix is read from HBM once and LDS is written once.  Matrices are whole
-  // numbers of chunks and all equally aligned, so the choice holds for every matrix of the batch.
-  const bool vec = (cols % 8 == 0) && ((((uintptr_t)in) & 15) == 0) && n_pad * 8 <= CH * kThreads;
-  const int cpr = tall ? 8 : n_pad / 8;  // chunks per 64-wide (tall) or n_pad-wide (wide) input row
-  const int nchunks = 8 * n_pad;         // 64 * n_pad / 8
-  uint4 raw[CH];
-  auto fetch = [&](int64_t mat) {
-    const T* src = in + mat * mat_elems;
-    // (the chunk coordinates are recomputed per matrix from a value the compiler cannot see through: hoisted out of
-    // the matrix loop they would sit in registers through every iteration phase)
-    int tid_l = tid;
-    asm volatile("" : "+v"(tid_l));
+  const int m = tall ? cols : rows, n = tall ? rows : cols;
+  const int64_t first = (int64_t)blockIdx.x * rows * cols;
+  const T* const src = in + first;
+  bf16_t* const dst = out + first;
+  const bool vec = cols % 8 == 0 && (((uintptr_t)in) & 15) == 0;
+  const bool ovec = cols % 8 == 0 && (((uintptr_t)out) & 15) == 0;
+  auto col0 = [&](int g) { return (wave + g * NW) * 32; };       // first column of the wavefront's group g
+  auto absent = [&](int g) { return g >= KF && col0(g) >= n; };
+  const int sub = 8 * (l16 >> 2) + (l16 & 3);                     // index l16 of tile 2 s + h is 32 s + sub + 4 h
+  const uint32_t one = 0x3f80u;
+  const uint32_t i0 = (4 * q == l16 ? one : 0u) | (4 * q + 1 == l16 ? one << 16 : 0u);
+  const uint32_t i1 = (4 * q + 2 == l16 ? one : 0u) | (4 * q + 3 == l16 ? one << 16 : 0u);
+  const rx4 eye[2] = {rx4{i0, i1, 0u, 0u}, rx4{0u, 0u, i0, i1}};
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+  // eight consecutive elements from `at` on, those at or past `left` zero
+  auto fetch = [&](const T* at, bool ok, int left) -> rx4 {
+    rx4 w = {0u, 0u, 0u, 0u};
+    if (!ok) return w;
+    if (vec) return load8_bf16<T>(at);
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int idx = tid_l + c * kThreads;
-      raw[c] = make_uint4(0, 0, 0, 0);
-      if (idx < nchunks) {
-        const int r = idx / cpr, c0 = (idx - r * cpr) * 8;  // input row, first input column
-        if (r < rows && c0 < cols) {
-          if (sizeof(T) == 2) {
-            raw[c] = *(const uint4*)((const bf16_t*)src + (int64_t)r * cols + c0);
-          } else {
-            const float4 f0 = *(const float4*)((const float*)src + (int64_t)r * cols + c0);
-            const float4 f1 = *(const float4*)((const float*)src + (int64_t)r * cols + c0 + 4);
-            raw[c].x = pack_bf16x2(f0.x, f0.y);
-            raw[c].y = pack_bf16x2(f0.z, f0.w);
-            raw[c].z = pack_bf16x2(f1.x, f1.y);
-            raw[c].w = pack_bf16x2(f1.z, f1.w);
-          }
-        }
-      }
+    for (int e = 0; e < 4; ++e) {
+      uint32_t lo = 0, hi = 0;
+      if (2 * e < left) lo = sizeof(T) == 2 ? (uint32_t)(uint16_t)((const bf16_t*)at)[2 * e] : (uint32_t)(uint16_t)f32_to_bf16(((const float*)at)[2 * e]);
+      if (2 * e + 1 < left) hi = sizeof(T) == 2 ? (uint32_t)(uint16_t)((const bf16_t*)at)[2 * e + 1] : (uint32_t)(uint16_t)f32_to_bf16(((const float*)at)[2 * e + 1]);
+      w[e] = lo | (hi << 16);
+    }
+    return w;
+  };
+  auto store = [&](bf16_t* at, bool ok, int left, rx4 w) {
+    if (!ok) return;
+    if (ovec) {
+      *(rx4*)at = w;
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (2 * e < left) at[2 * e] = (bf16_t)(w[e] & 0xffffu);
+      if (2 * e + 1 < left) at[2 * e + 1] = (bf16_t)(w[e] >> 16);
     }
   };
-  if (kPrefetch && vec && (int64_t)blockIdx.x < batch) fetch(blockIdx.x);
 
-  for (int64_t mat = blockIdx.x; mat < batch; mat += gridDim.x) {
-  const T* src = in + mat * mat_elems;
-  bf16_t* dst = out + mat * mat_elems;
-
-  // ---- (raw bf16 values in registers), sum of squares, scale, store to LDS
-  float ss = 0.f;
-  if (vec) {
-    if (!kPrefetch) fetch(mat);
+  rx4 x[KC][MT];
+  // ---- load.  A tall matrix lies with its columns contiguous: fetched with lanes along columns and turned.
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const uint32_t w[4] = {raw[c].x, raw[c].y, raw[c].z, raw[c].w};
+  for (int g = 0; g < KC; ++g) {
+    const int c0 = col0(g);
+    if (!tall) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int r = 32 * (t >> 1) + sub + 4 * (t & 1), c = c0 + 8 * q;
+        x[g][t] = fetch(src + (int64_t)r * cols + c, r < m && c < n, n - c);
+      }
+    } else {
+      rx4 p[2][ST];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+          const int c = c0 + sub + 4 * h, r = 32 * s + 8 * q;
+          p[h][s] = fetch(src + (int64_t)c * cols + r, r < m && c < n, m - r);
+        }
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 d = mfma_rx(p[h][t >> 1], eye[t & 1], zero);
+          x[g][t][2 * h] = pack_bf16x2(d[0], d[1]);
+          x[g][t][2 * h + 1] = pack_bf16x2(d[2], d[3]);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // ---- Frobenius norm, scale
+  float ss = 0.f;
+#pragma unroll
+  for (int g = 0; g < KC; ++g)
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float lo = __uint_as_float(w[e] << 16), hi = __uint_as_float(w[e] & 0xffff0000u);
+        const float lo = __uint_as_float(x[g][t][e] << 16), hi = __uint_as_float(x[g][t][e] & 0xffff0000u);
         ss += lo * lo;
         ss += hi * hi;
       }
-    }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-    if (lane == 0) red[wave] = ss;
-    __syncthreads();
-    const float total = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
-    const float sc = 1.0f / (sqrtf(total) * norm_scale + eps);
-    int tid_l = tid;
-    asm volatile("" : "+v"(tid_l));
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int idx = tid_l + c * kThreads;
-      if (idx < nchunks) {
-        const int r = idx / cpr, c0 = (idx - r * cpr) * 8;
-        const uint32_t w[4] = {raw[c].x, raw[c].y, raw[c].z, raw[c].w};
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[2 * e] = __uint_as_float(w[e] << 16) * sc;
-          v[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u) * sc;
-        }
-        if (!tall) {  // X[r][c0..c0+7]
-          uint4 o;
-          o.x = pack_bf16x2(v[0], v[1]);
-          o.y = pack_bf16x2(v[2], v[3]);
-          o.z = pack_bf16x2(v[4], v[5]);
-          o.w = pack_bf16x2(v[6], v[7]);
-          *(uint4*)(Xs + r * xp + c0 * 2) = o;
-        } else {  // X[c0+e][r]
-#pragma unroll
-          for (int e = 0; e < 8; ++e) *(bf16_t*)(Xs + (c0 + e) * xp + r * 2) = f32_to_bf16(v[e]);
-        }
-      }
-    }
-    // the registers are free again: the next matrix of this workgroup travels while this one is iterated
-    if (kPrefetch && mat + gridDim.x < batch) fetch(mat + gridDim.x);
-  } else {
-    for (int idx = tid; idx < 64 * n_pad; idx += kThreads) {
-      const int i = idx / n_pad, j = idx - i * n_pad;  // X[i][j]
-      float v = 0.f;
-      if (i < m && j < n) {
-        const int64_t g = tall ? (int64_t)j * cols + i : (int64_t)i * cols + j;
-        v = sizeof(T) == 2 ? bf16_to_f32(((const bf16_t*)src)[g])
-                           : bf16_to_f32(f32_to_bf16(((const float*)src)[g]));
-      }
-      ss += v * v;
-      *(bf16_t*)(Xs + i * xp + j * 2) = f32_to_bf16(v);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-    if (lane == 0) red[wave] = ss;
-    __syncthreads();
-    const float total = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
-    const float sc = 1.0f / (sqrtf(total) * norm_scale + eps);
-    for (int idx = tid; idx < 64 * n_pad; idx += kThreads) {
-      const int i = idx / n_pad, j = idx - i * n_pad;
-      bf16_t* p = (bf16_t*)(Xs + i * xp + j * 2);
-      *p = f32_to_bf16(bf16_to_f32(*p) * sc);
-    }
-  }
+  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  if (lane == 0) red[wave] = ss;
   __syncthreads();
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) total += red[w];
+  const float sc = 1.0f / (sqrtf(total) * norm_scale + eps);
+#pragma unroll
+  for (int g = 0; g < KC; ++g)
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[g][t][e] = pack_bf16x2(__uint_as_float(x[g][t][e] << 16) * sc, __uint_as_float(x[g][t][e] & 0xffff0000u) * sc);
 
-  const int frow = lane & 31, fhalf = lane >> 5;
-  // A and B (64 x 64) are computed as 16x16 tiles with v_mfma_f32_16x16x32_bf16: lane l holds row / column
-  // l % 16 and the eight k values 8 * (l / 16) .. + 7 of a 32-deep step; accumulator element r is row
-  // 4 * (l / 16) + r, column l % 16.
-  const int r16 = lane & 15, kq = lane >> 4;
-  const int ti = wave >> 1, tj0 = (wave & 1) * 2;  // B = poly(A): two neighbouring tiles of one tile row
-  const int nstep = n_pad / 32;
-  // A = X X^T is symmetric: ten of its sixteen tiles are computed, the others are their mirror images.
-  // Four groups of wavefronts take the tiles (row block, column block)
-  //   (0,0) (0,1) (0,2) | (3,3) (3,0) (3,1) | (1,1) (1,2) | (2,2) (2,3)
-  // -- always the group's first row block against itself and its one or two other row blocks, so a k step
-  // costs a group three (two) fragment reads for three (two) MFMAs, the same fragments serving as both
-  // operands -- and the two wavefronts of a group split the k steps, even and odd.  (One tile row per
-  // wavefront pair over the full k range, the previous form, read 2.4 times as many fragment bytes and
-  // computed all sixteen tiles; this phase was LDS-bound.)
-  const int ag = wave >> 1, akh = wave & 1;
-  const int rb0 = ag == 0 ? 0 : ag == 1 ? 3 : ag == 2 ? 1 : 2;
-  const int rb1 = ag == 0 ? 1 : ag == 1 ? 0 : ag == 2 ? 2 : 3;
-  const int rb2 = ag == 0 ? 2 : 1;
-  const bool three = ag < 2;
-  float* Ps = (float*)(Bs + 64 * ap);  // partial sums of the odd-k wavefronts: [group][tile][lane] f32x4
+  // group g with lanes along columns: p[h][s] holds, of column tile h, the rows of tiles 2 s and 2 s + 1
+  auto turn = [&](int g, rx4 (&p)[2][ST]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const f32x4 d = mfma_rx(x[g][t], eye[h], zero);
+        p[h][t >> 1][2 * (t & 1)] = pack_bf16x2(d[0], d[1]);
+        p[h][t >> 1][2 * (t & 1) + 1] = pack_bf16x2(d[2], d[3]);
+      }
+  };
 
-  // wide result with 16-byte aligned rows: written out from LDS as whole rows after the last iteration
-  const bool out_rows = !tall && (cols % 8 == 0) && ((((uintptr_t)out) & 15) == 0);
-  auto last_it = [&](int it) { return it == co.n - 1; };
   for (int it = 0; it < co.n; ++it) {
     const float a = co.c[it][0], b = co.c[it][1], c = co.c[it][2];
-    // ---- A = X X^T
-    {
-      f32x4 acc[3];
+    // ---- A = X X^T, GT tiles at a time: every wavefront's share, then one wavefront per tile adds them in order
 #pragma unroll
-      for (int t = 0; t < 3; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const char* p0 = Xs + (rb0 * 16 + r16) * xp + kq * 16;
-      const char* p1 = Xs + (rb1 * 16 + r16) * xp + kq * 16;
-      const char* p2 = Xs + (rb2 * 16 + r16) * xp + kq * 16;
-      // fragments of the step after next are requested before the MFMAs of this one (two register sets)
-      if (three) {
-        bf16x8 f[2][3];
-        f[0][0] = *(const bf16x8*)(p0 + akh * 64);
-        f[0][1] = *(const bf16x8*)(p1 + akh * 64);
-        f[0][2] = *(const bf16x8*)(p2 + akh * 64);
-        int s = akh;
-        for (; s + 2 < nstep; s += 4) {
-          f[1][0] = *(const bf16x8*)(p0 + (s + 2) * 64);
-          f[1][1] = *(const bf16x8*)(p1 + (s + 2) * 64);
-          f[1][2] = *(const bf16x8*)(p2 + (s + 2) * 64);
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][0], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][1], acc[1], 0, 0, 0);
-          acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][2], acc[2], 0, 0, 0);
-          if (s + 4 < nstep) {
-            f[0][0] = *(const bf16x8*)(p0 + (s + 4) * 64);
-            f[0][1] = *(const bf16x8*)(p1 + (s + 4) * 64);
-            f[0][2] = *(const bf16x8*)(p2 + (s + 4) * 64);
-          }
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][0], f[1][0], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][0], f[1][1], acc[1], 0, 0, 0);
-          acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][0], f[1][2], acc[2], 0, 0, 0);
-        }
-        if (s < nstep) {  // an odd number of steps for this wavefront: the last one sits in set 0
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][0], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][1], acc[1], 0, 0, 0);
-          acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][2], acc[2], 0, 0, 0);
-        }
-      } else {
-        bf16x8 f[2][2];
-        f[0][0] = *(const bf16x8*)(p0 + akh * 64);
-        f[0][1] = *(const bf16x8*)(p1 + akh * 64);
-        int s = akh;
-        for (; s + 2 < nstep; s += 4) {
-          f[1][0] = *(const bf16x8*)(p0 + (s + 2) * 64);
-          f[1][1] = *(const bf16x8*)(p1 + (s + 2) * 64);
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][0], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][1], acc[1], 0, 0, 0);
-          if (s + 4 < nstep) {
-            f[0][0] = *(const bf16x8*)(p0 + (s + 4) * 64);
-            f[0][1] = *(const bf16x8*)(p1 + (s + 4) * 64);
-          }
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][0], f[1][0], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[1][0], f[1][1], acc[1], 0, 0, 0);
-        }
-        if (s < nstep) {
-          acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][0], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[0][0], f[0][1], acc[1], 0, 0, 0);
-        }
-      }
-      float* pp = Ps + ((ag * 3) * 64 + lane) * 4;
-      if (akh == 1) {
+    for (int ps = 0; ps < C::PASSES; ++ps) {
+      f32x4 acc[GT];
 #pragma unroll
-        for (int t = 0; t < 3; ++t) *(f32x4*)(pp + t * 256) = acc[t];
+      for (int k = 0; k < GT; ++k) acc[k] = zero;
+#pragma unroll
+      for (int g = 0; g < KC; ++g) {
+        if (absent(g)) continue;
+#pragma unroll
+        for (int t1 = 0; t1 < MT; ++t1)
+#pragma unroll
+          for (int t2 = t1; t2 < MT; ++t2) {
+            const int k = t1 * MT - t1 * (t1 - 1) / 2 + (t2 - t1) - ps * GT;
+            if (k >= 0 && k < GT) acc[k] = mfma_rx(x[g][t1], x[g][t2], acc[k]);
+          }
       }
+      if (ps > 0) __syncthreads();  // the sums of the tiles before have been read
+#pragma unroll
+      for (int k = 0; k < GT; ++k) Ps[(wave * GT + k) * 64 + lane] = acc[k];
       __syncthreads();
-      if (akh == 0) {
 #pragma unroll
-        for (int t = 0; t < 3; ++t) {
-          if (t == 2 && !three) break;
-          const f32x4 o = *(const f32x4*)(pp + t * 256);
-          const int cb = t == 0 ? rb0 : t == 1 ? rb1 : rb2;
+      for (int i = 0; i < (GT + NW - 1) / NW; ++i) {
+        const int k = wave + i * NW;
+        if (k >= GT || ps * GT + k >= C::NTILE) continue;
+        int t1 = 0, t2 = ps * GT + k;
+        while (t2 >= MT - t1) {
+          t2 -= MT - t1;
+          ++t1;
+        }
+        t2 += t1;
+        f32x4 s = Ps[k * 64 + lane];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int row = rb0 * 16 + kq * 4 + r, col = cb * 16 + r16;
-            const bf16_t v = f32_to_bf16(acc[t][r] + o[r]);
-            *(bf16_t*)(As + row * ap + col * 2) = v;
-            if (t > 0) *(bf16_t*)(As + col * ap + row * 2) = v;
-          }
+        for (int w = 1; w < NW; ++w) s += Ps[(w * GT + k) * 64 + lane];
+        const uint32_t w0 = pack_bf16x2(s[0], s[1]), w1 = pack_bf16x2(s[2], s[3]);
+        const int row = 16 * t1 + 4 * q, col = 16 * t2 + l16;
+        *(uint2*)(As + col * AP + row * 2) = make_uint2(w0, w1);
+        if (t1 != t2) {
+          *(uint16_t*)(As + row * AP + col * 2) = (uint16_t)w0;
+          *(uint16_t*)(As + (row + 1) * AP + col * 2) = (uint16_t)(w0 >> 16);
+          *(uint16_t*)(As + (row + 2) * AP + col * 2) = (uint16_t)w1;
+          *(uint16_t*)(As + (row + 3) * AP + col * 2) = (uint16_t)(w1 >> 16);
         }
       }
     }
     __syncthreads();
-    // ---- B = c A A + b A + a I  (A symmetric: rows of A serve both operands)
-    {
-      f32x4 acc[2];
-      acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // ---- B = c A A + b A + a I.  A is symmetric, and so, bit for bit, is B: element (row, col) is stored as (col, row).
+#pragma unroll 4
+    for (int i = 0; i < (MT * MT + NW - 1) / NW; ++i) {
+      const int u = wave + i * NW;
+      if (MT * MT % NW != 0 && u >= MT * MT) continue;
+      const int t1 = u / MT, t2 = u - t1 * MT;
+      f32x4 acc = zero;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const bf16x8 fa = *(const bf16x8*)(As + (ti * 16 + r16) * ap + s * 64 + kq * 16);
-        const bf16x8 f0 = *(const bf16x8*)(As + (tj0 * 16 + r16) * ap + s * 64 + kq * 16);
-        const bf16x8 f1 = *(const bf16x8*)(As + ((tj0 + 1) * 16 + r16) * ap + s * 64 + kq * 16);
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, f0, acc[0], 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, f1, acc[1], 0, 0, 0);
-      }
+      for (int s = 0; s < ST; ++s)
+        acc = mfma_rx(*(const rx4*)(As + (16 * t1 + l16) * AP + s * 64 + q * 16),
+                      *(const rx4*)(As + (16 * t2 + l16) * AP + s * 64 + q * 16), acc);
+      const int row = 16 * t1 + 4 * q, col = 16 * t2 + l16;
+      const uint2 av = *(const uint2*)(As + col * AP + row * 2);
+      float v[4];
+      v[0] = c * acc[0] + b * __uint_as_float(av.x << 16);
+      v[1] = c * acc[1] + b * __uint_as_float(av.x & 0xffff0000u);
+      v[2] = c * acc[2] + b * __uint_as_float(av.y << 16);
+      v[3] = c * acc[3] + b * __uint_as_float(av.y & 0xffff0000u);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = ti * 16 + kq * 4 + r;
-          const int col = (tj0 + j) * 16 + r16;
-          float v = c * acc[j][r] + b * bf16_to_f32(*(const bf16_t*)(As + row * ap + col * 2));
-          if (row == col) v += a;
-          *(bf16_t*)(Bs + row * ap + col * 2) = f32_to_bf16(v);
-        }
+      for (int r = 0; r < 4; ++r)
+        if (row + r == col) v[r] += a;
+      // (columns of B in the order a turned fragment holds its rows)
+      *(uint2*)(Bs + col * AP + (32 * (t1 >> 1) + 8 * q + 4 * (t1 & 1)) * 2) =
+          make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
     }
     __syncthreads();
-    // ---- X = B X: wavefront w owns column tiles w, w+8, ...; both row tiles per column tile, so
-    // the whole 64 x 32 column block is read before it is overwritten.
-    {
-      bf16x8 fB[2][4];
+    // ---- X = B X
+    auto bfrag = [&](int t, int s) { return *(const rx4*)(Bs + (16 * t + l16) * AP + s * 64 + q * 16); };
+    rx4 bf[BREG ? MT : 1][ST];
+    if constexpr (BREG)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-          fB[i][s] = *(const bf16x8*)(Bs + (i * 32 + frow) * ap + s * 32 + fhalf * 16);
-      // transposed-read addressing: 16-lane group g covers columns (g&1)*16.., k rows 8*(g>>1)..;
-      // lane t of the group points at row t/4, 4-element column chunk t%4.
-      const int g16 = lane >> 4, t16 = lane & 15;
-      const int trow = 8 * (g16 >> 1) + (t16 >> 2);
-      const int tcol = (g16 & 1) * 16 + (t16 & 3) * 4;
-      const bool last = (it == co.n - 1);
-      // The MFMA operands are swapped (X fragment first): the accumulators then hold (B X)^T tiles, i.e.
-      // lane l owns output row i*32 + l%32 and, per group of four accumulator elements, four consecutive
-      // output columns -- one 8-byte store per group instead of four 2-byte ones.
-      const int ntile = n_pad / 32;
-      auto load_tile = [&](int jt, s16x4 (&lo)[4], s16x4 (&hi)[4]) {
-        const char* px = Xs + trow * xp + (jt * 32 + tcol) * 2;
+        for (int s = 0; s < ST; ++s) bf[t][s] = bfrag(t, s);
+    // (where the registers reach for it, the next group is turned beside the products of this one)
+    rx4 p[2][2][ST];
+    if (PIPE && !absent(0)) turn(0, p[0]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          lo[s] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS3(px + (s * 16) * xp));
-          hi[s] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS3(px + (s * 16 + 4) * xp));
+    for (int g = 0; g < KC; ++g) {
+      if (absent(g)) continue;
+      if constexpr (!PIPE) turn(g, p[g & 1]);
+      else if (g + 1 < KC && !absent(g + 1)) turn(g + 1, p[(g + 1) & 1]);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        rx4 b1[ST];
+#pragma unroll
+        for (int k = 0; k < ST; ++k) b1[k] = BREG ? bf[BREG ? t : 0][k] : bfrag(t, k);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          f32x4 acc = zero;
+#pragma unroll
+          for (int k = 0; k < ST; ++k) acc = mfma_rx(p[g & 1][h][k], b1[k], acc);
+          x[g][t][2 * h] = pack_bf16x2(acc[0], acc[1]);
+          x[g][t][2 * h + 1] = pack_bf16x2(acc[2], acc[3]);
         }
-      };
-      auto do_tile = [&](int jt, s16x4 (&clo)[4], s16x4 (&chi)[4], s16x4 (&nlo)[4], s16x4 (&nhi)[4]) {
-        f32x16 acc[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
-        // the next column tile's fragments are requested before this tile's MFMAs and stores
-        if (jt + 8 < ntile) load_tile(jt + 8, nlo, nhi);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const bf16x8 fx = join_tr(clo[s], chi[s]);
-          acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx, fB[0][s], acc[0], 0, 0, 0);
-          acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx, fB[1][s], acc[1], 0, 0, 0);
-        }
-        const int col0 = jt * 32 + 4 * fhalf;  // + 8 * g: first of four consecutive columns
-        // The last X' of a wide matrix goes through LDS like the others and leaves as whole rows below (16 bytes
-        // per lane): stored from the accumulators it would be 8-byte pieces 1.5 KB apart.
-        if (!last || out_rows) {
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              uint2 o;
-              o.x = pack_bf16x2(acc[i][4 * g], acc[i][4 * g + 1]);
-              o.y = pack_bf16x2(acc[i][4 * g + 2], acc[i][4 * g + 3]);
-              *(uint2*)(Xs + (i * 32 + frow) * xp + (col0 + 8 * g) * 2) = o;
-            }
-        } else if (!tall) {
-          const bool vec4 = (cols % 4 == 0) && ((((uintptr_t)dst) & 7) == 0);
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int row = i * 32 + frow;
-            if (row >= m) continue;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const int col = col0 + 8 * g;
-              bf16_t* q = dst + row * cols + col;
-              if (vec4 && col + 3 < n) {
-                uint2 o;
-                o.x = pack_bf16x2(acc[i][4 * g], acc[i][4 * g + 1]);
-                o.y = pack_bf16x2(acc[i][4 * g + 2], acc[i][4 * g + 3]);
-                *(uint2*)q = o;
-              } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (col + e < n) q[e] = f32_to_bf16(acc[i][4 * g + e]);
-              }
-            }
-          }
-        } else {
-          // tall input: X holds the transpose, output element (col, row); lanes run along `row`
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int row = i * 32 + frow;
-            if (row >= m) continue;
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const int col = col0 + 8 * g + e;
-                if (col < n) dst[col * cols + row] = f32_to_bf16(acc[i][4 * g + e]);
-              }
-          }
-        }
-      };
-      s16x4 lo0[4], hi0[4], lo1[4], hi1[4];
-      if (wave < ntile) load_tile(wave, lo0, hi0);
-      for (int jt = wave; jt < ntile; jt += 16) {
-        do_tile(jt, lo0, hi0, lo1, hi1);
-        if (jt + 8 < ntile) do_tile(jt + 8, lo1, hi1, lo0, hi0);
       }
-    }
-    __syncthreads();
-    if (last_it(it) && out_rows) {
-      // X [m][n] in LDS -> dst [rows][cols], 16 bytes per lane, lanes side by side along a row
-      const int cpr8 = cols / 8;
-      for (int idx = tid; idx < m * cpr8; idx += kThreads) {
-        const int r = idx / cpr8, c8 = idx - r * cpr8;
-        *(uint4*)(dst + (int64_t)r * cols + c8 * 8) = *(const uint4*)(Xs + r * xp + c8 * 16);
-      }
-      __syncthreads();  // X is rewritten by the next matrix
+      __builtin_amdgcn_sched_barrier(0);  // no more than two groups' temporaries at a time
     }
   }
-  if (co.n == 0) {  // normalisation only
-    for (int idx = tid; idx < m * n; idx += kThreads) {
-      const int i = idx / n, j = idx - i * n;
-      const int64_t g = tall ? (int64_t)j * cols + i : (int64_t)i * cols + j;
-      dst[g] = *(const bf16_t*)(Xs + i * xp + j * 2);
+  // ---- out
+#pragma unroll
+  for (int g = 0; g < KC; ++g) {
+    if (absent(g)) continue;
+    if (!tall) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int r = 32 * (t >> 1) + sub + 4 * (t & 1), c = col0(g) + 8 * q;
+        store(dst + (int64_t)r * cols + c, r < m && c < n, n - c, x[g][t]);
+      }
+    } else {
+      rx4 p[2][ST];
+      turn(g, p);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+          const int c = col0(g) + sub + 4 * h, r = 32 * s + 8 * q;
+          store(dst + (int64_t)c * cols + r, r < m && c < n, m - r, p[h][s]);
+        }
     }
-    __syncthreads();  // X is rewritten by the next matrix
+    __builtin_amdgcn_sched_barrier(0);
   }
-  }  // matrices of this workgroup
 }
 
-bool ns_small_fits(int rows, int cols) {
-  const int m = rows < cols ? rows : cols, n = rows < cols ? cols : rows;
-  if (m > 64) return false;
-  const int n_pad = (n + 63) / 64 * 64;
-  const size_t bytes = (size_t)64 * (n_pad * 2 + 16) + 2 * 64 * (64 * 2 + 16) + kPartialBytes;
-  return bytes <= kMaxLds;
-}
-
-hipError_t launch_ns_small(const void* in, int in_dtype, bf16_t* out, int batch, int rows, int cols,
-                           const NsCoeffs& co, float norm_scale, float eps, hipStream_t st) {
-  const int n = rows < cols ? cols : rows;
-  const int n_pad = (n + 63) / 64 * 64;
-  const size_t bytes = (size_t)64 * (n_pad * 2 + 16) + 2 * 64 * (64 * 2 + 16) + kPartialBytes;
-  static std::atomic<uint64_t> done[4];
-  const bool small = n_pad * 8 <= 12 * kThreads;
-  const void* kern = in_dtype == 0 ? (small ? (const void*)ns_small_kernel<bf16_t, 12> : (const void*)ns_small_kernel<bf16_t, kMaxChunks>)
-                                   : (small ? (const void*)ns_small_kernel<float, 12> : (const void*)ns_small_kernel<float, kMaxChunks>);
-  if (hipError_t e = set_max_dynamic_lds_once(kern, kMaxLds, done[(in_dtype == 0 ? 0 : 2) + (small ? 0 : 1)])) return e;
-  // one workgroup per CU (the LDS footprint admits no second one), each walking its share of the batch
-  static std::atomic<int> cu_count[64];
-  int dev = 0;
-  if (hipError_t e = hipGetDevice(&dev)) return e;
-  int cus = cu_count[dev & 63].load(std::memory_order_relaxed);
-  if (cus == 0) {
-    if (hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) return e;
-    if (cus <= 0) return hipErrorInvalidValue;
-    cu_count[dev & 63].store(cus, std::memory_order_relaxed);
-  }
-  const int grid = batch < cus ? batch : cus;
-#define SMALL_LAUNCH(T, CHN)                                                                                   \
-  hipLaunchKernelGGL((ns_small_kernel<T, CHN>), dim3(grid), dim3(kThreads), bytes, st, (const T*)in, out, batch, \
-                     rows, cols, n_pad, co, norm_scale, eps)
+template <int MT, int KC, int NW, int KF>
+static hipError_t launch_reg(const void* in, int in_dtype, bf16_t* out, int batch, int rows, int cols, const NsCoeffs& co,
+                             float norm_scale, float eps, hipStream_t st) {
+  static std::atomic<uint64_t> done[2];
+  constexpr int bytes = RegCfg<MT, NW>::LDS;
+  static_assert(bytes <= kMaxLds, "");
   if (in_dtype == 0) {
-    if (small) SMALL_LAUNCH(bf16_t, 12); else SMALL_LAUNCH(bf16_t, kMaxChunks);
+    if (hipError_t e = set_max_dynamic_lds_once((const void*)ns_reg_kernel<MT, KC, NW, KF, bf16_t>, bytes, done[0])) return e;
+    hipLaunchKernelGGL((ns_reg_kernel<MT, KC, NW, KF, bf16_t>), dim3(batch), dim3(NW * 64), bytes, st, (const bf16_t*)in, out,
+                       rows, cols, co, norm_scale, eps);
   } else {
-    if (small) SMALL_LAUNCH(float, 12); else SMALL_LAUNCH(float, kMaxChunks);
+    if (hipError_t e = set_max_dynamic_lds_once((const void*)ns_reg_kernel<MT, KC, NW, KF, float>, bytes, done[1])) return e;
+    hipLaunchKernelGGL((ns_reg_kernel<MT, KC, NW, KF, float>), dim3(batch), dim3(NW * 64), bytes, st, (const float*)in, out,
+                       rows, cols, co, norm_scale, eps);
   }
-#undef SMALL_LAUNCH
   return hipGetLastError();
+}
+
+// Longest long side the kernel takes at a short side of m: 128 registers of X per lane; 0: none.
+static int ns_reg_max_cols(int m) { return m <= 32 ? 4096 : m <= 64 ? 2048 : m <= 96 ? 1280 : m <= 128 ? 1024 : 0; }
+
+hipError_t launch_ns_small(const void* in, int in_dtype, bf16_t* out, int batch, int rows, int cols, const NsCoeffs& co,
+                           float norm_scale, float eps, hipStream_t st) {
+  const int m = rows < cols ? rows : cols, n = rows < cols ? cols : rows;
+  const int groups = (n + 31) / 32;
+  // Up to a workgroup per CU eight wavefronts share a matrix (24 x (64 x 768): 26.8 -> 22.0 us), past that four, two
+  // workgroups per CU.  The forms of 128 registers of X check every group for being there: the straight-line code of
+  // the others makes the compiler keep more of them in flight than fit (256 x (64 x 2048): 76 -> 104 us).
+  const bool wide = batch <= 256;
+#define REG(MT, KC, NW, KF)                                                                               \
+  if (groups <= KC * NW && groups >= KF * NW)                                                             \
+  return launch_reg<MT, KC, NW, KF>(in, in_dtype, out, batch, rows, cols, co, norm_scale, eps, st)
+  if (m <= 32) {
+    if (!wide) {
+      REG(2, 2, 4, 0); REG(2, 4, 4, 2); REG(2, 8, 4, 4);
+    }
+    REG(2, 4, 8, 0); REG(2, 8, 8, 4); REG(2, 16, 8, 0);
+  } else if (m <= 64) {
+    if (!wide) {
+      REG(4, 2, 4, 0); REG(4, 4, 4, 2); REG(4, 6, 4, 4);
+    }
+    REG(4, 1, 8, 0); REG(4, 2, 8, 1); REG(4, 3, 8, 2); REG(4, 4, 8, 3); REG(4, 6, 8, 4); REG(4, 8, 8, 0);
+  } else if (m <= 96) {
+    REG(6, 2, 8, 0); REG(6, 3, 8, 2); REG(6, 4, 8, 3); REG(6, 5, 8, 0);
+  } else if (m <= 128) {
+    REG(8, 2, 8, 0); REG(8, 3, 8, 2); REG(8, 4, 8, 0);
+  }
+#undef REG
+  return hipErrorInvalidValue;
+}
+
+// Short sides up to 64 and long sides up to 1024 whatever the batch.  Past that a matrix is more work for one CU (128 x
+// 1024: 16 us an iteration) than its share of a few GEMM launches: only batches of 16 and more, from 256 columns on (a group
+// for every wavefront): 24 x (128 x 1024) 85 us against 123, 16 x (128 x 256) 42 against 90, 64 x (32 x 4096) 46 against 403.
+bool ns_small_fits(int batch, int rows, int cols) {
+  const int m = rows < cols ? rows : cols, n = rows < cols ? cols : rows;
+  if (m <= 64 && n <= 1024) return true;
+  return batch >= 16 && n >= 256 && n <= ns_reg_max_cols(m);
 }
 
 }  // namespace dion
