@@ -77,6 +77,10 @@ SIGNATURES = {
     "dion_dion2_gather": (c_int, [_u64p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float,
                                   c_void_p, c_void_p]),
     "dion_dion2_gather_sumsq_blocks": (c_int, [c_int, c_int, c_int, c_int]),
+    "dion_dion2_column_norms": (c_int, [_u64p, c_int, _u64p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                                        c_size_t, c_void_p]),
+    "dion_dion2_add_gather_columns": (c_int, [_u64p, c_int, _u64p, c_int, c_int, c_int, c_int, c_int, c_void_p,
+                                              c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p]),
     "dion_dion2_gather_prepared": (c_int, [_u64p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float,
                                            c_void_p, c_void_p, c_void_p]),
     "dion_dion2_post": (c_int, [_u64p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p,

@@ -1327,22 +1327,21 @@ extern "C" size_t dion_dion2_accumulate_scratch_bytes(int n_mat, int rows, int c
   return slabs > 1 ? (size_t)slabs * n_mat * cols * sizeof(float) : 0;
 }
 
-extern "C" int dion_dion2_accumulate(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs,
-                                     int m_dtype, int n, int mats_per_ptr, int rows, int cols, int select_dim,
-                                     float* norms, void* scratch, size_t scratch_bytes,
-                                     void* stream) {
-  if (int rc = check_select_dim("dion_dion2_accumulate", select_dim)) return rc;
-  if (int rc = check_state_dtype("dion_dion2_accumulate", "m_dtype", m_dtype)) return rc;
-  if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0)
-    return fail(DION_E_INVALID, "dion_dion2_accumulate: bad size");
-  if (g_dtype != DION_BF16 && g_dtype != DION_F32)
-    return fail(DION_E_INVALID, "dion_dion2_accumulate: g_dtype");
+static int dion2_norms_impl(const char* who, bool store, const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs,
+                            int m_dtype, int n, int mats_per_ptr, int rows, int cols, int select_dim, float* norms,
+                            void* scratch, size_t scratch_bytes, void* stream) {
+  if (int rc = check_select_dim(who, select_dim)) return rc;
+  if (int rc = check_state_dtype(who, "m_dtype", m_dtype)) return rc;
+  if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0) return fail(DION_E_INVALID, "%s: bad size", who);
+  if (g_dtype != DION_BF16 && g_dtype != DION_F32) return fail(DION_E_INVALID, "%s: g_dtype", who);
   if (n == 0 || rows == 0 || cols == 0) return DION_OK;
-  if (!G_ptrs || !M_ptrs || !norms) return fail(DION_E_INVALID, "dion_dion2_accumulate: null argument");
+  if (!G_ptrs || !M_ptrs || !norms) return fail(DION_E_INVALID, "%s: null argument", who);
   const int dim = select_dim == -2 ? rows : cols;
   // 16-byte accesses need 4-column alignment of every row of every matrix
   const bool vec4 = (cols % 4 == 0) && table_aligned(G_ptrs, n) && table_aligned(M_ptrs, n) &&
                     aligned16((uint64_t)norms);
+  if (!store && !vec4)
+    return fail(DION_E_INVALID, "%s: cols (%d) must be a multiple of 4, every pointer 16-byte aligned", who, cols);
   // Row slabs (column sums only): sized for the whole group, used if the scratch holds them.
   int slabs = 1;
   if (select_dim == -1 && vec4 && scratch && aligned16((uint64_t)scratch)) {
@@ -1359,9 +1358,55 @@ extern "C" int dion_dion2_accumulate(const uint64_t* G_ptrs, int g_dtype, const 
     fill_tab(m, M_ptrs + i0, c);
     HIP_TRY(launch_dion2_accumulate(g, dt(g_dtype), m, dt(m_dtype), c * mats_per_ptr, mats_per_ptr, rows, cols,
                                     select_dim == -2, norms + (int64_t)i0 * mats_per_ptr * dim, vec4,
-                                    slabs > 1 ? (float*)scratch : nullptr, slabs,
+                                    slabs > 1 ? (float*)scratch : nullptr, slabs, store,
                                     (hipStream_t)stream),
-            "dion_dion2_accumulate");
+            who);
+  }
+  return DION_OK;
+}
+
+extern "C" int dion_dion2_accumulate(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs,
+                                     int m_dtype, int n, int mats_per_ptr, int rows, int cols, int select_dim,
+                                     float* norms, void* scratch, size_t scratch_bytes,
+                                     void* stream) {
+  return dion2_norms_impl("dion_dion2_accumulate", true, G_ptrs, g_dtype, M_ptrs, m_dtype, n, mats_per_ptr, rows, cols,
+                          select_dim, norms, scratch, scratch_bytes, stream);
+}
+
+extern "C" int dion_dion2_column_norms(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, int n,
+                                       int mats_per_ptr, int rows, int cols, float* norms, void* scratch,
+                                       size_t scratch_bytes, void* stream) {
+  return dion2_norms_impl("dion_dion2_column_norms", false, G_ptrs, g_dtype, M_ptrs, m_dtype, n, mats_per_ptr, rows, cols,
+                          -1, norms, scratch, scratch_bytes, stream);
+}
+
+extern "C" int dion_dion2_add_gather_columns(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype,
+                                             int n, int mats_per_ptr, int rows, int cols, const int32_t* idx,
+                                             const int32_t* map, int k, float ef_decay, void* U_sel, float* sumsq,
+                                             void* stream) {
+  const char* who = "dion_dion2_add_gather_columns";
+  if (int rc = check_state_dtype(who, "m_dtype", m_dtype)) return rc;
+  if (g_dtype != DION_BF16 && g_dtype != DION_F32) return fail(DION_E_INVALID, "%s: g_dtype", who);
+  if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0 || k < 0) return fail(DION_E_INVALID, "%s: bad size", who);
+  if (n == 0 || rows == 0 || cols == 0 || k == 0) return DION_OK;
+  if (!G_ptrs || !M_ptrs || !idx || !map || !U_sel || !sumsq) return fail(DION_E_INVALID, "%s: null argument", who);
+  if (k > cols || rows <= k || rows % 64 || k % 64 || cols % 4 || rows / 64 > 65535)
+    return fail(DION_E_INVALID, "%s: %d columns of %d x %d", who, k, rows, cols);
+  if (!table_aligned(G_ptrs, n) || !table_aligned(M_ptrs, n) || !aligned16((uint64_t)U_sel) || !aligned16((uint64_t)map))
+    return fail(DION_E_INVALID, "%s: pointers must be 16-byte aligned", who);
+  const int cmax = ptr_chunk(mats_per_ptr);
+  if (cmax == 0) return fail(DION_E_INVALID, "more than 65535 matrices behind one pointer");
+  const int64_t blocks = (int64_t)(rows / 64) * (k / 64);
+  for (int i0 = 0; i0 < n; i0 += cmax) {
+    const int c = (n - i0) < cmax ? (n - i0) : cmax;
+    PtrTab g, m;
+    fill_tab(g, G_ptrs + i0, c);
+    fill_tab(m, M_ptrs + i0, c);
+    const int64_t mat0 = (int64_t)i0 * mats_per_ptr;
+    HIP_TRY(launch_dion2_add_gather_cols(g, dt(g_dtype), m, dt(m_dtype), c * mats_per_ptr, mats_per_ptr, rows, cols,
+                                         idx + mat0 * k, map + mat0 * cols, k, ef_decay,
+                                         (bf16_t*)U_sel + mat0 * rows * k, sumsq + mat0 * blocks, (hipStream_t)stream),
+            who);
   }
   return DION_OK;
 }

@@ -64,8 +64,13 @@ hipError_t launch_normuon_stats(const bf16_t* U, const PtrTab& V, int v_dtype, i
                                 float* row_scale, hipStream_t st);
 hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, int n_mat,
                                    int mats_per_ptr, int rows, int cols, int select_rows,
-                                   float* norms, bool vec4, float* slab_scratch, int slabs,
+                                   float* norms, bool vec4, float* slab_scratch, int slabs, bool store,
                                    hipStream_t st);
+// M += G, selected columns to U^T and decayed, partial sums as launch_dion2_gather_prepared's tall form: rows % 64 == 0,
+// k % 64 == 0, cols % 4 == 0, G and M 16-byte aligned.
+hipError_t launch_dion2_add_gather_cols(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, int n_mat,
+                                        int mats_per_ptr, int rows, int cols, const int32_t* idx, const int32_t* map,
+                                        int k, float ef_decay, bf16_t* U, float* sumsq, hipStream_t st);
 // Row slabs the column-sum path of launch_dion2_accumulate wants for this shape (1 = no scratch).
 int dion2_acc_slabs(int n_mat, int rows, int cols);
 hipError_t launch_dion2_topk(const float* norms, int n_mat, int dim, int k, int32_t* idx,

@@ -905,7 +905,7 @@ __global__ __launch_bounds__(256) void dion2_acc_cols_kernel(PtrTab G, PtrTab M,
                                      (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
-template <int B, typename GT, typename MT, bool NT>
+template <int B, typename GT, typename MT, bool NT, bool STORE>
 static __device__ __forceinline__ void acc_cols_batch(const GT* __restrict__ g, MT* __restrict__ m, int64_t i, int cols,
                                                       float4& s) {
   float gv[B][4], mv[B][4];
@@ -918,7 +918,7 @@ static __device__ __forceinline__ void acc_cols_batch(const GT* __restrict__ g, 
   for (int b = 0; b < B; ++b) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) mv[b][e] = st_round<MT>(__fadd_rn(mv[b][e], gv[b][e]));
-    st_store4<MT, NT>(m, (i >> 2) + (int64_t)b * cols, mv[b]);
+    if (STORE) st_store4<MT, NT>(m, (i >> 2) + (int64_t)b * cols, mv[b]);
     s.x += fabsf(mv[b][0]);
     s.y += fabsf(mv[b][1]);
     s.z += fabsf(mv[b][2]);
@@ -931,7 +931,8 @@ static __device__ __forceinline__ void acc_cols_batch(const GT* __restrict__ g, 
 // gradients: 844 us (4.8 TB/s) with four -> 717 us (5.6 TB/s); 12 x (3072 x 768) 52 us either way).
 // With gridDim.z row slabs the block writes its slab's partial sums to out[(slab*n_mat + mat)*cols]
 // (n_mat = gridDim.y); dion2_sum_slabs_kernel adds the slabs in a fixed order.
-template <typename GT, typename MT, bool NT>
+// STORE false: the norms alone, M stays as it is (dion2_add_gather_cols_kernel updates it).
+template <typename GT, typename MT, bool NT, bool STORE = true>
 __global__ __launch_bounds__(256) void dion2_acc_cols_vec_kernel(PtrTab G, PtrTab M, int mats_per_ptr,
                                                                  int rows, int cols, int slab_rows,
                                                                  float* __restrict__ norms) {
@@ -949,8 +950,8 @@ __global__ __launch_bounds__(256) void dion2_acc_cols_vec_kernel(PtrTab G, PtrTa
   if (c < cols) {
     int r = r0 + ry;
     // eight rows' loads in flight, added in row order
-    for (; r + 28 < r1; r += 32) acc_cols_batch<8, GT, MT, NT>(g, m, (int64_t)r * cols + c, cols, s);
-    for (; r < r1; r += 4) acc_cols_batch<1, GT, MT, NT>(g, m, (int64_t)r * cols + c, cols, s);
+    for (; r + 28 < r1; r += 32) acc_cols_batch<8, GT, MT, NT, STORE>(g, m, (int64_t)r * cols + c, cols, s);
+    for (; r < r1; r += 4) acc_cols_batch<1, GT, MT, NT, STORE>(g, m, (int64_t)r * cols + c, cols, s);
   }
   red[ry][threadIdx.x & 63] = s;
   __syncthreads();
@@ -986,8 +987,9 @@ int dion2_acc_slabs(int n_mat, int rows, int cols) {
 
 hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, int n_mat,
                                    int mats_per_ptr, int rows, int cols, int select_rows,
-                                   float* norms, bool vec4, float* slab_scratch, int slabs,
+                                   float* norms, bool vec4, float* slab_scratch, int slabs, bool store,
                                    hipStream_t st) {
+  if (!store && (select_rows || !vec4)) return hipErrorInvalidValue;
   const bool nt = exceeds_caches((int64_t)n_mat * rows * cols * ((m_dtype == 0 ? 4 : 8) + (g_dtype == 0 ? 2 : 4)));
   // the four (gradient, momentum) dtype pairs; NTV... is empty for kernels without a non-temporal form
 #define ACC_LAUNCH_T(K, GRID, NTV, ...)                                                                 \
@@ -1003,6 +1005,8 @@ hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M
   } while (0)
 #define ACC_NT , true
 #define ACC_T , false
+#define ACC_NT_NORMS , true, false
+#define ACC_T_NORMS , false, false
 #define ACC_LAUNCH(K, GRID, ...)                             \
   do {                                                       \
     if (nt) ACC_LAUNCH_T(K, GRID, ACC_NT, __VA_ARGS__);      \
@@ -1017,7 +1021,9 @@ hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M
     slabs = (rows + slab_rows - 1) / slab_rows;
     float* dst = slabs > 1 ? slab_scratch : norms;
     dim3 grid((cols / 4 + 63) / 64, n_mat, slabs);
-    ACC_LAUNCH(dion2_acc_cols_vec_kernel, grid, G, M, mats_per_ptr, rows, cols, slab_rows, dst);
+    if (store) ACC_LAUNCH(dion2_acc_cols_vec_kernel, grid, G, M, mats_per_ptr, rows, cols, slab_rows, dst);
+    else if (nt) ACC_LAUNCH_T(dion2_acc_cols_vec_kernel, grid, ACC_NT_NORMS, G, M, mats_per_ptr, rows, cols, slab_rows, dst);
+    else ACC_LAUNCH_T(dion2_acc_cols_vec_kernel, grid, ACC_T_NORMS, G, M, mats_per_ptr, rows, cols, slab_rows, dst);
     if (slabs > 1) {
       const int64_t n = (int64_t)n_mat * cols;
       hipLaunchKernelGGL(dion2_sum_slabs_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
@@ -1029,6 +1035,8 @@ hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M
   }
 #undef ACC_NT
 #undef ACC_T
+#undef ACC_NT_NORMS
+#undef ACC_T_NORMS
 #undef ACC_LAUNCH_T
 #undef ACC_LAUNCH
   return hipGetLastError();
@@ -1270,6 +1278,107 @@ __global__ __launch_bounds__(256) void dion2_gather_cols_transposed_kernel(PtrTa
       w[e] = (uint32_t)tile[chunk * 8 + 2 * e][col] | ((uint32_t)tile[chunk * 8 + 2 * e + 1][col] << 16);
     *(uint4*)(ut + (int64_t)(j0 + col) * rows + r0 + chunk * 8) = make_uint4(w[0], w[1], w[2], w[3]);
   }
+}
+
+// The same U^T and decay with M += G in the same pass over whole rows: every element of M is read and written once, in
+// whole lines.  A workgroup takes 64 rows and the columns from its 64 selected ones' first up to the next workgroup's
+// (the outermost to the matrix's edge), both rounded down to 64 columns -- with ranges that ended inside a line the launch
+// below took 1058 us.  It writes the selected columns that fall into its range (at most 127) and one partial sum of their
+// squares; the partial sums of a matrix add up as those of the kernel above do.
+// map [n_mat][cols]: position among the selected, or -1.  cols % 4 == 0, G and M 16-byte aligned, rows % 64 == 0, k % 64 == 0.
+// Bound by HBM.  Beside norms that do not write M this moves 16 bytes an element of an fp32 momentum with bf16 gradients
+// where accumulating first (715 us) and gathering a scattered quarter of every line (754) moved 18: 24 x (8192 x 2048).
+template <typename GT, typename MT, bool NT>
+__global__ __launch_bounds__(256) void dion2_add_gather_cols_kernel(PtrTab G, PtrTab M, int mats_per_ptr, int rows,
+                                                                    int cols, const int32_t* __restrict__ idx,
+                                                                    const int32_t* __restrict__ map, int k,
+                                                                    float ef_decay, bf16_t* __restrict__ U,
+                                                                    float* __restrict__ sumsq) {
+  __shared__ __attribute__((aligned(16))) bf16_t tile[128][72];  // [selected column][row]
+  __shared__ float red[16];
+  const int mat = blockIdx.z, lane = threadIdx.x & 63;
+  const int64_t base = (int64_t)(mat % mats_per_ptr) * rows * cols;
+  const int r0 = blockIdx.y * 64, j0 = blockIdx.x * 64, j1 = j0 + 64;
+  const GT* __restrict__ g = (const GT*)G.p[mat / mats_per_ptr] + base + (int64_t)r0 * cols;
+  MT* __restrict__ m = (MT*)M.p[mat / mats_per_ptr] + base + (int64_t)r0 * cols;
+  const int32_t* id = idx + (int64_t)mat * k;
+  const int c_lo = j0 == 0 ? 0 : id[j0] & ~63, c_hi = j1 == k ? cols : id[j1] & ~63;
+  // selected columns of the range: [s_lo, s_hi); at most 63 of those before a bound's own share its 64 columns
+  const int s_lo = j0 - __popcll(__ballot(j0 > lane && id[j0 > lane ? j0 - 1 - lane : 0] >= c_lo));
+  const int s_hi = j1 == k ? k : j1 - __popcll(__ballot(id[j1 - 1 - lane] >= c_hi));
+  const int q0 = c_lo >> 2;
+  const unsigned nq = (unsigned)((c_hi >> 2) - q0), total = nq * 64;  // groups of four columns a row, in the tile
+  const int4* mp = (const int4*)(map + (int64_t)mat * cols) + q0;
+  constexpr int B = 8;  // groups in flight a thread
+  for (unsigned t0 = threadIdx.x; t0 < total; t0 += B * 256) {
+    float mv[B][4], gv[B][4];
+    int4 slot[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const unsigned t = t0 + b * 256;
+      if (t >= total) continue;
+      const unsigned row = t / nq, grp = t - row * nq;
+      const int64_t i4 = (((int64_t)row * cols) >> 2) + q0 + grp;
+      st_load4<MT, NT>(m, i4, mv[b]);
+      st_load4<GT, NT>(g, i4, gv[b]);
+      slot[b] = mp[grp];
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const unsigned t = t0 + b * 256;
+      if (t >= total) continue;
+      const unsigned row = t / nq, grp = t - row * nq;
+      const int s[4] = {slot[b].x, slot[b].y, slot[b].z, slot[b].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        mv[b][e] = st_round<MT>(__fadd_rn(mv[b][e], gv[b][e]));
+        if (s[e] >= s_lo && s[e] < s_hi) {
+          tile[s[e] - s_lo][row] = f32_to_bf16(mv[b][e]);
+          mv[b][e] = __fmul_rn(mv[b][e], ef_decay);
+        }
+      }
+      st_store4<MT, NT>(m, (((int64_t)row * cols) >> 2) + q0 + grp, mv[b]);
+    }
+  }
+  __syncthreads();
+  bf16_t* ut = U + ((int64_t)mat * k + s_lo) * rows + r0;
+  float ss = 0.f;
+  for (int i = threadIdx.x; i < (s_hi - s_lo) * 8; i += 256) {
+    const int col = i >> 3, chunk = i & 7;
+    const u32x4_t w = *(const u32x4_t*)&tile[col][chunk * 8];
+    *(u32x4_t*)(ut + (int64_t)col * rows + chunk * 8) = w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = __uint_as_float(w[e] << 16), hi = __uint_as_float(w[e] & 0xffff0000u);
+      ss += lo * lo;
+      ss += hi * hi;
+    }
+  }
+  ss = block_sum(ss, red);
+  if (threadIdx.x == 0) sumsq[((int64_t)mat * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = ss;
+}
+
+hipError_t launch_dion2_add_gather_cols(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, int n_mat,
+                                        int mats_per_ptr, int rows, int cols, const int32_t* idx, const int32_t* map,
+                                        int k, float ef_decay, bf16_t* U, float* sumsq, hipStream_t st) {
+  const bool nt = exceeds_caches((int64_t)n_mat * rows * cols * ((m_dtype == 0 ? 2 : 4) + (g_dtype == 0 ? 2 : 4)));
+  const dim3 grid(k / 64, rows / 64, n_mat);
+#define ADDG_LAUNCH(GT, MT)                                                                                           \
+  do {                                                                                                                \
+    if (nt)                                                                                                           \
+      hipLaunchKernelGGL((dion2_add_gather_cols_kernel<GT, MT, true>), grid, dim3(256), 0, st, G, M, mats_per_ptr, rows, \
+                         cols, idx, map, k, ef_decay, U, sumsq);                                                      \
+    else                                                                                                              \
+      hipLaunchKernelGGL((dion2_add_gather_cols_kernel<GT, MT, false>), grid, dim3(256), 0, st, G, M, mats_per_ptr,    \
+                         rows, cols, idx, map, k, ef_decay, U, sumsq);                                                \
+  } while (0)
+  if (g_dtype == 0) {
+    if (m_dtype == 0) ADDG_LAUNCH(bf16_t, bf16_t); else ADDG_LAUNCH(bf16_t, float);
+  } else {
+    if (m_dtype == 0) ADDG_LAUNCH(float, bf16_t); else ADDG_LAUNCH(float, float);
+  }
+#undef ADDG_LAUNCH
+  return hipGetLastError();
 }
 
 hipError_t launch_dion2_gather(const PtrTab& M, int m_dtype, int n_mat, int mats_per_ptr, int rows, int cols,

@@ -561,9 +561,18 @@ def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_d
     st = _stream_handle(dev)
     sbytes = lib.dion_dion2_accumulate_scratch_bytes(n_mat, rows, cols, select_dim)
     scratch = torch.empty(sbytes, dtype=torch.uint8, device=dev) if sbytes else None
-    check(lib.dion_dion2_accumulate(gp, _dtype_code(G[0], "G"), mp, mcode, n, mats_per_ptr, rows, cols, select_dim,
-                                    norms.data_ptr(), scratch.data_ptr() if sbytes else None, sbytes, st),
-          "dion2_accumulate")
+    gcode = _dtype_code(G[0], "G")
+    # Columns of tall matrices in the prepared form: the norms first, without a write of M; the pass that gathers the
+    # selected columns, and would touch every line of M for them anyway, adds G.
+    add_late = prepared and select_dim == -1 and rows > k and cols % 4 == 0 and \
+        not any(p & 15 for p in gp) and not any(p & 15 for p in mp)
+    if add_late:
+        check(lib.dion_dion2_column_norms(gp, gcode, mp, mcode, n, mats_per_ptr, rows, cols, norms.data_ptr(),
+                                          scratch.data_ptr() if sbytes else None, sbytes, st), "dion2_column_norms")
+    else:
+        check(lib.dion_dion2_accumulate(gp, gcode, mp, mcode, n, mats_per_ptr, rows, cols, select_dim,
+                                        norms.data_ptr(), scratch.data_ptr() if sbytes else None, sbytes, st),
+              "dion2_accumulate")
     check(lib.dion_dion2_topk(norms.data_ptr(), n_mat, dim, k, idx.data_ptr(), imap.data_ptr(), st),
           "dion2_topk")
     if prepared:
@@ -573,6 +582,11 @@ def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_d
         sr, sc = (k, cols) if select_dim == -2 else (rows, k)
         U = U.view(n_mat, min(sr, sc), max(sr, sc))
         sumsq = torch.empty(n_mat, blocks, dtype=torch.float32, device=dev)
+        if add_late:
+            check(lib.dion_dion2_add_gather_columns(gp, gcode, mp, mcode, n, mats_per_ptr, rows, cols, idx.data_ptr(),
+                                                    imap.data_ptr(), k, float(ef_decay), U.data_ptr(), sumsq.data_ptr(),
+                                                    st), "dion2_add_gather_columns")
+            return U, idx, imap, sumsq
         check(lib.dion_dion2_gather_prepared(mp, mcode, n, mats_per_ptr, rows, cols, select_dim, idx.data_ptr(), k,
                                              float(ef_decay), U.data_ptr(), sumsq.data_ptr(), st),
               "dion2_gather_prepared")

@@ -318,6 +318,18 @@ int dion_dion2_gather_prepared(const uint64_t* M_ptrs, int m_dtype, int n, int m
                                int select_dim, const int32_t* idx, int k, float ef_decay, void* U_sel,
                                float* sumsq, void* stream);
 
+/* The tall form (select_dim -1, rows > k) with M += G in the gather: dion_dion2_column_norms gives the norms of
+ * dion_dion2_accumulate, bit for bit, without writing M, and dion_dion2_add_gather_columns then adds G, writes U_sel
+ * and sumsq as dion_dion2_gather_prepared does and decays the selected columns, in one pass.  M ends as after
+ * dion_dion2_accumulate and dion_dion2_gather_prepared.  idx and map as dion_dion2_topk writes them; cols a multiple
+ * of 4, G, M and map 16-byte aligned.  Replaces dion/dion2.py:439-545. */
+int dion_dion2_column_norms(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, int n,
+                            int mats_per_ptr, int rows, int cols, float* norms, void* scratch, size_t scratch_bytes,
+                            void* stream);
+int dion_dion2_add_gather_columns(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, int n,
+                                  int mats_per_ptr, int rows, int cols, const int32_t* idx, const int32_t* map, int k,
+                                  float ef_decay, void* U_sel, float* sumsq, void* stream);
+
 /* Dion2 fused weight decay + selective update, single rounding:
  *   x = (1 - lr wd) x - b u[map]   on selected slices,  x = (1 - lr wd) x elsewhere
  *   b = lr * adj_ratio, or (*adj_lr_dev) * adj_ratio when adj_lr_dev (nullable, device fp32 scalar:
