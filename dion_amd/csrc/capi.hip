@@ -196,9 +196,9 @@ struct PostSpec {
   int cautious;
 };
 
-// per-head regime: whole iteration resident in LDS, one workgroup per matrix, no workspace.  The Gram
+// per-head regime: whole iteration in the registers of one workgroup per matrix, no workspace.  The Gram
 // flag changes nothing here: the recurrence saves memory traffic of rectangular GEMMs, and a matrix
-// that never leaves LDS has none; the standard iteration applies the same polynomial.
+// that never leaves its workgroup has none; the standard iteration applies the same polynomial.
 bool ns_small_path(int batch, int rows, int cols, int flags, int n_iters) {
   (void)flags;
   return n_iters <= kMaxSmallIters && ns_small_fits(batch, rows, cols);
@@ -214,7 +214,7 @@ bool ns_padded(int batch, int rows, int cols, int flags, int n_iters, int* mp = 
   return pl.mp != pl.m || pl.np != pl.n;
 }
 
-// The update rides on the last GEMM: at least one iteration, not the LDS-resident kernel.  (Padded matrices had a separate
+// The update rides on the last GEMM: at least one iteration, not the small-matrix kernel.  (Padded matrices had a separate
 // update pass, without a limit to the number of parameters, before they fused: past what a launch list holds they
 // still take it.)
 constexpr int kMaxFusedPadded = 4096;
@@ -225,13 +225,20 @@ bool ns_update_fuses(int batch, int rows, int cols, int flags, int n_iters) {
 
 // A prepared input (short side along rows, unnormalised, with partial sums of squares) is taken when
 // the matrices fill whole tiles -- no padding, so the input can be the first GEMMs' operand as it lies --
-// outside the LDS-resident kernel and with at least one iteration to carry the normalisation.
-bool ns_accepts_prepared(int batch, int rows, int cols, int flags, int n_iters) {
+// and there is at least one iteration to carry the normalisation.  Taken, not advised, where the small-matrix kernel
+// runs plain calls of the batch and a single such matrix would go to the GEMMs (from 65 rows or 1025 columns on): a
+// caller who prepares those runs the GEMMs.
+bool ns_takes_prepared(int batch, int rows, int cols, int flags, int n_iters) {
   if (batch <= 0 || batch > 65535 || rows <= 0 || cols <= 0 || n_iters <= 0) return false;
-  if (ns_small_path(batch, rows, cols, flags, n_iters)) return false;
+  if (ns_small_path(1, rows, cols, flags, n_iters)) return false;
   if (((int64_t)rows * cols) % 4096) return false;
   const NsPlan pl = make_plan(batch, rows, cols, flags);
   return pl.mp == pl.m && pl.np == pl.n;
+}
+
+// ... and the GEMMs are also what a plain call of these matrices runs.
+bool ns_accepts_prepared(int batch, int rows, int cols, int flags, int n_iters) {
+  return !ns_small_path(batch, rows, cols, flags, n_iters) && ns_takes_prepared(batch, rows, cols, flags, n_iters);
 }
 
 // One kernel launch of a planned call.
@@ -335,7 +342,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
   const bool padded = ns_padded(batch, rows, cols, flags, n_iters, &pad_m, &pad_n);
   if (sumsq) {
     if (in_padded) call.in_hi = call.in_lo + (size_t)batch * pad_m * pad_n * 2;
-    if (!(in_padded ? padded : ns_accepts_prepared(batch, rows, cols, flags, n_iters)) || in_dtype != DION_BF16 ||
+    if (!(in_padded ? padded : ns_takes_prepared(batch, rows, cols, flags, n_iters)) || in_dtype != DION_BF16 ||
         sumsq_blocks <= 0)
       return fail(DION_E_INVALID,
                   "dion_ns_orthogonalize_prepared: %d x (%d x %d), %d iterations does not take a prepared input "
@@ -345,7 +352,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     call.sq_lo = (const char*)sumsq;
     call.sq_hi = call.sq_lo + (size_t)batch * sumsq_blocks * 4;
   }
-  if (ns_small_path(batch, rows, cols, flags, n_iters)) {
+  if (!sumsq && ns_small_path(batch, rows, cols, flags, n_iters)) {
     NsStep s = blank_step(NsStep::kSmall, "small-matrix Newton-Schulz");
     s.in = in;
     s.in_dtype = in_dtype;
@@ -937,9 +944,11 @@ extern "C" int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* 
 
 extern "C" size_t dion_ns_update_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  const size_t ns = ns_small_path(batch, rows, cols, flags, n_iters) ? 0 : align256(make_plan(batch, rows, cols, flags).total);
-  if (ns_update_fuses(batch, rows, cols, flags, n_iters)) return ns;
-  return ns + align256((size_t)batch * rows * cols * 2);
+  const bool small = ns_small_path(batch, rows, cols, flags, n_iters);
+  const size_t plan = align256(make_plan(batch, rows, cols, flags).total), tail = align256((size_t)batch * rows * cols * 2);
+  if (small && ns_takes_prepared(batch, rows, cols, flags, n_iters)) return plan > tail ? plan : tail;
+  if (ns_update_fuses(batch, rows, cols, flags, n_iters)) return plan;
+  return (small ? 0 : plan) + tail;
 }
 
 extern "C" int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X_ptrs, int x_dtype,
@@ -966,7 +975,7 @@ extern "C" int dion_ns_orthogonalize_update(const void* in, int in_dtype, const 
     return ns_run(in, in_dtype, nullptr, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset,
                   workspace, workspace_bytes, stream, &ps);
   }
-  // the LDS-resident kernel: orthogonalize into the tail of the workspace (the
+  // the small-matrix kernel: orthogonalize into the tail of the workspace (the
   // last align256(batch * rows * cols * 2) bytes of what dion_ns_update_workspace_bytes reports),
   // then the plain update pass
   const size_t tail = align256((size_t)batch * rows * cols * 2);
@@ -1011,7 +1020,7 @@ static int update_prepared(const char* who, bool in_padded, const void* in, cons
   if (!X_ptrs || !lr_dev || !sumsq) return fail(DION_E_INVALID, "%s: null argument", who);
   for (int i = 0; i < n_ptrs; ++i)
     if (!X_ptrs[i]) return fail(DION_E_INVALID, "%s: parameter %d is null", who, i);
-  if (!(in_padded ? ns_padded(batch, rows, cols, flags, n_iters) : ns_accepts_prepared(batch, rows, cols, flags, n_iters)))
+  if (!(in_padded ? ns_padded(batch, rows, cols, flags, n_iters) : ns_takes_prepared(batch, rows, cols, flags, n_iters)))
     return fail(DION_E_INVALID, "%s: %d x (%d x %d) does not take a prepared input (see %s)", who, batch, rows, cols,
                 in_padded ? "dion_ns_padded_extents" : "dion_ns_accepts_prepared");
   const PostSpec ps = {X_ptrs, x_dtype, n_ptrs, mats_per_ptr, lr_dev, adj_ratio, wd_dev, wd_host, cautious};
@@ -1080,7 +1089,7 @@ static int plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters, 
   if (int rc = check_state_dtype("dion_ns_plan_audit", "x_dtype", x_dtype)) return rc;
   float coeffs[48];
   for (int i = 0; i < 48; ++i) coeffs[i] = 1.0f;
-  const bool small = ns_small_path(batch, rows, cols, flags, n_iters);
+  const bool small = !prepared && ns_small_path(batch, rows, cols, flags, n_iters);
   const size_t ws_bytes = small ? 0 : make_plan(batch, rows, cols, flags).total;
   // disjoint synthetic regions, 1 TiB apart
   char* const base = (char*)(uintptr_t)0x100000000000ull;
@@ -1094,7 +1103,9 @@ static int plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters, 
   std::vector<uint64_t> xp;
   PostSpec ps;
   // (with_update == 1 asks about matrices that fill whole tiles; 2 about any)
-  const bool fused = with_update && ns_update_fuses(batch, rows, cols, flags, n_iters) &&
+  const bool fused = with_update &&
+                     (prepared ? ns_takes_prepared(batch, rows, cols, flags, n_iters)
+                               : ns_update_fuses(batch, rows, cols, flags, n_iters)) &&
                      (with_update == 2 || !ns_padded(batch, rows, cols, flags, n_iters));
   if (with_update && !fused)
     return fail(DION_E_INVALID, "dion_ns_plan_audit: this shape does not take the fused update");

@@ -121,8 +121,8 @@ int dion_ns_plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters,
  * `muon_update_newton_schulz` + `muon_update_post_orthogonalize`, dion/muon.py:249-277.
  * in: [n_ptrs * mats_per_ptr, rows, cols] as for dion_ns_orthogonalize; X_ptrs: host array of n_ptrs
  * device pointers, each to mats_per_ptr contiguous [rows, cols] matrices of x_dtype, updated in place.
- * With more than 64 rows or columns on the short side the last GEMM applies the update in its epilogue;
- * otherwise the library runs the two passes itself, through the tail of the workspace.  Workspace size from
+ * The last GEMM applies the update in its epilogue; where one workgroup takes a whole matrix instead (short sides up
+ * to 128) the library runs the two passes itself, through the tail of the workspace.  Workspace size from
  * dion_ns_update_workspace_bytes (same flags and n_iters).  lr / weight decay as for dion_muon_post. */
 size_t dion_ns_update_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters);
 int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X_ptrs, int x_dtype, int n_ptrs,
@@ -142,9 +142,11 @@ int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X
  * parameters), as in dion_ns_orthogonalize; all other arguments as there.
  *   in     bf16 [batch, m, n], m = min(rows, cols), n = max(rows, cols), 16-byte aligned
  *   sumsq  fp32 [batch, sumsq_blocks]; the sum of row b is ||in[b]||_F^2
- * Taken only when dion_ns_accepts_prepared() returns 1: rows and cols multiples of the GEMM tile
- * (no padding), rows * cols a multiple of 4096, at least one iteration, more than 64 rows or columns
- * on the short side, at most 65535 matrices; DION_E_INVALID otherwise (use dion_ns_orthogonalize).
+ * Taken when dion_ns_accepts_prepared() returns 1: rows and cols multiples of the GEMM tile
+ * (no padding), rows * cols a multiple of 4096, at least one iteration, at most 65535 matrices, and not a batch whose
+ * plain calls give every matrix to one workgroup; DION_E_INVALID otherwise (use dion_ns_orthogonalize).  Such a batch
+ * of whole-tile matrices with more than 64 rows or columns on the short side (16 and more matrices of 128 x up to 1024) is
+ * taken all the same: it runs the GEMMs, slower than the plain call.
  * Results differ from dion_ns_orthogonalize in the last bf16 bit (X0 is not rounded to bf16 once
  * more before the first products).
  * ------------------------------------------------------------------------------------------ */
@@ -165,8 +167,8 @@ int dion_ns_orthogonalize_update_prepared(const void* in, const float* sumsq, in
 /* The same for matrices that do not fill whole tiles: the producer (dion_muon_pre_padded) writes them into the
  * zero-padded form they are iterated in -- bf16 [batch, mp, np], short side along rows, zero outside
  * min(rows, cols) x max(rows, cols), 16-byte aligned -- with partial sums of squares as above.
- * dion_ns_padded_extents returns 1 and the extents when such a call pads its matrices (at least one iteration, more
- * than 64 rows or columns on the short side, at most 4096 matrices), 0 otherwise.  Results differ from
+ * dion_ns_padded_extents returns 1 and the extents when such a call pads its matrices (at least one iteration, at most
+ * 4096 matrices, not a batch whose plain calls give every matrix to one workgroup), 0 otherwise.  Results differ from
  * dion_ns_orthogonalize on the same matrices by nothing: it makes the same copy itself. */
 int dion_ns_padded_extents(int batch, int rows, int cols, int flags, int n_iters, int* mp, int* np);
 int dion_ns_orthogonalize_padded(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch, int rows,

@@ -97,12 +97,37 @@ def test_prepared_orthogonalization_vs_exact_and_unprepared(variant, shape):
     assert float(per.max()) <= float(per_plain.max()) * 1.15 + 1e-3
 
 
+@pytest.mark.parametrize("shape", [(24, 128, 1024), (24, 256, 128)])
+def test_prepared_input_of_matrices_the_small_kernel_takes(shape):
+    """A batch whose plain calls run the small-matrix kernel: the prepared form runs the GEMMs, with the bits of a batch
+    that is too small for that kernel."""
+    from dion_amd import newton_schulz as ns
+    from dion_amd import ops
+
+    batch, rows, cols = shape
+    assert not ops.ns_accepts_prepared(batch, rows, cols, 5)
+    gen = torch.Generator().manual_seed(batch + rows + cols)
+    G = (torch.randn(shape, generator=gen) * 0.02).to(torch.bfloat16).to(DEV)
+    U = (G.mT if rows > cols else G).contiguous()
+    sumsq = U.float().pow(2).sum(dim=2).contiguous()
+    out = ns.orthogonalize_prepared(ns.polar_express, U, sumsq, rows, cols, 1e-8)
+    exact = _ns_fp64_on_device(G, oracle.POLAR_EXPRESS_COEFFS, 1.02, 1e-8)
+    per = (out.double() - exact).flatten(1).norm(dim=1) / exact.flatten(1).norm(dim=1)
+    assert float(per.max()) <= 2e-2
+    X = [torch.randn(rows, cols, device=DEV) for _ in range(batch)]
+    want = [x.clone() for x in X]
+    lr = torch.tensor(0.02, device=DEV)
+    ops.ns_orthogonalize_update_prepared(U, sumsq, rows, cols, X, ns.POLAR_EXPRESS_COEFFS, 1.02, 1e-8, lr, 0.5, 0.01)
+    ops.muon_post(want, out, lr, 0.5, 0.01)
+    assert all(torch.equal(a, b) for a, b in zip(X, want))
+
+
 def test_prepared_input_is_refused_where_it_does_not_apply():
     from dion_amd import newton_schulz as ns
     from dion_amd import ops
 
     assert not ops.ns_accepts_prepared(4, 96, 160, 5)        # padded to the tile
-    assert not ops.ns_accepts_prepared(4, 64, 768, 5)        # the LDS-resident small-matrix kernel
+    assert not ops.ns_accepts_prepared(4, 64, 768, 5)        # the small-matrix kernel
     assert not ops.ns_accepts_prepared(4, 256, 512, 0)       # nothing to carry the normalisation
     assert ops.ns_accepts_prepared(4, 256, 512, 5)
     U = torch.zeros(4, 128, 160, dtype=torch.bfloat16, device=DEV)

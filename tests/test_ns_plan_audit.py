@@ -150,6 +150,20 @@ def test_prepared_input_plans(shape):
         assert _audit_prepared(lib, shape, 5, flags, ws=4096) == -1
 
 
+@pytest.mark.parametrize("shape", [(16, 128, 256), (24, 128, 1024), (20, 768, 128)])
+def test_prepared_input_of_matrices_the_small_kernel_takes(shape):
+    """Where plain calls of a batch run the small-matrix kernel, a prepared input is not advised but still taken: the GEMMs
+    of a batch too small for that kernel, within the workspace the library reports."""
+    lib = _lib.load()
+    b, r, c = shape
+    assert not lib.dion_ns_accepts_prepared(b, r, c, 0, 5) and lib.dion_ns_accepts_prepared(15, r, c, 0, 5)
+    assert _audit(lib, shape, 5, 0) == 1
+    for with_update in (0, 1):
+        n = _audit_prepared(lib, shape, 5, 0, with_update=with_update)
+        assert n == _audit_prepared(lib, (15, r, c), 5, 0, with_update=with_update) > 1
+    assert lib.dion_ns_update_workspace_bytes(b, r, c, 0, 5) >= lib.dion_ns_workspace_bytes(b, r, c, 0)
+
+
 @pytest.mark.parametrize("shape", [s for s in RAGGED_SHAPES if min(s[1:]) > 64 and (s[1] % 128 or s[2] % 128)])
 def test_padded_plans_with_the_update(shape):
     """Matrices with padding: one copy in, the update in the last product, stored extents without the padding."""
