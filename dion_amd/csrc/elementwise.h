@@ -10,7 +10,7 @@ namespace dion {
 // 356 us, 2 x (32000 x 1000) bf16, 0.51 GB, 181 -> 166; 2 x (32000 x 320) fp32, 0.29 GB, would go from 87 to 98.
 inline bool exceeds_caches(int64_t bytes) { return bytes >= (384LL << 20); }
 
-// Coefficient schedule passed by value to the LDS-resident small-matrix kernel.
+// Coefficient schedule passed by value to the small-matrix kernel.
 constexpr int kMaxSmallIters = 8;
 struct NsCoeffs {
   int n;

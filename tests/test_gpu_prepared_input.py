@@ -99,8 +99,9 @@ def test_prepared_orthogonalization_vs_exact_and_unprepared(variant, shape):
 
 @pytest.mark.parametrize("shape", [(24, 128, 1024), (24, 256, 128)])
 def test_prepared_input_of_matrices_the_small_kernel_takes(shape):
-    """A batch whose plain calls run the small-matrix kernel: the prepared form runs the GEMMs, with the bits of a batch
-    that is too small for that kernel."""
+    """A batch whose plain calls run the small-matrix kernel: the prepared form runs the GEMMs.  The
+    reference is float64; the bound is the error of the same iteration in float32 with A, B and X rounded to bf16 where the
+    kernels round them (factor 1.5: the sums run in another order), which these steep polynomials carry to about 2e-2."""
     from dion_amd import newton_schulz as ns
     from dion_amd import ops
 
@@ -112,8 +113,14 @@ def test_prepared_input_of_matrices_the_small_kernel_takes(shape):
     sumsq = U.float().pow(2).sum(dim=2).contiguous()
     out = ns.orthogonalize_prepared(ns.polar_express, U, sumsq, rows, cols, 1e-8)
     exact = _ns_fp64_on_device(G, oracle.POLAR_EXPRESS_COEFFS, 1.02, 1e-8)
-    per = (out.double() - exact).flatten(1).norm(dim=1) / exact.flatten(1).norm(dim=1)
-    assert float(per.max()) <= 2e-2
+    same = U.float()
+    same = same / (same.flatten(1).norm(dim=1)[:, None, None] * 1.02 + 1e-8)
+    for a, b, c in oracle.POLAR_EXPRESS_COEFFS:
+        A = (same @ same.mT.contiguous()).bfloat16().float()
+        B = (b * A + c * (A @ A) + a * torch.eye(A.shape[-1], device=DEV)).bfloat16().float()
+        same = (B @ same).bfloat16().float()
+    per = lambda t: ((t.double() - exact).flatten(1).norm(dim=1) / exact.flatten(1).norm(dim=1)).max()
+    assert float(per(out)) <= 1.5 * float(per(same.mT if rows > cols else same)) + 1e-4
     X = [torch.randn(rows, cols, device=DEV) for _ in range(batch)]
     want = [x.clone() for x in X]
     lr = torch.tensor(0.02, device=DEV)
