@@ -28,7 +28,8 @@ constexpr int kMaxLds = 160 * 1024 - 1024;  // dynamic LDS of one workgroup; the
 //
 // What bounds it, 432 x (64 x 768), 43 us: 17 us are the 84 MB in and out (5 TB/s, no iteration), 4.7 us an iteration of
 // two matrices on one CU, of which 2.8 are MFMA time (the turning products are a quarter of it); the rest is the latency
-// of three barriers and A's partial sums through LDS.  The form with X in LDS and one workgroup per CU took 60.
+// of three barriers and A's partial sums through LDS.  The form with X in LDS and one workgroup per CU took 60 on the same box
+// (38.7 against 55.0 us, call by call, on another).
 // 256 x (64 x 2048) 76 us, 300 x (128 x 768) 135, 200 x (80 x 1000) 54, 1000 x (128 x 1024) 453, where the GEMM chain on
 // matrices padded to 128 rows took 1074, 724, 296 and 2626; 16 x (128 x 256) 42 against 90.
 // ------------------------------------------------------------------------------------------
