@@ -54,6 +54,7 @@ SIGNATURES = {
                                                     c_int, _f32p, c_int, c_float, c_float, c_int, c_int, c_void_p,
                                                     c_float, c_void_p, c_float, c_int, c_void_p, c_size_t,
                                                     c_void_p]),
+    "dion_ns_plan_audit_overlap": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64]),
     "dion_ns_plan_audit_prepared": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                             c_size_t]),
     "dion_gemm_tile_edge": (c_int, [c_int, c_int, c_int, c_int]),

@@ -204,6 +204,22 @@ bool ns_small_path(int batch, int rows, int cols, int flags, int n_iters) {
   return n_iters <= kMaxSmallIters && ns_small_fits(batch, rows, cols);
 }
 
+bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+  return (const char*)a < (const char*)b + b_bytes && (const char*)b < (const char*)a + a_bytes;
+}
+
+// Whether the small-matrix kernel may run a call with these buffers.  Its workgroups do not wait for each other: one
+// stores its result while others have not read their matrices yet.  A bf16 call in place is sound all the same, a
+// workgroup holds its whole matrix before it stores; where `out` overlaps `in` in any other way the GEMMs take the call,
+// which copy such an input first.  (Short sides up to 64 with long sides up to 1024 run here at any batch: a call of
+// those has disjoint buffers or is in place in bf16.)
+bool ns_small_buffers(const void* in, int in_dtype, const void* out, int batch, int rows, int cols, int flags,
+                      int n_iters) {
+  const size_t n = (size_t)batch * rows * cols;
+  if (!out || !overlap(in, n * (in_dtype == DION_BF16 ? 2 : 4), out, n * 2)) return true;
+  return (in == out && in_dtype == DION_BF16) || ns_small_path(1, rows, cols, flags, n_iters);
+}
+
 // The matrices do not fill whole tiles: they are iterated in zero-padded copies, mp x np each.
 bool ns_padded(int batch, int rows, int cols, int flags, int n_iters, int* mp = nullptr, int* np = nullptr) {
   if (batch <= 0 || batch > 65535 || rows <= 0 || cols <= 0 || n_iters <= 0) return false;
@@ -338,12 +354,14 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     call.n_ptrs = post->n_ptrs;
     call.x_bytes = (size_t)post->mats_per_ptr * mat_elems * (post->x_dtype == DION_BF16 ? 2 : 4);
   }
-  int pad_m = 0, pad_n = 0;
-  const bool padded = ns_padded(batch, rows, cols, flags, n_iters, &pad_m, &pad_n);
+  const bool small = !sumsq && ns_small_path(batch, rows, cols, flags, n_iters) &&
+                     ns_small_buffers(in, in_dtype, out, batch, rows, cols, flags, n_iters);
   if (sumsq) {
+    int pad_m = 0, pad_n = 0;
+    const bool takes = in_padded ? ns_padded(batch, rows, cols, flags, n_iters, &pad_m, &pad_n)
+                                 : ns_takes_prepared(batch, rows, cols, flags, n_iters);
     if (in_padded) call.in_hi = call.in_lo + (size_t)batch * pad_m * pad_n * 2;
-    if (!(in_padded ? padded : ns_takes_prepared(batch, rows, cols, flags, n_iters)) || in_dtype != DION_BF16 ||
-        sumsq_blocks <= 0)
+    if (!takes || in_dtype != DION_BF16 || sumsq_blocks <= 0)
       return fail(DION_E_INVALID,
                   "dion_ns_orthogonalize_prepared: %d x (%d x %d), %d iterations does not take a prepared input "
                   "(see dion_ns_accepts_prepared)", batch, rows, cols, n_iters);
@@ -352,7 +370,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
     call.sq_lo = (const char*)sumsq;
     call.sq_hi = call.sq_lo + (size_t)batch * sumsq_blocks * 4;
   }
-  if (!sumsq && ns_small_path(batch, rows, cols, flags, n_iters)) {
+  if (small) {
     NsStep s = blank_step(NsStep::kSmall, "small-matrix Newton-Schulz");
     s.in = in;
     s.in_dtype = in_dtype;
@@ -398,15 +416,16 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
   float* inv = (float*)w; w += pl.inv_bytes;
 
   const int mp = pl.mp, np = pl.np;
+  const bool padded = n_iters > 0 && (mp != pl.m || np != pl.n);
   const int64_t sX = (int64_t)mp * np, sA = (int64_t)mp * mp;
   // An input that fills whole tiles is not scaled on its way in either: a wide bf16 one is read by the first
   // GEMMs where it lies, any other is copied (rounded to bf16, transposed if tall) value for value, and the
   // normalisation rides on the first two GEMMs as for a prepared input -- one pass over a wide bf16 input instead
   // of two, and the same arithmetic whichever way (orientation, fp32 or bf16) a matrix is handed over.
   const bool self_prep = !sumsq && aligned16((uint64_t)(uintptr_t)in) &&
-                         ns_accepts_prepared(batch, rows, cols, flags, n_iters);
+                         ns_takes_prepared(batch, rows, cols, flags, n_iters);
   // (not when `out` overlaps `in`: the copy is then what keeps a caller's in-place call working)
-  const bool aliased = out && call.out_lo < call.in_hi && call.in_lo < call.out_hi;
+  const bool aliased = out && overlap(call.in_lo, call.in_hi - call.in_lo, call.out_lo, call.out_hi - call.out_lo);
   const bool in_place = self_prep && !pl.tall && in_dtype == DION_BF16 && !aliased;
   const bool copy_first = self_prep && pl.tall;
   // A matrix that needs padding is copied, rounded to bf16 and unscaled, into its padded form; the copy delivers the
@@ -804,12 +823,13 @@ int ns_audit(const NsCall& call) {
         const size_t es = s.in_dtype == DION_BF16 ? 2 : 4;
         if (!rd(s.in, (size_t)s.batch * s.R * s.C * es)) bad = "input";
         else if (!wr(s.dst, (size_t)s.batch * s.R * s.C * 2)) bad = "output";
+        else if (!ns_small_buffers(s.in, s.in_dtype, s.dst, s.batch, s.R, s.C, 0, s.co.n)) bad = "unread input";
         break;
       }
     }
     if (bad)
-      return fail(DION_E_INVALID, "dion_ns_orthogonalize: launch %d (%s) would access its %s outside the call's buffers",
-                  idx, s.what, bad);
+      return fail(DION_E_INVALID, "dion_ns_orthogonalize: launch %d (%s) would access its %s outside the call's buffers%s",
+                  idx, s.what, bad, s.kind == NsStep::kSmall ? " or overwrite it" : "");
   }
   return DION_OK;
 }
@@ -926,7 +946,8 @@ extern "C" int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* 
                                             float eps, int flags, int gram_reset, void* stream) {
   size_t need = 0;
   if (batch > 0 && rows > 0 && cols > 0 && !(flags & ~DION_NS_GRAM) && n_iters >= 0 &&
-      !ns_small_path(batch, rows, cols, flags, n_iters))
+      !(ns_small_path(batch, rows, cols, flags, n_iters) &&
+        ns_small_buffers(in, in_dtype, out, batch, rows, cols, flags, n_iters)))
     need = make_plan(batch, rows, cols, flags).total;
   if (need > (size_t)DION_NS_STATIC_SCRATCH_BYTES)
     return fail(DION_E_WORKSPACE,
@@ -1083,19 +1104,20 @@ extern "C" int dion_gemm_tile_edge(int batch, int m, int n, int symmetric) {
 // is checked before its first launch.  audit_ws_bytes > 0 checks against a workspace of that size
 // instead of the size the plan was laid out for.
 static int plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters, int flags, int gram_reset,
-                      int with_update, int x_dtype, int mats_per_ptr, size_t audit_ws_bytes, bool prepared) {
+                      int with_update, int x_dtype, int mats_per_ptr, size_t audit_ws_bytes, bool prepared,
+                      const int64_t* out_offset = nullptr) {
   if (batch <= 0 || rows <= 0 || cols <= 0 || n_iters < 0 || n_iters > 16 || mats_per_ptr <= 0)
     return fail(DION_E_INVALID, "dion_ns_plan_audit: bad size");
   if (int rc = check_state_dtype("dion_ns_plan_audit", "x_dtype", x_dtype)) return rc;
   float coeffs[48];
   for (int i = 0; i < 48; ++i) coeffs[i] = 1.0f;
-  const bool small = !prepared && ns_small_path(batch, rows, cols, flags, n_iters);
+  const bool small = !prepared && !out_offset && ns_small_path(batch, rows, cols, flags, n_iters);
   const size_t ws_bytes = small ? 0 : make_plan(batch, rows, cols, flags).total;
   // disjoint synthetic regions, 1 TiB apart
   char* const base = (char*)(uintptr_t)0x100000000000ull;
   const size_t gap = (size_t)1 << 40;
   void* in = base;
-  void* out = base + gap;
+  void* out = out_offset ? base + *out_offset : base + gap;
   void* ws = base + 2 * gap;
   const float* sumsq = prepared ? (const float*)(base + 3 * gap + (gap >> 1)) : nullptr;
   const int sumsq_blocks = prepared ? (int)((int64_t)rows * cols / 4096) : 0;
@@ -1129,6 +1151,13 @@ extern "C" int dion_ns_plan_audit(int batch, int rows, int cols, int in_dtype, i
                                   size_t audit_ws_bytes) {
   return plan_audit(batch, rows, cols, in_dtype, n_iters, flags, gram_reset, with_update, x_dtype, mats_per_ptr,
                     audit_ws_bytes, false);
+}
+
+extern "C" int dion_ns_plan_audit_overlap(int batch, int rows, int cols, int in_dtype, int n_iters, int flags,
+                                          int gram_reset, int64_t out_offset) {
+  if (out_offset < -((int64_t)1 << 40) || out_offset > ((int64_t)1 << 40))
+    return fail(DION_E_INVALID, "dion_ns_plan_audit_overlap: offset");
+  return plan_audit(batch, rows, cols, in_dtype, n_iters, flags, gram_reset, 0, DION_BF16, 1, 0, false, &out_offset);
 }
 
 extern "C" int dion_ns_plan_audit_prepared(int batch, int rows, int cols, int n_iters, int flags, int gram_reset,

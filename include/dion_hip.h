@@ -73,6 +73,8 @@ int dion_ns_line_3(const void* B, const void* X, void* C, int batch, int m, int 
  *   A = X X^T; B = b A + c A A; X = a X + B X   on the orientation with rows <= cols.
  *   (For matrices that fill whole GEMM tiles the division is not a pass of its own: the factor is applied
  *   in the fp32 epilogue of the first two GEMMs, and a wide bf16 `in` is read where it lies.)
+ *   `out` may overlap `in`: the input is then copied first, through the workspace.  Not so for matrices whose short side is
+ *   at most 64 and whose long side is at most 1024: those take disjoint buffers, or a bf16 call in place (out == in).
  *   flags: DION_NS_GRAM selects the Gram-matrix recurrence (call site
  *   dion/megabatch_base.py:77-94) with a restart at iteration `gram_reset` (<=0: none).  Both forms
  *   apply the same polynomial; the recurrence only saves work for long matrices, so it is used
@@ -114,6 +116,9 @@ int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* out, int ba
  * size the plan was laid out for.  No counterpart in the reference. */
 int dion_ns_plan_audit(int batch, int rows, int cols, int in_dtype, int n_iters, int flags, int gram_reset,
                        int with_update, int x_dtype, int mats_per_ptr, size_t audit_ws_bytes);
+/* The same for a dion_ns_orthogonalize call whose `out` lies out_offset bytes behind (or, negative, before) its `in`. */
+int dion_ns_plan_audit_overlap(int batch, int rows, int cols, int in_dtype, int n_iters, int flags, int gram_reset,
+                               int64_t out_offset);
 
 /* Orthogonalization and Muon update in one call: what dion_ns_orthogonalize followed by dion_muon_post
  * (bf16 update, no row_scale) does to the parameters, bit for bit, without the pass that writes the

@@ -176,3 +176,36 @@ def test_padded_plans_with_the_update(shape):
                 assert n > 0, lib.dion_last_error().decode()
                 if not flags or max(shape[1:]) < 3 * min(shape[1:]):
                     assert n == 2 + 3 * 4 + 2 + (b + 63) // 64
+
+
+@pytest.mark.parametrize("shape", [(16, 128, 256), (400, 128, 1024), (24, 1024, 128), (17, 64, 2048), (40, 100, 500)])
+def test_an_output_over_another_matrix_keeps_a_batch_off_the_small_kernel(shape):
+    """One workgroup per matrix stores its result while others have not read their input: a batch of that kernel whose
+    output overlaps the input runs the GEMMs, which copy the input first.  In place in bf16 every workgroup holds its own
+    matrix before it stores."""
+    lib = _lib.load()
+    b, r, c = shape
+    mat = 2 * r * c
+    for in_dtype in (BF16, F32):
+        size = b * mat * (1 if in_dtype == BF16 else 2)
+        audit = lambda offset, n=5: lib.dion_ns_plan_audit_overlap(b, r, c, in_dtype, n, 0, 0, offset)
+        assert audit(size) == 1 and audit(-b * mat) == 1  # side by side
+        assert audit(0) == 1 if in_dtype == BF16 else audit(0) > 1
+        for offset in (mat, -mat, 2, size - 2, 2 - b * mat):
+            if offset % 16 == 0:
+                assert audit(offset) > 1 and audit(offset, 0) > 1, offset
+            else:  # what the GEMM path refuses anyway
+                assert audit(offset) == -1 and "16-byte" in lib.dion_last_error().decode()
+    # the GEMMs need the workspace that is reported for the shape: refused on the host without it
+    import ctypes
+    co = (ctypes.c_float * 15)(*[1.0] * 15)
+    base = 0x100000000000
+    assert lib.dion_ns_orthogonalize(base, BF16, base + mat, b, r, c, co, 5, 1.0, 0.0, 0, 0, None, 0, None) == -2
+    if lib.dion_ns_workspace_bytes(b, r, c, 0) > _lib.DION_NS_STATIC_SCRATCH_BYTES:
+        assert lib.dion_ns_orthogonalize_static(base, BF16, base + mat, b, r, c, co, 5, 1.0, 0.0, 0, 0, None) == -2
+
+
+def test_overlap_of_matrices_that_only_the_small_kernel_takes():
+    lib = _lib.load()
+    for offset in (0, 64 * 768 * 2, -64 * 768 * 2):
+        assert lib.dion_ns_plan_audit_overlap(432, 64, 768, BF16, 5, 0, 0, offset) == 1
