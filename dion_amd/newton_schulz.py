@@ -13,21 +13,21 @@ from . import ops
 
 # Quintic coefficient schedules (a, b, c), one triple per iteration.
 # dion/newton_schulz_triton.py:500-506
-NS5_COEFFS: Sequence[Tuple[float, float, float]] = (
+NS5_COEFFS: Sequence[Tuple[float, float, float]] = ops.Schedule((
     (4.0848, -6.8946, 2.9270),
     (3.9505, -6.3029, 2.6377),
     (3.7418, -5.5913, 2.3037),
     (2.8769, -3.1427, 1.2046),
     (2.8366, -3.0525, 1.2012),
-)
+))
 # dion/polar_express.py:10-16 (safety factor 1.02 baked into all but the last polynomial)
-POLAR_EXPRESS_COEFFS: Sequence[Tuple[float, float, float]] = (
+POLAR_EXPRESS_COEFFS: Sequence[Tuple[float, float, float]] = ops.Schedule((
     (8.156554524902461, -22.48329292557795, 15.878769915207462),
     (4.042929935166739, -2.808917465908714, 0.5000178451051316),
     (3.8916678022926607, -2.772484153217685, 0.5060648178503393),
     (3.285753657755655, -2.3681294933425376, 0.46449024233003106),
     (2.3465413258596377, -1.7097828382687081, 0.42323551169305323),
-)
+))
 POLAR_EXPRESS_SAFETY = 1.02  # dion/polar_express.py:35
 # dion/muon_reference.py:16 (Keller Jordan's fixed quintic)
 KJ_COEFFS: Tuple[float, float, float] = (3.4445, -4.7750, 2.0315)

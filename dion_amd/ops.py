@@ -5,7 +5,6 @@ hands raw device pointers and the current stream to the library, and returns tor
 torch is used for device memory and streams only; all arithmetic happens in the HIP kernels.
 There is no CPU implementation behind these functions: CPU tensors raise.
 """
-import functools
 import math
 from typing import List, Optional, Sequence, Tuple
 
@@ -203,19 +202,29 @@ def ns_orthogonalize(G: Tensor, coeffs: Sequence[Sequence[float]], norm_scale: f
     return out.reshape(shape)
 
 
-def _flat_coeffs(coeffs):
-    return _tuple_coeffs(coeffs) if type(coeffs) is tuple else _list_coeffs(coeffs)
+class Schedule(tuple):
+    """A schedule that stays as it is: ``(a, b, c)`` triples of Python floats, with the arguments the library takes for
+    them (it only reads them) made once."""
+
+    def __new__(cls, triples):
+        self = super().__new__(cls, (tuple(float(v) for v in abc) for abc in triples))
+        self.args = _coeff_args(self)
+        return self
+
+    def __reduce__(self):
+        return Schedule, (tuple(self),)
 
 
-def _list_coeffs(coeffs):
+def _coeff_args(coeffs):
     flat = [float(v) for abc in coeffs for v in abc]
     if len(flat) % 3:
         raise ValueError("coeffs must be (a, b, c) triples")
     return (_lib.ctypes.c_float * max(1, len(flat)))(*flat), len(flat) // 3
 
 
-# the built-in schedules, as the library takes them (which only reads them)
-_tuple_coeffs = functools.lru_cache(maxsize=16)(_list_coeffs)
+def _flat_coeffs(coeffs):
+    # (any other sequence is read anew: its rows may be tensors or lists that the caller changes between calls)
+    return coeffs.args if type(coeffs) is Schedule else _coeff_args(coeffs)
 
 
 def ns_orthogonalize_update(G: Tensor, X: List[Tensor], coeffs: Sequence[Sequence[float]], norm_scale: float,
