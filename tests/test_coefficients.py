@@ -22,6 +22,7 @@ def _values(coeffs):
                                   [tuple(r) for r in ROWS]], ids=["lists", "numpy", "tensors", "tuples"])
 @pytest.mark.parametrize("outer", [tuple, list])
 def test_rows_of_any_kind_are_read_at_every_call(outer, rows):
+    rows = copy.deepcopy(rows)
     coeffs = outer(rows)
     assert _values(coeffs) == ([4.0, -6.5, 2.5, 3.0, -2.0, 1.0], 2)
     if isinstance(rows[0], tuple):
