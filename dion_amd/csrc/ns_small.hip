@@ -30,8 +30,8 @@ constexpr int kMaxLds = 160 * 1024 - 1024;  // dynamic LDS of one workgroup; the
 // two matrices on one CU, of which 2.8 are MFMA time (the turning products are a quarter of it); the rest is the latency
 // of three barriers and A's partial sums through LDS.  The form with X in LDS and one workgroup per CU took 60 on the same box
 // (38.7 against 55.0 us, call by call, on another).
-// 256 x (64 x 2048) 76 us, 300 x (128 x 768) 135, 200 x (80 x 1000) 54, 1000 x (128 x 1024) 453, where the GEMM chain on
-// matrices padded to 128 rows took 1074, 724, 296 and 2626; 16 x (128 x 256) 42 against 90.
+// 256 x (64 x 2048) 53 us, 300 x (128 x 768) 133, 200 x (80 x 1000) 53, 400 x (128 x 1024) 163, where the GEMM chain on
+// matrices padded to 128 rows took many times that (1074, 724, 296 for the first three); 16 x (128 x 256) 41 against 90.
 // ------------------------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) unsigned rx4;
 static __device__ __forceinline__ f32x4 mfma_rx(rx4 a, rx4 b, f32x4 c) {
@@ -144,6 +144,16 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  // Between two passes over x: without this the compiler keeps the values it unpacked for one as floats for the next, twice
+  // the registers of x, and the forms of 96 and 128 registers of x went through scratch memory (up to 444 bytes a lane:
+  // 256 x (64 x 2048) 72 us, 53 without; 256 x (32 x 4096) 73 and 51; 400 x (128 x 1024) 211 and 163).
+  auto settle = [&]() {
+    if constexpr (MT * KC < 24) return;
+#pragma unroll
+    for (int g = 0; g < KC; ++g)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) asm volatile("" : "+v"(x[g][t]));
+  };
   // ---- Frobenius norm, scale
   float ss = 0.f;
 #pragma unroll
@@ -156,6 +166,7 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
         ss += lo * lo;
         ss += hi * hi;
       }
+  settle();
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
   if (lane == 0) red[wave] = ss;
