@@ -5,7 +5,6 @@
 // Follows the same arithmetic as the batched driver (dion/newton_schulz_triton.py:508-522,
 // dion/polar_express.py:30-50): X = bf16(G) / (||.||_F * s + eps); A = X X^T; B = c A A + b A + a I;
 // X = B X, with A, B and X rounded to bf16 once per iteration and fp32 MFMA accumulation.
-//
 #include "elementwise.h"
 
 namespace dion {
@@ -30,8 +29,8 @@ constexpr int kMaxLds = 160 * 1024 - 1024;  // dynamic LDS of one workgroup; the
 // two matrices on one CU, of which 2.8 are MFMA time (the turning products are a quarter of it); the rest is the latency
 // of three barriers and A's partial sums through LDS.  The form with X in LDS and one workgroup per CU took 60 on the same box
 // (38.7 against 55.0 us, call by call, on another).
-// 256 x (64 x 2048) 53 us, 300 x (128 x 768) 133, 200 x (80 x 1000) 53, 400 x (128 x 1024) 163, where the GEMM chain on
-// matrices padded to 128 rows took many times that (1074, 724, 296 for the first three); 16 x (128 x 256) 41 against 90.
+// 256 x (64 x 2048) 55 us, 300 x (128 x 768) 135, 200 x (80 x 1000) 54, 400 x (128 x 1024) 163, where the GEMM chain on
+// matrices padded to 128 rows took many times that (1074, 724, 296 for the first three); 16 x (128 x 256) 42 against 90.
 // ------------------------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(4))) unsigned rx4;
 static __device__ __forceinline__ f32x4 mfma_rx(rx4 a, rx4 b, f32x4 c) {
@@ -62,6 +61,9 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
   constexpr int MR = C::MR, AP = C::AP, GT = C::GT, ST = MT / 2;
   // x takes 4 MT KC registers: past 96 there is no room for a second turned group (256 x (64 x 2048) 76 -> 130 us)
   constexpr bool PIPE = MT * KC <= 24;
+  // Matrices the GEMMs would take otherwise are not rounded after the scaling there, and so not here; the multiplications cost
+  // 5 % of an iteration, which the shapes that never ran anywhere else (up to 64 x 1024) are spared.
+  constexpr bool LATE = MT > 4 || KC * NW > 32;
   constexpr bool BREG = MT <= 4;  // B's fragments stay in registers over the column groups
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   __shared__ float red[NW];
@@ -146,9 +148,9 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
   }
   // Between two passes over x: without this the compiler keeps the values it unpacked for one as floats for the next, twice
   // the registers of x, and the forms of 96 and 128 registers of x went through scratch memory (up to 444 bytes a lane:
-  // 256 x (64 x 2048) 72 us, 53 without; 256 x (32 x 4096) 73 and 51; 400 x (128 x 1024) 211 and 163).
+  // 256 x (64 x 2048) 72 us, 55 without; 256 x (32 x 4096) 73 and 52; 400 x (128 x 1024) 211 and 163).
   auto settle = [&]() {
-    if constexpr (MT * KC < 24) return;
+    if constexpr (!LATE && MT * KC < 24) return;
 #pragma unroll
     for (int g = 0; g < KC; ++g)
 #pragma unroll
@@ -175,13 +177,25 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
 #pragma unroll
   for (int w = 0; w < NW; ++w) total += red[w];
   const float sc = 1.0f / (sqrtf(total) * norm_scale + eps);
+  // LATE: the factor rides on the fp32 sums of the first iteration, squared on A's and once on those of X'.  Scaled here, x is
+  // rounded a second time, which the steep first polynomials carry far (16 x (128 x 256), singular values over 2.5 decades,
+  // Polar-Express, distance to float64: 5.8e-2, and 4.1e-2 without; folded into B before B is rounded, it shifts all of B's
+  // diagonal by one rounding, 64 x (32 x 4096) of Gaussian values 1.23e-2 -> 1.65e-2).  It is scaled here all the same where no
+  // iteration follows and where sums of products of the values as they came would leave the normal range of fp32.
+  const bool late = LATE && co.n > 0 && total > 0x1p-80f && total < 0x1p80f;
+  if (!late) {
 #pragma unroll
-  for (int g = 0; g < KC; ++g)
+    for (int g = 0; g < KC; ++g)
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        x[g][t][e] = pack_bf16x2(__uint_as_float(x[g][t][e] << 16) * sc, __uint_as_float(x[g][t][e] & 0xffff0000u) * sc);
+        for (int e = 0; e < 4; ++e)
+          x[g][t][e] = pack_bf16x2(__uint_as_float(x[g][t][e] << 16) * sc, __uint_as_float(x[g][t][e] & 0xffff0000u) * sc);
+    if (LATE) settle();
+  }
+  // (the same for every lane: say so, the factors live in scalar registers)
+  auto uniform = [](float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v))); };
+  float sa = uniform(late ? sc * sc : 1.0f), sx = uniform(late ? sc : 1.0f);
 
   // group g with lanes along columns: p[h][s] holds, of column tile h, the rows of tiles 2 s and 2 s + 1
   auto turn = [&](int g, rx4 (&p)[2][ST]) {
@@ -231,6 +245,7 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
         f32x4 s = Ps[k * 64 + lane];
 #pragma unroll
         for (int w = 1; w < NW; ++w) s += Ps[(w * GT + k) * 64 + lane];
+        if (LATE) s *= sa;
         const uint32_t w0 = pack_bf16x2(s[0], s[1]), w1 = pack_bf16x2(s[2], s[3]);
         const int row = 16 * t1 + 4 * q, col = 16 * t2 + l16;
         *(uint2*)(As + col * AP + row * 2) = make_uint2(w0, w1);
@@ -295,12 +310,14 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
           f32x4 acc = zero;
 #pragma unroll
           for (int k = 0; k < ST; ++k) acc = mfma_rx(p[g & 1][h][k], b1[k], acc);
+          if (LATE) acc *= sx;
           x[g][t][2 * h] = pack_bf16x2(acc[0], acc[1]);
           x[g][t][2 * h + 1] = pack_bf16x2(acc[2], acc[3]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);  // no more than two groups' temporaries at a time
     }
+    sa = sx = 1.0f;
   }
   // ---- out
 #pragma unroll

@@ -72,7 +72,9 @@ int dion_ns_line_3(const void* B, const void* X, void* C, int batch, int m, int 
  *   X0 = bf16(in) / (||bf16(in)||_F * norm_scale + eps)  per matrix, then n_iters times
  *   A = X X^T; B = b A + c A A; X = a X + B X   on the orientation with rows <= cols.
  *   (For matrices that fill whole GEMM tiles the division is not a pass of its own: the factor is applied
- *   in the fp32 epilogue of the first two GEMMs, and a wide bf16 `in` is read where it lies.)
+ *   in the fp32 epilogue of the first two GEMMs, and a wide bf16 `in` is read where it lies.  The small-matrix kernel
+ *   applies it to the fp32 sums of the first iteration too, except for matrices of up to 64 x 1024: there X0 is scaled
+ *   and rounded to bf16 first.)
  *   `out` may overlap `in`: the input is then copied first, through the workspace.  Not so for matrices whose short side is
  *   at most 64 and whose long side is at most 1024: those take disjoint buffers, or a bf16 call in place (out == in).
  *   flags: DION_NS_GRAM selects the Gram-matrix recurrence (call site
@@ -152,8 +154,8 @@ int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X
  * plain calls give every matrix to one workgroup; DION_E_INVALID otherwise (use dion_ns_orthogonalize).  Such a batch
  * of whole-tile matrices with more than 64 rows or columns on the short side (16 and more matrices of 128 x up to 1024) is
  * taken all the same: it runs the GEMMs, slower than the plain call.
- * Results differ from dion_ns_orthogonalize in the last bf16 bit (X0 is not rounded to bf16 once
- * more before the first products).
+ * Results may differ from dion_ns_orthogonalize in the last bf16 bit (the norm is summed in another order; where that
+ * call runs the small-matrix kernel, every sum is).
  * ------------------------------------------------------------------------------------------ */
 int dion_ns_accepts_prepared(int batch, int rows, int cols, int flags, int n_iters);
 int dion_ns_orthogonalize_prepared(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch,

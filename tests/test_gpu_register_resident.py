@@ -81,3 +81,50 @@ def test_nothing_is_written_beside_the_result(shape):
                                              torch.cuda.current_stream().cuda_stream), "ns")
         assert torch.equal(buf[offset:offset + n].view(shape), want)
         assert bool((buf[:offset] == 3).all()) and bool((buf[offset + n:] == 3).all())
+
+
+def _decaying(b, m, n, tall, seed):
+    """Matrices whose singular values fall over 2.5 decades, as a gradient's do."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    Q = torch.linalg.qr(torch.randn(m, m, device=DEV, generator=g))[0] * torch.logspace(0, -2.5, m, device=DEV)
+    G = Q @ torch.randn(b, m, n, device=DEV, generator=g).mul_(0.02)
+    return (G.mT if tall else G).contiguous().bfloat16()
+
+
+@pytest.mark.parametrize("tall", [False, True])
+@pytest.mark.parametrize("shape", [(16, 128, 256), (24, 128, 1024), (17, 96, 1280), (260, 96, 512), (24, 64, 1536), (17, 64, 2048), (24, 32, 2048), (16, 32, 4096)])
+def test_the_norm_is_no_rounding_of_its_own(shape, tall):
+    """Shapes that single matrices run on the GEMMs: the distance to float64 is that of the iteration whose first products take
+    the values as they came (rounded to bf16 once), A, B and X rounded once per iteration.  Sums in another order move single roundings, and with them a
+    distance over this many elements by a few per cent; X rounded once more after the scaling is 1.3 to 1.4 times as far."""
+    b, m, n = shape
+    G = _decaying(b, m, n, tall, m + n)
+    exact = _iterate(G.bfloat16().double(), CO, lambda t: t)
+    to_bf16 = lambda t: t.bfloat16().float()
+    first = []  # the first value _iterate rounds is the scaled X
+    round_ = lambda t: to_bf16(t) if first else (first.append(1), t)[1]
+    err = lambda t: float((t.double() - exact).norm() / exact.norm())
+    as_it_came, rounded = err(_iterate(G.float(), CO, round_)), err(_iterate(G.float(), CO, to_bf16))
+    got = err(ops.ns_orthogonalize(G, CO, 1.02, 1e-6))
+    print(f"{shape} {tall}: {got:.3e}, emulated {as_it_came:.3e}, with X rounded again {rounded:.3e}")
+    assert got <= 1.1 * as_it_came
+
+
+@pytest.mark.parametrize("tall", [False, True])
+@pytest.mark.parametrize("exponent", [-58, -46, -34, -20, 20, 34, 46, 54])
+def test_inputs_of_any_magnitude(exponent, tall):
+    """The scale of the input cancels: powers of two on both sides of where the factor moves from the sums into X (squared
+    norms of 2^-80 and 2^80), with the bound of the iteration that rounds the scaled X."""
+    g = torch.Generator(device=DEV).manual_seed(7)
+    G = torch.randn((24, 256, 128) if tall else (24, 128, 256), device=DEV, generator=g).bfloat16()
+    O = ops.ns_orthogonalize(torch.ldexp(G.float(), torch.tensor(exponent, device=DEV)).bfloat16(), CO, 1.02, 0.0)
+    exact = _iterate(G.double(), CO, lambda t: t)
+    same = _iterate(G.float(), CO, lambda t: t.bfloat16().float())
+    err = lambda t: float((t.double() - exact).norm() / exact.norm())
+    assert err(O) <= 1.5 * err(same) + 1e-4, (err(O), err(same))
+
+
+def test_a_norm_past_the_range_of_fp32_gives_zeros():
+    """X / (inf * s + eps)."""
+    G = torch.full((24, 128, 256), 2.0 ** 64, device=DEV).bfloat16()
+    assert not bool(ops.ns_orthogonalize(G, CO, 1.02, 1e-6).any())

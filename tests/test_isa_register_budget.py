@@ -1,7 +1,7 @@
 """The small-matrix kernel keeps a whole matrix in the registers of one workgroup: up to 128 registers of X a lane beside
 the operands of the products.  What does not fit goes through scratch memory, once per iteration, and the point of the kernel is
-gone.  This test compiles ns_small.hip for gfx950 and reads the compiler's own account of every instantiation: 16 bytes a
-lane (a pointer put aside over the iterations) is what it may use.  Needs hipcc, no GPU."""
+gone.  This test compiles ns_small.hip for gfx950 and reads the compiler's own account of every instantiation: 32 bytes a
+lane (addresses put aside over the iterations, six registers) is what it may use.  Needs hipcc, no GPU."""
 import os
 import re
 import shutil
@@ -29,4 +29,4 @@ def test_no_form_of_the_small_matrix_kernel_keeps_its_matrix_in_scratch_memory(t
             scratch[name] = int(m.group(1))
     forms = {k: v for k, v in scratch.items() if "ns_reg_kernel" in k}
     assert len(forms) >= 40, sorted(scratch)
-    assert not {k: v for k, v in forms.items() if v > 16}
+    assert not {k: v for k, v in forms.items() if v > 32}
