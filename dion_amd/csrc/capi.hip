@@ -1428,7 +1428,8 @@ extern "C" int dion_dion2_add_gather_columns(const uint64_t* G_ptrs, int g_dtype
   if (int rc = check_state_dtype(who, "m_dtype", m_dtype)) return rc;
   if (g_dtype != DION_BF16 && g_dtype != DION_F32) return fail(DION_E_INVALID, "%s: g_dtype", who);
   if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0 || k < 0) return fail(DION_E_INVALID, "%s: bad size", who);
-  if (n == 0 || rows == 0 || cols == 0 || k == 0) return DION_OK;
+  if (n == 0 || rows == 0 || cols == 0) return DION_OK;
+  if (k == 0) return fail(DION_E_INVALID, "%s: k == 0 (no column selected: dion_dion2_accumulate adds the gradients)", who);
   if (!G_ptrs || !M_ptrs || !idx || !map || !U_sel || !sumsq) return fail(DION_E_INVALID, "%s: null argument", who);
   if (k > cols || rows <= k || rows % 64 || k % 64 || cols % 4 || rows / 64 > 65535)
     return fail(DION_E_INVALID, "%s: %d columns of %d x %d", who, k, rows, cols);

@@ -331,7 +331,7 @@ int dion_dion2_gather_prepared(const uint64_t* M_ptrs, int m_dtype, int n, int m
  * dion_dion2_accumulate, bit for bit, without writing M, and dion_dion2_add_gather_columns then adds G, writes U_sel
  * and sumsq as dion_dion2_gather_prepared does and decays the selected columns, in one pass.  M ends as after
  * dion_dion2_accumulate and dion_dion2_gather_prepared.  idx and map as dion_dion2_topk writes them; cols a multiple
- * of 4, G, M and map 16-byte aligned.  Replaces dion/dion2.py:439-545. */
+ * of 4, G, M and map 16-byte aligned, k at least 1 (DION_E_INVALID otherwise).  Replaces dion/dion2.py:439-545. */
 int dion_dion2_column_norms(const uint64_t* G_ptrs, int g_dtype, const uint64_t* M_ptrs, int m_dtype, int n,
                             int mats_per_ptr, int rows, int cols, float* norms, void* scratch, size_t scratch_bytes,
                             void* stream);

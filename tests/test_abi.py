@@ -150,3 +150,19 @@ def test_argument_validation_happens_before_any_device_work():
     assert lib.dion_slice_l1(None, 0, 0, 8, 8, -2, 0, None, None) == 0
     assert lib.dion_gather_slices(None, 0, 1, 8, 8, -2, None, 0, None, None) == 0
     assert lib.dion_dion2_index_map(None, 0, 0, 8, None, None) == 0
+
+
+def test_adding_the_gradients_with_no_column_selected_is_refused():
+    """dion_dion2_add_gather_columns is what adds G to M behind norms that do not: without a column to gather it has no
+    workgroup to do so, and may not report success."""
+    import ctypes
+
+    from dion_amd import _lib
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("libdion_hip.so not built in this checkout")
+    lib = _lib.load()
+    call = lambda n, k: lib.dion_dion2_add_gather_columns(None, 0, None, 1, n, 1, 128, 64, None, None, k, ctypes.c_float(0.9),
+                                                          None, None, None)
+    assert call(1, 0) == -1 and "k == 0" in lib.dion_last_error().decode()
+    assert call(0, 0) == 0 and call(0, 64) == 0  # no matrix: nothing to add
