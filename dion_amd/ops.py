@@ -168,6 +168,14 @@ def ns_line_3(B: Tensor, X: Tensor, a: float, *, out: Optional[Tensor] = None) -
     return res.contiguous()
 
 
+def _calls(batch: int, most: int = 32768) -> List[Tuple[int, int]]:
+    """(first matrix, matrices) of the library calls for ``batch`` matrices (one call takes at most 65535), of nearly equal
+    size: a short last one could run another kernel than the rest, and sum in another order."""
+    n = -(-batch // most)
+    bounds = [batch * i // n for i in range(n + 1)]
+    return [(lo, hi - lo) for lo, hi in zip(bounds, bounds[1:])]
+
+
 def ns_orthogonalize(G: Tensor, coeffs: Sequence[Sequence[float]], norm_scale: float, epsilon: float,
                      gram: bool = False, gram_reset: int = 0) -> Tensor:
     """Batched Newton-Schulz / Polar-Express orthogonalization of ``G[..., rows, cols]``.
@@ -190,9 +198,7 @@ def ns_orthogonalize(G: Tensor, coeffs: Sequence[Sequence[float]], norm_scale: f
     carr, n_iters = _flat_coeffs(coeffs)
     flags = DION_NS_GRAM if gram else 0
     lib = _lib.load()
-    chunk = 32768  # one library call takes at most 65535 matrices
-    for b0 in range(0, batch, chunk):
-        nb = min(chunk, batch - b0)
+    for b0, nb in _calls(batch):
         nbytes = lib.dion_ns_workspace_bytes(nb, rows, cols, flags)
         ws = _workspace(G.device, nbytes)
         check(lib.dion_ns_orthogonalize(G3[b0:].data_ptr(), _dtype_code(G3, "G"), out[b0:].data_ptr(), nb, rows,

@@ -209,3 +209,20 @@ def test_overlap_of_matrices_that_only_the_small_kernel_takes():
     lib = _lib.load()
     for offset in (0, 64 * 768 * 2, -64 * 768 * 2):
         assert lib.dion_ns_plan_audit_overlap(432, 64, 768, BF16, 5, 0, 0, offset) == 1
+
+
+@pytest.mark.parametrize("batch", [1, 15, 32768, 32769, 32773, 65537, 98305, 200001])
+def test_a_batch_of_several_calls_runs_one_kernel(batch):
+    """The calls that ops.ns_orthogonalize cuts a batch into cover it once and plan the same launches: a matrix's result does
+    not depend on which of them it falls into."""
+    from dion_amd import ops
+    lib = _lib.load()
+    calls = ops._calls(batch)
+    assert [b0 for b0, _n in calls] == [sum(n for _b, n in calls[:i]) for i in range(len(calls))]
+    assert sum(n for _b, n in calls) == batch and all(0 < n <= 32768 for _b, n in calls)
+    sizes = sorted({n for _b, n in calls})
+    assert sizes[-1] - sizes[0] <= 1
+    for shape in [(128, 256), (64, 2048), (100, 500), (128, 128), (256, 256), (300, 40)]:
+        for flags in (0, GRAM):
+            plans = {(_audit(lib, (n, *shape), 5, flags), lib.dion_gemm_tile_edge(n, 256, 256, 1)) for n in sizes}
+            assert len(plans) == 1 and min(plans)[0] > 0, (shape, plans)
