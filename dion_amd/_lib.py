@@ -30,6 +30,7 @@ SIGNATURES = {
     "dion_ns_line_2": (c_int, [c_void_p, c_void_p, c_int, c_int, c_float, c_float, c_void_p]),
     "dion_ns_line_3": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_void_p]),
     "dion_ns_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "dion_ns_call_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "dion_ns_orthogonalize": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, _f32p, c_int,
                                       c_float, c_float, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "dion_ns_orthogonalize_static": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, _f32p, c_int,

@@ -963,13 +963,21 @@ extern "C" int dion_ns_orthogonalize_static(const void* in, int in_dtype, void* 
                 need, stream, nullptr);
 }
 
-extern "C" size_t dion_ns_update_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters) {
+extern "C" size_t dion_ns_call_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters, int with_update) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  const bool small = ns_small_path(batch, rows, cols, flags, n_iters);
-  const size_t plan = align256(make_plan(batch, rows, cols, flags).total), tail = align256((size_t)batch * rows * cols * 2);
-  if (small && ns_takes_prepared(batch, rows, cols, flags, n_iters)) return plan > tail ? plan : tail;
-  if (ns_update_fuses(batch, rows, cols, flags, n_iters)) return plan;
-  return (small ? 0 : plan) + tail;
+  const size_t tail = align256((size_t)batch * rows * cols * 2);
+  if (ns_small_path(batch, rows, cols, flags, n_iters)) return with_update ? tail : 0;
+  const size_t plan = make_plan(batch, rows, cols, flags).total;
+  if (!with_update) return plan;
+  return align256(plan) + (ns_update_fuses(batch, rows, cols, flags, n_iters) ? 0 : tail);
+}
+
+extern "C" size_t dion_ns_update_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters) {
+  const size_t call = dion_ns_call_workspace_bytes(batch, rows, cols, flags, n_iters, 1);
+  // (a prepared input runs the GEMMs also where plain calls run the small-matrix kernel)
+  if (!ns_takes_prepared(batch, rows, cols, flags, n_iters)) return call;
+  const size_t plan = align256(make_plan(batch, rows, cols, flags).total);
+  return plan > call ? plan : call;
 }
 
 extern "C" int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X_ptrs, int x_dtype,
@@ -988,7 +996,7 @@ extern "C" int dion_ns_orthogonalize_update(const void* in, int in_dtype, const 
   if (!X_ptrs || !lr_dev) return fail(DION_E_INVALID, "dion_ns_orthogonalize_update: null argument");
   for (int i = 0; i < n_ptrs; ++i)
     if (!X_ptrs[i]) return fail(DION_E_INVALID, "dion_ns_orthogonalize_update: parameter %d is null", i);
-  const size_t need = dion_ns_update_workspace_bytes(batch, rows, cols, flags, n_iters);
+  const size_t need = dion_ns_call_workspace_bytes(batch, rows, cols, flags, n_iters, 1);
   if (workspace_bytes < need)
     return fail(DION_E_WORKSPACE, "dion_ns_orthogonalize_update: workspace %zu < %zu bytes", workspace_bytes, need);
   if (ns_update_fuses(batch, rows, cols, flags, n_iters)) {
@@ -996,9 +1004,8 @@ extern "C" int dion_ns_orthogonalize_update(const void* in, int in_dtype, const 
     return ns_run(in, in_dtype, nullptr, batch, rows, cols, coeffs, n_iters, norm_scale, eps, flags, gram_reset,
                   workspace, workspace_bytes, stream, &ps);
   }
-  // the small-matrix kernel: orthogonalize into the tail of the workspace (the
-  // last align256(batch * rows * cols * 2) bytes of what dion_ns_update_workspace_bytes reports),
-  // then the plain update pass
+  // the small-matrix kernel: orthogonalize into the tail of the workspace (the last
+  // align256(batch * rows * cols * 2) bytes of what the call needs), then the plain update pass
   const size_t tail = align256((size_t)batch * rows * cols * 2);
   const size_t ns = need - tail;
   if (!workspace) return fail(DION_E_WORKSPACE, "dion_ns_orthogonalize_update: workspace is null");

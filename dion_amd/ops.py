@@ -199,11 +199,12 @@ def ns_orthogonalize(G: Tensor, coeffs: Sequence[Sequence[float]], norm_scale: f
     flags = DION_NS_GRAM if gram else 0
     lib = _lib.load()
     for b0, nb in _calls(batch):
-        nbytes = lib.dion_ns_workspace_bytes(nb, rows, cols, flags)
-        ws = _workspace(G.device, nbytes)
+        nbytes = lib.dion_ns_call_workspace_bytes(nb, rows, cols, flags, n_iters, 0)
+        ws = _workspace(G.device, nbytes) if nbytes else None  # the small-matrix kernel needs none
         check(lib.dion_ns_orthogonalize(G3[b0:].data_ptr(), _dtype_code(G3, "G"), out[b0:].data_ptr(), nb, rows,
                                         cols, carr, n_iters, float(norm_scale), float(epsilon), flags,
-                                        int(gram_reset), ws.data_ptr(), ws.numel(), _stream_handle(G.device)),
+                                        int(gram_reset), ws.data_ptr() if nbytes else None, ws.numel() if nbytes else 0,
+                                        _stream_handle(G.device)),
               "ns_orthogonalize")
     return out.reshape(shape)
 
@@ -266,7 +267,7 @@ def ns_orthogonalize_update(G: Tensor, X: List[Tensor], coeffs: Sequence[Sequenc
     carr, n_iters = _flat_coeffs(coeffs)
     flags = DION_NS_GRAM if gram else 0
     lib = _lib.load()
-    ws = _workspace(G.device, lib.dion_ns_update_workspace_bytes(batch, rows, cols, flags, n_iters))
+    ws = _workspace(G.device, lib.dion_ns_call_workspace_bytes(batch, rows, cols, flags, n_iters, 1))
     check(lib.dion_ns_orthogonalize_update(G3.data_ptr(), _dtype_code(G3, "G"), xp, xcode, n, mats_per_ptr, rows,
                                            cols, carr, n_iters, float(norm_scale), float(epsilon), flags,
                                            int(gram_reset), lr_p, float(adj_ratio), wd_p, wd_h,

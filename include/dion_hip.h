@@ -87,6 +87,10 @@ int dion_ns_line_3(const void* B, const void* X, void* C, int batch, int m, int 
  * ------------------------------------------------------------------------------------------ */
 #define DION_NS_GRAM 1
 size_t dion_ns_workspace_bytes(int batch, int rows, int cols, int flags);
+/* What a call on plain, disjoint buffers uses of that: nothing where the small-matrix kernel runs (a null workspace is
+ * accepted there).  with_update 0: dion_ns_orthogonalize; 1: dion_ns_orthogonalize_update, whose workspace may be this
+ * small where its input is not a prepared one. */
+size_t dion_ns_call_workspace_bytes(int batch, int rows, int cols, int flags, int n_iters, int with_update);
 int dion_ns_orthogonalize(const void* in, int in_dtype, void* out, int batch, int rows, int cols,
                           const float* coeffs, int n_iters, float norm_scale, float eps, int flags,
                           int gram_reset, void* workspace, size_t workspace_bytes, void* stream);

@@ -128,3 +128,15 @@ def test_a_norm_past_the_range_of_fp32_gives_zeros():
     """X / (inf * s + eps)."""
     G = torch.full((24, 128, 256), 2.0 ** 64, device=DEV).bfloat16()
     assert not bool(ops.ns_orthogonalize(G, CO, 1.02, 1e-6).any())
+
+
+@pytest.mark.parametrize("shape", [(100, 64, 768), (100, 128, 1024)])
+def test_no_workspace_is_allocated(shape):
+    ops.release_workspaces()
+    G = torch.randn(shape, device=DEV).bfloat16()
+    ns.polar_express(G)
+    assert not ops._workspaces
+    X = [torch.zeros(shape[1:], device=DEV) for _ in range(shape[0])]
+    ops.ns_orthogonalize_update(G, X, CO, 1.02, 1e-6, torch.tensor(0.1, device=DEV), 1.0, 0.0)
+    assert [w.numel() for w in ops._workspaces.values()] == [G.numel() * 2]
+    assert torch.equal(torch.stack(X), -0.1 * ns.polar_express(G).float())

@@ -226,3 +226,23 @@ def test_a_batch_of_several_calls_runs_one_kernel(batch):
         for flags in (0, GRAM):
             plans = {(_audit(lib, (n, *shape), 5, flags), lib.dion_gemm_tile_edge(n, 256, 256, 1)) for n in sizes}
             assert len(plans) == 1 and min(plans)[0] > 0, (shape, plans)
+
+
+@pytest.mark.parametrize("shape", CONFIG_SHAPES + RAGGED_SHAPES + [(1000, 128, 1024), (1024, 32, 4096), (24, 1024, 128)])
+def test_the_workspace_of_a_plain_call(shape):
+    """What a call uses: nothing where one workgroup takes a whole matrix (432 x (64 x 768) would report 0.6 GB of GEMM
+    buffers), the orthogonalized matrices alone where the update follows."""
+    lib = _lib.load()
+    b, r, c = shape
+    for flags in (0, GRAM):
+        for n_iters in (0, 5, 9):
+            full = lib.dion_ns_workspace_bytes(b, r, c, flags)
+            plain = lib.dion_ns_call_workspace_bytes(b, r, c, flags, n_iters, 0)
+            update = lib.dion_ns_call_workspace_bytes(b, r, c, flags, n_iters, 1)
+            tail = -(-b * r * c * 2 // 256) * 256
+            small = _audit(lib, shape, n_iters, flags) == 1
+            assert plain == (0 if small else full)
+            fuses = not small and n_iters > 0
+            assert update == (tail if small else full + (0 if fuses else tail))
+            # an upper bound for prepared inputs too, as before
+            assert lib.dion_ns_update_workspace_bytes(b, r, c, flags, n_iters) >= update
