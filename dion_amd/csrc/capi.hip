@@ -1100,6 +1100,7 @@ extern "C" int dion_gemm_tile_edge(int batch, int m, int n, int symmetric) {
   memset(&p, 0, sizeof(p));
   p.M = m;
   p.N = symmetric ? m : n;
+  p.K = m;
   p.batch = batch;
   p.tri = symmetric ? 1 : 0;
   return gemm_tile_edge(p);

@@ -1528,9 +1528,14 @@ int gemm_pad_granule(int m, int n, int batch) {
 //    that are not full cost less than their geometry says: the part is power-limited, and the CUs that are busy run
 //    faster while others idle.
 //  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
-//    per CU, for symmetric products (whose 128-wide form has only a quarter as many) two per CU: X X^T of one
-//    768 x 3072 matrix 28.4 -> 10.0, of 1024 x 4096 42.9 -> 15.8; at two rounds 12 x (512 x 2048) 22.8 -> 16.8 (18.4
-//    with the form below), at three 4 x (1024 x 2816) 28.4 against 23.4; B X at 576 tiles (768 x 3072) 14.0 against 9.3.
+//    per CU, for symmetric products (whose 128-wide form has only a quarter as many) two per CU unless the reduction is
+//    short: X X^T of one 768 x 3072 matrix 28.4 -> 10.0, of 1024 x 4096 42.9 -> 15.8; at two rounds 12 x (512 x 2048)
+//    22.8 -> 16.8 (18.4 with the form below), at three 4 x (1024 x 2816) 28.4 against 23.4; one 2048 x 2048, 528 tiles, 17.6
+//    against 12.4.  Two rounds of a short reduction against the form below: X X^T of 128 x (128 x 128) 6.8 against 5.1,
+//    of 40 x (256 x 256) 7.6 against 6.6, of 150 x (128 x 512) 8.7 against 7.7; but of 32 x (256 x 512) 8.0 against 8.1, of
+//    100 x (128 x 1024) 9.8 against 10.5, A A of 13 x 384 7.9 against 8.3.  B X: 256 tiles (1024 x 1024) 9.8 -> 6.3; past
+//    that the last form, at 288 (2 x (768 x 768)) 9.4 against 8.4, at 512 (4 x (512 x 1024)) 8.7 against 7.4, at 576
+//    (768 x 3072) 14.0 against 8.9.
 //  * 128-wide tiles, at most one per CU: the CU is one workgroup's alone, and a ring of four slots keeps three slabs
 //    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
 //    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
@@ -1542,7 +1547,8 @@ static TileKind pick_tile(const GemmParams& p) {
     return (p.tri ? T * (T + 1) / 2 : T * (p.N / edge)) * (p.rule_batch > 0 ? p.rule_batch : p.batch);
   };
   if (p.M % 256 == 0 && p.N % 256 == 0 && tiles(256) >= (p.tri ? 160 : 384)) return kTile256;
-  if (tiles(64) <= (p.tri ? 512 : 256) && !(p.D && !p.tri)) return kTile64;
+  const int short_k = p.M < 256 ? 1024 : p.M < 384 ? 512 : 384;
+  if (tiles(64) <= (p.tri && p.K >= short_k ? 512 : 256) && !(p.D && !p.tri)) return kTile64;
   if (tiles(128) <= 256 && (p.tri || p.K > 1024)) return kTile128Deep;
   return kTile128;
 }

@@ -195,7 +195,7 @@ int dion_ns_orthogonalize_update_padded(const void* in, const float* sumsq, int 
 int dion_ns_plan_audit_prepared(int batch, int rows, int cols, int n_iters, int flags, int gram_reset,
                                 int with_update, int x_dtype, int mats_per_ptr, size_t audit_ws_bytes);
 
-/* Tile edge (64, 128 or 256) the GEMM launcher picks for `batch` products of an m x n result
+/* Tile edge (64, 128 or 256) the GEMM launcher picks for `batch` products of an m x n result over a reduction of m
  * (symmetric != 0: an m x m symmetric product, upper tiles only).  Lets a benchmark count executed
  * FLOP with the library's own rule.  No counterpart in the reference. */
 int dion_gemm_tile_edge(int batch, int m, int n, int symmetric);

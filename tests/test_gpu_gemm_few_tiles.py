@@ -77,3 +77,10 @@ def test_fused_update_of_few_tiles(shape, cautious, dtype):
     ops.ns_orthogonalize_update(G, X, NS5_COEFFS, 1.0, 1e-7, lr, 0.7, 0.01, cautious)
     ops.muon_post(X2, ops.ns_orthogonalize(G, NS5_COEFFS, 1.0, 1e-7).view(batch, -1), lr, 0.7, 0.01, cautious)
     assert all(torch.equal(a, b) for a, b in zip(X, X2))
+
+
+@pytest.mark.parametrize("batch,m,n,sym_edge,full_edge", [(86, 128, 128, 128, 128), (128, 128, 256, 128, 128), (100, 128, 1024, 128, 128),
+                                                          (26, 256, 256, 128, 128), (26, 256, 512, 128, 128), (13, 384, 384, 64, 128),
+                                                          (14, 512, 256, 64, 128)])
+def test_products_at_the_line_of_short_reductions(batch, m, n, sym_edge, full_edge):
+    test_products_of_few_tiles(batch, m, n, sym_edge, full_edge)

@@ -246,3 +246,11 @@ def test_the_workspace_of_a_plain_call(shape):
             assert update == (tail if small else full + (0 if fuses else tail))
             # an upper bound for prepared inputs too, as before
             assert lib.dion_ns_update_workspace_bytes(b, r, c, flags, n_iters) >= update
+
+
+@pytest.mark.parametrize("batch,m,edge", [(85, 128, 64), (86, 128, 128), (128, 128, 128), (25, 256, 64), (26, 256, 128), (51, 256, 128),
+                                          (13, 384, 64), (24, 384, 64), (25, 384, 128), (14, 512, 64), (15, 512, 128)])
+def test_tiles_of_symmetric_products_with_short_reductions(batch, m, edge):
+    """64-wide tiles split a reduction over four wavefronts; past one such tile per CU a short one is left with less than it
+    costs to add the parts (128 x (128 x 128): 6.8 us against 5.1)."""
+    assert _lib.load().dion_gemm_tile_edge(batch, m, m, 1) == edge
