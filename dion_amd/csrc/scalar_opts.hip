@@ -2,9 +2,9 @@
 // biases) of a model whose matrices are updated by Muon / NorMuon / Dion2 / NorDion2.
 //
 // One launch updates up to kMtaTensors tensors of different sizes: their pointers and element
-// counts travel by value in the kernel-argument segment, each workgroup owns one run of kMtaChunk
-// consecutive elements of one tensor (found by bisection in a table of first workgroups), and a thread has
-// the loads of sixteen elements in flight at once.  All traffic is HBM streaming: AdamW reads X, G, M, V
+// counts travel by value in the kernel-argument segment, each workgroup owns one run of consecutive elements of one
+// tensor: kMtaChunk of them (the tensor found by bisection in a table of first workgroups, a thread with the loads
+// of sixteen elements in flight at once), or in small launches a short run (mta_run; BRIEF).  All traffic is HBM streaming: AdamW reads X, G, M, V
 // and writes X, M, V (28 B/element with fp32 state and gradients, 26 with bf16 gradients), Lion 20 / 18
 // B/element.  The state tensors X, M, V of one launch share a dtype, fp32 or bf16 (half the bytes);
 // arithmetic is fp32 either way.
@@ -24,6 +24,7 @@ struct MtaTensors {
   uint64_t x[kMtaTensors], g[kMtaTensors], m[kMtaTensors], v[kMtaTensors], step[kMtaTensors];
   int64_t numel[kMtaTensors];
   unsigned wg0[kMtaTensors + 1];  // first workgroup of each tensor; wg0[n] = workgroups of the launch
+  int run;                        // elements per workgroup (mta_run)
 };
 
 // Elements one workgroup updates: two rounds of 256 threads x kMtaGroups groups of four.
@@ -73,13 +74,14 @@ static __device__ __forceinline__ void adamw_one(float& x, float g, float& m, fl
   x = x - adj_lr * upd;
 }
 
-template <typename GT, typename ST, bool NT>
+template <typename GT, typename ST, bool NT, bool BRIEF = false>
 __global__ __launch_bounds__(256) void adamw_mt_kernel(MtaTensors a, int n, const float* __restrict__ lr_dev,
                                                        const float* __restrict__ wd_dev,
                                                        AdamwScalars sc) {
-  const int t = mta_tensor(a, n, blockIdx.x);
-  const int64_t first = (int64_t)(blockIdx.x - a.wg0[t]) * kMtaChunk;
-  const int64_t end = a.numel[t] < first + kMtaChunk ? a.numel[t] : first + kMtaChunk;
+  const int t = BRIEF ? blockIdx.y : mta_tensor(a, n, blockIdx.x);
+  const int64_t first = (int64_t)(blockIdx.x - (BRIEF ? 0 : a.wg0[t])) * a.run;
+  if (BRIEF && first >= a.numel[t]) return;
+  const int64_t end = a.numel[t] < first + a.run ? a.numel[t] : first + a.run;
   ST* __restrict__ x = (ST*)a.x[t];
   const GT* __restrict__ g = (const GT*)a.g[t];
   ST* __restrict__ m = (ST*)a.m[t];
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(256) void adamw_mt_kernel(MtaTensors a, int n, cons
     w1 = 1.0f - sc.beta1;
     w2 = 1.0f - sc.beta2;
   };
-  if (vec && end - first == kMtaChunk) {
+  if (!BRIEF && vec && end - first == kMtaChunk) {
     float xv[kMtaGroups][4], mv[kMtaGroups][4], vv[kMtaGroups][4], gv[kMtaGroups][4];
 #pragma unroll 1
     for (int r = 0; r < 2; ++r) {
@@ -127,15 +129,20 @@ __global__ __launch_bounds__(256) void adamw_mt_kernel(MtaTensors a, int n, cons
     }
     return;
   }
-  // the last run of a tensor, and tensors that are not aligned
-  scalars();
+  // short runs, the last run of a tensor, and tensors that are not aligned
   const int64_t vend = vec ? end & ~(int64_t)3 : first;
-  for (int64_t q = first / 4 + threadIdx.x; q < vend / 4; q += 256) {
-    float xv[4], mv[4], vv[4], gv[4];
+  int64_t q = first / 4 + threadIdx.x;
+  float xv[4], mv[4], vv[4], gv[4];
+  auto load = [&]() {
+    if (q >= vend / 4) return;
     st_load4<ST>(x, q, xv);
     st_load4<ST>(m, q, mv);
     st_load4<ST>(v, q, vv);
     st_load4<GT>(g, q, gv);
+  };
+  load();
+  scalars();
+  for (; q < vend / 4; q += 256, load()) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       adamw_one<GT>(xv[e], gv[e], mv[e], vv[e], w1, sc.beta2, w2, inv_bc2_sqrt, sc.eps, adj_lr, aa, coeff,
@@ -167,13 +174,14 @@ static __device__ __forceinline__ void lion_one(float& x, float g, float& m, flo
   x = x - lr * u;
 }
 
-template <typename GT, typename ST, bool NT>
+template <typename GT, typename ST, bool NT, bool BRIEF = false>
 __global__ __launch_bounds__(256) void lion_mt_kernel(MtaTensors a, int n, const float* __restrict__ lr_dev,
                                                       const float* __restrict__ wd_dev, float beta1,
                                                       float beta2, float wd_host, int cautious) {
-  const int t = mta_tensor(a, n, blockIdx.x);
-  const int64_t first = (int64_t)(blockIdx.x - a.wg0[t]) * kMtaChunk;
-  const int64_t end = a.numel[t] < first + kMtaChunk ? a.numel[t] : first + kMtaChunk;
+  const int t = BRIEF ? blockIdx.y : mta_tensor(a, n, blockIdx.x);
+  const int64_t first = (int64_t)(blockIdx.x - (BRIEF ? 0 : a.wg0[t])) * a.run;
+  if (BRIEF && first >= a.numel[t]) return;
+  const int64_t end = a.numel[t] < first + a.run ? a.numel[t] : first + a.run;
   ST* __restrict__ x = (ST*)a.x[t];
   const GT* __restrict__ g = (const GT*)a.g[t];
   ST* __restrict__ m = (ST*)a.m[t];
@@ -184,7 +192,7 @@ __global__ __launch_bounds__(256) void lion_mt_kernel(MtaTensors a, int n, const
   const float w1 = 1.0f - beta1, w2 = 1.0f - beta2;
   const bool vec = (((a.x[t] | a.m[t]) & (sizeof(ST) == 2 ? 7 : 15)) == 0) &&
                    ((a.g[t] & (sizeof(GT) == 2 ? 7 : 15)) == 0);
-  if (vec && end - first == kMtaChunk) {
+  if (!BRIEF && vec && end - first == kMtaChunk) {
     float xv[kMtaGroups][4], mv[kMtaGroups][4], gv[kMtaGroups][4];
 #pragma unroll 1
     for (int r = 0; r < 2; ++r) {
@@ -230,6 +238,13 @@ static bool past_caches(const int64_t* numel, int n, int bytes_per_element) {
   return exceeds_caches(total * bytes_per_element);
 }
 
+// Elements per workgroup.  A launch of up to 5 M elements does not fill the chip with runs of kMtaChunk: it takes short ones, a
+// grid row per tensor, from a kernel of half the registers.  fp32 state, bf16 gradients, runs of 1024 / 2048 / 8192
+// elements, us, AdamW: 49 x 2048 14.3 / 15.9 / 15.7, 60 x 5000 15.9 / 17.6 / 22.0, 1 M in one tensor 8.4 / 8.2 / 10.9, 4 M 22.5 /
+// 20.8 / 21.9, 6 M 29.9 / 29.2 / 27.8, 38.6 M 191 / 196 / 174; Lion: 60 x 5000 4.5 / 5.4 / 8.3, 4 M 13.0 / 12.5 / 12.6,
+// 38.6 M 121 / 126 / 128.
+static int mta_run(int64_t total) { return total < (1 << 20) ? 1024 : total < (5 << 20) ? 2048 : kMtaChunk; }
+
 // false: more workgroups than one launch can have
 static bool fill(MtaTensors& a, const uint64_t* X, const uint64_t* G, const uint64_t* M, const uint64_t* V,
                  const uint64_t* S, const int64_t* numel, int n) {
@@ -242,13 +257,23 @@ static bool fill(MtaTensors& a, const uint64_t* X, const uint64_t* G, const uint
     a.step[i] = S ? S[j] : 0;
     a.numel[i] = i < n ? numel[j] : 0;
   }
-  int64_t wg = 0;
+  int64_t wg = 0, total = 0;
+  for (int i = 0; i < n; ++i) total += numel[i];
+  a.run = mta_run(total);
   for (int i = 0; i <= kMtaTensors; ++i) {
     a.wg0[i] = (unsigned)wg;
-    if (i < n) wg += (numel[i] + kMtaChunk - 1) / kMtaChunk;
+    if (i < n) wg += (numel[i] + a.run - 1) / a.run;
     if (wg > 0x7fffffff) return false;
   }
   return true;
+}
+
+// a grid row per tensor where the runs are short
+static dim3 mta_grid(const MtaTensors& a, const int64_t* numel, int n) {
+  if (a.run == kMtaChunk) return dim3(a.wg0[n]);
+  int64_t longest = 0;
+  for (int i = 0; i < n; ++i) longest = numel[i] > longest ? numel[i] : longest;
+  return dim3((unsigned)((longest + a.run - 1) / a.run), n);
 }
 
 hipError_t launch_adamw_mt(const uint64_t* X, const uint64_t* G, int g_dtype, const uint64_t* M,
@@ -261,10 +286,12 @@ hipError_t launch_adamw_mt(const uint64_t* X, const uint64_t* G, int g_dtype, co
   if (a.wg0[n] == 0) return hipGetLastError();
   const bool nt = past_caches(numel, n, 3 * (s_dtype == 0 ? 2 : 4) + (g_dtype == 0 ? 2 : 4));
   AdamwScalars sc{beta1, beta2, eps, wd_host, cautious};
-  const dim3 grid(a.wg0[n]);
+  const dim3 grid = mta_grid(a, numel, n);
 #define ADAMW_LAUNCH(GT, ST)                                                                                       \
   do {                                                                                                             \
-    if (nt) hipLaunchKernelGGL((adamw_mt_kernel<GT, ST, true>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, sc); \
+    if (a.run != kMtaChunk)                                                                                        \
+      hipLaunchKernelGGL((adamw_mt_kernel<GT, ST, false, true>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, sc); \
+    else if (nt) hipLaunchKernelGGL((adamw_mt_kernel<GT, ST, true>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, sc); \
     else hipLaunchKernelGGL((adamw_mt_kernel<GT, ST, false>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, sc);   \
   } while (0)
   if (g_dtype == 0) {
@@ -282,11 +309,14 @@ hipError_t launch_lion_mt(const uint64_t* X, const uint64_t* G, int g_dtype, con
   MtaTensors a;
   if (!fill(a, X, G, M, nullptr, nullptr, numel, n)) return hipErrorInvalidValue;
   if (a.wg0[n] == 0) return hipSuccess;
-  const dim3 grid(a.wg0[n]);
+  const dim3 grid = mta_grid(a, numel, n);
   const bool nt = past_caches(numel, n, 2 * (s_dtype == 0 ? 2 : 4) + (g_dtype == 0 ? 2 : 4));
 #define LION_LAUNCH(GT, ST)                                                                                \
   do {                                                                                                     \
-    if (nt) hipLaunchKernelGGL((lion_mt_kernel<GT, ST, true>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, \
+    if (a.run != kMtaChunk)                                                                                \
+      hipLaunchKernelGGL((lion_mt_kernel<GT, ST, false, true>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, \
+                         beta1, beta2, wd_host, cautious);                                                 \
+    else if (nt) hipLaunchKernelGGL((lion_mt_kernel<GT, ST, true>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, \
                                beta1, beta2, wd_host, cautious);                                           \
     else hipLaunchKernelGGL((lion_mt_kernel<GT, ST, false>), grid, dim3(256), 0, st, a, n, lr_dev, wd_dev, \
                             beta1, beta2, wd_host, cautious);                                              \

@@ -40,3 +40,12 @@ def test_runs_and_rests(kind, sdt, gdt, sizes):
                     [torch.full((), 3.0, device=DEV) for _ in parts[0][lo:lo + 48]], lr)
     for a, b in zip(X + M + (V if kind == "adamw" else []), Xc + Mc + (Vc if kind == "adamw" else [])):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kind", ["adamw", "lion"])
+@pytest.mark.parametrize("sdt,gdt", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("sizes", [[1, 1023, 0, 1024, 1025, 3 * 1024 + 5], [(1 << 20) - 1], [(1 << 20) - 4095, 2047, 2048, 2049, 0, 7],
+                                   [(5 << 20) - 8192, 8191], [(5 << 20) - 8192, 8192, 8193, 3]])
+def test_short_runs_and_rests(kind, sdt, gdt, sizes):
+    """The same at the edges of the short runs (1024, 2048 elements) and of the launch sizes that take them."""
+    test_runs_and_rests(kind, sdt, gdt, sizes)
