@@ -546,6 +546,14 @@ def dion2_prepared_blocks(rows: int, cols: int, select_dim: int, k: int) -> int:
     return int(_lib.load().dion_dion2_gather_sumsq_blocks(int(rows), int(cols), int(select_dim), int(k)))
 
 
+def _late_add_pays(m_dtype: int, elements: int) -> bool:
+    """Adding the gradients in the gathering pass reads G and M twice and saves a write and a scattered read of M: less
+    traffic for an fp32 momentum, from where that is what the launches are bound by.  us, added late / first, bf16 gradients,
+    a quarter of the columns: fp32 momentum 24 x (8192 x 2048) 1194 / 1474, 12 x (3072 x 768) 94 / 103, 2 x (4096 x
+    1024) 46 / 48, 4 x (2048 x 512) 37 / 29; bf16 momentum 24 x (8192 x 2048) 899 / 852, 12 x (3072 x 768) 77 / 69."""
+    return m_dtype == DION_F32 and elements >= 1 << 23
+
+
 def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_decay: float, prepared: bool = False):
     """``M += G``; pick the ``k`` slices of largest L1 norm along ``select_dim`` of every matrix; return
     (U_sel bf16 arena, idx int32 [n_mat, k] ascending, map int32 [n_mat, dim]) and decay the selected
@@ -580,7 +588,7 @@ def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_d
     gcode = _dtype_code(G[0], "G")
     # Columns of tall matrices in the prepared form: the norms first, without a write of M; the pass that gathers the
     # selected columns, and would touch every line of M for them anyway, adds G.
-    add_late = prepared and select_dim == -1 and rows > k and cols % 4 == 0 and \
+    add_late = prepared and select_dim == -1 and rows > k and cols % 4 == 0 and _late_add_pays(mcode, n * numel) and \
         not any(p & 15 for p in gp) and not any(p & 15 for p in mp)
     if add_late:
         check(lib.dion_dion2_column_norms(gp, gcode, mp, mcode, n, mats_per_ptr, rows, cols, norms.data_ptr(),

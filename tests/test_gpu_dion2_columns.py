@@ -9,6 +9,13 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+@pytest.fixture(autouse=True, params=[True, False], ids=["late", "by the rule"])
+def late(request, monkeypatch):
+    """Both forms at every size: the rule leaves small launches and bf16 momenta to the other one."""
+    if request.param:
+        monkeypatch.setattr(ops, "_late_add_pays", lambda *a: True)
+
+
 @pytest.mark.parametrize("sdt,gdt", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16),
                                      (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("where", ["anywhere", "first", "last", "ends", "every fourth"])
