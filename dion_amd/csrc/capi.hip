@@ -441,6 +441,11 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
       s.partial = sumsq ? const_cast<float*>(sumsq) : (float*)Xt;
       s.nblk = sumsq ? sumsq_blocks : (mp / 64) * (np / 64);
       s.inv = inv;
+      if (padded) {  // (a copy in either case: the caller's tensors themselves are never scaled)
+        s.same = sumsq ? (bf16_t*)const_cast<void*>(in) : X[0];
+        s.Rp = mp;
+        s.Cp = np;
+      }
       call.push(s);
     } else {
       // (over the transposed copy of a tall input that is copied unscaled: the sum then runs in the order it
@@ -752,6 +757,7 @@ int ns_audit(const NsCall& call) {
                                         : rd(s.partial, (size_t)s.batch * s.nblk * 4)))
           bad = "norm partials";
         else if (!wr(s.inv, (size_t)s.batch * 4)) bad = "reciprocal norms";
+        else if (s.same && !rd(s.same, (size_t)s.batch * s.Rp * s.Cp * 2)) bad = "X";
         break;
       case NsStep::kNorm: {
         const size_t es = s.in_dtype == DION_BF16 ? 2 : 4;
@@ -840,7 +846,8 @@ int ns_execute(const NsCall& call, hipStream_t st) {
     hipError_t e = hipSuccess;
     switch (s.kind) {
       case NsStep::kNormFinalize:
-        e = launch_norm_finalize(s.partial, s.nblk, s.batch, s.norm_scale, s.eps, s.inv, st);
+        e = launch_norm_finalize(s.partial, s.nblk, s.batch, s.norm_scale, s.eps, s.inv, s.same,
+                                 (int64_t)s.Rp * s.Cp, st);
         break;
       case NsStep::kNorm:
         e = launch_frobenius_inv(s.in, s.in_dtype, s.batch, (int64_t)s.R * s.C, s.norm_scale, s.eps, s.partial,
@@ -1073,7 +1080,7 @@ extern "C" int dion_ns_padded_extents(int batch, int rows, int cols, int flags, 
   return ns_padded(batch, rows, cols, flags, n_iters, mp, np) ? 1 : 0;
 }
 
-extern "C" int dion_ns_orthogonalize_padded(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch,
+extern "C" int dion_ns_orthogonalize_padded(void* in, const float* sumsq, int sumsq_blocks, void* out, int batch,
                                             int rows, int cols, const float* coeffs, int n_iters, float norm_scale,
                                             float eps, int flags, int gram_reset, void* workspace,
                                             size_t workspace_bytes, void* stream) {
@@ -1083,7 +1090,7 @@ extern "C" int dion_ns_orthogonalize_padded(const void* in, const float* sumsq, 
                 workspace_bytes, stream, nullptr, sumsq, sumsq_blocks, true);
 }
 
-extern "C" int dion_ns_orthogonalize_update_padded(const void* in, const float* sumsq, int sumsq_blocks,
+extern "C" int dion_ns_orthogonalize_update_padded(void* in, const float* sumsq, int sumsq_blocks,
                                                    const uint64_t* X_ptrs, int x_dtype, int n_ptrs, int mats_per_ptr,
                                                    int rows, int cols, const float* coeffs, int n_iters,
                                                    float norm_scale, float eps, int flags, int gram_reset,

@@ -24,9 +24,10 @@ hipError_t launch_ns_small(const void* in, int in_dtype, bf16_t* out, int batch,
 hipError_t launch_frobenius_inv(const void* in, int in_dtype, int batch, int64_t numel,
                                 float norm_scale, float eps, float* partial, int nblk,
                                 float* inv_norm, hipStream_t st);
-// inv_norm[b] = 1 / (sqrt(sum of partial[b][0..nblk)) * norm_scale + eps), fixed summation order.
+// inv_norm[b] = 1 / (sqrt(sum of partial[b][0..nblk)) * norm_scale + eps), fixed summation order.  X (may be null): [batch][elems],
+// elems % 8 == 0, 16-byte aligned; a matrix whose squared norm is outside 2^-80 ... 2^80 is scaled there, its inv_norm 1.
 hipError_t launch_norm_finalize(const float* partial, int nblk, int batch, float norm_scale, float eps,
-                                float* inv_norm, hipStream_t st);
+                                float* inv_norm, bf16_t* X, int64_t elems, hipStream_t st);
 hipError_t launch_ns_prepare(const void* in, int in_dtype, int batch, int R, int C,
                              const float* inv_norm, bf16_t* same, int Rp, int Cp, int ld_same,
                              int64_t stride_same, bf16_t* trans, int ld_trans, int64_t stride_trans,

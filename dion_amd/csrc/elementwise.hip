@@ -92,7 +92,8 @@ __global__ __launch_bounds__(256) void sumsq_partial_kernel(const T* __restrict_
 
 __global__ __launch_bounds__(256) void norm_finalize_kernel(const float* __restrict__ partial, int nblk,
                                                             float norm_scale, float eps,
-                                                            float* __restrict__ inv_norm) {
+                                                            float* __restrict__ inv_norm, bf16_t* __restrict__ X,
+                                                            int64_t elems) {
   // Fixed summation order: thread t adds partials t, t + 256, ... (four independent running sums,
   // so four loads are in flight), then the block sum.
   __shared__ float red[16];
@@ -106,7 +107,22 @@ __global__ __launch_bounds__(256) void norm_finalize_kernel(const float* __restr
   }
   for (int j = 0; i < nblk; i += 256, ++j) s4[j] += src[i];
   const float s = block_sum((s4[0] + s4[1]) + (s4[2] + s4[3]), red);
-  if (threadIdx.x == 0) inv_norm[b] = 1.0f / (sqrtf(s) * norm_scale + eps);
+  float inv = 1.0f / (sqrtf(s) * norm_scale + eps);
+  // X (may be null): the matrices as they came, whose products the factor is applied to.  Where sums of such products, or
+  // the factor's square, would leave the normal range of fp32, the matrix is scaled here instead (an overflown norm, a factor
+  // of 0, leaves zeros; one value that is not finite, NaN).
+  if (X && s != 0.f && !(s > 0x1p-80f && s < 0x1p80f)) {
+    bf16_t* x = X + (int64_t)b * elems;
+    for (int64_t i8 = threadIdx.x; i8 < elems / 8; i8 += 256) {
+      float v[8];
+      st_load8<bf16_t>(x, i8, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= inv;
+      st_store8<bf16_t>(x, i8, v);
+    }
+    inv = 1.0f;
+  }
+  if (threadIdx.x == 0) inv_norm[b] = inv;
 }
 
 // in [B,R,C] -> same [B,Rp,Cp] (scaled, zero padded) and trans [B,Cp,Rp] = same^T, both bf16.
@@ -213,13 +229,13 @@ hipError_t launch_frobenius_inv(const void* in, int in_dtype, int batch, int64_t
     if (vec) SUMSQ_LAUNCH(float, true); else SUMSQ_LAUNCH(float, false);
   }
 #undef SUMSQ_LAUNCH
-  return launch_norm_finalize(partial, nblk, batch, norm_scale, eps, inv_norm, st);
+  return launch_norm_finalize(partial, nblk, batch, norm_scale, eps, inv_norm, nullptr, 0, st);
 }
 
 hipError_t launch_norm_finalize(const float* partial, int nblk, int batch, float norm_scale, float eps,
-                                float* inv_norm, hipStream_t st) {
+                                float* inv_norm, bf16_t* X, int64_t elems, hipStream_t st) {
   hipLaunchKernelGGL(norm_finalize_kernel, dim3(batch), dim3(256), 0, st, partial, nblk, norm_scale, eps,
-                     inv_norm);
+                     inv_norm, X, elems);
   return hipGetLastError();
 }
 

@@ -178,14 +178,15 @@ int dion_ns_orthogonalize_update_prepared(const void* in, const float* sumsq, in
 /* The same for matrices that do not fill whole tiles: the producer (dion_muon_pre_padded) writes them into the
  * zero-padded form they are iterated in -- bf16 [batch, mp, np], short side along rows, zero outside
  * min(rows, cols) x max(rows, cols), 16-byte aligned -- with partial sums of squares as above.
+ * A matrix whose squared norm lies outside 2^-80 ... 2^80 is scaled in place before the iteration.
  * dion_ns_padded_extents returns 1 and the extents when such a call pads its matrices (at least one iteration, at most
  * 4096 matrices, not a batch whose plain calls give every matrix to one workgroup), 0 otherwise.  Results differ from
  * dion_ns_orthogonalize on the same matrices by nothing: it makes the same copy itself. */
 int dion_ns_padded_extents(int batch, int rows, int cols, int flags, int n_iters, int* mp, int* np);
-int dion_ns_orthogonalize_padded(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch, int rows,
+int dion_ns_orthogonalize_padded(void* in, const float* sumsq, int sumsq_blocks, void* out, int batch, int rows,
                                  int cols, const float* coeffs, int n_iters, float norm_scale, float eps, int flags,
                                  int gram_reset, void* workspace, size_t workspace_bytes, void* stream);
-int dion_ns_orthogonalize_update_padded(const void* in, const float* sumsq, int sumsq_blocks, const uint64_t* X_ptrs,
+int dion_ns_orthogonalize_update_padded(void* in, const float* sumsq, int sumsq_blocks, const uint64_t* X_ptrs,
                                         int x_dtype, int n_ptrs, int mats_per_ptr, int rows, int cols,
                                         const float* coeffs, int n_iters, float norm_scale, float eps, int flags,
                                         int gram_reset, const float* lr_dev, float adj_ratio, const float* wd_dev,

@@ -149,3 +149,39 @@ def test_step_with_and_without_the_padded_hand_over(shape, cls):
         return [p.data for p in ps] + [opt.state[p]["momentum"] for p in ps]
 
     assert all(torch.equal(a, b) for a, b in zip(build(True), build(False)))
+
+
+def _both_forms(G, func, eps):
+    """The operator on G, and on its padded form from the momentum pass (M = 0, no momentum: U = G)."""
+    b, r, c = G.shape
+    yield func(G, eps)
+    extents = ns.padded_extents(func, b, r, c)
+    U, sumsq = ops.muon_pre_padded([G], [torch.zeros_like(G)], 0.0, False, b, r, c, extents)
+    yield ns.orthogonalize_prepared(func, U, sumsq, r, c, eps, padded=True)
+
+
+@pytest.mark.parametrize("shape", [(2, 130, 200), (2, 200, 130), (3, 1100, 1151), (40, 130, 201)])
+@pytest.mark.parametrize("exponent", [-58, -46, -34, 34, 46, 54])
+def test_inputs_of_any_magnitude(shape, exponent):
+    """The scale of the input cancels, also where squares of the values as they came leave the range of fp32: powers of two
+    on both sides of where the copy is scaled (squared norms of 2^-80 and 2^80).  The bound is the error without the power
+    of two; one more rounding of the scaled matrix is within the factor."""
+    G = _rand(shape, 5)
+    exact = torch.stack([torch.from_numpy(oracle.ns_fp64(g.double().cpu().numpy(), oracle.NS5_COEFFS, 1.0, 0.0)) for g in G[:2]]).to(DEV)
+    bound = 1.5 * _rel(ns.zeropower_via_newtonschulz5(G, 0.0)[:2], exact) + 1e-4
+    scaled = torch.ldexp(G.float(), torch.tensor(exponent, device=DEV)).bfloat16()
+    for O in _both_forms(scaled, ns.zeropower_via_newtonschulz5, 0.0):
+        assert _rel(O[:2], exact) <= bound
+
+
+@pytest.mark.parametrize("shape", [(3, 130, 200), (3, 200, 130)])
+def test_norms_past_fp32_and_values_that_are_not_finite(shape):
+    """X / inf is 0 where X is finite; a value that is not makes its own matrix NaN and no other."""
+    G = _rand(shape, 6)
+    G[0] = 2.0 ** 64
+    G[1, 5, 7] = float("inf")
+    want = ns.polar_express(_rand(shape, 6))[2]
+    for O in _both_forms(G, ns.polar_express, 1e-6):
+        assert not bool(O[0].any())
+        assert bool(O[1].isnan().all())
+        assert torch.equal(O[2], want)
