@@ -367,7 +367,7 @@ def main() -> int:
         ms3 = time_kernel(lambda: lib.dion_ns_line_3(Bm.data_ptr(), X.data_ptr(), C.data_ptr(), B, m, n, 0.0, st))
         # the vendor library's bf16 GEMM (hipBLASLt behind torch.bmm) on the same operands, same box, same
         # run: the full product X X^T and B X ("NN": X read as it lies, the form of the dominant launch).  X^T is
-        # a contiguous copy: the library's batched bf16 product has faulted the GPU on a transposed right operand.
+        # a contiguous copy: a test run with the transposed view in its place ended in an illegal access.
         XT = X.mT.contiguous()
         ms_v_nt = time_kernel(lambda: torch.bmm(X, XT, out=A))
         del XT
@@ -421,7 +421,7 @@ def main() -> int:
         }
         del X
         if args.workload == "gpt_small_heads":
-            # the per-head group on its own: 36 heads x 12 layers of 64 x 768, one LDS-resident launch
+            # the per-head group on its own: 36 heads x 12 layers of 64 x 768, one launch of the small-matrix kernel
             Xh = (torch.randn(432, 64, 768, device=dev) * 0.01).to(torch.bfloat16)
             ms_h = time_kernel(lambda: fn(Xh, 1e-8), iters=20)
             h_tf = 432 * ns_flops(64, 768) / (ms_h * 1e-3) * 1e-12

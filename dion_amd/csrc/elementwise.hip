@@ -1064,8 +1064,10 @@ hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M
 // and stops as soon as a candidate has exactly k entries above it; a pass over 1024 entries at a time then places the
 // selected ones in index order.  Bound by the chain of at most sixteen counting steps (about 0.2 us each), not by
 // its dim * 4 bytes.  Keys stay in registers up to 1024 * 8 entries; longer rows are read again at every step.
-// 24 rows of 2048 (k = 512): 43.4 us counting every entry's rank (2048^2 compares a row) and compacting in a second launch
-// -> 9.4 us; 12 rows of 768: 20.9 -> 7.5.
+// 24 rows of 2048 (k = 512), the launch alone: 43.4 us counting every entry's rank (2048^2 compares a row) and compacting in a
+// second launch -> 8.2 us; 12 rows of 768: 20.9 -> 7.0; 300 rows of 64: 6.2 -> 7.0.  Inside a step it takes longer: a workgroup
+// of 16 wavefronts waits for a CU that another stream's kernels leave (205 us a launch on average in a Dion2 step
+// over matrices of 2048 x 8192).
 // unsigned keys in the order of the values (NaN = +inf, -0 = +0); never 0
 static __device__ __forceinline__ uint32_t topk_key(float x) {
   if (x != x) x = INFINITY;

@@ -25,10 +25,10 @@ constexpr int kMaxLds = 160 * 1024 - 1024;  // dynamic LDS of one workgroup; the
 // wavefront), NW wavefronts.  NW = 4 leaves room for two workgroups per CU: one's reduction and load phases run under the
 // other's MFMAs.
 //
-// What bounds it, 432 x (64 x 768), 43 us: 17 us are the 84 MB in and out (5 TB/s, no iteration), 4.7 us an iteration of
-// two matrices on one CU, of which 2.8 are MFMA time (the turning products are a quarter of it); the rest is the latency
-// of three barriers and A's partial sums through LDS.  The form with X in LDS and one workgroup per CU took 60 on the same box
-// (38.7 against 55.0 us, call by call, on another).
+// What bounds it, 432 x (64 x 768), 38.8 us: 16.8 us are the 84 MB in and out (5 TB/s, no iteration), 4.4 us an iteration of
+// two matrices on one CU (20.6, 25.2, 29.6, 34.4, 38.8 us with one to five), of which 2.8 are MFMA time (the turning products
+// are a quarter of it); the rest is the latency of three barriers and A's partial sums through LDS.  The form with X in
+// LDS and one workgroup per CU took 55.0.
 // 256 x (64 x 2048) 55 us, 300 x (128 x 768) 135, 200 x (80 x 1000) 54, 400 x (128 x 1024) 163, where the GEMM chain on
 // matrices padded to 128 rows took many times that (1074, 724, 296 for the first three); 16 x (128 x 256) 42 against 90.
 // ------------------------------------------------------------------------------------------
@@ -59,7 +59,8 @@ __global__ __launch_bounds__(NW * 64, 2) void ns_reg_kernel(const T* __restrict_
                                                             int cols, NsCoeffs co, float norm_scale, float eps) {
   typedef RegCfg<MT, NW> C;
   constexpr int MR = C::MR, AP = C::AP, GT = C::GT, ST = MT / 2;
-  // x takes 4 MT KC registers: past 96 there is no room for a second turned group (256 x (64 x 2048) 76 -> 130 us)
+  // x takes 4 MT KC registers: past 96 a second turned group gains nothing (256 x (64 x 2048) 54.8 us, 54.7 with it; 400 x (128 x
+  // 1024) 162 and 167)
   constexpr bool PIPE = MT * KC <= 24;
   // Matrices the GEMMs would take otherwise are not rounded after the scaling there, and so not here; the multiplications cost
   // 5 % of an iteration, which the shapes that never ran anywhere else (up to 64 x 1024) are spared.
@@ -371,7 +372,7 @@ hipError_t launch_ns_small(const void* in, int in_dtype, bf16_t* out, int batch,
   const int groups = (n + 31) / 32;
   // Up to a workgroup per CU eight wavefronts share a matrix (24 x (64 x 768): 26.8 -> 22.0 us), past that four, two
   // workgroups per CU.  The forms of 128 registers of X check every group for being there: the straight-line code of
-  // the others makes the compiler keep more of them in flight than fit (256 x (64 x 2048): 76 -> 104 us).
+  // the others makes the compiler keep more of them in flight than fit (256 x (64 x 2048) 55 -> 82 us).
   const bool wide = batch <= 256;
 #define REG(MT, KC, NW, KF)                                                                               \
   if (groups <= KC * NW && groups >= KF * NW)                                                             \
@@ -395,9 +396,12 @@ hipError_t launch_ns_small(const void* in, int in_dtype, bf16_t* out, int batch,
   return hipErrorInvalidValue;
 }
 
-// Short sides up to 64 and long sides up to 1024 whatever the batch.  Past that a matrix is more work for one CU (128 x
-// 1024: 16 us an iteration) than its share of a few GEMM launches: only batches of 16 and more, from 256 columns on (a group
-// for every wavefront): 24 x (128 x 1024) 85 us against 123, 16 x (128 x 256) 42 against 90, 64 x (32 x 4096) 46 against 403.
+// Short sides up to 64 and long sides up to 1024 whatever the batch.  Past that only batches of 16 and more, from 256 columns
+// on (a group for every wavefront).  The line is where the widest matrices break even, a whole call in us, GEMM chain / this
+// kernel: 128 x 1024, one of them 78 / 77, 15 85 / 79, 128 of them 196 (the chain before 64-wide tiles) / 82.  It is
+// on the safe side for the others, which would gain below it too: 15 x (128 x 256) 71 / 43, 15 x (96 x 768) 83 / 43,
+// 15 x (64 x 2048) 107 / 49, one of 32 x 4096 125 / 40, 16 x (128 x 128) 67 / 38, 128 x (96 x 192) 101 / 28.  Rows that are no
+// multiple of 16 bytes are fetched element by element and lose at short batches: 16 x (100 x 500) 75 / 81.
 bool ns_small_fits(int batch, int rows, int cols) {
   const int m = rows < cols ? rows : cols, n = rows < cols ? cols : rows;
   if (m <= 64 && n <= 1024) return true;

@@ -67,7 +67,7 @@ int dion_ns_line_3(const void* B, const void* X, void* C, int batch, int m, int 
  *
  *   in   [batch, rows, cols]  bf16 or fp32 (in_dtype), dense
  *   out  [batch, rows, cols]  bf16, dense, 16-byte aligned (DION_E_INVALID otherwise; batches that take
- *        the LDS-resident small-matrix kernel are exempt)
+ *        the small-matrix kernel are exempt)
  *   coeffs  host array of n_iters*3 floats (a,b,c per iteration)
  *   X0 = bf16(in) / (||bf16(in)||_F * norm_scale + eps)  per matrix, then n_iters times
  *   A = X X^T; B = b A + c A A; X = a X + B X   on the orientation with rows <= cols.

@@ -43,7 +43,7 @@ def test_line_1_and_2_all_tile_paths(batch, m, n):
     x64 = X.float().cpu().numpy().astype(np.float64)
     ref = x64 @ np.swapaxes(x64, -2, -1)
     mean, mx = _err(A, ref)
-    # (contiguous: batched bf16 products with a transposed right operand have faulted the GPU)
+    # (contiguous: a run with the transposed view here ended in an illegal access, reported after this product)
     bmean, bmx = _err(X @ X.mT.contiguous(), ref)
     assert mean <= bmean * 1.05 + 1e-6 and mx <= bmx * 1.5 + 1e-6
     assert torch.equal(A, A.mT)

@@ -1,7 +1,7 @@
 """The one-workgroup-per-matrix kernel (X in registers) at the edges of its row tiles, column groups and wavefront counts,
 tall and wide, at every alignment.  The reference is float64; the bound is the error of the same iteration carried out
 with torch in float32 with A, B and X rounded to bf16 where the kernel rounds them (factor 1.5: the sums run in another
-order)."""
+order; the scaled X too, which the forms beyond 64 x 1024 leave unrounded: test_the_norm_is_no_rounding_of_its_own)."""
 import pytest
 import torch
 
