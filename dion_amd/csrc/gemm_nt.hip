@@ -29,10 +29,11 @@ namespace dion {
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 #define GLB_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
 
-template <int BM_, int BN_, int BK_, int WM_, int WN_, int NSTAGE_>
+template <int BM_, int BN_, int BK_, int WM_, int WN_, int NSTAGE_, bool AHEAD_ = false>
 struct TileCfg {
+  static constexpr bool AHEAD = AHEAD_;  // fragments of a whole slab requested one slab ahead (see the kernel)
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, NSTAGE = NSTAGE_;
-  static_assert(NSTAGE_ == 2 || NSTAGE_ == 4, "two-slot ring, or a four-slot one for launches that leave a CU one workgroup");
+  static_assert(NSTAGE_ == 2 || (AHEAD_ && NSTAGE_ == 4), "two-slot ring, or a four-slot one for launches that leave a CU one workgroup");
   static constexpr int NT = WM * WN * 64;
   static constexpr int CPR = BK / 8;            // 16-byte chunks per tile row
   static constexpr int ROWS_PER_LOAD = NT / CPR; // tile rows covered by one load instruction
@@ -386,7 +387,7 @@ __device__ __forceinline__ void store_lines_bounded(const char* stg, int pitch, 
 // product of a call then needs no pass that drops the padding (4 x (2730 x 1000): 22 us; 12 x: 100), and no separate
 // update pass (65 us more).  256-wide tiles take this kernel for it, not the tile-walking one.
 template <class Cfg, bool HAS_D, bool HAS_C, bool HAS_CT, bool QK = false, int POST = 0, bool BND = false>
-__global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
+__global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, ST = Cfg::ST, HALVES = Cfg::HALVES, NSTAGE = Cfg::NSTAGE;
   constexpr int HP = HALVES * ST;  // halves (sixteen MFMAs each) per slab
@@ -494,81 +495,178 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
                                       (t16 & 3) * 8);
   }
 
-  typedef FragSched<HALVES, ST, QK> FS;
-  // A fragments: two sets of four, alternating by half; B fragments: two sets of TN, alternating by step
-  bf16x8 fa[2][4], fb[2][TN];
-  // Read r of the fragments half hn (0..HP-1) of ring slot buf needs: the first half of a step takes
-  // A0 B0 B1 B2 B3 A1 A2 A3 (r = 0..7), a second half its A fragments 4..7 (r = 0..3).  All compile-time
-  // constants, which end up in the instruction's offset field.
-  auto read_frag = [&](auto bufc, auto hnc, auto rc) {
-    constexpr int buf = decltype(bufc)::value, hn = decltype(hnc)::value, r = decltype(rc)::value;
-    constexpr int st = hn / HALVES, part = hn % HALVES, fs = hn & 1, bs = st & 1;
-    if constexpr (part != 0) {
-      lds_read16<buf * Cfg::P_BYTES + (4 + r) * (16 * BK * 2)>(fa[fs][r], aoff[st]);
-    } else if constexpr (r == 0 || r > 4) {
-      constexpr int i = r == 0 ? 0 : r - 4;
-      lds_read16<buf * Cfg::P_BYTES + i * (16 * BK * 2)>(fa[fs][i], aoff[st]);
-    } else if constexpr (QK) {
-      constexpr int j = r - 1;
-      lds_read_tr<buf * Cfg::Q_BYTES + st * (32 * BN * 2), 4 * BN * 2>(fb[bs][j], qoff[j]);
-    } else {
-      constexpr int j = r - 1;
-      lds_read16<buf * Cfg::Q_BYTES + j * (16 * BK * 2)>(fb[bs][j], boff[st]);
-    }
-  };
-  typedef std::integral_constant<int, 0> ic0;
-
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  typedef std::integral_constant<int, 0> ic0;
 
-  // ---- prologue: fill NSTAGE-1 ring slots, wait for slab 0, read its first fragments, start the
-  // last free slot.
-  constexpr bool DEEP = NSTAGE > 2;
-  auto ring_barrier = [&](int newer) {
-    // slabs newer than the one waited for that may still be in flight
-    constexpr int PL = Cfg::P_LOADS;
-    if (newer >= 2) { if (one_operand) pipeline_barrier<2 * PL>(); else pipeline_barrier<2 * LPS>(); }
-    else if (newer == 1) { if (one_operand) pipeline_barrier<PL>(); else pipeline_barrier<LPS>(); }
-    else pipeline_barrier<0>();
-  };
+  if constexpr (Cfg::AHEAD) {
+    // ---- main loop of 64 x 64 wavefront tiles (128-wide tiles).  A wavefront holds the fragments of a whole slab and
+    // requests those of the next one behind this one's MFMAs: one wait and one barrier per slab, and the slot of a
+    // slab is free for its refill a slab earlier than with fragments read half a slab ahead.  Four wavefronts share a
+    // CU's four SIMDs here, or eight with two workgroups, so nothing hides what a wavefront issues besides its MFMAs:
+    // an instruction costs four cycles, an MFMA sixteen, hence slots as constants of the unrolled loop and
+    // refills without address arithmetic.  What bounds it is the LDS: 64 KB of fragments and 32 KB of refills a slab are
+    // 750 cycles at 128 bytes per cycle, 512 are MFMA time; measured 0.31 us a slab (0.42 with half-slab fragments and
+    // accumulators in AGPRs, which the compiler copied around every MFMA: __launch_bounds__' second figure keeps
+    // them out).  X X^T of 12 x (768 x 3072) 29.1 -> 25.1 us, of 4 x (1024 x 2816) 24.1 -> 20.3, of 24 x (512 x 8192)
+    // 63.0 -> 54.1, of 8 x (1024 x 4096), two workgroups per CU, 49.1 -> 42.5; B X of 12 x (768 x 3072) 55.8 -> 46.4.  256 x 128 tiles
+    // on the same loop (eight wavefronts, three slots) are bound by the LDS alike: 0.57 us for twice the work, slower in a
+    // launch than either neighbour (12 x (768 x 768): 14.7 against 13.8 us).
+    static_assert(TM == 4 && ST == 2 && LPS <= 8, "64 x 64 wavefront tiles");
+    bf16x8 fa[2][ST][4], fb[2][ST][TN];  // by parity of the slab
+    // read r (0..15) of the fragments of the slab in ring slot `slotc`
+    auto read_frag = [&](auto slotc, auto rc) {
+      constexpr int slot = decltype(slotc)::value, par = slot & 1;
+      constexpr int r = decltype(rc)::value, st = r / 8, f = r % 8;
+      if constexpr (f < 4) lds_read16<slot * Cfg::P_BYTES + f * (16 * BK * 2)>(fa[par][st][f], aoff[st]);
+      else if constexpr (QK) lds_read_tr<slot * Cfg::Q_BYTES + st * (32 * BN * 2), 4 * BN * 2>(fb[par][st][f - 4], qoff[f - 4]);
+      else lds_read16<slot * Cfg::Q_BYTES + (f - 4) * (16 * BK * 2)>(fb[par][st][f - 4], boff[st]);
+    };
+    // every fragment of that parity has arrived
+    auto landed = [&](auto parc) {
+      auto& a = fa[decltype(parc)::value];
+      auto& b = fb[decltype(parc)::value];
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(a[0][0]), "+v"(a[0][1]), "+v"(a[0][2]), "+v"(a[0][3]), "+v"(a[1][0]), "+v"(a[1][1]), "+v"(a[1][2]),
+                     "+v"(a[1][3]));
+      asm volatile("" : "+v"(b[0][0]), "+v"(b[0][1]), "+v"(b[0][2]), "+v"(b[0][3]), "+v"(b[1][0]), "+v"(b[1][1]),
+                        "+v"(b[1][2]), "+v"(b[1][3]));
+    };
+    // Refills.  The slab is in the scalar base, the rows a load covers in a per-lane offset of its own: two scalar
+    // additions fewer per load (not for a K-major Q, 64 of whose rows may span more than a 32-bit offset).
+    constexpr int VOFF = QK ? Cfg::P_LOADS : LPS;
+    uint32_t voff[LPS];
 #pragma unroll
-  for (int s = 0; s < NSTAGE - 1; ++s)
-    if (!DEEP || s < KT)
+    for (int j = 0; j < LPS; ++j)
+      voff[j] = j < Cfg::P_LOADS ? offP + j * stepP : QK ? offQ : offQ + (j - Cfg::P_LOADS) * stepQ;
+    const char *nextP = gP, *nextQ = gQ;  // slab to load next
+    auto load = [&](int slot, auto jc) {
+      constexpr int j = decltype(jc)::value, jq = j - Cfg::P_LOADS;
+      if (one_operand && jq >= 0) return;
+      const char* src = jq < 0 ? nextP : j < VOFF ? nextQ : nextQ + (uint64_t)(jq < 0 ? 0 : jq) * stepQ;
+      char* l = jq < 0 ? lds + slot * Cfg::P_BYTES + j * (Cfg::NT * 16)
+                       : lds + NSTAGE * Cfg::P_BYTES + slot * Cfg::Q_BYTES + jq * (Cfg::NT * 16);
+      asm volatile("" : "+s"(src), "+v"(voff[j]));
+      __builtin_amdgcn_global_load_lds(GLB_PTR(src + voff[j]), LDS_PTR(l + wave * (64 * 16)), 16, 0, 0);
+    };
+    auto loaded = [&]() {
+      nextP += BK * 2;
+      nextQ += slabQ;
+    };
+    auto ring_barrier = [&](int newer) {
+      // slabs newer than the one waited for that may still be in flight
+      constexpr int PL = Cfg::P_LOADS;
+      if (NSTAGE > 3 && newer >= 3) { if (one_operand) pipeline_barrier<3 * PL>(); else pipeline_barrier<3 * LPS>(); }
+      else if (NSTAGE > 2 && newer == 2) { if (one_operand) pipeline_barrier<2 * PL>(); else pipeline_barrier<2 * LPS>(); }
+      else if (newer == 1) { if (one_operand) pipeline_barrier<PL>(); else pipeline_barrier<LPS>(); }
+      else pipeline_barrier<0>();
+    };
+    static_for<0, NSTAGE>([&](auto sc) {
+      if (decltype(sc)::value < KT) {
+        static_for<0, LPS>([&](auto jc) { load(decltype(sc)::value, jc); });
+        loaded();
+      }
+    });
+    ring_barrier((KT < NSTAGE ? KT : NSTAGE) - 1);
+    static_for<0, 16>([&](auto rc) { read_frag(ic0(), rc); });
+    // Slab kt, in slot kt % NSTAGE: its fragments are on their way or there, slab kt + 1 has to be in the ring, and slab
+    // kt + NSTAGE goes where this one was.
+    auto slab = [&](int kt, auto slotc, auto steady) {
+      constexpr int slot = decltype(slotc)::value, par = slot & 1;
+      typedef std::integral_constant<int, (slot + 1) % NSTAGE> nextc;
+      bool fill = true;
+      if constexpr (decltype(steady)::value) {
+        if (one_operand) pipeline_barrier<(NSTAGE - 2) * Cfg::P_LOADS>();
+        else pipeline_barrier<(NSTAGE - 2) * LPS>();
+      } else {
+        const int newest = kt + NSTAGE - 1 < KT - 1 ? kt + NSTAGE - 1 : KT - 1;
+        ring_barrier(newest - kt - 1);
+        fill = kt + NSTAGE < KT;
+      }
+      landed(std::integral_constant<int, par>());
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, 32>([&](auto qc) {
+        constexpr int q = decltype(qc)::value, st = q / 16, i = (q % 16) / 4, j = q % 4;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[par][st][i], fb[par][st][j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        // a refill behind every E-th MFMA: spread over the slab, or early in it where it is needed a slab later
+        constexpr int E = NSTAGE == 2 ? 2 : 4;
+        constexpr bool refill = q % E == E - 1 && q / E < LPS;
+        constexpr int before = q / E < LPS ? q / E : LPS;  // refills behind the MFMAs before this one
+        constexpr int r = q - before;
+        if constexpr (refill) {
+          if (fill) load(slot, std::integral_constant<int, q / E>());
+        } else if constexpr (r < 16) {
+          read_frag(nextc(), std::integral_constant<int, r>());
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      loaded();
+    };
+    int kt = 0;
+    for (; kt + 2 * NSTAGE <= KT; kt += NSTAGE)
+      static_for<0, NSTAGE>([&](auto sc) { slab(kt + decltype(sc)::value, sc, std::true_type()); });
+    for (; kt < KT; kt += NSTAGE)  // (KT is even)
+      static_for<0, NSTAGE>([&](auto sc) {
+        if (decltype(sc)::value < 2 || kt + decltype(sc)::value < KT) slab(kt + decltype(sc)::value, sc, std::false_type());
+      });
+    wait_vmcnt<0>();
+    landed(ic0());  // the reads behind the last slab's MFMAs, which nobody uses, before their registers are let go
 #pragma unroll
-      for (int j = 0; j < LPS; ++j) issue_load(s, s, j);
-  if constexpr (DEEP) ring_barrier((KT < NSTAGE - 1 ? KT : NSTAGE - 1) - 1);
-  else pipeline_barrier<(NSTAGE - 2) * LPS>();
-  static_for<0, 8>([&](auto rc) { read_frag(ic0(), ic0(), rc); });
-  if (!DEEP || NSTAGE - 1 < KT)
+    for (int st = 0; st < ST; ++st)
 #pragma unroll
-    for (int j = 0; j < (SPREAD ? LPS / 2 : LPS); ++j) issue_load(NSTAGE - 1, NSTAGE - 1, j);
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (DEEP) {
-    static_assert(!SPREAD, "");
-    int slot = 0;
-    auto slab = [&](int kt, auto refill) {
-      const int next = slot == NSTAGE - 1 ? 0 : slot + 1;
-      static_for<0, HP>([&](auto hc) {
-        constexpr int hp = decltype(hc)::value;
+      for (int i = 0; i < 4; ++i) {
+        asm volatile("" ::"v"(fa[0][st][i]));
+        asm volatile("" ::"v"(fb[0][st][i]));
+      }
+  } else {
+    typedef FragSched<HALVES, ST, QK> FS;
+    // A fragments: two sets of four, alternating by half; B fragments: two sets of TN, alternating by step
+    bf16x8 fa[2][4], fb[2][TN];
+    // Read r of the fragments half hn (0..HP-1) of ring slot buf needs: the first half of a step takes
+    // A0 B0 B1 B2 B3 A1 A2 A3 (r = 0..7), a second half its A fragments 4..7 (r = 0..3).  All compile-time
+    // constants, which end up in the instruction's offset field.
+    auto read_frag = [&](auto bufc, auto hnc, auto rc) {
+      constexpr int buf = decltype(bufc)::value, hn = decltype(hnc)::value, r = decltype(rc)::value;
+      constexpr int st = hn / HALVES, part = hn % HALVES, fs = hn & 1, bs = st & 1;
+      if constexpr (part != 0) {
+        lds_read16<buf * Cfg::P_BYTES + (4 + r) * (16 * BK * 2)>(fa[fs][r], aoff[st]);
+      } else if constexpr (r == 0 || r > 4) {
+        constexpr int i = r == 0 ? 0 : r - 4;
+        lds_read16<buf * Cfg::P_BYTES + i * (16 * BK * 2)>(fa[fs][i], aoff[st]);
+      } else if constexpr (QK) {
+        constexpr int j = r - 1;
+        lds_read_tr<buf * Cfg::Q_BYTES + st * (32 * BN * 2), 4 * BN * 2>(fb[bs][j], qoff[j]);
+      } else {
+        constexpr int j = r - 1;
+        lds_read16<buf * Cfg::Q_BYTES + j * (16 * BK * 2)>(fb[bs][j], boff[st]);
+      }
+    };
+
+    // ---- prologue: fill one ring slot, wait for slab 0, read its first fragments, start the other slot.
+    static_assert(NSTAGE == 2, "");
+#pragma unroll
+    for (int j = 0; j < LPS; ++j) issue_load(0, 0, j);
+    pipeline_barrier<0>();
+    static_for<0, 8>([&](auto rc) { read_frag(ic0(), ic0(), rc); });
+#pragma unroll
+    for (int j = 0; j < (SPREAD ? LPS / 2 : LPS); ++j) issue_load(1, 1, j);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- main loop.  Halves run back to back across slab boundaries: while the MFMAs of one half issue, the
+    // fragment reads of the next half (and, from the last half of a slab on, the refill of the slot that slab
+    // occupied) are slotted behind them.  sched_barrier pins that order.  KT is a multiple of NSTAGE
+    // (launcher checks) so ring slots are compile-time constants.
+    for (int kt0 = 0; kt0 < KT; kt0 += NSTAGE) {
+      static_for<0, NSTAGE * HP>([&](auto shc) {
+        constexpr int s = decltype(shc)::value / HP, hp = decltype(shc)::value % HP;
         constexpr int st = hp / HALVES, part = hp % HALVES, fs = hp & 1, bs = st & 1;
         constexpr bool last = (hp == HP - 1);
-        if constexpr (last) {
-          if constexpr (decltype(refill)::value) {
-            if (one_operand) pipeline_barrier<(NSTAGE - 2) * Cfg::P_LOADS>();
-            else pipeline_barrier<(NSTAGE - 2) * LPS>();
-          } else ring_barrier(KT - 2 - kt);
-          // every read of this slab has been issued and has returned: the address registers move to the next slot
-          const uint32_t d = (uint32_t)(next - slot) * (uint32_t)Cfg::P_BYTES;
-#pragma unroll
-          for (int t = 0; t < ST; ++t) { aoff[t] += d; if (!QK) boff[t] += d; }
-          if (QK)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) qoff[j] += d;
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        // slab kt+1 landed, slab kt fully read
+        if constexpr (last) pipeline_barrier<(NSTAGE - 2) * LPS>();
         static_for<0, NM>([&](auto qc) {
           constexpr int q = decltype(qc)::value, i = q / 4, j = q % 4;
           frag_wait<FS::allowed(hp, q)>(fa[fs][i], fb[bs][j]);
@@ -577,67 +675,34 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_nt_kernel(const GemmParams p, co
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (FS::read_behind(hp, q) >= 0) {
             typedef std::integral_constant<int, FS::read_behind(hp, q)> rc;
-            if constexpr (last) read_frag(ic0(), ic0(), rc());
-            else read_frag(ic0(), std::integral_constant<int, hp + 1>(), rc());
+            if constexpr (last) read_frag(std::integral_constant<int, (s + 1) % NSTAGE>(), ic0(), rc());
+            else read_frag(std::integral_constant<int, s>(), std::integral_constant<int, hp + 1>(), rc());
           }
-          if constexpr (decltype(refill)::value)
-            if constexpr (last && (q & 1) && q / 2 < LPS) issue_load(kt + NSTAGE, slot, q / 2);
+          if constexpr (SPREAD) {
+            if constexpr (last && q % 4 == 3 && q / 4 < LPS / 2) issue_load(kt0 + s + NSTAGE, s, q / 4);
+            if constexpr (hp == 0 && q % 4 == 3 && LPS / 2 + q / 4 < LPS)
+              issue_load(kt0 + s - 1 + NSTAGE, (s + NSTAGE - 1) % NSTAGE, LPS / 2 + q / 4);
+          } else {
+            if constexpr (last && (q & 1) && q / 2 < LPS) issue_load(kt0 + s + NSTAGE, s, q / 2);
+          }
           __builtin_amdgcn_sched_barrier(0);
         });
       });
-      slot = next;
-    };
-    int kt = 0;
-    for (; kt + NSTAGE < KT; ++kt) slab(kt, std::true_type());
-    for (; kt < KT; ++kt) slab(kt, std::false_type());
-  } else
-
-  // ---- main loop.  Halves run back to back across slab boundaries: while the MFMAs of one half issue, the
-  // fragment reads of the next half (and, from the last half of a slab on, the refill of the slot that slab
-  // occupied) are slotted behind them.  sched_barrier pins that order.  KT is a multiple of NSTAGE
-  // (launcher checks) so ring slots are compile-time constants.
-  for (int kt0 = 0; kt0 < KT; kt0 += NSTAGE) {
-    static_for<0, NSTAGE * HP>([&](auto shc) {
-      constexpr int s = decltype(shc)::value / HP, hp = decltype(shc)::value % HP;
-      constexpr int st = hp / HALVES, part = hp % HALVES, fs = hp & 1, bs = st & 1;
-      constexpr bool last = (hp == HP - 1);
-      // slab kt+1 landed, slab kt fully read
-      if constexpr (last) pipeline_barrier<(NSTAGE - 2) * LPS>();
-      static_for<0, NM>([&](auto qc) {
-        constexpr int q = decltype(qc)::value, i = q / 4, j = q % 4;
-        frag_wait<FS::allowed(hp, q)>(fa[fs][i], fb[bs][j]);
-        acc[part * 4 + i][j] =
-            __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[fs][i], fb[bs][j], acc[part * 4 + i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (FS::read_behind(hp, q) >= 0) {
-          typedef std::integral_constant<int, FS::read_behind(hp, q)> rc;
-          if constexpr (last) read_frag(std::integral_constant<int, (s + 1) % NSTAGE>(), ic0(), rc());
-          else read_frag(std::integral_constant<int, s>(), std::integral_constant<int, hp + 1>(), rc());
-        }
-        if constexpr (SPREAD) {
-          if constexpr (last && q % 4 == 3 && q / 4 < LPS / 2) issue_load(kt0 + s + NSTAGE, s, q / 4);
-          if constexpr (hp == 0 && q % 4 == 3 && LPS / 2 + q / 4 < LPS)
-            issue_load(kt0 + s - 1 + NSTAGE, (s + NSTAGE - 1) % NSTAGE, LPS / 2 + q / 4);
-        } else {
-          if constexpr (last && (q & 1) && q / 2 < LPS) issue_load(kt0 + s + NSTAGE, s, q / 2);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      });
-    });
-  }
-  wait_vmcnt<0>();  // drain the redundant tail refills before LDS is reused / the wave exits
-  // The read-ahead of the last half issued reads whose results nobody uses.  The compiler does not know
-  // they are in flight; were their destination registers dead here, it would hand them to whatever comes
-  // next (the lane index, store addresses) and a read landing late would overwrite that.  So: wait for the
-  // LDS queue to drain, and only then let go of the fragment registers -- the empty asm statements below
-  // are their last use and sit behind the wait.
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    wait_vmcnt<0>();  // drain the redundant tail refills before LDS is reused / the wave exits
+    // The read-ahead of the last half issued reads whose results nobody uses.  The compiler does not know
+    // they are in flight; were their destination registers dead here, it would hand them to whatever comes
+    // next (the lane index, store addresses) and a read landing late would overwrite that.  So: wait for the
+    // LDS queue to drain, and only then let go of the fragment registers -- the empty asm statements below
+    // are their last use and sit behind the wait.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-  for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < 2; ++f) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) asm volatile("" ::"v"(fa[f][i]));
+      for (int i = 0; i < 4; ++i) asm volatile("" ::"v"(fa[f][i]));
 #pragma unroll
-    for (int j = 0; j < TN; ++j) asm volatile("" ::"v"(fb[f][j]));
+      for (int j = 0; j < TN; ++j) asm volatile("" ::"v"(fb[f][j]));
+    }
   }
 
   // ---- epilogue.  Accumulator element e of lane l holds row 4 * (l / 16) + e, column l % 16 of its 16 x 16
@@ -1118,7 +1183,7 @@ struct CfgK64 {
 };
 
 template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0, bool BND = false>
-__global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
+__global__ __launch_bounds__(CfgK64::NT, 2) void gemm_k64_kernel(const GemmParams p, const typename PostSel<POST>::arg post) {
   typedef CfgK64 Cfg;
   typedef typename PostSel<POST>::xt XT;
   constexpr int OPB = Cfg::OP_BYTES, KW = Cfg::KW, BK = Cfg::BK;
@@ -1388,9 +1453,9 @@ __global__ __launch_bounds__(CfgK64::NT) void gemm_k64_kernel(const GemmParams p
 }
 
 // ---------------------------------------------------------------------------------------------
-typedef TileCfg<128, 128, 64, 2, 2, 2> Cfg128;     // 4 wavefronts, 64x64 each; two workgroups per CU
-typedef TileCfg<128, 128, 64, 2, 2, 4> Cfg128d;    // the same on a four-slot ring: one workgroup per CU
-typedef TileCfg<256, 256, 64, 2, 4, 2> Cfg256w8;   // 8 wavefronts, 128x64 each: two per SIMD, one workgroup per CU
+typedef TileCfg<128, 128, 64, 2, 2, 2, true> Cfg128;   // 4 wavefronts, 64x64 each; two workgroups per CU
+typedef TileCfg<128, 128, 64, 2, 2, 4, true> Cfg128d;  // the same on a four-slot ring: one workgroup per CU
+typedef TileCfg<256, 256, 64, 2, 4, 2> Cfg256w8;       // 8 wavefronts, 128x64 each: two per SIMD, one workgroup per CU
 constexpr int kWalkMaxK = 2048;                    // longest reduction the tile-walking kernel is used for
 
 // Tile list dealt to the XCDs in interleaved 32-tile chunks (see the kernel) when the first operand of

@@ -84,3 +84,30 @@ def test_fused_update_of_few_tiles(shape, cautious, dtype):
                                                           (14, 512, 256, 64, 128)])
 def test_products_at_the_line_of_short_reductions(batch, m, n, sym_edge, full_edge):
     test_products_of_few_tiles(batch, m, n, sym_edge, full_edge)
+
+
+# Slab counts (64 columns of the reduction each) from fewer than a ring has slots, remainders of its length among them.
+@pytest.mark.parametrize("batch", [14, 30])  # 140 tiles on the four-slot ring, 300 on the two-slot one
+@pytest.mark.parametrize("n", [128, 256, 384, 512, 640, 768, 896, 1152])
+def test_reduction_lengths_of_symmetric_products(batch, n):
+    lib, check, st = _lib()
+    g = torch.Generator(device=DEV).manual_seed(n)
+    X = torch.randn(batch, 512, n, device=DEV, generator=g).to(torch.bfloat16)
+    A = torch.full((batch, 512, 512), float("nan"), device=DEV, dtype=torch.bfloat16)
+    check(lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), batch, 512, n, st), "line_1")
+    _close(A, X.double() @ X.double().mT.contiguous())
+    assert torch.equal(A, A.mT)
+
+
+@pytest.mark.parametrize("m", [128, 256, 384, 512, 640, 1152])
+def test_reduction_lengths_of_products_with_a_k_major_operand(m):
+    lib, check, st = _lib()
+    batch, n = -(-38400 // m), 256  # 300 tiles and a few more
+    assert lib.dion_gemm_tile_edge(batch, m, n, 0) == 128
+    g = torch.Generator(device=DEV).manual_seed(m)
+    B = torch.randn(batch, m, m, device=DEV, generator=g)
+    B = (B + B.mT).to(torch.bfloat16)
+    X = torch.randn(batch, m, n, device=DEV, generator=g).to(torch.bfloat16)
+    Y = torch.full_like(X, float("nan"))
+    check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, n, ctypes.c_float(0.0), st), "line_3")
+    _close(Y, B.double() @ X.double())
