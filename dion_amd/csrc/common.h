@@ -234,6 +234,7 @@ struct GemmParams {
   int tri;           // 1: Q == P, only tiles with tile_row <= tile_col are computed, Ct mirrors
   int q_kmajor;      // 1: Q is stored [K][N] (reduction index along rows); not with tri
   int xcd_interleave;  // set by the launcher: tile list dealt to the XCDs in interleaved 32-tile chunks
+  uint32_t inv_mat, inv_group, inv_tail;  // set by the launcher: reciprocals of the tile list's divisors
   float alpha, beta;
   float diag;        // added to C[i][i] (global diagonal); used with tri to fold a*I into B
   // Optional per-matrix factor of the product, read on the device: matrix b is scaled by
@@ -244,10 +245,9 @@ struct GemmParams {
   int scale_pow;
 };
 
-// alpha of matrix b of a launch (see GemmParams::scale_vec)
-__device__ __forceinline__ float gemm_alpha(const GemmParams& p, int b) {
+// alpha of a matrix whose entry of GemmParams::scale_vec is s
+__device__ __forceinline__ float gemm_alpha(const GemmParams& p, float s) {
   if (!p.scale_vec) return p.alpha;
-  const float s = p.scale_vec[b];
   return p.alpha * (p.scale_pow == 2 ? s * s : s);
 }
 

@@ -152,6 +152,18 @@ __device__ __forceinline__ void lds_read_tr(bf16x8& dst, uint32_t addr) {
   dst = __builtin_bit_cast(bf16x8, v);
 }
 
+// Eight transposing reads and the wait for them in one statement (through the builtin, the compiler waits for every
+// outstanding store before each of them).
+typedef __attribute__((ext_vector_type(2))) unsigned tr_u32x2;
+__device__ __forceinline__ void lds_read_tr8(tr_u32x2 (&d)[8], const uint32_t (&a)[8]) {
+  asm volatile("ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %9\n\tds_read_b64_tr_b16 %2, %10\n\t"
+               "ds_read_b64_tr_b16 %3, %11\n\tds_read_b64_tr_b16 %4, %12\n\tds_read_b64_tr_b16 %5, %13\n\t"
+               "ds_read_b64_tr_b16 %6, %14\n\tds_read_b64_tr_b16 %7, %15\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(d[0]), "=&v"(d[1]), "=&v"(d[2]), "=&v"(d[3]), "=&v"(d[4]), "=&v"(d[5]), "=&v"(d[6]), "=&v"(d[7])
+               : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7])
+               : "memory");
+}
+
 // Enumeration of the upper triangle (ti <= tj) of a T x T tile grid in super-blocks of SB x SB
 // tiles, so that the ~32 workgroups an XCD runs side by side touch as few distinct operand row
 // blocks as possible (their L2 is what feeds the LDS): a diagonal super-block has SB(SB+1)/2
@@ -192,15 +204,27 @@ __device__ __forceinline__ void tri_tile(int t, int T, int& ti, int& tj) {
   ti = tj = 0;  // unreachable for t < T(T+1)/2
 }
 
+// Quotient and remainder by a divisor the host knows: inv = (2^32 - 1) / d gives the quotient or one less for x < 2^31.
+__device__ __forceinline__ int div_known(int x, int d, uint32_t inv, int& rem) {
+  int q = (int)__umulhi((uint32_t)x, inv);
+  rem = x - q * d;
+  if (rem >= d) {
+    rem -= d;
+    ++q;
+  }
+  return q;
+}
+
 // Tile number `pid` of a launch of `total` tiles -> (batch, tile row, tile column).  Hardware deals workgroups
 // round-robin over the 8 XCDs; each XCD (own L2) gets one contiguous run of the tile list, so that neighbours share
 // operands, or -- xcd_interleave -- 32 consecutive tiles of every 256: the 8 XCDs then work on neighbouring tile
 // groups (same matrix, same operand row panels) at the same time, and what one of them fetches from memory the
 // others find in the memory-side cache.  The latter pays when a matrix's operands are much larger than an XCD's L2.
-template <int BM, int BN>
+// Every workgroup starts with this, alone on its CU: no division by a number the host can divide by (four of them and
+// the triangle's loop were 0.5 us of the 9 us a launch of 10 x (640 x 640) takes).
+template <int BM, int BN, bool TRI>
 __device__ __forceinline__ void tile_of(const GemmParams& p, int pid, int total, int& b, int& ti, int& tj) {
   const int tilesM = p.M / BM, tilesN = p.N / BN;
-  const int tiles_per_mat = p.tri ? (tilesM * (tilesM + 1)) / 2 : tilesM * tilesN;
   int lt;
   if (p.xcd_interleave && pid < (total & ~255)) {
     const int j = pid & 255;
@@ -212,24 +236,60 @@ __device__ __forceinline__ void tile_of(const GemmParams& p, int pid, int total,
     const int q = total >> 3, r = total & 7;
     lt = xcd * q + (xcd < r ? xcd : r) + loc;
   }
-  b = lt / tiles_per_mat;
-  const int t = lt - b * tiles_per_mat;
-  if (p.tri) {
-    tri_tile(t, tilesM, ti, tj);
+  int t;
+  if constexpr (TRI) {
+    b = div_known(lt, (tilesM * (tilesM + 1)) / 2, p.inv_mat, t);
+    if (tilesM <= 8) {
+      // row-major triangle: tile row i starts at i * tilesM - i (i - 1) / 2.  The root is off by less than one.  (Wider ones
+      // stay in super-blocks: X X^T of one 768 x 3072 on 64-wide tiles 10.2 us so, 12.9 row by row.)
+      const float e = (float)(2 * tilesM + 1);
+      int i = (int)(0.5f * (e - __builtin_amdgcn_sqrtf(e * e - 8.0f * (float)t)));
+      i = __builtin_amdgcn_readfirstlane(i);
+      int start = i * tilesM - i * (i - 1) / 2;
+      if (t < start) {
+        --i;
+        start -= tilesM - i;
+      } else if (t >= start + tilesM - i) {
+        start += tilesM - i;
+        ++i;
+      }
+      ti = i;
+      tj = i + t - start;
+    } else {
+      tri_tile(t, tilesM, ti, tj);
+    }
   } else {
     constexpr int GM = 8;
     const int per_group = GM * tilesN;
-    const int g = t / per_group;
-    const int first = g * GM;
-    const int gsz = (tilesM - first) < GM ? (tilesM - first) : GM;
-    const int tg = t - g * per_group;
-    ti = first + tg % gsz;
-    tj = tg / gsz;
+    b = div_known(lt, tilesM * tilesN, p.inv_mat, t);
+    int tg;
+    const int first = div_known(t, per_group, p.inv_group, tg) * GM;
+    if (tilesM - first >= GM) {
+      ti = first + (tg & (GM - 1));
+      tj = tg / GM;
+    } else {
+      int row;
+      tj = div_known(tg, tilesM - first, p.inv_tail, row);
+      ti = first + row;
+    }
   }
   // (the same for every lane: say so, tile bases live in scalar registers)
   b = __builtin_amdgcn_readfirstlane(b);
   ti = __builtin_amdgcn_readfirstlane(ti);
   tj = __builtin_amdgcn_readfirstlane(tj);
+}
+
+// What tile_of needs of the host: the reciprocals of its divisors (tiles of a matrix, of a group of eight tile rows, rows
+// of the last group), and the order of the list.
+static void set_tile_order(GemmParams& p, int bm, int bn) {
+  const int64_t tm = p.M / bm, tn = p.N / bn;
+  const int64_t per_mat = p.tri ? tm * (tm + 1) / 2 : tm * tn;
+  p.inv_mat = (uint32_t)(0xffffffffu / per_mat);
+  p.inv_group = (uint32_t)(0xffffffffu / (8 * tn));
+  p.inv_tail = tm % 8 ? (uint32_t)(0xffffffffu / (tm % 8)) : 0;
+  // interleaved 32-tile chunks when the first operand of one matrix is at least 16 MB; below that a contiguous run per
+  // XCD keeps whole matrices in one L2
+  p.xcd_interleave = (int64_t)p.M * p.K * 2 >= (16L << 20) ? 1 : 0;
 }
 
 // Workgroup barrier preceded by the counter waits the software pipeline needs: every LDS read
@@ -408,7 +468,9 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
 
   int b, ti, tj;
-  tile_of<BM, BN>(p, blockIdx.x, gridDim.x, b, ti, tj);
+  constexpr bool TRI = HAS_C && HAS_CT && !QK;  // (the launcher's combinations)
+  tile_of<BM, BN, TRI>(p, blockIdx.x, gridDim.x, b, ti, tj);
+  const float factor = p.scale_vec ? p.scale_vec[b] : 1.0f;  // (requested here, used behind the main loop)
 
   // ---- global -> LDS addressing.  Chunk q = j*NT + tid of a tile lands at LDS byte q*16; it holds
   // logical 16-byte chunk (q % CPR) ^ swz(row) of tile row q / CPR.
@@ -441,7 +503,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
   // A diagonal tile of a symmetric product of one matrix with itself (A = X X^T, A A) needs one operand
   // tile, not two: Q's loads are skipped and its fragments are read from P's half of the slot.  (With a
   // two-slot ring the barrier waits for every outstanding load, so the load count per slab is free to vary.)
-  const bool one_operand = !QK && p.tri && ti == tj && p.P == p.Q && p.ldp == p.ldq && p.strideP == p.strideQ;
+  const bool one_operand = !QK && TRI && ti == tj && p.P == p.Q && p.ldp == p.ldq && p.strideP == p.strideQ;
   // LDS layout of the ring: [P slot 0][P slot 1][Q slot 0][Q slot 1].  With the two slots of an operand
   // side by side, slot, wavefront-tile row block and k step all fit the offset field of the LDS read
   // instructions: the per-lane address registers below are all the address arithmetic the loop needs.
@@ -465,6 +527,22 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
       __builtin_amdgcn_global_load_lds(GLB_PTR(src + offQ), LDS_PTR(l + NSTAGE * Cfg::P_BYTES + jq * (Cfg::NT * 16)),
                                        16, 0, 0);
     }
+  };
+
+  // ---- addend.  A wavefront fetches its part of D with direct-to-LDS loads into its own eighths of a ring slot that is
+  // no longer needed: 64 rows of 128 bytes, load n brings rows 8 n .. 8 n + 7, the 16-byte chunk c of row r lies at
+  // c ^ 2 * ((r >> 1) & 3), so that the transposing reads of the epilogue cover all banks.
+  constexpr int D_LOADS = 8;
+  static_assert(!HAS_D || LPS == D_LOADS, "a wavefront's share of a slot is 64 rows of 64 columns");
+  const char* gD = HAS_D ? (const char*)(p.D + (int64_t)b * p.strideD + (int64_t)(ti * BM + wm * Cfg::WTM) * p.ldd +
+                                         tj * BN + wn * Cfg::WTN)
+                         : nullptr;
+  uint32_t offD = HAS_D ? (uint32_t)((lane >> 3) * p.ldd + ((lane & 7) ^ ((lane >> 4) << 1)) * 8) * 2u : 0;
+  auto issue_addend = [&](int buf, int h, int n) {  // rows 64 h + 8 n .. of the wavefront tile, into slot buf
+    const char* src = gD + (int64_t)(h * 64 + n * 8) * p.ldd * 2;
+    char* l = lds + buf * Cfg::P_BYTES + wave * (64 * 16) + (n & 3) * (Cfg::NT * 16) + (n >> 2) * (NSTAGE * Cfg::P_BYTES);
+    asm volatile("" : "+s"(src), "+v"(offD));
+    __builtin_amdgcn_global_load_lds(GLB_PTR(src + offD), LDS_PTR(l), 16, 0, 0);
   };
 
   // ---- LDS -> register fragment addressing.  A fragment of v_mfma_f32_16x16x32_bf16: lane l holds row (or
@@ -509,17 +587,19 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
     // CU's four SIMDs here, or eight with two workgroups, so nothing hides what a wavefront issues besides its MFMAs:
     // an instruction costs four cycles, an MFMA sixteen, hence slots as constants of the unrolled loop and
     // refills without address arithmetic.  What bounds it is the LDS: 64 KB of fragments and 32 KB of refills a slab are
-    // 750 cycles at 128 bytes per cycle, 512 are MFMA time; measured 0.31 us a slab (0.42 with half-slab fragments and
-    // accumulators in AGPRs, which the compiler copied around every MFMA: __launch_bounds__' second figure keeps
-    // them out).  X X^T of 12 x (768 x 3072) 29.1 -> 25.1 us, of 4 x (1024 x 2816) 24.1 -> 20.3, of 24 x (512 x 8192)
-    // 63.0 -> 54.1, of 8 x (1024 x 4096), two workgroups per CU, 49.1 -> 42.5; B X of 12 x (768 x 3072) 55.8 -> 46.4.  256 x 128 tiles
+    // 750 cycles at 128 bytes per cycle, 512 are MFMA time; measured 0.31 us a slab of a long reduction (0.42 with half-slab
+    // fragments and accumulators in AGPRs, which the compiler copied around every MFMA: __launch_bounds__' second figure
+    // keeps them out).  Short reductions pay for what is outside: first loads 1.3 us behind the tile's coordinates, the
+    // epilogue 1.4.  X X^T of 12 x (768 x 3072) 27.1 -> 24.4 us, of 4 x (1024 x 2816) 23.1 -> 19.8, of 24 x (512 x 8192)
+    // 62.6 -> 51.7, of 8 x (1024 x 4096), two workgroups per CU, 49.6 -> 41.2, of 10 x (640 x 640) 9.5 -> 8.3, A A of
+    // those 10.6 -> 9.1, of 24 x (512 x 512) 10.4 -> 9.1; B X of 10 x (640 x 640) 9.5 -> 8.7.  256 x 128 tiles
     // on the same loop (eight wavefronts, three slots) are bound by the LDS alike: 0.57 us for twice the work, slower in a
     // launch than either neighbour (12 x (768 x 768): 14.7 against 13.8 us).
     static_assert(TM == 4 && ST == 2 && LPS <= 8, "64 x 64 wavefront tiles");
     bf16x8 fa[2][ST][4], fb[2][ST][TN];  // by parity of the slab
-    // read r (0..15) of the fragments of the slab in ring slot `slotc`
+    // read r (0..15) of the fragments of the slab in ring slot `slotc` (0, 1) of the pair the offsets point to
     auto read_frag = [&](auto slotc, auto rc) {
-      constexpr int slot = decltype(slotc)::value, par = slot & 1;
+      constexpr int slot = decltype(slotc)::value, par = slot;
       constexpr int r = decltype(rc)::value, st = r / 8, f = r % 8;
       if constexpr (f < 4) lds_read16<slot * Cfg::P_BYTES + f * (16 * BK * 2)>(fa[par][st][f], aoff[st]);
       else if constexpr (QK) lds_read_tr<slot * Cfg::Q_BYTES + st * (32 * BN * 2), 4 * BN * 2>(fb[par][st][f - 4], qoff[f - 4]);
@@ -535,84 +615,97 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
       asm volatile("" : "+v"(b[0][0]), "+v"(b[0][1]), "+v"(b[0][2]), "+v"(b[0][3]), "+v"(b[1][0]), "+v"(b[1][1]),
                         "+v"(b[1][2]), "+v"(b[1][3]));
     };
-    // Refills.  The slab is in the scalar base, the rows a load covers in a per-lane offset of its own: two scalar
-    // additions fewer per load (not for a K-major Q, 64 of whose rows may span more than a 32-bit offset).
-    constexpr int VOFF = QK ? Cfg::P_LOADS : LPS;
+    // Refills go through buffer descriptors, always LPS of them per slab.  Those past the last slab -- and all of Q's on a
+    // tile that has one operand -- have a descriptor of no records, so they touch no memory; the loop is the same
+    // code for every slab, and the waits are constants.  (With branches around the loads of the last slabs those slabs
+    // ran in a second copy of the loop, cold, with a branch per load: X X^T of 10 x (640 x 640) had six of its ten slabs
+    // there.)  The place behind the last slab is the addend's.
+    const char *nextP = gP, *nextQ = gQ;  // what to load next
     uint32_t voff[LPS];
 #pragma unroll
     for (int j = 0; j < LPS; ++j)
       voff[j] = j < Cfg::P_LOADS ? offP + j * stepP : QK ? offQ : offQ + (j - Cfg::P_LOADS) * stepQ;
-    const char *nextP = gP, *nextQ = gQ;  // slab to load next
-    auto load = [&](int slot, auto jc) {
-      constexpr int j = decltype(jc)::value, jq = j - Cfg::P_LOADS;
-      if (one_operand && jq >= 0) return;
-      const char* src = jq < 0 ? nextP : j < VOFF ? nextQ : nextQ + (uint64_t)(jq < 0 ? 0 : jq) * stepQ;
-      char* l = jq < 0 ? lds + slot * Cfg::P_BYTES + j * (Cfg::NT * 16)
-                       : lds + NSTAGE * Cfg::P_BYTES + slot * Cfg::Q_BYTES + jq * (Cfg::NT * 16);
-      asm volatile("" : "+s"(src), "+v"(voff[j]));
-      __builtin_amdgcn_global_load_lds(GLB_PTR(src + voff[j]), LDS_PTR(l + wave * (64 * 16)), 16, 0, 0);
+    uint64_t rowsQ = QK ? stepQ : 0;  // between two loads of a K-major Q, 64 of whose rows may span more than a 32-bit offset
+    const int keepQ = __builtin_amdgcn_readfirstlane(one_operand ? 0 : -1);
+    int recsP = -1, recsQ = keepQ, nxt = 0;
+    auto load = [&](int slot_at, auto jc) {  // slot_at: offset of the slot in either operand's half of the ring
+      constexpr int j = decltype(jc)::value, jq = j < Cfg::P_LOADS ? 0 : j - Cfg::P_LOADS;
+      const char* src = j < Cfg::P_LOADS ? nextP : QK ? nextQ + jq * rowsQ : nextQ;
+      char* l = lds + slot_at + (j < Cfg::P_LOADS ? j * (Cfg::NT * 16) : NSTAGE * Cfg::P_BYTES + jq * (Cfg::NT * 16));
+      const __amdgpu_buffer_rsrc_t rs =
+          __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, j < Cfg::P_LOADS ? recsP : recsQ, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS_PTR(l + wave * (64 * 16)), 16, (int)voff[j], 0, 0, 0);
     };
     auto loaded = [&]() {
-      nextP += BK * 2;
-      nextQ += slabQ;
-    };
-    auto ring_barrier = [&](int newer) {
-      // slabs newer than the one waited for that may still be in flight
-      constexpr int PL = Cfg::P_LOADS;
-      if (NSTAGE > 3 && newer >= 3) { if (one_operand) pipeline_barrier<3 * PL>(); else pipeline_barrier<3 * LPS>(); }
-      else if (NSTAGE > 2 && newer == 2) { if (one_operand) pipeline_barrier<2 * PL>(); else pipeline_barrier<2 * LPS>(); }
-      else if (newer == 1) { if (one_operand) pipeline_barrier<PL>(); else pipeline_barrier<LPS>(); }
-      else pipeline_barrier<0>();
+      ++nxt;
+      int left = nxt - KT;
+      asm volatile("" : "+s"(left));  // (recognised as a comparison, its result would come through vector registers)
+      recsP = left >> 31;  // all ones while there are slabs
+      recsQ = recsP & keepQ;
+      nextP += recsP & (BK * 2);
+      nextQ += (int64_t)recsP & slabQ;
+      if constexpr (HAS_D) {
+        if (nxt == KT) {
+          // loads 0-3 bring rows 0-31 of the wavefront's part of D, loads 4-7 rows 32-63
+          nextP = gD;
+          nextQ = gD + (int64_t)32 * p.ldd * 2;
+          rowsQ = 0;
+          recsP = recsQ = -1;
+#pragma unroll
+          for (int j = 0; j < LPS; ++j) voff[j] = offD + (uint32_t)((j & 3) * 8 * p.ldd) * 2u;
+        }
+      }
     };
     static_for<0, NSTAGE>([&](auto sc) {
-      if (decltype(sc)::value < KT) {
-        static_for<0, LPS>([&](auto jc) { load(decltype(sc)::value, jc); });
-        loaded();
-      }
+      static_for<0, LPS>([&](auto jc) { load(decltype(sc)::value * Cfg::P_BYTES, jc); });
+      loaded();
     });
-    ring_barrier((KT < NSTAGE ? KT : NSTAGE) - 1);
+    pipeline_barrier<(NSTAGE - 1) * LPS>();
     static_for<0, 16>([&](auto rc) { read_frag(ic0(), rc); });
     // Slab kt, in slot kt % NSTAGE: its fragments are on their way or there, slab kt + 1 has to be in the ring, and slab
-    // kt + NSTAGE goes where this one was.
-    auto slab = [&](int kt, auto slotc, auto steady) {
-      constexpr int slot = decltype(slotc)::value, par = slot & 1;
-      typedef std::integral_constant<int, (slot + 1) % NSTAGE> nextc;
-      bool fill = true;
-      if constexpr (decltype(steady)::value) {
-        if (one_operand) pipeline_barrier<(NSTAGE - 2) * Cfg::P_LOADS>();
-        else pipeline_barrier<(NSTAGE - 2) * LPS>();
-      } else {
-        const int newest = kt + NSTAGE - 1 < KT - 1 ? kt + NSTAGE - 1 : KT - 1;
-        ring_barrier(newest - kt - 1);
-        fill = kt + NSTAGE < KT;
+    // kt + NSTAGE goes where this one was.  The loop is two slabs long; in a four-slot ring the addresses alternate
+    // between the two pairs of slots.
+    uint32_t to_pair = NSTAGE == 4 ? 2 * Cfg::P_BYTES : 0;  // from this pair to the other, then back
+    int pair_at = 0;
+    auto slab = [&](auto slotc) {
+      constexpr int slot = decltype(slotc)::value;
+      typedef std::integral_constant<int, slot ^ 1> nextc;
+      pipeline_barrier<(NSTAGE - 2) * LPS>();
+      landed(slotc);
+      if constexpr (NSTAGE == 4 && slot == 1) {
+#pragma unroll
+        for (int st = 0; st < ST; ++st) {
+          aoff[st] += to_pair;
+          if (!QK) boff[st] += to_pair;
+        }
+        if (QK)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) qoff[j] += to_pair;
       }
-      landed(std::integral_constant<int, par>());
       __builtin_amdgcn_sched_barrier(0);
       static_for<0, 32>([&](auto qc) {
         constexpr int q = decltype(qc)::value, st = q / 16, i = (q % 16) / 4, j = q % 4;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[par][st][i], fb[par][st][j], acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[slot][st][i], fb[slot][st][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         // a refill behind every E-th MFMA: spread over the slab, or early in it where it is needed a slab later
         constexpr int E = NSTAGE == 2 ? 2 : 4;
         constexpr bool refill = q % E == E - 1 && q / E < LPS;
         constexpr int before = q / E < LPS ? q / E : LPS;  // refills behind the MFMAs before this one
         constexpr int r = q - before;
-        if constexpr (refill) {
-          if (fill) load(slot, std::integral_constant<int, q / E>());
-        } else if constexpr (r < 16) {
-          read_frag(nextc(), std::integral_constant<int, r>());
-        }
+        if constexpr (refill) load(pair_at + slot * Cfg::P_BYTES, std::integral_constant<int, q / E>());
+        else if constexpr (r < 16) read_frag(nextc(), std::integral_constant<int, r>());
         __builtin_amdgcn_sched_barrier(0);
       });
       loaded();
+      if constexpr (NSTAGE == 4 && slot == 1) {
+        pair_at += (int)to_pair;
+        to_pair = 0u - to_pair;
+      }
     };
-    int kt = 0;
-    for (; kt + 2 * NSTAGE <= KT; kt += NSTAGE)
-      static_for<0, NSTAGE>([&](auto sc) { slab(kt + decltype(sc)::value, sc, std::true_type()); });
-    for (; kt < KT; kt += NSTAGE)  // (KT is even)
-      static_for<0, NSTAGE>([&](auto sc) {
-        if (decltype(sc)::value < 2 || kt + decltype(sc)::value < KT) slab(kt + decltype(sc)::value, sc, std::false_type());
-      });
+    for (int kt = 0; kt < KT; kt += 2) {  // (KT is even)
+      slab(ic0());
+      slab(std::integral_constant<int, 1>());
+    }
     wait_vmcnt<0>();
     landed(ic0());  // the reads behind the last slab's MFMAs, which nobody uses, before their registers are let go
 #pragma unroll
@@ -659,8 +752,9 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
     // ---- main loop.  Halves run back to back across slab boundaries: while the MFMAs of one half issue, the
     // fragment reads of the next half (and, from the last half of a slab on, the refill of the slot that slab
     // occupied) are slotted behind them.  sched_barrier pins that order.  KT is a multiple of NSTAGE
-    // (launcher checks) so ring slots are compile-time constants.
-    for (int kt0 = 0; kt0 < KT; kt0 += NSTAGE) {
+    // (launcher checks) so ring slots are compile-time constants.  The refills of the last round have no slab to
+    // fetch: they bring the addend, whose 64-row blocks are as large as a wavefront's share of a slot.
+    auto round = [&](int kt0, auto finalc) {
       static_for<0, NSTAGE * HP>([&](auto shc) {
         constexpr int s = decltype(shc)::value / HP, hp = decltype(shc)::value % HP;
         constexpr int st = hp / HALVES, part = hp % HALVES, fs = hp & 1, bs = st & 1;
@@ -682,13 +776,17 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
             if constexpr (last && q % 4 == 3 && q / 4 < LPS / 2) issue_load(kt0 + s + NSTAGE, s, q / 4);
             if constexpr (hp == 0 && q % 4 == 3 && LPS / 2 + q / 4 < LPS)
               issue_load(kt0 + s - 1 + NSTAGE, (s + NSTAGE - 1) % NSTAGE, LPS / 2 + q / 4);
-          } else {
-            if constexpr (last && (q & 1) && q / 2 < LPS) issue_load(kt0 + s + NSTAGE, s, q / 2);
+          } else if constexpr (last && (q & 1) && q / 2 < LPS) {
+            if constexpr (HAS_D && decltype(finalc)::value) issue_addend(s, s, q / 2);
+            else issue_load(kt0 + s + NSTAGE, s, q / 2);
           }
           __builtin_amdgcn_sched_barrier(0);
         });
       });
-    }
+    };
+    int kt0 = 0;
+    for (; kt0 + (HAS_D ? NSTAGE : 0) < KT; kt0 += NSTAGE) round(kt0, std::false_type());
+    if constexpr (HAS_D) round(kt0, std::true_type());
     wait_vmcnt<0>();  // drain the redundant tail refills before LDS is reused / the wave exits
     // The read-ahead of the last half issued reads whose results nobody uses.  The compiler does not know
     // they are in flight; were their destination registers dead here, it would hand them to whatever comes
@@ -706,22 +804,96 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
   }
 
   // ---- epilogue.  Accumulator element e of lane l holds row 4 * (l / 16) + e, column l % 16 of its 16 x 16
-  // tile.  Whole tiles are stored: destinations are padded to the tile.  C goes out straight from registers
-  // (16 lanes x 2 B = one 32-byte run per row and instruction, neighbouring tiles completing the lines).
-  // The transposed copy would be 8-byte pieces scattered over 16 rows per instruction, so it is staged
-  // through LDS ([column][row], this wavefront's private slice) and stored as 16 bytes per lane with
-  // 256-byte runs per row.
-  const float alpha = gemm_alpha(p, b), beta = p.beta;
+  // tile.  Whole tiles are stored: destinations are padded to the tile.
+  const float alpha = gemm_alpha(p, factor), beta = p.beta;
   const int row_base = ti * BM + wm * Cfg::WTM;
   const int col_base = tj * BN + wn * Cfg::WTN;
-  const bool mirror = HAS_CT && !(p.tri && ti == tj);  // a diagonal tile is its own mirror
-  const bf16_t* Dp = HAS_D ? p.D + (int64_t)b * p.strideD + (int64_t)(row_base + 4 * quad) * p.ldd +
-                                 col_base + l16
-                           : nullptr;
-  bf16_t* Cp = (HAS_C && POST == 0) ? p.C + (int64_t)b * p.strideC +
-                                           (int64_t)(row_base + 4 * quad) * p.ldc + col_base + l16
-                                     : nullptr;
-  const int ldd = p.ldd, ldc = p.ldc, ldct = p.ldct;
+  const bool mirror = HAS_CT && !(TRI && ti == tj);  // a diagonal tile is its own mirror
+  const bool on_diag = TRI && ti == tj && p.diag != 0.0f;
+  const int ldc = p.ldc, ldct = p.ldct;
+
+  // Whole tiles.  C goes out straight from registers (16 lanes x 2 B = one 32-byte run per row and instruction, neighbouring
+  // tiles completing the lines; staged through LDS and stored as 16 bytes per lane it took 0.3-0.5 us longer, two LDS
+  // round trips with nothing beside them).  The transposed copy would be 8-byte pieces scattered over 16 rows per
+  // instruction, so 64 x 64 blocks of it are staged [column][row] in the wavefront's own part of a ring slot nobody
+  // reads any more.  The addend lies there already (see issue_addend); loaded here, 2 bytes per lane, it made the
+  // epilogue 0.8 us longer.
+  if constexpr (POST == 0 && !BND) {
+    constexpr int PIECE = Cfg::NT * 16, FAR = NSTAGE * Cfg::P_BYTES;  // lines 8 n .. of a block: n % 4 pieces on, n / 4 far
+    const int slot0 = Cfg::AHEAD ? KT % NSTAGE : 0;
+    bf16_t* Cp = HAS_C ? p.C + (int64_t)b * p.strideC + (int64_t)(row_base + 4 * quad) * ldc + col_base + l16 : nullptr;
+    const int line = (l16 >> 2), half = (l16 & 1) * 8, pair = (l16 >> 1) & 1;  // transposing reads: line of four, piece
+    const int sw_w = ((l16 >> 1) & 1) << 1 | ((l16 >> 3) & 1) << 2 | ((l16 >> 2) & 1);
+    static_for<0, TM / 4>([&](auto hc) {
+      constexpr int h = decltype(hc)::value;
+      char* const blk = lds + (slot0 + h) * Cfg::P_BYTES + wave * (64 * 16);
+      const uint32_t blk_a = lds_base + (uint32_t)((slot0 + h) * Cfg::P_BYTES + wave * (64 * 16));
+      tr_u32x2 dv[2][8];  // [row block / 2][row block % 2, column block]
+      if constexpr (HAS_D) {
+        // lane: column l16 of the tile, rows 4 quad ..: a transposing read over four rows of D
+        const uint32_t q = blk_a + (quad >> 1) * PIECE + ((quad & 1) * 4 + line) * 128 + half;
+        const int sw = ((line >> 1) | (quad & 1) << 1) << 1;
+        uint32_t at[8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) at[i * 4 + j] = q + i * 2 * PIECE + ((2 * j + pair) ^ sw) * 16;
+        lds_read_tr8(dv[0], at);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) at[r] += FAR;
+        lds_read_tr8(dv[1], at);
+      }
+      // line j * 16 + l16 (a column) of the staged block: chunk c (rows 8 c ..) lies at c ^ f(column), so that the writes of
+      // sixteen columns cover all banks
+      char* const w = blk + (l16 >> 3) * PIECE + (l16 & 7) * 128 + (quad & 1) * 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = alpha * acc[h * 4 + i][j][e];
+          if (HAS_D) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const uint32_t d = dv[i >> 1][(i & 1) * 4 + j][e >> 1];
+              v[e] = fmaf(alpha, acc[h * 4 + i][j][e], beta * __uint_as_float((e & 1) ? (d & 0xffff0000u) : (d << 16)));
+            }
+          }
+          if (i == j && on_diag && row_base + h * 64 == col_base) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = l16 - 4 * quad == e ? v[e] + p.diag : v[e];
+          }
+          if (HAS_C) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Cp[(int64_t)(h * 64 + i * 16 + e) * ldc + j * 16] = f32_to_bf16(v[e]);
+          }
+          if (!HAS_CT) continue;
+          uint2 pk;
+          pk.x = pack_bf16x2(v[0], v[1]);
+          pk.y = pack_bf16x2(v[2], v[3]);
+          *(uint2*)(w + (j & 1) * 2 * PIECE + (j >> 1) * FAR + (((2 * i + (quad >> 1)) ^ sw_w) * 16)) = pk;
+        }
+      asm volatile("" ::: "memory");
+    });
+    if (HAS_CT && mirror) {
+      // lines of TM / 4 * 128 bytes
+      constexpr int LL = TM * 2, LPI = 64 / LL;  // lanes per line, lines per instruction
+      const int sub = lane / LL, h = (lane >> 3) & (TM / 4 - 1), ch = lane & 7;
+      bf16_t* o = p.Ct + (int64_t)b * p.strideCt + (int64_t)(col_base + sub) * ldct + row_base + h * 64 + ch * 8;
+      const char* blk = lds + (slot0 + h) * Cfg::P_BYTES + wave * (64 * 16) + sub * 128;
+#pragma unroll
+      for (int n = 0; n < 64 / LPI; ++n) {
+        const int c = n * LPI + sub;
+        const int sw = ((c >> 1) & 1) << 1 | ((c >> 3) & 1) << 2 | ((c >> 2) & 1);
+        const int piece = n * LPI / 8, in_piece = n * LPI % 8;
+        const uint4 q = *(const uint4*)(blk + (piece & 3) * PIECE + (piece >> 2) * FAR + in_piece * 128 + ((ch ^ sw) * 16));
+        *(uint4*)(o + (int64_t)(n * LPI) * ldct) = q;
+      }
+    }
+    return;
+  }
+
   // BND: rows / columns of this wavefront's tile that exist; per lane, those left from its first row / column on
   const int rows_in = BND ? p.out_rows - row_base : 0, cols_in = BND ? p.out_cols - col_base : 0;
   const int lrows = rows_in - 4 * quad, lcols = cols_in - l16;
@@ -739,7 +911,6 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
     xmat = (XT*)post.X.p[pi] + (int64_t)(b - pi * post.mats_per_ptr) * (HAS_C ? p.strideC : p.strideCt);
   }
   char* stg = lds + wave * Cfg::STG_BYTES;
-  const bool on_diag = p.tri && ti == tj && p.diag != 0.0f;
   if (HAS_CT) __syncthreads();  // every wavefront is done with the operand ring
 
   if constexpr (POST != 0 && HAS_C) {
@@ -796,42 +967,19 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
     return;
   }
 
-  // The addend is loaded one row of tiles (TN tiles) at a time, one row ahead: the loads of a row are issued
-  // before the stores of the row before it, so they neither wait for those stores (the memory counter retires
-  // in order) nor cost a round trip to memory per tile.
-  bf16_t dreg[HAS_D ? 2 : 1][TN][4];
-  auto load_addend = [&](int i) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dreg[i & 1][j][e] = Dp[(int64_t)(i * 16 + e) * ldd + j * 16];
-  };
-  if (HAS_D) load_addend(0);
-
+  // (here: the update of a transposed parameter, or a bounded destination)
+  bf16_t* Cp = HAS_C ? p.C + (int64_t)b * p.strideC + (int64_t)(row_base + 4 * quad) * ldc + col_base + l16 : nullptr;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    if (HAS_D && i + 1 < TM) load_addend(i + 1);
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = alpha * acc[i][j][e];
-      if (HAS_D) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += beta * bf16_to_f32(dreg[i & 1][j][e]);
-      }
-      if (on_diag) {
-        // element (row, col) of this tile sits on the global diagonal
-        const int dcol = col_base + j * 16 + l16 - (row_base + i * 16 + 4 * quad);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (dcol == e) v[e] += p.diag;
-      }
-      if (HAS_C && POST == 0) {
+      if (HAS_C) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if constexpr (BND)
-            if (i * 16 + e >= lrows || j * 16 >= lcols) continue;
+          if (i * 16 + e >= lrows || j * 16 >= lcols) continue;
           Cp[(int64_t)(i * 16 + e) * ldc + j * 16] = f32_to_bf16(v[e]);
         }
       }
@@ -856,76 +1004,60 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
     }
     if (pair) store_lines_bounded<2, Cfg::WTM, Cfg::WTN, POST>(stg, Cfg::STG_PITCH, lane, dst, ldct, cols_in, rows_in, pa, pcoeff, pb, pcautious);
     else store_lines_bounded<1, Cfg::WTM, Cfg::WTN, POST>(stg, Cfg::STG_PITCH, lane, dst, ldct, cols_in, rows_in, pa, pcoeff, pb, pcautious);
-  } else if (HAS_CT) {
-    if (mirror) {
-      constexpr int CH = Cfg::WTM / 8;  // 16-byte chunks per staged row
-      constexpr int RPI = 64 / CH;      // staged rows per store instruction
-      const int srow = lane / CH, schunk = lane % CH;
-      const char* sp = stg + srow * Cfg::STG_PITCH + schunk * 16;
-      if constexpr (POST != 0) {
-        // The staged bf16 tile is the update.  One 16-byte access of X per lane and step (4 fp32 or 8 bf16
-        // elements), lanes side by side along the row: every instruction covers whole contiguous runs.
-        constexpr int EPL = 16 / (int)sizeof(XT);   // elements per lane
-        constexpr int PCH = Cfg::WTM / EPL;          // lanes per staged row
-        constexpr int PRPI = 64 / PCH;               // staged rows per instruction
-        constexpr int NIT = Cfg::WTN / PRPI;
-        constexpr int BI = NIT < (EPL == 4 ? 16 : 8) ? NIT : (EPL == 4 ? 16 : 8);
-        static_assert(64 % PCH == 0 && Cfg::WTN % PRPI == 0 && NIT % BI == 0, "staged rows per wavefront");
-        const int prow = lane / PCH, pchunk = lane % PCH;
-        const char* pp = stg + prow * Cfg::STG_PITCH + pchunk * (EPL * 2);
-        const __amdgpu_buffer_rsrc_t xr = bx_resource(uniform_ptr(xmat + (int64_t)col_base * ldct + row_base));
-        const int xl = (prow * ldct + pchunk * EPL) * (int)sizeof(XT);  // per lane
-        auto run = [&](auto caut) {
-          constexpr int CAUT = decltype(caut)::value;
+  } else if constexpr (HAS_CT && POST != 0) {
+    // The staged bf16 tile is the update.  One 16-byte access of X per lane and step (4 fp32 or 8 bf16
+    // elements), lanes side by side along the row: every instruction covers whole contiguous runs.
+    constexpr int EPL = 16 / (int)sizeof(XT);   // elements per lane
+    constexpr int PCH = Cfg::WTM / EPL;          // lanes per staged row
+    constexpr int PRPI = 64 / PCH;               // staged rows per instruction
+    constexpr int NIT = Cfg::WTN / PRPI;
+    constexpr int BI = NIT < (EPL == 4 ? 16 : 8) ? NIT : (EPL == 4 ? 16 : 8);
+    static_assert(64 % PCH == 0 && Cfg::WTN % PRPI == 0 && NIT % BI == 0, "staged rows per wavefront");
+    const int prow = lane / PCH, pchunk = lane % PCH;
+    const char* pp = stg + prow * Cfg::STG_PITCH + pchunk * (EPL * 2);
+    const __amdgpu_buffer_rsrc_t xr = bx_resource(uniform_ptr(xmat + (int64_t)col_base * ldct + row_base));
+    const int xl = (prow * ldct + pchunk * EPL) * (int)sizeof(XT);  // per lane
+    auto run = [&](auto caut) {
+      constexpr int CAUT = decltype(caut)::value;
 #pragma unroll
-          for (int it0 = 0; it0 < NIT; it0 += BI) {
-            float uv[BI][EPL], xv[BI][EPL];
+      for (int it0 = 0; it0 < NIT; it0 += BI) {
+        float uv[BI][EPL], xv[BI][EPL];
 #pragma unroll
-            for (int k = 0; k < BI; ++k) {
-              const char* q = pp + (it0 + k) * PRPI * Cfg::STG_PITCH;
-              if constexpr (EPL == 8) st_load8<bf16_t>((const bf16_t*)q, 0, uv[k]);
-              else st_load4<bf16_t>((const bf16_t*)q, 0, uv[k]);
-            }
-            if (pvec) {
+        for (int k = 0; k < BI; ++k) {
+          const char* q = pp + (it0 + k) * PRPI * Cfg::STG_PITCH;
+          if constexpr (EPL == 8) st_load8<bf16_t>((const bf16_t*)q, 0, uv[k]);
+          else st_load4<bf16_t>((const bf16_t*)q, 0, uv[k]);
+        }
+        if (pvec) {
 #pragma unroll
-              for (int k = 0; k < BI; ++k)
-                bx_load16<XT>(xr, xl, (it0 + k) * PRPI * ldct * (int)sizeof(XT), xv[k]);
-            } else {
+          for (int k = 0; k < BI; ++k)
+            bx_load16<XT>(xr, xl, (it0 + k) * PRPI * ldct * (int)sizeof(XT), xv[k]);
+        } else {
 #pragma unroll
-              for (int k = 0; k < BI; ++k)
+          for (int k = 0; k < BI; ++k)
 #pragma unroll
-                for (int e = 0; e < EPL; ++e)
-                  xv[k][e] = bx_load<XT>(xr, xl, ((it0 + k) * PRPI * ldct + e) * (int)sizeof(XT));
-            }
+            for (int e = 0; e < EPL; ++e)
+              xv[k][e] = bx_load<XT>(xr, xl, ((it0 + k) * PRPI * ldct + e) * (int)sizeof(XT));
+        }
 #pragma unroll
-            for (int k = 0; k < BI; ++k)
+        for (int k = 0; k < BI; ++k)
 #pragma unroll
-              for (int e = 0; e < EPL; ++e) xv[k][e] = muon_post_one(xv[k][e], uv[k][e], pa, pcoeff, pb, CAUT);
-            if (pvec) {
+          for (int e = 0; e < EPL; ++e) xv[k][e] = muon_post_one(xv[k][e], uv[k][e], pa, pcoeff, pb, CAUT);
+        if (pvec) {
 #pragma unroll
-              for (int k = 0; k < BI; ++k)
-                bx_store16<XT>(xr, xl, (it0 + k) * PRPI * ldct * (int)sizeof(XT), xv[k]);
-            } else {
+          for (int k = 0; k < BI; ++k)
+            bx_store16<XT>(xr, xl, (it0 + k) * PRPI * ldct * (int)sizeof(XT), xv[k]);
+        } else {
 #pragma unroll
-              for (int k = 0; k < BI; ++k)
+          for (int k = 0; k < BI; ++k)
 #pragma unroll
-                for (int e = 0; e < EPL; ++e)
-                  bx_store<XT>(xr, xl, ((it0 + k) * PRPI * ldct + e) * (int)sizeof(XT), xv[k][e]);
-            }
-          }
-        };
-        if (pcautious) run(std::integral_constant<int, 1>());
-        else run(std::integral_constant<int, 0>());
-      } else {
-        bf16_t* Ctp =
-            p.Ct + (int64_t)b * p.strideCt + (int64_t)(col_base + srow) * ldct + row_base + schunk * 8;
-#pragma unroll 8
-        for (int it = 0; it < Cfg::WTN / RPI; ++it) {
-          const uint4 q = *(const uint4*)(sp + it * RPI * Cfg::STG_PITCH);
-          *(uint4*)(Ctp + (int64_t)(it * RPI) * ldct) = q;
+            for (int e = 0; e < EPL; ++e)
+              bx_store<XT>(xr, xl, ((it0 + k) * PRPI * ldct + e) * (int)sizeof(XT), xv[k][e]);
         }
       }
-    }
+    };
+    if (pcautious) run(std::integral_constant<int, 1>());
+    else run(std::integral_constant<int, 0>());
   }
 }
 
@@ -981,7 +1113,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
 
   int b_c, ti_c, tj_c, b_n, ti_n, tj_n;
   int pid = blockIdx.x;
-  tile_of<BM, BN>(p, pid, total_tiles, b_c, ti_c, tj_c);
+  tile_of<BM, BN, false>(p, pid, total_tiles, b_c, ti_c, tj_c);
   auto base_p = [&](int b, int ti) { return (const char*)(p.P + (int64_t)b * p.strideP + (int64_t)(ti * BM) * p.ldp); };
   auto base_q = [&](int b, int tj) { return (const char*)(p.Q + (int64_t)b * p.strideQ + tj * BN); };
   const char* gP_c = base_p(b_c, ti_c);
@@ -992,7 +1124,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
     // fetched again and never read, which keeps the load count per slab fixed)
     const int np = pid + (int)gridDim.x;
     if (np < total_tiles) {
-      tile_of<BM, BN>(p, np, total_tiles, b_n, ti_n, tj_n);
+      tile_of<BM, BN, false>(p, np, total_tiles, b_n, ti_n, tj_n);
       gP_n = base_p(b_n, ti_n);
       gQ_n = base_q(b_n, tj_n);
     } else {
@@ -1074,7 +1206,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
                         : p.C + (int64_t)b * p.strideC + (int64_t)row_base * ld_out + col_base;
     const __amdgpu_buffer_rsrc_t rs = bx_resource(uniform_ptr(out));
     const int lane_bytes = (rl * ld_out + rq * 8) * 2;
-    const float alpha = gemm_alpha(p, b);  // 1 unless a per-matrix factor rides on this launch
+    const float alpha = gemm_alpha(p, p.scale_vec ? p.scale_vec[b] : 1.0f);  // 1 unless a per-matrix factor rides on this launch
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       // chunk c: 32 output lines of 128 bytes.  OUT_T false: C rows 32 c .. 32 c + 31 of the wavefront tile
@@ -1192,8 +1324,10 @@ __global__ __launch_bounds__(CfgK64::NT, 2) void gemm_k64_kernel(const GemmParam
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int b, ti, tj;
-  tile_of<64, 64>(p, blockIdx.x, gridDim.x, b, ti, tj);
-  const bool one_operand = !QK && p.tri && ti == tj && p.P == p.Q && p.ldp == p.ldq && p.strideP == p.strideQ;
+  constexpr bool TRI = HAS_C && HAS_CT && !QK;
+  tile_of<64, 64, TRI>(p, blockIdx.x, gridDim.x, b, ti, tj);
+  const float factor = p.scale_vec ? p.scale_vec[b] : 1.0f;
+  const bool one_operand = !QK && TRI && ti == tj && p.P == p.Q && p.ldp == p.ldq && p.strideP == p.strideQ;
 
   // ---- global -> LDS: a load moves 8 tile rows of 128 bytes; lane l brings 16-byte chunk l % 8 of row l / 8.  The
   // swizzles are those of the kernel above; a load's first row is a multiple of 8, and they differ between
@@ -1366,8 +1500,8 @@ __global__ __launch_bounds__(CfgK64::NT, 2) void gemm_k64_kernel(const GemmParam
     for (int j = 0; j < 4; ++j) part[((wave * 4 + i) * 4 + j) * 64 + lane] = acc[i][j];
   });
   __syncthreads();
-  const float alpha = gemm_alpha(p, b), beta = p.beta;
-  const bool on_diag = p.tri && ti == tj && p.diag != 0.0f;
+  const float alpha = gemm_alpha(p, factor), beta = p.beta;
+  const bool on_diag = TRI && ti == tj && p.diag != 0.0f;
   char* stg = lds + Cfg::PART_BYTES;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -1441,7 +1575,7 @@ __global__ __launch_bounds__(CfgK64::NT, 2) void gemm_k64_kernel(const GemmParam
         const int64_t at = (int64_t)c * p.ldct;
         st_store<XT>(xt, at, muon_post_one(st_load<XT>(xt, at), u, pa, pcoeff, pb, post.cautious));
       }
-    } else if (!(p.tri && ti == tj)) {  // a diagonal tile is its own mirror
+    } else if (!(TRI && ti == tj)) {  // a diagonal tile is its own mirror
       bf16_t* Ctp = p.Ct + (int64_t)b * p.strideCt + (int64_t)col_base * p.ldct + ti * 64;
 #pragma unroll
       for (int it = 0; it < 2; ++it) {
@@ -1458,10 +1592,6 @@ typedef TileCfg<128, 128, 64, 2, 2, 4, true> Cfg128d;  // the same on a four-slo
 typedef TileCfg<256, 256, 64, 2, 4, 2> Cfg256w8;       // 8 wavefronts, 128x64 each: two per SIMD, one workgroup per CU
 constexpr int kWalkMaxK = 2048;                    // longest reduction the tile-walking kernel is used for
 
-// Tile list dealt to the XCDs in interleaved 32-tile chunks (see the kernel) when the first operand of
-// one matrix is at least 16 MB; below that a contiguous run per XCD keeps whole matrices in one L2.
-static bool xcd_interleave_pays(const GemmParams& p) { return (int64_t)p.M * p.K * 2 >= (16L << 20); }
-
 template <class Cfg, bool HAS_D, bool HAS_C, bool HAS_CT, bool QK = false, int POST = 0, bool BND = false>
 static hipError_t launch_epi(const GemmParams& p, hipStream_t stream,
                              const typename PostSel<POST>::arg& post = typename PostSel<POST>::arg()) {
@@ -1474,7 +1604,7 @@ static hipError_t launch_epi(const GemmParams& p, hipStream_t stream,
   if (total <= 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidValue;
   GemmParams pp = p;
-  pp.xcd_interleave = xcd_interleave_pays(p) ? 1 : 0;
+  set_tile_order(pp, Cfg::BM, Cfg::BN);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, pp, post);
   return hipGetLastError();
 }
@@ -1491,7 +1621,7 @@ static hipError_t launch_k64_epi(const GemmParams& p, hipStream_t stream,
   if (total <= 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidValue;
   GemmParams pp = p;
-  pp.xcd_interleave = xcd_interleave_pays(p) ? 1 : 0;
+  set_tile_order(pp, 64, 64);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(CfgK64::NT), CfgK64::LDS_BYTES, stream, pp, post);
   return hipGetLastError();
 }
@@ -1518,7 +1648,7 @@ static hipError_t launch_walk(const GemmParams& p, hipStream_t stream) {
     cu_count[dev & 63].store(cus, std::memory_order_relaxed);
   }
   GemmParams pp = p;
-  pp.xcd_interleave = xcd_interleave_pays(p) ? 1 : 0;
+  set_tile_order(pp, Cfg::BM, Cfg::BN);
   const unsigned grid = (unsigned)(total < cus ? total : cus);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(Cfg::NT), kLds, stream, pp, (int)total);
   return hipGetLastError();

@@ -111,3 +111,23 @@ def test_reduction_lengths_of_products_with_a_k_major_operand(m):
     Y = torch.full_like(X, float("nan"))
     check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, n, ctypes.c_float(0.0), st), "line_3")
     _close(Y, B.double() @ X.double())
+
+
+# The addend travels through the ring behind the last slab: slab counts (m / 64) from two, remainders of the ring's length,
+# more than eight tile rows; four-slot and two-slot rings of 128-wide tiles, and 256-wide tiles.
+@pytest.mark.parametrize("m,batch,sym_edge", [(128, 300, 128), (256, 70, 128), (256, 200, 256), (384, 42, 128), (384, 60, 128), (512, 20, 128),
+                                              (512, 60, 256), (640, 16, 128), (768, 30, 256), (1152, 3, 128), (1152, 8, 128), (2304, 4, 256)])
+def test_addend_at_every_slab_count(m, batch, sym_edge):
+    lib, check, st = _lib()
+    assert lib.dion_gemm_tile_edge(batch, m, m, 1) == sym_edge
+    g = torch.Generator(device=DEV).manual_seed(m + batch)
+    S = torch.randn(batch, m, m, device=DEV, generator=g)
+    S = ((S + S.mT) * (0.5 / m ** 0.5)).to(torch.bfloat16)
+    X = torch.randn(batch, m, m, device=DEV, generator=g).to(torch.bfloat16)
+    B, Y = (torch.full_like(S, float("nan")) for _ in range(2))
+    Sd = S.double()
+    check(lib.dion_ns_line_2(S.data_ptr(), B.data_ptr(), batch, m, ctypes.c_float(0.5), ctypes.c_float(2.0), st), "line_2")
+    _close(B, 0.5 * (Sd @ Sd) + 2.0 * Sd)
+    assert torch.equal(B, B.mT)
+    check(lib.dion_ns_line_3(S.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, m, ctypes.c_float(0.75), st), "line_3")
+    _close(Y, Sd @ X.double() + 0.75 * X.double())
