@@ -1717,11 +1717,13 @@ int gemm_pad_granule(int m, int n, int batch) {
 }
 
 // Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box.
-//  * 256-wide tiles when there are enough of them: a full product from 384 (one and a half rounds of the 256 CUs;
-//    432 tiles of 12 x (768 x 3072) run 14 % faster than the 1728 128-wide ones, 108 tiles of 12 x (768 x 768) 20 %
-//    slower), a symmetric one from 160 (16 x 1024-wide: 5 % faster; 72 tiles of 12 x 768-wide: 70 % slower).  Rounds
-//    that are not full cost less than their geometry says: the part is power-limited, and the CUs that are busy run
-//    faster while others idle.
+//  * 256-wide tiles when there are enough of them: a symmetric product from 160 (16 x 1024-wide: 5 % faster; 72 tiles of
+//    12 x 768-wide: 70 % slower), a full one when they make one round of the CUs where 128-wide ones make more than one of
+//    two workgroups each (129-256 tiles), or most of two (from 336, with reductions past 1024 from 384).  B X on 128- /
+//    256-wide tiles: 128 tiles of 8 x (1024 x 1024) 20.5 / 25.2, 144 of 9 x 29.3 / 25.9, 256 of 16 x 36.9 / 32.9, 272 of 17 x
+//    46.6 / 49.1, 336 of 21 x 51.0 / 49.8; 135 of 15 x (768 x 768) 24.1 / 21.8, 243 of 27 x 30.7 / 26.8; 129 of 43 x
+//    (256 x 768) 13.2 / 11.4, 256 of 32 x (512 x 1024) 26.2 / 21.8, 336 of 42 x 33.5 / 30.7; 252 of 7 x (1536 x 1536) 50.0 /
+//    44.1, 360 of 10 x 71.4 / 72.1.
 //  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
 //    per CU, for symmetric products (whose 128-wide form has only a quarter as many) two per CU unless the reduction is
 //    short: X X^T of one 768 x 3072 matrix 28.4 -> 10.0, of 1024 x 4096 42.9 -> 15.8; at two rounds 12 x (512 x 2048)
@@ -1741,7 +1743,10 @@ static TileKind pick_tile(const GemmParams& p) {
     const int64_t T = p.M / edge;
     return (p.tri ? T * (T + 1) / 2 : T * (p.N / edge)) * (p.rule_batch > 0 ? p.rule_batch : p.batch);
   };
-  if (p.M % 256 == 0 && p.N % 256 == 0 && tiles(256) >= (p.tri ? 160 : 384)) return kTile256;
+  if (p.M % 256 == 0 && p.N % 256 == 0) {
+    const int64_t t = tiles(256);
+    if (p.tri ? t >= 160 : t >= 384 || (t > 128 && t <= 256) || (t >= 336 && p.K <= 1024)) return kTile256;
+  }
   const int short_k = p.M < 256 ? 1024 : p.M < 384 ? 512 : 384;
   if (tiles(64) <= (p.tri && p.K >= short_k ? 512 : 256) && !(p.D && !p.tri)) return kTile64;
   if (tiles(128) <= 256 && (p.tri || p.K > 1024)) return kTile128Deep;

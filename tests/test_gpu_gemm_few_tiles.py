@@ -102,7 +102,7 @@ def test_reduction_lengths_of_symmetric_products(batch, n):
 @pytest.mark.parametrize("m", [128, 256, 384, 512, 640, 1152])
 def test_reduction_lengths_of_products_with_a_k_major_operand(m):
     lib, check, st = _lib()
-    batch, n = -(-38400 // m), 256  # 300 tiles and a few more
+    batch, n = -(-12800 // m), 384  # 300 tiles and a few more, of a width that has no 256-wide ones
     assert lib.dion_gemm_tile_edge(batch, m, n, 0) == 128
     g = torch.Generator(device=DEV).manual_seed(m)
     B = torch.randn(batch, m, m, device=DEV, generator=g)
@@ -131,3 +131,18 @@ def test_addend_at_every_slab_count(m, batch, sym_edge):
     assert torch.equal(B, B.mT)
     check(lib.dion_ns_line_3(S.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, m, ctypes.c_float(0.75), st), "line_3")
     _close(Y, Sd @ X.double() + 0.75 * X.double())
+
+
+# Full products on both sides of the lines between 128- and 256-wide tiles: one round of the CUs, and most of two.
+@pytest.mark.parametrize("batch,m,n,edge", [(32, 512, 512, 128), (43, 256, 768, 256), (32, 512, 1024, 256), (17, 1024, 1024, 128),
+                                            (42, 512, 1024, 256), (7, 1536, 1536, 256), (10, 1536, 1536, 128), (9, 1024, 1152, 128)])
+def test_full_products_at_the_lines_of_256_wide_tiles(batch, m, n, edge):
+    lib, check, st = _lib()
+    assert lib.dion_gemm_tile_edge(batch, m, n, 0) == edge
+    g = torch.Generator(device=DEV).manual_seed(batch)
+    B = torch.randn(batch, m, m, device=DEV, generator=g)
+    B = ((B + B.mT) * (0.5 / m ** 0.5)).to(torch.bfloat16)
+    X = torch.randn(batch, m, n, device=DEV, generator=g).to(torch.bfloat16)
+    Y = torch.full_like(X, float("nan"))
+    check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, n, ctypes.c_float(0.0), st), "line_3")
+    _close(Y, B.double() @ X.double())
