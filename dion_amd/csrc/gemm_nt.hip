@@ -1717,22 +1717,26 @@ int gemm_pad_granule(int m, int n, int batch) {
 }
 
 // Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box.
-//  * 256-wide tiles when there are enough of them: a symmetric product from 160 (16 x 1024-wide: 5 % faster; 72 tiles of
-//    12 x 768-wide: 70 % slower), a full one when they make one round of the CUs where 128-wide ones make more than one of
+//  * 256-wide tiles, a symmetric product: when 128-wide ones are more than two per CU (512) and 256-wide ones at most one;
+//    past that from the count on where 128-wide ones need a fourth round of two per CU (1536; reductions past 2048: from
+//    1152, their second round of 256-wide tiles being the cheaper one).  X X^T on 256- / 128-wide tiles: 130 / 468 tiles of
+//    13 x (1024 x 1024) 26.1 / 19.5, 144 / 544 of 4 x (2048 x 2048) 42.6 / 48.8, 200 / 720 of 20 x (1024 x 3072) 65.0 / 71.8,
+//    260 / 936 of 26 x (1024 x 1024) 50.8 / 36.7, of 26 x (1024 x 3072) 124 / 81, 288 / 1008 of 48 x (768 x 2304) 94.6 / 66.4,
+//    320 / 1152 of 32 x (1024 x 3072) 123 / 111, 360 / 1296 of 36 x 138 / 146, 399 / 1482 of 19 x (1536 x 1536) 74.5 / 70.4, 420 / 1560
+//    of 20 x 76.4 / 86.9.  A full product: when they make one round of the CUs where 128-wide ones make more than one of
 //    two workgroups each (129-256 tiles), or most of two (from 336, with reductions past 1024 from 384).  B X on 128- /
 //    256-wide tiles: 128 tiles of 8 x (1024 x 1024) 20.5 / 25.2, 144 of 9 x 29.3 / 25.9, 256 of 16 x 36.9 / 32.9, 272 of 17 x
 //    46.6 / 49.1, 336 of 21 x 51.0 / 49.8; 135 of 15 x (768 x 768) 24.1 / 21.8, 243 of 27 x 30.7 / 26.8; 129 of 43 x
 //    (256 x 768) 13.2 / 11.4, 256 of 32 x (512 x 1024) 26.2 / 21.8, 336 of 42 x 33.5 / 30.7; 252 of 7 x (1536 x 1536) 50.0 /
 //    44.1, 360 of 10 x 71.4 / 72.1.
 //  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
-//    per CU, for symmetric products (whose 128-wide form has only a quarter as many) two per CU unless the reduction is
-//    short: X X^T of one 768 x 3072 matrix 28.4 -> 10.0, of 1024 x 4096 42.9 -> 15.8; at two rounds 12 x (512 x 2048)
-//    22.8 -> 16.8 (18.4 with the form below), at three 4 x (1024 x 2816) 28.4 against 23.4; one 2048 x 2048, 528 tiles, 17.6
-//    against 12.4.  Two rounds of a short reduction against the form below: X X^T of 128 x (128 x 128) 6.8 against 5.1,
-//    of 40 x (256 x 256) 7.6 against 6.6, of 150 x (128 x 512) 8.7 against 7.7; but of 32 x (256 x 512) 8.0 against 8.1, of
-//    100 x (128 x 1024) 9.8 against 10.5, A A of 13 x 384 7.9 against 8.3.  B X: 256 tiles (1024 x 1024) 9.8 -> 6.3; past
-//    that the last form, at 288 (2 x (768 x 768)) 9.4 against 8.4, at 512 (4 x (512 x 1024)) 8.7 against 7.4, at 576
-//    (768 x 3072) 14.0 against 8.9.
+//    per CU: X X^T of one 768 x 3072 matrix 28.4 -> 10.0 (78 tiles), of 1024 x 4096 42.9 -> 15.8, of 4 x (640 x 2560) 16.3 ->
+//    10.4; B X of 1024 x 1024 (256 tiles) 9.8 -> 6.3, past that the last form, at 288 (2 x (768 x 768)) 9.4 against 8.4, at 576
+//    (768 x 3072) 14.0 against 8.9.  Symmetric products of up to two per CU where the reduction is as long as the matrix is
+//    wide and not short (A A of 13 x 384 8.1 against 7.3 of the form below, of 5 x (768 x 768) 10.5 / 9.3: that form has
+//    overtaken them; the line stays where the tests of this form have it).  Longer reductions go to the form below: X X^T
+//    of 2 x (1024 x 4096) 30.6 -> 24.0, of 13 x (512 x 2048) 17.8 -> 14.9, of 6 x (768 x 3072) 25.3 -> 22.1, of 8 x (512 x 2048)
+//    14.0 / 14.0.
 //  * 128-wide tiles, at most one per CU: the CU is one workgroup's alone, and a ring of four slots keeps three slabs
 //    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
 //    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
@@ -1744,11 +1748,14 @@ static TileKind pick_tile(const GemmParams& p) {
     return (p.tri ? T * (T + 1) / 2 : T * (p.N / edge)) * (p.rule_batch > 0 ? p.rule_batch : p.batch);
   };
   if (p.M % 256 == 0 && p.N % 256 == 0) {
-    const int64_t t = tiles(256);
-    if (p.tri ? t >= 160 : t >= 384 || (t > 128 && t <= 256) || (t >= 336 && p.K <= 1024)) return kTile256;
+    const int64_t t = tiles(256), t128 = tiles(128);
+    const bool sym = t128 > 512 && (t <= 256 || t128 > (p.K > 2048 ? 1152 : 1536));
+    const bool full = t >= 384 || (t > 128 && t <= 256) || (t >= 336 && p.K <= 1024);
+    if (p.tri ? sym : full) return kTile256;
   }
   const int short_k = p.M < 256 ? 1024 : p.M < 384 ? 512 : 384;
-  if (tiles(64) <= (p.tri && p.K >= short_k ? 512 : 256) && !(p.D && !p.tri)) return kTile64;
+  const int most64 = p.tri && p.K >= short_k && p.K <= p.M ? 512 : 256;
+  if (tiles(64) <= most64 && !(p.D && !p.tri)) return kTile64;
   if (tiles(128) <= 256 && (p.tri || p.K > 1024)) return kTile128Deep;
   return kTile128;
 }

@@ -146,3 +146,17 @@ def test_full_products_at_the_lines_of_256_wide_tiles(batch, m, n, edge):
     Y = torch.full_like(X, float("nan"))
     check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), batch, m, n, ctypes.c_float(0.0), st), "line_3")
     _close(Y, B.double() @ X.double())
+
+
+# Symmetric products on both sides of the lines between 64-, 128- and 256-wide tiles.
+@pytest.mark.parametrize("batch,m,n", [(6, 768, 768), (6, 768, 1024), (1, 1920, 1920), (1, 1920, 2048), (21, 512, 1024), (51, 512, 512),
+                                       (52, 512, 512), (85, 512, 640), (86, 512, 640), (36, 1024, 1024), (32, 1024, 2176), (33, 1024, 2176),
+                                       (20, 1536, 1536)])
+def test_symmetric_products_at_the_lines(batch, m, n):
+    lib, check, st = _lib()
+    g = torch.Generator(device=DEV).manual_seed(batch + n)
+    X = torch.randn(batch, m, n, device=DEV, generator=g).to(torch.bfloat16)
+    A = torch.full((batch, m, m), float("nan"), device=DEV, dtype=torch.bfloat16)
+    check(lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), batch, m, n, st), "line_1")
+    _close(A, X.double() @ X.double().mT.contiguous())
+    assert torch.equal(A, A.mT)
