@@ -457,7 +457,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
   static_assert(!BND || (QK && !HAS_D && HAS_C != HAS_CT), "bounded destinations: the last product of a call");
   // Refill of the slot a slab occupied: all of it during the slab's last half, or -- the plain product of two
   // K-contiguous operands on 256-wide tiles, i.e. X X^T -- half then and half during the next slab's first half.
-  // Measured: X X^T 2-3 % faster that way; the polynomial GEMM (addend loads in the epilogue) 1 % slower, the
+  // Measured: X X^T 2-3 % faster that way; the polynomial GEMM (its last refills bring the addend) 1 % slower, the
   // K-major form (two-instruction fragment reads in the same half) 3 % slower, 128-wide tiles 10 % slower.
   constexpr bool SPREAD = !QK && !HAS_D && BM == 256;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
