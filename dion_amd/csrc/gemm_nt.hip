@@ -1732,11 +1732,11 @@ int gemm_pad_granule(int m, int n, int batch) {
 //  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
 //    per CU: X X^T of one 768 x 3072 matrix 28.4 -> 10.0 (78 tiles), of 1024 x 4096 42.9 -> 15.8, of 4 x (640 x 2560) 16.3 ->
 //    10.4; B X of 1024 x 1024 (256 tiles) 9.8 -> 6.3, past that the last form, at 288 (2 x (768 x 768)) 9.4 against 8.4, at 576
-//    (768 x 3072) 14.0 against 8.9.  Symmetric products of up to two per CU where the reduction is as long as the matrix is
-//    wide and not short (A A of 13 x 384 8.1 against 7.3 of the form below, of 5 x (768 x 768) 10.5 / 9.3: that form has
-//    overtaken them; the line stays where the tests of this form have it).  Longer reductions go to the form below: X X^T
-//    of 2 x (1024 x 4096) 30.6 -> 24.0, of 13 x (512 x 2048) 17.8 -> 14.9, of 6 x (768 x 3072) 25.3 -> 22.1, of 8 x (512 x 2048)
-//    14.0 / 14.0.
+//    (768 x 3072) 14.0 against 8.9.  Symmetric products of up to two per CU where the reduction is not short: the form
+//    below takes less time there (X X^T of 2 x (1024 x 4096) 24.0 against 30.6, of 13 x (512 x 2048) 14.9 / 17.8, of
+//    113 x (128 x 2048) 14.1 / 17.4, of 6 x (768 x 3072) 22.1 / 25.3, of 8 x (512 x 2048) 14.0 / 14.0; A A of 5 x (768 x 768)
+//    9.3 / 10.5), but adds a reduction up in one chain where this one has four partial sums, and one chain carries twice
+//    the rounding error: sums of 2048 products of unit variance that cancel, 3.7e-6 rms here, 8.1e-6 there.
 //  * 128-wide tiles, at most one per CU: the CU is one workgroup's alone, and a ring of four slots keeps three slabs
 //    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
 //    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
@@ -1754,7 +1754,7 @@ static TileKind pick_tile(const GemmParams& p) {
     if (p.tri ? sym : full) return kTile256;
   }
   const int short_k = p.M < 256 ? 1024 : p.M < 384 ? 512 : 384;
-  const int most64 = p.tri && p.K >= short_k && p.K <= p.M ? 512 : 256;
+  const int most64 = p.tri && p.K >= short_k ? 512 : 256;
   if (tiles(64) <= most64 && !(p.D && !p.tri)) return kTile64;
   if (tiles(128) <= 256 && (p.tri || p.K > 1024)) return kTile128Deep;
   return kTile128;

@@ -160,3 +160,21 @@ def test_symmetric_products_at_the_lines(batch, m, n):
     check(lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), batch, m, n, st), "line_1")
     _close(A, X.double() @ X.double().mT.contiguous())
     assert torch.equal(A, A.mT)
+
+
+# 257-512 tiles of 64: the reduction is added up in four partial sums, slab (64 columns) by slab in turn, whether it is
+# longer than the matrix is wide or not.  Slabs 0 and 4 bring 2^26 and -2^26 to one partial sum, slab 1 a 1 to another: exact
+# there, lost in one chain, where 2^26 + 1 rounds to 2^26.
+@pytest.mark.parametrize("batch,m,n", [(86, 128, 1024), (113, 128, 2048), (26, 256, 512), (13, 512, 2048), (6, 768, 3072), (2, 1024, 4096),
+                                       (1, 1920, 2176), (14, 512, 512), (2, 1024, 1024)])
+def test_partial_sums_of_symmetric_products(batch, m, n):
+    lib, check, st = _lib()
+    X = torch.zeros(batch, m, n, device=DEV, dtype=torch.bfloat16)
+    X[:, :, 0] = 2.0 ** 13
+    X[:, :, 64] = 1.0
+    X[:, 0::2, 256] = 2.0 ** 13
+    X[:, 1::2, 256] = -(2.0 ** 13)
+    A = torch.full((batch, m, m), float("nan"), device=DEV, dtype=torch.bfloat16)
+    check(lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), batch, m, n, st), "line_1")
+    assert bool((A[:, 0::2, 1::2] == 1).all())
+    assert torch.equal(A, A.mT)
