@@ -59,6 +59,7 @@ SIGNATURES = {
     "dion_ns_plan_audit_prepared": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                             c_size_t]),
     "dion_gemm_tile_edge": (c_int, [c_int, c_int, c_int, c_int]),
+    "dion_ns_line_kernel": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "dion_muon_pre_sumsq_blocks": (c_int, [c_int, c_int]),
     "dion_muon_pre_prepared": (c_int, [_u64p, c_int, _u64p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                        c_float, c_int, c_void_p]),

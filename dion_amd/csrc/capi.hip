@@ -56,13 +56,7 @@ static int check_gemm_ptr(const char* who, const char* arg, const void* ptr) {
   return DION_OK;
 }
 
-extern "C" int dion_ns_line_1(const void* X, void* A, int batch, int m, int k, void* stream) {
-  if (int rc = check_gemm_dims("dion_ns_line_1", batch, m, k)) return rc;
-  if (batch == 0 || m == 0) return DION_OK;
-  if (k == 0) return fail(DION_E_INVALID, "dion_ns_line_1: k == 0");
-  if (!X || !A) return fail(DION_E_INVALID, "dion_ns_line_1: null argument");
-  if (int rc = check_gemm_ptr("dion_ns_line_1", "X", X)) return rc;
-  if (int rc = check_gemm_ptr("dion_ns_line_1", "A", A)) return rc;
+static GemmParams line_1_params(const void* X, void* A, int batch, int m, int k) {
   GemmParams p;
   memset(&p, 0, sizeof(p));
   p.P = p.Q = (const bf16_t*)X;
@@ -76,18 +70,10 @@ extern "C" int dion_ns_line_1(const void* X, void* A, int batch, int m, int k, v
   p.batch = batch;
   p.tri = 1;
   p.alpha = 1.0f;
-  HIP_TRY(launch_gemm_nt(p, (hipStream_t)stream), "dion_ns_line_1");
-  return DION_OK;
+  return p;
 }
 
-extern "C" int dion_ns_line_2(const void* A, void* B, int batch, int m, float alpha, float beta,
-                              void* stream) {
-  if (int rc = check_gemm_dims("dion_ns_line_2", batch, m, m)) return rc;
-  if (batch == 0 || m == 0) return DION_OK;
-  if (!A || !B) return fail(DION_E_INVALID, "dion_ns_line_2: null argument");
-  if (A == B) return fail(DION_E_INVALID, "dion_ns_line_2: in-place not supported");
-  if (int rc = check_gemm_ptr("dion_ns_line_2", "A", A)) return rc;
-  if (int rc = check_gemm_ptr("dion_ns_line_2", "B", B)) return rc;
+static GemmParams line_2_params(const void* A, void* B, int batch, int m, float alpha, float beta) {
   GemmParams p;
   memset(&p, 0, sizeof(p));
   p.P = p.Q = p.D = (const bf16_t*)A;
@@ -99,19 +85,10 @@ extern "C" int dion_ns_line_2(const void* A, void* B, int batch, int m, float al
   p.tri = 1;
   p.alpha = alpha;
   p.beta = beta;
-  HIP_TRY(launch_gemm_nt(p, (hipStream_t)stream), "dion_ns_line_2");
-  return DION_OK;
+  return p;
 }
 
-extern "C" int dion_ns_line_3(const void* B, const void* X, void* C, int batch, int m, int n, float a,
-                              void* stream) {
-  if (int rc = check_gemm_dims("dion_ns_line_3", batch, m, n)) return rc;
-  if (batch == 0 || m == 0 || n == 0) return DION_OK;
-  if (!B || !X || !C) return fail(DION_E_INVALID, "dion_ns_line_3: null argument");
-  if (C == X) return fail(DION_E_INVALID, "dion_ns_line_3: in-place not supported");
-  if (int rc = check_gemm_ptr("dion_ns_line_3", "B", B)) return rc;
-  if (int rc = check_gemm_ptr("dion_ns_line_3", "X", X)) return rc;
-  if (int rc = check_gemm_ptr("dion_ns_line_3", "C", C)) return rc;
+static GemmParams line_3_params(const void* B, const void* X, void* C, int batch, int m, int n, float a) {
   GemmParams p;
   memset(&p, 0, sizeof(p));
   p.P = (const bf16_t*)B;
@@ -129,8 +106,57 @@ extern "C" int dion_ns_line_3(const void* B, const void* X, void* C, int batch, 
   p.batch = batch;
   p.alpha = 1.0f;
   p.beta = a;
+  return p;
+}
+
+extern "C" int dion_ns_line_1(const void* X, void* A, int batch, int m, int k, void* stream) {
+  if (int rc = check_gemm_dims("dion_ns_line_1", batch, m, k)) return rc;
+  if (batch == 0 || m == 0) return DION_OK;
+  if (k == 0) return fail(DION_E_INVALID, "dion_ns_line_1: k == 0");
+  if (!X || !A) return fail(DION_E_INVALID, "dion_ns_line_1: null argument");
+  if (int rc = check_gemm_ptr("dion_ns_line_1", "X", X)) return rc;
+  if (int rc = check_gemm_ptr("dion_ns_line_1", "A", A)) return rc;
+  const GemmParams p = line_1_params(X, A, batch, m, k);
+  HIP_TRY(launch_gemm_nt(p, (hipStream_t)stream), "dion_ns_line_1");
+  return DION_OK;
+}
+
+extern "C" int dion_ns_line_2(const void* A, void* B, int batch, int m, float alpha, float beta,
+                              void* stream) {
+  if (int rc = check_gemm_dims("dion_ns_line_2", batch, m, m)) return rc;
+  if (batch == 0 || m == 0) return DION_OK;
+  if (!A || !B) return fail(DION_E_INVALID, "dion_ns_line_2: null argument");
+  if (A == B) return fail(DION_E_INVALID, "dion_ns_line_2: in-place not supported");
+  if (int rc = check_gemm_ptr("dion_ns_line_2", "A", A)) return rc;
+  if (int rc = check_gemm_ptr("dion_ns_line_2", "B", B)) return rc;
+  const GemmParams p = line_2_params(A, B, batch, m, alpha, beta);
+  HIP_TRY(launch_gemm_nt(p, (hipStream_t)stream), "dion_ns_line_2");
+  return DION_OK;
+}
+
+extern "C" int dion_ns_line_3(const void* B, const void* X, void* C, int batch, int m, int n, float a,
+                              void* stream) {
+  if (int rc = check_gemm_dims("dion_ns_line_3", batch, m, n)) return rc;
+  if (batch == 0 || m == 0 || n == 0) return DION_OK;
+  if (!B || !X || !C) return fail(DION_E_INVALID, "dion_ns_line_3: null argument");
+  if (C == X) return fail(DION_E_INVALID, "dion_ns_line_3: in-place not supported");
+  if (int rc = check_gemm_ptr("dion_ns_line_3", "B", B)) return rc;
+  if (int rc = check_gemm_ptr("dion_ns_line_3", "X", X)) return rc;
+  if (int rc = check_gemm_ptr("dion_ns_line_3", "C", C)) return rc;
+  const GemmParams p = line_3_params(B, X, C, batch, m, n, a);
   HIP_TRY(launch_gemm_nt(p, (hipStream_t)stream), "dion_ns_line_3");
   return DION_OK;
+}
+
+extern "C" int dion_ns_line_kernel(int line, int batch, int m, int n, int with_addend) {
+  if (int rc = check_gemm_dims("dion_ns_line_kernel", batch, m, line == 2 ? m : n)) return rc;
+  if (line < 1 || line > 3 || batch == 0 || m == 0 || (line != 2 && n == 0))
+    return fail(DION_E_INVALID, "dion_ns_line_kernel: line %d, %d x (%d x %d)", line, batch, m, n);
+  // (addresses are not looked at, only whether there is an addend)
+  static const bf16_t any = 0;
+  return gemm_kernel(line == 1   ? line_1_params(&any, nullptr, batch, m, n)
+                     : line == 2 ? line_2_params(&any, nullptr, batch, m, 1.0f, 1.0f)
+                                 : line_3_params(&any, &any, nullptr, batch, m, n, with_addend ? 1.0f : 0.0f));
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -1609,13 +1609,25 @@ static hipError_t launch_epi(const GemmParams& p, hipStream_t stream,
   return hipGetLastError();
 }
 
+enum TileKind { kTile64, kTile128Deep, kTile128, kTile256 };
+
+// The kernels keep the byte offset of a lane's row from its tile's first one in 32 bits (and some of the products it is
+// made of in an int): 128 rows of a K-contiguous operand, 64 with 256-wide tiles; 16 rows of a K-major one; 32 of the addend,
+// 8 with 256-wide tiles.  The 64-wide kernel spans 8 rows of an operand, and the addend's rows have 64-bit addresses there.
+static bool rows_addressable(const GemmParams& p, TileKind k) {
+  auto fits = [](int64_t rows, int ld) { return rows * ld < (int64_t(1) << 31); };
+  if (k == kTile64) return fits(8, p.ldp) && fits(8, p.ldq);
+  const int rows = k == kTile256 ? 64 : 128;
+  return fits(rows, p.ldp) && fits(p.q_kmajor ? 16 : rows, p.ldq) && (!p.D || fits(k == kTile256 ? 8 : 32, p.ldd));
+}
+
 template <bool HAS_D, bool HAS_C, bool HAS_CT, bool QK, int POST = 0, bool BND = false>
 static hipError_t launch_k64_epi(const GemmParams& p, hipStream_t stream,
                                  const typename PostSel<POST>::arg& post = typename PostSel<POST>::arg()) {
   static std::atomic<uint64_t> attr_done{0};
   auto kern = gemm_k64_kernel<HAS_D, HAS_C, HAS_CT, QK, POST, BND>;
   if (hipError_t e = set_max_dynamic_lds_once((const void*)kern, CfgK64::LDS_BYTES, attr_done)) return e;
-  if (p.M % 64 || p.N % 64 || p.K % 64) return hipErrorInvalidValue;
+  if (p.M % 64 || p.N % 64 || p.K % 64 || !rows_addressable(p, kTile64)) return hipErrorInvalidValue;
   const int64_t T = p.M / 64;
   const int64_t total = (p.tri ? T * (T + 1) / 2 : T * (p.N / 64)) * p.batch;
   if (total <= 0) return hipSuccess;
@@ -1700,6 +1712,7 @@ static hipError_t launch_k64(const GemmParams& p, hipStream_t stream) {
   if (p.q_kmajor && !p.tri) {
     if (!d && c && !ct) return launch_k64_epi<false, true, false, true>(p, stream);
     if (!d && !c && ct) return launch_k64_epi<false, false, true, true>(p, stream);
+    if (d && c && !ct) return launch_k64_epi<true, true, false, true>(p, stream);  // (rows too long for the other kernels)
     return hipErrorInvalidValue;
   }
   if (p.tri && !d && c && ct) return launch_k64_epi<false, true, true, false>(p, stream);
@@ -1741,8 +1754,7 @@ int gemm_pad_granule(int m, int n, int batch) {
 //    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
 //    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
 //  * else 128-wide tiles on a two-slot ring, two workgroups per CU (288 tiles of 8 x (1024 x 4096): 50 against 62).
-enum TileKind { kTile64, kTile128Deep, kTile128, kTile256 };
-static TileKind pick_tile(const GemmParams& p) {
+static TileKind tile_by_count(const GemmParams& p) {
   auto tiles = [&](int edge) -> int64_t {
     const int64_t T = p.M / edge;
     return (p.tri ? T * (T + 1) / 2 : T * (p.N / edge)) * (p.rule_batch > 0 ? p.rule_batch : p.batch);
@@ -1760,9 +1772,19 @@ static TileKind pick_tile(const GemmParams& p) {
   return kTile128;
 }
 
+static TileKind pick_tile(const GemmParams& p) {
+  const TileKind k = tile_by_count(p);
+  return rows_addressable(p, k) ? k : kTile64;
+}
+
 int gemm_tile_edge(const GemmParams& p) {
   const TileKind k = pick_tile(p);
   return k == kTile256 ? 256 : k == kTile64 ? 64 : 128;
+}
+
+int gemm_kernel(const GemmParams& p) {
+  const TileKind k = pick_tile(p);
+  return k == kTile256 ? 256 : k == kTile64 ? 64 : k == kTile128Deep ? 129 : 128;
 }
 
 template <class Cfg, int POST, bool BND>

@@ -201,6 +201,12 @@ int dion_ns_plan_audit_prepared(int batch, int rows, int cols, int n_iters, int 
  * FLOP with the library's own rule.  No counterpart in the reference. */
 int dion_gemm_tile_edge(int batch, int m, int n, int symmetric);
 
+/* The kernel that dion_ns_line_1 (m x n matrices), dion_ns_line_2 (m x m; n is not looked at) or dion_ns_line_3 (m x n,
+ * with_addend: a != 0) runs: the edge of its tiles, 64, 128 or 256, or 129 for 128-wide tiles on a four-slot ring; a negative
+ * status for what these refuse.  Host only.  Unlike dion_gemm_tile_edge it knows the reduction length of X X^T.
+ * No counterpart in the reference. */
+int dion_ns_line_kernel(int line, int batch, int m, int n, int with_addend);
+
 /* --------------------------------------------------------------------------------------------
  * Memory-bound fused kernels of the optimizer step.
  * Optimizer state -- parameters X, momentum M, second moments V -- is fp32 or bf16 in memory, as the

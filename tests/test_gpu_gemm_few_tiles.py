@@ -178,3 +178,23 @@ def test_partial_sums_of_symmetric_products(batch, m, n):
     check(lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), batch, m, n, st), "line_1")
     assert bool((A[:, 0::2, 1::2] == 1).all())
     assert torch.equal(A, A.mT)
+
+
+def test_addend_with_rows_too_long_for_32_bit_offsets():
+    lib, check, st = _lib()
+    m, n = 128, 1 << 26
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 35 GB")
+    assert lib.dion_ns_line_kernel(3, 1, m, n, 1) == 64
+    g = torch.Generator(device=DEV).manual_seed(1)
+    B = torch.randn(1, m, m, device=DEV, generator=g).to(torch.bfloat16)
+    X = torch.zeros(1, m, n, device=DEV, dtype=torch.bfloat16)
+    Y = torch.empty_like(X)
+    parts = [slice(c, c + 4096) for c in (0, n // 2 - 2048, n - 4096)]
+    for p in parts:
+        X[:, :, p] = torch.randn(1, m, 4096, device=DEV, generator=g).to(torch.bfloat16)
+    check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), 1, m, n, ctypes.c_float(0.75), st), "line_3")
+    for p in parts:
+        Xd = X[:, :, p].double()
+        _close(Y[:, :, p], B.double() @ Xd + 0.75 * Xd)
+    assert not bool(Y[:, :, 4096:n // 2 - 2048].any()) and not bool(Y[:, :, n // 2 + 2048:n - 4096].any())

@@ -254,3 +254,13 @@ def test_tiles_of_symmetric_products_with_short_reductions(batch, m, edge):
     """64-wide tiles split a reduction over four wavefronts; past one such tile per CU a short one is left with less than it
     costs to add the parts (128 x (128 x 128): 6.8 us against 5.1)."""
     assert _lib.load().dion_gemm_tile_edge(batch, m, m, 1) == edge
+
+
+@pytest.mark.parametrize("line,m,n,addend,edge", [
+    (1, 2048, 1 << 24, 0, 64), (1, 2048, (1 << 24) - 128, 0, 129), (1, 2048, 16911104, 0, 64),  # 128 rows past 2^31 elements
+    (1, 4096, 1 << 25, 0, 64), (1, 4096, 1 << 24, 0, 256),
+    (3, 128, 1 << 26, 1, 64), (3, 128, (1 << 26) - 128, 1, 128), (3, 128, 1 << 26, 0, 128), (3, 128, 1 << 27, 0, 64)])
+def test_rows_too_long_for_32_bit_offsets(line, m, n, addend, edge):
+    """128- and 256-wide tiles address a tile's rows with 32-bit offsets, which the rows of X X^T from 2^24 columns on (2^25 with
+    256-wide tiles), of the addend from 2^26, of the K-major operand from 2^27 do not fit: 64-wide tiles take those."""
+    assert _lib.load().dion_ns_line_kernel(line, 1, m, n, addend) == edge
