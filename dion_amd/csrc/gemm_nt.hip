@@ -1731,12 +1731,17 @@ int gemm_pad_granule(int m, int n, int batch) {
 
 // Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box.
 //  * 256-wide tiles, a symmetric product: when 128-wide ones are more than two per CU (512) and 256-wide ones at most one;
-//    past that from the count on where 128-wide ones need a fourth round of two per CU (1536; reductions past 2048: from
-//    1152, their second round of 256-wide tiles being the cheaper one).  X X^T on 256- / 128-wide tiles: 130 / 468 tiles of
-//    13 x (1024 x 1024) 26.1 / 19.5, 144 / 544 of 4 x (2048 x 2048) 42.6 / 48.8, 200 / 720 of 20 x (1024 x 3072) 65.0 / 71.8,
-//    260 / 936 of 26 x (1024 x 1024) 50.8 / 36.7, of 26 x (1024 x 3072) 124 / 81, 288 / 1008 of 48 x (768 x 2304) 94.6 / 66.4,
-//    320 / 1152 of 32 x (1024 x 3072) 123 / 111, 360 / 1296 of 36 x 138 / 146, 399 / 1482 of 19 x (1536 x 1536) 74.5 / 70.4, 420 / 1560
-//    of 20 x 76.4 / 86.9.  A full product: when they make one round of the CUs where 128-wide ones make more than one of
+//    past that from the count on where 128-wide ones need a fourth round of two per CU (1536) where the reduction is as long
+//    as the matrix is wide, and soon into the third (1152, or its begin, 1024) where it is longer.  X X^T on 256- / 128-wide
+//    tiles, repeated on one operand: 130 / 468 tiles of 13 x (1024 x 1024) 26.1 / 19.5, 144 / 544 of 4 x (2048 x 2048) 42.6 /
+//    48.8, 200 / 720 of 20 x (1024 x 3072) 65.0 / 71.8, 260 / 936 of 26 x (1024 x 1024) 50.8 / 36.7, of 26 x (1024 x 3072) 124 /
+//    81, 270 / 900 of 90 x (512 x 2048) 84.9 / 55.8, 399 / 1482 of 19 x (1536 x 1536) 74.5 / 70.4, 420 / 1560 of 20 x 76.4 / 86.9.
+//    The third round's lines are those of whole calls, whose X the product before has just written (five NS5 iterations, X X^T
+//    on 256- / 128-wide tiles): 1344 tiles of 64 x (768 x 1536) 1303 / 1343, 1296 of 36 x (1024 x 2048) 1574 / 1622, 1512 of
+//    42 x 1781 / 1846, but 1050 of 10 x (1792 x 3584) 2127 / 2085, 1044 of 29 x (1024 x 2048) 1339 / 1315, 1152 of
+//    32 x (1024 x 1280) 1032 / 1025; from reductions four times the width on 1100 of 110 x (512 x 2048) 1412 / 1467, 1134 of
+//    54 x (768 x 3072) 2018 / 2053, outside these widths 1026 of 342 x (256 x 1024) 855 / 836, 1050 of 10 x (1792 x 7168) 3835 /
+//    3755.  A full product: when they make one round of the CUs where 128-wide ones make more than one of
 //    two workgroups each (129-256 tiles), or most of two (from 336, with reductions past 1024 from 384).  B X on 128- /
 //    256-wide tiles: 128 tiles of 8 x (1024 x 1024) 20.5 / 25.2, 144 of 9 x 29.3 / 25.9, 256 of 16 x 36.9 / 32.9, 272 of 17 x
 //    46.6 / 49.1, 336 of 21 x 51.0 / 49.8; 135 of 15 x (768 x 768) 24.1 / 21.8, 243 of 27 x 30.7 / 26.8; 129 of 43 x
@@ -1761,7 +1766,8 @@ static TileKind tile_by_count(const GemmParams& p) {
   };
   if (p.M % 256 == 0 && p.N % 256 == 0) {
     const int64_t t = tiles(256), t128 = tiles(128);
-    const bool sym = t128 > 512 && (t <= 256 || t128 > (p.K > 2048 ? 1152 : 1536));
+    const int most128 = p.K / 4 >= p.M && p.M >= 512 && p.M <= 1024 ? 1024 : p.K > p.M || p.K > 2048 ? 1152 : 1536;
+    const bool sym = t128 > 512 && (t <= 256 || t128 > most128);
     const bool full = t >= 384 || (t > 128 && t <= 256) || (t >= 336 && p.K <= 1024);
     if (p.tri ? sym : full) return kTile256;
   }

@@ -264,3 +264,14 @@ def test_rows_too_long_for_32_bit_offsets(line, m, n, addend, edge):
     """128- and 256-wide tiles address a tile's rows with 32-bit offsets, which the rows of X X^T from 2^24 columns on (2^25 with
     256-wide tiles), of the addend from 2^26, of the K-major operand from 2^27 do not fit: 64-wide tiles take those."""
     assert _lib.load().dion_ns_line_kernel(line, 1, m, n, addend) == edge
+
+
+@pytest.mark.parametrize("line,batch,m,n,edge", [
+    (1, 64, 768, 1536, 256), (1, 36, 1024, 2048, 256), (1, 32, 1024, 1280, 128), (1, 33, 1024, 1280, 256),  # 1152 | 1188 128-wide tiles
+    (1, 110, 512, 2048, 256), (1, 110, 512, 1920, 128), (1, 102, 512, 2048, 128), (1, 54, 768, 3072, 256), (1, 342, 256, 1024, 128),
+    (1, 10, 1792, 7168, 128), (1, 42, 1024, 1024, 128), (1, 43, 1024, 1024, 256), (2, 42, 1024, 1024, 128), (2, 43, 1024, 1024, 256),
+    (1, 13, 1024, 3072, 128), (1, 16, 1024, 3072, 256), (1, 26, 1024, 3072, 128)])
+def test_tiles_of_symmetric_products_by_rounds(line, batch, m, n, edge):
+    """128-wide tiles of a symmetric product in their third round of two per CU: no more than soon after its begin where the
+    reduction is longer than the matrix is wide (a call on 42 x (1024 x 2048) took 1846 us so, 1781 with 256-wide ones)."""
+    assert _lib.load().dion_ns_line_kernel(line, batch, m, n, 0) == edge
