@@ -148,15 +148,20 @@ extern "C" int dion_ns_line_3(const void* B, const void* X, void* C, int batch, 
   return DION_OK;
 }
 
-extern "C" int dion_ns_line_kernel(int line, int batch, int m, int n, int with_addend) {
+extern "C" int dion_ns_line_kernel(int line, int batch, int m, int n, int form) {
   if (int rc = check_gemm_dims("dion_ns_line_kernel", batch, m, line == 2 ? m : n)) return rc;
-  if (line < 1 || line > 3 || batch == 0 || m == 0 || (line != 2 && n == 0))
-    return fail(DION_E_INVALID, "dion_ns_line_kernel: line %d, %d x (%d x %d)", line, batch, m, n);
+  if (line < 1 || line > 3 || form < 0 || form > 5 || (form && line != 3) || batch == 0 || m == 0 || (line != 2 && n == 0))
+    return fail(DION_E_INVALID, "dion_ns_line_kernel: line %d, form %d, %d x (%d x %d)", line, form, batch, m, n);
   // (addresses are not looked at, only whether there is an addend)
   static const bf16_t any = 0;
-  return gemm_kernel(line == 1   ? line_1_params(&any, nullptr, batch, m, n)
-                     : line == 2 ? line_2_params(&any, nullptr, batch, m, 1.0f, 1.0f)
-                                 : line_3_params(&any, &any, nullptr, batch, m, n, with_addend ? 1.0f : 0.0f));
+  GemmParams p = line == 1   ? line_1_params(&any, nullptr, batch, m, n)
+                 : line == 2 ? line_2_params(&any, nullptr, batch, m, 1.0f, 1.0f)
+                             : line_3_params(&any, &any, nullptr, batch, m, n, form == 1 ? 1.0f : 0.0f);
+  if (form >= 4) {
+    p.out_rows = m - 1;
+    p.out_cols = n - 1;
+  }
+  return gemm_kernel(p, form < 2 ? kNoUpdate : form % 2 ? kUpdateTransposed : kUpdate);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -257,7 +257,8 @@ hipError_t launch_gemm_nt(const GemmParams& p, hipStream_t stream);
 // multiples of it, K of 128.
 int gemm_tile_edge(const GemmParams& p);
 // The kernel they use: 64, 128 (two-slot ring), 256, or 129 for 128-wide tiles on the four-slot ring.
-int gemm_kernel(const GemmParams& p);
+enum UpdateKind { kNoUpdate, kUpdate, kUpdateTransposed };  // launch_gemm_nt, launch_gemm_nt_post by `transposed`
+int gemm_kernel(const GemmParams& p, UpdateKind update);
 // C = P * Q with Q K-major (p.q_kmajor, no tri, no D), the product consumed by the fused Muon update
 // instead of being stored: `transposed` false updates X[row][col] (ldc / strideC describe X),
 // true updates X[col][row] (ldct / strideCt).  x_dtype 0 = bf16, 1 = fp32.  p.batch <= kMaxPtrs *

@@ -1742,11 +1742,17 @@ int gemm_pad_granule(int m, int n, int batch) {
 //    32 x (1024 x 1280) 1032 / 1025; from reductions four times the width on 1100 of 110 x (512 x 2048) 1412 / 1467, 1134 of
 //    54 x (768 x 3072) 2018 / 2053, outside these widths 1026 of 342 x (256 x 1024) 855 / 836, 1050 of 10 x (1792 x 7168) 3835 /
 //    3755.  A full product: when they make one round of the CUs where 128-wide ones make more than one of
-//    two workgroups each (129-256 tiles), or most of two (from 336, with reductions past 1024 from 384).  B X on 128- /
-//    256-wide tiles: 128 tiles of 8 x (1024 x 1024) 20.5 / 25.2, 144 of 9 x 29.3 / 25.9, 256 of 16 x 36.9 / 32.9, 272 of 17 x
-//    46.6 / 49.1, 336 of 21 x 51.0 / 49.8; 135 of 15 x (768 x 768) 24.1 / 21.8, 243 of 27 x 30.7 / 26.8; 129 of 43 x
-//    (256 x 768) 13.2 / 11.4, 256 of 32 x (512 x 1024) 26.2 / 21.8, 336 of 42 x 33.5 / 30.7; 252 of 7 x (1536 x 1536) 50.0 /
-//    44.1, 360 of 10 x 71.4 / 72.1.
+//    two workgroups each (129-256 tiles), or most of two (from 336, with reductions past 1024 or an epilogue that reads memory --
+//    an addend, a fused update -- from 384); the update of transposed padded parameters, whose epilogue is the longest, not
+//    on one round of reductions up to 512.  B X on 128- / 256-wide tiles: 128 tiles of 8 x (1024 x 1024) 20.5 / 25.2, 144 of 9 x
+//    27.2 / 24.3, 256 of 16 x 33.7 / 31.4, 272 of 17 x 46.6 / 49.1, 135 of 15 x (768 x 768) 24.2 / 22.1, 129 of 43 x (256 x 768)
+//    12.4 / 11.4, 216 of 27 x (512 x 1024) 23.0 / 19.9, 252 of 7 x (1536 x 1536) 50.0 / 44.1, 360 of 10 x 71.4 / 72.1, 192 of one
+//    3072 x 4096 75.9 / 66.7, 256 of one 4096 x 4096 112 / 100, 336 of 42 x (512 x 1024) 33.9 / 31.2 (on another box 28.8 / 29.5),
+//    of 21 x (1024 x 1024) 52.0 / 50.6.  With an addend 144 of 9 x (1024 x 1024) 28.3 / 25.8, 129 of 43 x (256 x 768) 13.2 / 12.8,
+//    336 of 42 x (512 x 1024) 34.6 / 36.5.  Updates of fp32 parameters 144 of 9 x (1024 x 1024) 33.4 / 32.1, 192 of one
+//    3072 x 4096 81.6 / 71.4, 336 of 21 x (1024 x 1024) 65.8 / 71.8, 352 of 44 x (512 x 1024) 54.4 / 51.4; padded and transposed
+//    144 of 9 x (1024 x 1024) 50.7 / 49.7, 135 of 15 x (768 x 768) 46.0 / 46.3, 132 of 33 x (512 x 512) 40.1 / 42.3, 130 of
+//    65 x (256 x 512) 35.3 / 38.2, 336 of 42 x (512 x 1024) 70.7 / 84.3.
 //  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
 //    per CU: X X^T of one 768 x 3072 matrix 28.4 -> 10.0 (78 tiles), of 1024 x 4096 42.9 -> 15.8, of 4 x (640 x 2560) 16.3 ->
 //    10.4; B X of 1024 x 1024 (256 tiles) 9.8 -> 6.3, past that the last form, at 288 (2 x (768 x 768)) 9.4 against 8.4, at 576
@@ -1759,7 +1765,7 @@ int gemm_pad_granule(int m, int n, int batch) {
 //    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
 //    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
 //  * else 128-wide tiles on a two-slot ring, two workgroups per CU (288 tiles of 8 x (1024 x 4096): 50 against 62).
-static TileKind tile_by_count(const GemmParams& p) {
+static TileKind tile_by_count(const GemmParams& p, UpdateKind update) {
   auto tiles = [&](int edge) -> int64_t {
     const int64_t T = p.M / edge;
     return (p.tri ? T * (T + 1) / 2 : T * (p.N / edge)) * (p.rule_batch > 0 ? p.rule_batch : p.batch);
@@ -1768,7 +1774,8 @@ static TileKind tile_by_count(const GemmParams& p) {
     const int64_t t = tiles(256), t128 = tiles(128);
     const int most128 = p.K / 4 >= p.M && p.M >= 512 && p.M <= 1024 ? 1024 : p.K > p.M || p.K > 2048 ? 1152 : 1536;
     const bool sym = t128 > 512 && (t <= 256 || t128 > most128);
-    const bool full = t >= 384 || (t > 128 && t <= 256) || (t >= 336 && p.K <= 1024);
+    const bool one_round = t > 128 && t <= 256 && !(update == kUpdateTransposed && bounded(p) && p.K <= 512);
+    const bool full = t >= 384 || one_round || (t >= 336 && p.K <= 1024 && update == kNoUpdate && !p.D);
     if (p.tri ? sym : full) return kTile256;
   }
   const int short_k = p.M < 256 ? 1024 : p.M < 384 ? 512 : 384;
@@ -1778,8 +1785,8 @@ static TileKind tile_by_count(const GemmParams& p) {
   return kTile128;
 }
 
-static TileKind pick_tile(const GemmParams& p) {
-  const TileKind k = tile_by_count(p);
+static TileKind pick_tile(const GemmParams& p, UpdateKind update = kNoUpdate) {
+  const TileKind k = tile_by_count(p, update);
   return rows_addressable(p, k) ? k : kTile64;
 }
 
@@ -1788,8 +1795,8 @@ int gemm_tile_edge(const GemmParams& p) {
   return k == kTile256 ? 256 : k == kTile64 ? 64 : 128;
 }
 
-int gemm_kernel(const GemmParams& p) {
-  const TileKind k = pick_tile(p);
+int gemm_kernel(const GemmParams& p, UpdateKind update) {
+  const TileKind k = pick_tile(p, update);
   return k == kTile256 ? 256 : k == kTile64 ? 64 : k == kTile128Deep ? 129 : 128;
 }
 
@@ -1802,7 +1809,7 @@ static hipError_t launch_post_cfg(const GemmParams& p, const FusedPost& post, bo
 
 template <int POST, bool BND>
 static hipError_t launch_post(const GemmParams& p, const FusedPost& post, bool transposed, hipStream_t stream) {
-  switch (pick_tile(p)) {
+  switch (pick_tile(p, transposed ? kUpdateTransposed : kUpdate)) {
     case kTile256: return launch_post_cfg<Cfg256w8, POST, BND>(p, post, transposed, stream);
     case kTile128Deep: return launch_post_cfg<Cfg128d, POST, BND>(p, post, transposed, stream);
     case kTile64:

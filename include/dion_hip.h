@@ -201,11 +201,12 @@ int dion_ns_plan_audit_prepared(int batch, int rows, int cols, int n_iters, int 
  * FLOP with the library's own rule.  No counterpart in the reference. */
 int dion_gemm_tile_edge(int batch, int m, int n, int symmetric);
 
-/* The kernel that dion_ns_line_1 (m x n matrices), dion_ns_line_2 (m x m; n is not looked at) or dion_ns_line_3 (m x n,
- * with_addend: a != 0) runs: the edge of its tiles, 64, 128 or 256, or 129 for 128-wide tiles on a four-slot ring; a negative
- * status for what these refuse.  Host only.  Unlike dion_gemm_tile_edge it knows the reduction length of X X^T.
- * No counterpart in the reference. */
-int dion_ns_line_kernel(int line, int batch, int m, int n, int with_addend);
+/* The kernel that dion_ns_line_1 (m x n matrices), dion_ns_line_2 (m x m; n is not looked at) or dion_ns_line_3 (m x n) runs:
+ * the edge of its tiles, 64, 128 or 256, or 129 for 128-wide tiles on a four-slot ring; a negative status for what these
+ * refuse.  form, 0 but for line 3: 1 with an addend (a != 0); 2 or 3 for the last product of dion_ns_orthogonalize_update
+ * that updates m x n or n x m parameters, 4 or 5 for the same of parameters smaller than the padded m x n product.
+ * Host only.  Unlike dion_gemm_tile_edge it knows the reduction length of X X^T.  No counterpart in the reference. */
+int dion_ns_line_kernel(int line, int batch, int m, int n, int form);
 
 /* --------------------------------------------------------------------------------------------
  * Memory-bound fused kernels of the optimizer step.

@@ -275,3 +275,14 @@ def test_tiles_of_symmetric_products_by_rounds(line, batch, m, n, edge):
     """128-wide tiles of a symmetric product in their third round of two per CU: no more than soon after its begin where the
     reduction is longer than the matrix is wide (a call on 42 x (1024 x 2048) took 1846 us so, 1781 with 256-wide ones)."""
     assert _lib.load().dion_ns_line_kernel(line, batch, m, n, 0) == edge
+
+
+@pytest.mark.parametrize("batch,m,n,edges", [  # per form: stored, with an addend, update, transposed update, both of padded parameters
+    (42, 512, 1024, (256, 128, 128, 128, 128, 128)), (41, 512, 1024, (128,) * 6), (48, 512, 1024, (256,) * 6),
+    (11, 1024, 2048, (256, 128, 128, 128, 128, 128)), (10, 1536, 1536, (128,) * 6),
+    (27, 512, 1024, (256, 256, 256, 256, 256, 128)), (43, 256, 768, (256, 256, 256, 256, 256, 128)), (15, 768, 768, (256,) * 6),
+    (1, 4096, 4096, (256,) * 6), (8, 1024, 1024, (128,) * 6)])
+def test_tiles_of_full_products_by_form(batch, m, n, edges):
+    """The lines between 128- and 256-wide tiles of B X lie elsewhere where the epilogue reads memory (336 tiles of
+    42 x (512 x 1024): stored 33.9 us against 31.2, with an addend 34.6 / 36.5, updating padded transposed parameters 70.7 / 84.3)."""
+    assert tuple(_lib.load().dion_ns_line_kernel(3, batch, m, n, form) for form in range(6)) == edges
