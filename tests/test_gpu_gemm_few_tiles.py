@@ -87,10 +87,12 @@ def test_products_at_the_line_of_short_reductions(batch, m, n, sym_edge, full_ed
 
 
 # Slab counts (64 columns of the reduction each) from fewer than a ring has slots, remainders of its length among them.
-@pytest.mark.parametrize("batch", [14, 30])  # 140 tiles on the four-slot ring, 300 on the two-slot one
+# 504 tiles of 64 from n = 384 on and 140 of 128 on the four-slot ring below; 160 on the four-slot ring; 300 on the two-slot one
+@pytest.mark.parametrize("batch", [14, 16, 30])
 @pytest.mark.parametrize("n", [128, 256, 384, 512, 640, 768, 896, 1152])
 def test_reduction_lengths_of_symmetric_products(batch, n):
     lib, check, st = _lib()
+    assert lib.dion_ns_line_kernel(1, batch, 512, n, 0) == (128 if batch == 30 else 129 if batch == 16 or n < 384 else 64)
     g = torch.Generator(device=DEV).manual_seed(n)
     X = torch.randn(batch, 512, n, device=DEV, generator=g).to(torch.bfloat16)
     A = torch.full((batch, 512, 512), float("nan"), device=DEV, dtype=torch.bfloat16)
@@ -133,6 +135,20 @@ def test_addend_at_every_slab_count(m, batch, sym_edge):
     _close(Y, Sd @ X.double() + 0.75 * X.double())
 
 
+# K-major operand and addend on the four-slot ring: slab counts (m / 64) that leave the addend in either of its slots.
+@pytest.mark.parametrize("m", [1152, 1280, 1408, 1536])
+def test_k_major_products_on_the_four_slot_ring(m):
+    lib, check, st = _lib()
+    assert lib.dion_ns_line_kernel(3, 1, m, m, 0) == 129 and lib.dion_ns_line_kernel(3, 1, m, m, 1) == 129
+    g = torch.Generator(device=DEV).manual_seed(m)
+    B = (torch.randn(1, m, m, device=DEV, generator=g) / m ** 0.5).to(torch.bfloat16)
+    X = torch.randn(1, m, m, device=DEV, generator=g).to(torch.bfloat16)
+    for a in (0.0, 0.75):
+        Y = torch.full_like(X, float("nan"))
+        check(lib.dion_ns_line_3(B.data_ptr(), X.data_ptr(), Y.data_ptr(), 1, m, m, ctypes.c_float(a), st), "line_3")
+        _close(Y, B.double() @ X.double() + a * X.double())
+
+
 # Full products on both sides of the lines between 128- and 256-wide tiles: one round of the CUs, and most of two.
 @pytest.mark.parametrize("batch,m,n,edge", [(32, 512, 512, 128), (43, 256, 768, 256), (32, 512, 1024, 256), (17, 1024, 1024, 128),
                                             (42, 512, 1024, 256), (7, 1536, 1536, 256), (10, 1536, 1536, 128), (9, 1024, 1152, 128)])
@@ -148,12 +164,14 @@ def test_full_products_at_the_lines_of_256_wide_tiles(batch, m, n, edge):
     _close(Y, B.double() @ X.double())
 
 
-# Symmetric products on both sides of the lines between 64-, 128- and 256-wide tiles.
-@pytest.mark.parametrize("batch,m,n", [(6, 768, 768), (6, 768, 1024), (1, 1920, 1920), (1, 1920, 2048), (21, 512, 1024), (51, 512, 512),
-                                       (52, 512, 512), (85, 512, 640), (86, 512, 640), (36, 1024, 1024), (32, 1024, 2176), (33, 1024, 2176),
-                                       (20, 1536, 1536)])
-def test_symmetric_products_at_the_lines(batch, m, n):
+# Symmetric products on both sides of the lines between 64-, 128- (129: on the four-slot ring) and 256-wide tiles.
+@pytest.mark.parametrize("batch,m,n,kernel", [(6, 768, 768, 64), (6, 768, 1024, 64), (7, 768, 1024, 129), (1, 1920, 1920, 64),
+                                              (1, 1920, 2048, 64), (1, 2048, 2048, 129), (21, 512, 1024, 129), (51, 512, 512, 128),
+                                              (52, 512, 512, 256), (85, 512, 640, 256), (86, 512, 640, 128), (36, 1024, 1024, 128),
+                                              (32, 1024, 2176, 128), (33, 1024, 2176, 256), (20, 1536, 1536, 256)])
+def test_symmetric_products_at_the_lines(batch, m, n, kernel):
     lib, check, st = _lib()
+    assert lib.dion_ns_line_kernel(1, batch, m, n, 0) == kernel
     g = torch.Generator(device=DEV).manual_seed(batch + n)
     X = torch.randn(batch, m, n, device=DEV, generator=g).to(torch.bfloat16)
     A = torch.full((batch, m, m), float("nan"), device=DEV, dtype=torch.bfloat16)
