@@ -357,9 +357,11 @@ def main() -> int:
         # the launch stream.  "executed" counts the MFMA work actually issued (upper-triangle tiles only
         # for the two symmetric products), "algorithmic" the full product.
         A = torch.empty(B, m, m, device=dev, dtype=torch.bfloat16)
-        # executed share of a symmetric product: upper tiles only, with the tile edge the library picks
-        T = m // lib.dion_gemm_tile_edge(B, m, m, 1)
-        tri = (T + 1) / (2.0 * T)
+        # executed share of a symmetric product (line 1: X X^T, 2: A A): upper tiles only, with the tile edge the library picks
+        def tri(line):
+            T = m // (lib.dion_ns_line_kernel(line, B, m, n, 0) // 64 * 64)  # (129: 128-wide tiles, too)
+            return (T + 1) / (2.0 * T)
+
         ms1 = time_kernel(lambda: lib.dion_ns_line_1(X.data_ptr(), A.data_ptr(), B, m, n, st))
         ms2 = time_kernel(lambda: lib.dion_ns_line_2(Bm.data_ptr(), A.data_ptr(), B, m, 1.0, 1.0, st))
         # dominant kernel: X' = B X with a*I folded into B, reading X as it lies; one launch per NS
@@ -386,8 +388,8 @@ def main() -> int:
                     "tflops_algorithmic": round(flop_full / (ms * 1e-3) * 1e-12, 1)}
 
         result["gemms"] = {
-            "A = X X^T": gemm_row(ms1, 2.0 * B * m * m * n, tri),
-            "B = c A A + b A + a I": gemm_row(ms2, 2.0 * B * m * m * m, tri),
+            "A = X X^T": gemm_row(ms1, 2.0 * B * m * m * n, tri(1)),
+            "B = c A A + b A + a I": gemm_row(ms2, 2.0 * B * m * m * m, tri(2)),
             "X' = B X": gemm_row(ms3, 2.0 * B * m * m * n, 1.0),
         }
         flop3 = 2.0 * B * m * m * n
