@@ -17,9 +17,10 @@
 // Kernel structure: one workgroup per BM x BN output tile, WM x WN wavefronts (64 lanes) each
 // owning a (BM/WM) x (BN/WN) sub-tile as 16x16 MFMA accumulators (v_mfma_f32_16x16x32_bf16: per
 // FLOP half the accumulator register traffic of the 32x32x16 form, which on this power-limited part is
-// worth 5 % of clock).  Operand tiles reach a two-slot LDS ring through direct-to-LDS
-// loads (global_load_lds_dwordx4, no VGPR staging); XOR swizzles keep the LDS writes and the
-// fragment reads bank-conflict free.
+// worth 5 % of clock).  Operand tiles reach an LDS ring through direct-to-LDS loads, no VGPR staging: two slots
+// filled by global_load_lds_dwordx4 with 256-wide tiles, two or four filled by buffer loads with 128-wide ones, and
+// a two-slot ring of its own per wavefront with 64-wide ones (gemm_k64_kernel).  XOR swizzles keep the LDS writes and
+// the fragment reads bank-conflict free.
 #include <type_traits>
 
 #include "common.h"
@@ -586,15 +587,18 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_nt_kernel(const GemmParams p,
     // slab is free for its refill a slab earlier than with fragments read half a slab ahead.  Four wavefronts share a
     // CU's four SIMDs here, or eight with two workgroups, so nothing hides what a wavefront issues besides its MFMAs:
     // an instruction costs four cycles, an MFMA sixteen, hence slots as constants of the unrolled loop and
-    // refills without address arithmetic.  What bounds it is the LDS: 64 KB of fragments and 32 KB of refills a slab are
-    // 750 cycles at 128 bytes per cycle, 512 are MFMA time; measured 0.31 us a slab of a long reduction (0.42 with half-slab
-    // fragments and accumulators in AGPRs, which the compiler copied around every MFMA: __launch_bounds__' second figure
+    // refills without address arithmetic.  The LDS allows 0.3 us a slab: 64 KB of fragments and 32 KB of refills are
+    // 750 cycles at 128 bytes per cycle, 512 are MFMA time.  Measured, X X^T of b x (1024 x K) on the four-slot ring, K from
+    // 1024 to 4096: 0.28-0.31 us with up to 144 workgroups whatever the operands hold, 0.39 with 252.  Of those 0.39,
+    // operands of zeros give back 0.07 (the clock, on this power-limited part) and one matrix for all workgroups 0.02-0.04 (the
+    // way from memory to L2); both, 0.30.  (Half-slab fragments and accumulators in AGPRs, which the compiler copied
+    // around every MFMA, took 0.42 where this takes 0.31: __launch_bounds__' second figure
     // keeps them out).  Short reductions pay for what is outside: first loads 1.3 us behind the tile's coordinates, the
     // epilogue 1.4.  X X^T of 12 x (768 x 3072) 27.1 -> 24.4 us, of 4 x (1024 x 2816) 23.1 -> 19.8, of 24 x (512 x 8192)
     // 62.6 -> 51.7, of 8 x (1024 x 4096), two workgroups per CU, 49.6 -> 41.2, of 10 x (640 x 640) 9.5 -> 8.3, A A of
     // those 10.6 -> 9.1, of 24 x (512 x 512) 10.4 -> 9.1; B X of 10 x (640 x 640) 9.5 -> 8.7.  256 x 128 tiles
-    // on the same loop (eight wavefronts, three slots) are bound by the LDS alike: 0.57 us for twice the work, slower in a
-    // launch than either neighbour (12 x (768 x 768): 14.7 against 13.8 us).
+    // on the same loop (eight wavefronts, three slots) take 0.57 us a slab for twice the work, in a launch longer than either
+    // neighbour (12 x (768 x 768): 14.7 against 13.8 us).
     static_assert(TM == 4 && ST == 2 && LPS <= 8, "64 x 64 wavefront tiles");
     bf16x8 fa[2][ST][4], fb[2][ST][TN];  // by parity of the slab
     // read r (0..15) of the fragments of the slab in ring slot `slotc` (0, 1) of the pair the offsets point to
@@ -1298,7 +1302,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
 // ---------------------------------------------------------------------------------------------
 // The same product for launches of few tiles: 64 x 64 tiles, the reduction of a tile split over the four
 // wavefronts of its workgroup.  With a handful of 128-wide tiles most CUs idle and each busy one walks the whole
-// reduction at the pace of its own operand stream (0.4-0.6 us per 64-deep slab, 64 slabs for 1024 x 4096); four times
+// reduction at the pace of its own operand stream (0.3-0.4 us per 64-deep slab, 64 slabs for 1024 x 4096); four times
 // as many tiles, each pulling a quarter of the bytes at once through four private rings, use the CUs that are
 // there.  A wavefront takes every fourth slab (64 x 64 of each operand) into a two-slot ring of its own and never
 // meets a barrier until its partial sums are added; the 64 x 64 wavefront tile keeps the fragment schedule of the
@@ -1722,18 +1726,26 @@ static hipError_t launch_k64(const GemmParams& p, hipStream_t stream) {
 }
 
 int gemm_pad_granule(int m, int n, int batch) {
-  // 256-wide tiles need enough of them to fill 256 CUs; small problems use 128-wide tiles.
+  // To 256 once whole 256-wide tiles make more than one round of the CUs for the symmetric products, so that every product may
+  // use them.  Where the symmetric ones stay on 128-wide tiles all the same (the lines below), padding a multiple of 128
+  // costs more than 256-wide tiles of B X give back.  NS5, us a call padded to 256 / 128: 48 x (640 x 2560) 1474 / 1283,
+  // 18 x (1152 x 1152) 798 / 684, 16 x (1408 x 1408) 1313 / 1062, 100 x (384 x 1536) 1010 / 737, 30 x (896 x 3584) 2244 / 1839; where both
+  // pad to the same width 47 x (650 x 2550) 1502 / 1511, 18 x (1200 x 1200) 816 / 815; 5 x (2944 x 2944), 256-wide throughout,
+  // 2569 / 2667.  The granule is also the layout dion_ns_padded_extents and dion_ns_accepts_prepared report, and what is
+  // not padded has its norm added up in another order, so another granule is not the same bits.
   const int64_t m256 = (m + 255) / 256;
   const int64_t syrk_tiles = m256 * (m256 + 1) / 2 * batch;
   (void)n;
   return syrk_tiles >= 256 ? 256 : 128;
 }
 
-// Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box.
+// Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box, a launch
+// repeated on the same operands unless it says otherwise.  In a call, behind the launch that wrote an operand, a launch
+// of few tiles takes up to 3 us more (X X^T of one 768 x 3072 13.0, B X 10.1).
 //  * 256-wide tiles, a symmetric product: when 128-wide ones are more than two per CU (512) and 256-wide ones at most one;
 //    past that from the count on where 128-wide ones need a fourth round of two per CU (1536) where the reduction is as long
 //    as the matrix is wide, and soon into the third (1152, or its begin, 1024) where it is longer.  X X^T on 256- / 128-wide
-//    tiles, repeated on one operand: 130 / 468 tiles of 13 x (1024 x 1024) 26.1 / 19.5, 144 / 544 of 4 x (2048 x 2048) 42.6 /
+//    tiles: 130 / 468 tiles of 13 x (1024 x 1024) 26.1 / 19.5, 144 / 544 of 4 x (2048 x 2048) 42.6 /
 //    48.8, 200 / 720 of 20 x (1024 x 3072) 65.0 / 71.8, 260 / 936 of 26 x (1024 x 1024) 50.8 / 36.7, of 26 x (1024 x 3072) 124 /
 //    81, 270 / 900 of 90 x (512 x 2048) 84.9 / 55.8, 399 / 1482 of 19 x (1536 x 1536) 74.5 / 70.4, 420 / 1560 of 20 x 76.4 / 86.9.
 //    The third round's lines are those of whole calls, whose X the product before has just written (five NS5 iterations, X X^T
@@ -1754,17 +1766,21 @@ int gemm_pad_granule(int m, int n, int batch) {
 //    144 of 9 x (1024 x 1024) 50.7 / 49.7, 135 of 15 x (768 x 768) 46.0 / 46.3, 132 of 33 x (512 x 512) 40.1 / 42.3, 130 of
 //    65 x (256 x 512) 35.3 / 38.2, 336 of 42 x (512 x 1024) 70.7 / 84.3.
 //  * 64-wide tiles with the reduction split over a workgroup's wavefronts (gemm_k64_kernel) when they are at most one
-//    per CU: X X^T of one 768 x 3072 matrix 28.4 -> 10.0 (78 tiles), of 1024 x 4096 42.9 -> 15.8, of 4 x (640 x 2560) 16.3 ->
-//    10.4; B X of 1024 x 1024 (256 tiles) 9.8 -> 6.3, past that the last form, at 288 (2 x (768 x 768)) 9.4 against 8.4, at 576
-//    (768 x 3072) 14.0 against 8.9.  Symmetric products of up to two per CU where the reduction is not short: the form
-//    below takes less time there (X X^T of 2 x (1024 x 4096) 24.0 against 30.6, of 13 x (512 x 2048) 14.9 / 17.8, of
-//    113 x (128 x 2048) 14.1 / 17.4, of 6 x (768 x 3072) 22.1 / 25.3, of 8 x (512 x 2048) 14.0 / 14.0; A A of 5 x (768 x 768)
-//    9.3 / 10.5), but adds a reduction up in one chain where this one has four partial sums, and one chain carries twice
-//    the rounding error: sums of 2048 products of unit variance that cancel, 3.7e-6 rms here, 8.1e-6 there.
+//    per CU.  64- / 128-wide tiles: X X^T of one 768 x 3072 matrix 10.1 / 17.8 (78 tiles), of 1024 x 4096 16.3 / 23.7, of
+//    4 x (640 x 2560) 10.6 / 15.9, A A of one 1024 x 1024 6.4 / 9.8; B X of one 1024 x 1024 (256 tiles) 5.8 / 8.6, its update 8.0 /
+//    10.3, past that no more: 288 of 2 x (768 x 768) 8.6 / 7.3, 576 of one 768 x 3072 13.0 / 7.9.  Whole calls with X X^T on
+//    64- / 128-wide tiles: one 768 x 3072 163 / 200, 3 x (768 x 3072) 184 / 220, 60 x (128 x 2048) 155 / 169.
+//    Symmetric products of up to two per CU where the reduction is not short: 128-wide tiles take less time there (X X^T of
+//    2 x (1024 x 4096) 30.6 / 24.0, of 13 x (512 x 2048) 17.8 / 14.9, of 113 x (128 x 2048) 17.4 / 14.1, of 6 x (768 x 3072) 25.3 /
+//    22.1, of 8 x (512 x 2048) 14.0 / 14.0; A A of 5 x (768 x 768) 10.4 / 9.0), but add a reduction up in one chain where
+//    these have four partial sums, and one chain carries twice the rounding error: sums of 2048 products of unit variance
+//    that cancel, 3.7e-6 rms on 64-wide tiles, 8.1e-6 on others.  Short ones, a slab or two to a wavefront: X X^T of
+//    128 x (128 x 128) 6.6 / 4.7, of 40 x (256 x 256) 7.3 / 5.8, of 150 x (128 x 512) 8.4 / 6.8.
 //  * 128-wide tiles, at most one per CU: the CU is one workgroup's alone, and a ring of four slots keeps three slabs
-//    of loads in flight instead of one: X X^T of 12 x (768 x 3072) 34.7 -> 28.4, 4 x (1024 x 2816) 31.7 -> 23.4; a full
-//    product gains only when its reduction is long (B X of one 2048 x 2048 26.1 -> 19.3, of 1024 x 4096 12.9 -> 13.2).
-//  * else 128-wide tiles on a two-slot ring, two workgroups per CU (288 tiles of 8 x (1024 x 4096): 50 against 62).
+//    of loads in flight instead of one.  Four / two slots: X X^T of 12 x (768 x 3072) 25.6 / 32.1, of 4 x (1024 x 2816) 19.8 / 28.1, of
+//    12 x (768 x 768) 10.9 / 10.9; a full product gains only when its reduction is long (B X of one 2048 x 2048 17.9 / 24.7, of
+//    one 1536 x 2048 13.4 / 17.7, of one 1024 x 4096 11.5 / 11.4).
+//  * else 128-wide tiles on a two-slot ring, two workgroups per CU (288 tiles of 8 x (1024 x 4096): 42.0, on four slots 50.1).
 static TileKind tile_by_count(const GemmParams& p, UpdateKind update) {
   auto tiles = [&](int edge) -> int64_t {
     const int64_t T = p.M / edge;
