@@ -1727,16 +1727,21 @@ static hipError_t launch_k64(const GemmParams& p, hipStream_t stream) {
 
 int gemm_pad_granule(int m, int n, int batch) {
   // To 256 once whole 256-wide tiles make more than one round of the CUs for the symmetric products, so that every product may
-  // use them.  Where the symmetric ones stay on 128-wide tiles all the same (the lines below), padding a multiple of 128
-  // costs more than 256-wide tiles of B X give back.  NS5, us a call padded to 256 / 128: 48 x (640 x 2560) 1474 / 1283,
-  // 18 x (1152 x 1152) 798 / 684, 16 x (1408 x 1408) 1313 / 1062, 100 x (384 x 1536) 1010 / 737, 30 x (896 x 3584) 2244 / 1839; where both
-  // pad to the same width 47 x (650 x 2550) 1502 / 1511, 18 x (1200 x 1200) 816 / 815; 5 x (2944 x 2944), 256-wide throughout,
-  // 2569 / 2667.  The granule is also the layout dion_ns_padded_extents and dion_ns_accepts_prepared report, and what is
-  // not padded has its norm added up in another order, so another granule is not the same bits.
+  // use them -- unless the padding to 128 leaves 18 % of the operations out: 256-wide tiles take up to 13 % less time for the same
+  // operations, no more.  NS5, us a call padded to 256 / 128, and the operations to 256 over those to 128: 64 x (640 x 640) 862 / 553
+  // (1.73), 100 x (384 x 1536) 1017 / 742 (1.82), 48 x (640 x 2560) 1483 / 1290 (1.46), 18 x (1152 x 1152) 804 / 690 (1.37), 30 x
+  // (896 x 3584) 2257 / 1836 (1.32), 16 x (1408 x 1408) 1323 / 1072 and 40 x 3000 / 2841 (1.30), 50 x (1152 x 4608) 6165 / 6070
+  // (1.245); but 12 x (1920 x 1920) 1880 / 1936 (1.21), 40 x (1408 x 5632) 7970 / 8150 (1.20), 20 x (1664 x 6656) 6396 / 6702
+  // (1.17), 24 x (1920 x 7680) 11020 / 11777 (1.14), 3 x (4224 x 4224) 4150 / 4618 (1.09).  Between 1.1 and 1.2 rounds of the CUs
+  // decide some square ones the other way: 10 x (2176 x 2176) 2371 / 2195 (1.19), 8 x (2432 x 2432) 2569 / 2328 (1.17).
   const int64_t m256 = (m + 255) / 256;
   const int64_t syrk_tiles = m256 * (m256 + 1) / 2 * batch;
-  (void)n;
-  return syrk_tiles >= 256 ? 256 : 128;
+  if (syrk_tiles < 256) return 128;
+  auto padded_ops = [&](int64_t g) {
+    const int64_t mp = (m + g - 1) / g, np = (n + g - 1) / g;  // (in tiles: no overflow)
+    return (double)(g * mp) * (double)(g * mp) * (double)(g * (3 * np + mp));
+  };
+  return padded_ops(256) >= 1.22 * padded_ops(128) ? 128 : 256;
 }
 
 // Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box, a launch
