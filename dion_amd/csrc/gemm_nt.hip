@@ -342,7 +342,16 @@ __device__ __forceinline__ void bx_store(__amdgpu_buffer_rsrc_t rs, int lane_byt
     __builtin_amdgcn_raw_buffer_store_b16((unsigned short)f32_to_bf16(v), rs, lane_bytes, uni_bytes, 0);
   else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, lane_bytes, uni_bytes, 0);
 }
-// 16 bytes per lane: eight bf16 or four fp32 elements
+// 16 bytes per lane.  A store of more than 8 bytes reads its data after it has issued: a VALU instruction that writes one of
+// those registers within the next two wait states can get ahead of it, and the lanes read last store the new value.  The
+// compiler keeps that distance where the store has no scalar offset and relies on the hardware where it has one; here it does not
+// hold (32 wrong elements in 40 % of the tiles of a B X that had `v_mul v98` right behind a store of v[98:101]).  The
+// statement behind the store keeps the data's registers until the distance is there.
+__device__ __forceinline__ void bx_store_b128(__amdgpu_buffer_rsrc_t rs, int lane_bytes, int uni_bytes, bx_u32x4 o) {
+  __builtin_amdgcn_raw_buffer_store_b128(o, rs, lane_bytes, uni_bytes, 0);
+  asm volatile("s_nop 1" ::"v"(o));
+}
+// eight bf16 or four fp32 elements
 template <typename T>
 __device__ __forceinline__ void bx_load16(__amdgpu_buffer_rsrc_t rs, int lane_bytes, int uni_bytes, float* v) {
   const bx_u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_bytes, uni_bytes, 0);
@@ -368,7 +377,7 @@ __device__ __forceinline__ void bx_store16(__amdgpu_buffer_rsrc_t rs, int lane_b
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = __float_as_uint(v[e]);
   }
-  __builtin_amdgcn_raw_buffer_store_b128(o, rs, lane_bytes, uni_bytes, 0);
+  bx_store_b128(rs, lane_bytes, uni_bytes, o);
 }
 
 // POST: 0 stores the product; 1 / 2 feed it to the fused Muon update of fp32 / bf16 parameters
@@ -1240,7 +1249,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_qk_walk_kernel(const GemmParams 
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
         const bx_u32x4 o = {v[it].x, v[it].y, v[it].z, v[it].w};
-        __builtin_amdgcn_raw_buffer_store_b128(o, rs, lane_bytes, ((line0 + 8 * it) * ld_out + run0) * 2, 0);
+        bx_store_b128(rs, lane_bytes, ((line0 + 8 * it) * ld_out + run0) * 2, o);
       }
     }
   };
