@@ -47,6 +47,12 @@ def _as_matrices(tensors: List[Tensor], mats: int, rows: int, cols: int) -> List
     return [t.view(mats, rows, cols) for t in tensors]
 
 
+def _row_blocks(tensors: List[Tensor], blocks) -> List[Tensor]:
+    """The row blocks ``(rows of each, first rows)`` of every 2D tensor."""
+    rows, first = blocks
+    return [t[at:at + rows] for at in first for t in tensors]
+
+
 def _require_state_dtype(params: List[Tensor], who: str) -> None:
     """Parameters (and with them momentum / second moments, dion/megabatch_base.py:198-203) are kept in
     float32 or bfloat16; the kernels compute in fp32 and round a bf16 value once, on store."""
@@ -64,11 +70,26 @@ class _MomentumOrtho(OrthoOptimizer):
     # Muon only: run orthogonalization and update as one library call (False: the two-call sequence)
     fused_update = True
 
-    def _shape_group_phases(self, group: dict, params: List[Tensor]):
+    def _shape_groups(self, group: dict, params: List[Tensor]):
+        """``split_sizes``: row blocks are matrices of their own (dion/megabatch_base.py:911-949), each with the lr ratio
+        of its own shape (:952-981), and a block of a contiguous parameter is contiguous: equal blocks are a shape
+        group like any other.  (A caller's orthogonalization gets them stacked, as the reference stacks them.)"""
+        split_sizes = self._resolve_split_sizes(group)
+        if split_sizes is None or self._custom_ns:
+            return [(group, params, None)]
+        self._validate_split_shape(split_sizes, params[0].shape)
+        first = {}
+        row = 0
+        for rows in split_sizes:
+            first.setdefault(rows, []).append(row)
+            row += rows
+        return [(group, params, (rows, at)) for rows, at in first.items()]
+
+    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks):
         """Generator: [momentum / cast] yield [orthogonalization GEMMs] yield [normalise / update]."""
         num_heads = self._resolve_num_heads(group)
-        split_sizes = self._resolve_split_sizes(group)
-        shape = params[0].shape
+        split_sizes = self._resolve_split_sizes(group) if blocks is None else None
+        shape = params[0].shape if blocks is None else (blocks[0], params[0].shape[1])
         flatten = group["flatten"]
         split_scales = None
         if split_sizes is not None:
@@ -79,14 +100,18 @@ class _MomentumOrtho(OrthoOptimizer):
             ratio_shape = (mats, rows, cols)  # the per-head 3D view decides the lr adjustment
         else:
             rows, cols = shape[-2], shape[-1]
-            mats = params[0].numel() // (rows * cols)
+            mats = 1 if blocks is not None else params[0].numel() // (rows * cols)
             ratio_shape = shape
         _require_state_dtype(params, type(self).__name__)
-        n = len(params)
         X = [p.data for p in params]
         G = [p.grad.contiguous() for p in params]
         states = [self._get_or_initialize_state(p, self._algo_name) for p in params]
         M = [s["momentum"] for s in states]
+        V = [s["variance_neuron"] for s in states] if self._normalize else None
+        if blocks is not None:
+            X, G, M = (_row_blocks(t, blocks) for t in (X, G, M))
+            V = V and _row_blocks(V, blocks)
+        n = len(X)
         eps = float(group["epsilon"])
 
         ratio = adjust_lr_ratio(ratio_shape, group["adjust_lr"], flatten)
@@ -117,7 +142,7 @@ class _MomentumOrtho(OrthoOptimizer):
             del U, sumsq
             yield
             _note_stream(O)
-            self._normalize_and_update(group, X, states, O, n, mats, rows, cols, ratio, None)
+            self._normalize_and_update(group, X, V, O, n, mats, rows, cols, ratio, None)
             return
 
         U = ops.muon_pre(G, M, group["mu"], group["nesterov"])  # [n, *shape] bf16
@@ -143,13 +168,12 @@ class _MomentumOrtho(OrthoOptimizer):
         del U
         yield
         _note_stream(O)
-        self._normalize_and_update(group, X, states, O, n, mats, rows, cols, ratio, split_sizes)
+        self._normalize_and_update(group, X, V, O, n, mats, rows, cols, ratio, split_sizes)
 
-    def _normalize_and_update(self, group, X, states, O, n, mats, rows, cols, ratio, split_sizes) -> None:
+    def _normalize_and_update(self, group, X, V, O, n, mats, rows, cols, ratio, split_sizes) -> None:
         """NorMuon's neuron-wise normalisation (when this class normalises) and the update pass."""
         row_scale = None
         if self._normalize:
-            V = [s["variance_neuron"] for s in states]
             O3 = O.view(n, mats, rows, cols)
             if split_sizes is not None:
                 # per-block Frobenius-preserving rescale (dion/normuon.py:359-369)
@@ -262,7 +286,7 @@ class Dion2(OrthoOptimizer):
         self.verbose = verbose
         self._triton_post_ortho = bool(triton_post_ortho)
 
-    def _shape_group_phases(self, group: dict, params: List[Tensor]):
+    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks):
         """Generator: [accumulate / select / gather] yield [orthogonalization] yield [update]."""
         num_heads = self._resolve_num_heads(group)
         if group.get("split_sizes") is not None:
@@ -396,7 +420,7 @@ class NorDion2(OrthoOptimizer):
             state["variance_neuron"] = torch.zeros_like(param[..., 0:1])
         return state
 
-    def _shape_group_phases(self, group: dict, params: List[Tensor]):
+    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks):
         """Generator: [accumulate / select rows / gather] yield [orthogonalization] yield
         [normalise selected rows / update]."""
         num_heads = self._resolve_num_heads(group)
