@@ -230,12 +230,11 @@ __device__ __forceinline__ void tile_of(const GemmParams& p, int pid, int total,
   if (p.xcd_interleave && pid < (total & ~255)) {
     const int j = pid & 255;
     lt = (pid & ~255) + (j & 7) * 32 + (j >> 3);
-  } else if (p.xcd_interleave) {
-    lt = pid;
   } else {
-    const int xcd = pid & 7, loc = pid >> 3;
-    const int q = total >> 3, r = total & 7;
-    lt = xcd * q + (xcd < r ? xcd : r) + loc;
+    const int base = p.xcd_interleave ? total & ~255 : 0;
+    const int xcd = pid & 7, loc = (pid - base) >> 3;
+    const int q = (total - base) >> 3, r = total & 7;
+    lt = base + xcd * q + (xcd < r ? xcd : r) + loc;
   }
   int t;
   if constexpr (TRI) {
@@ -288,9 +287,22 @@ static void set_tile_order(GemmParams& p, int bm, int bn) {
   p.inv_mat = (uint32_t)(0xffffffffu / per_mat);
   p.inv_group = (uint32_t)(0xffffffffu / (8 * tn));
   p.inv_tail = tm % 8 ? (uint32_t)(0xffffffffu / (tm % 8)) : 0;
-  // interleaved 32-tile chunks when the first operand of one matrix is at least 16 MB; below that a contiguous run per
-  // XCD keeps whole matrices in one L2
-  p.xcd_interleave = (int64_t)p.M * p.K * 2 >= (16L << 20) ? 1 : 0;
+  // Interleaved 32-tile chunks for 256-wide tiles of large matrices.  us a launch, one contiguous run per XCD / interleaved:
+  //  * symmetric products from 16 MB of X and reductions of 3584 on: X X^T of 32 x (4096 x 14336) 6364 / 5688, of 4 x 967 / 877, of
+  //    12 x (2560 x 6912) 491 / 444, of 10 x (2304 x 9216) 461 / 415, of 20 x (1536 x 6144) 283 / 262, of 24 x (2048 x 8192)
+  //    699 / 682, of 32 x (1024 x 8192) 328 / 323, A A of 5 x (5120 x 5120) 622 / 574; shorter ones 4 x (6144 x 2048) 252 / 271,
+  //    8 x (3072 x 3072) 198 / 201.  (4 x (3584 x 3584), five iterations, 3310 / 3223 less 31 for the rest below.)
+  //  * full products from 16 MB of B on: B X of 32 x (4096 x 14336) 11310 / 11064, of 5 x (5120 x 5120) 1055 / 976, between 386 /
+  //    386 (8 x (3072 x 3072)) and 467 / 473 (4 x (3072 x 8192)).  (From 8 MB on, the walking kernel's 24 x (2048 x 8192) takes
+  //    1306 / 1279 alone, but a whole step of such groups on two streams no less.)
+  // 128-wide tiles are two to a CU, 64 of them side by side on an XCD: X X^T of 8 x (1024 x 14336) 132 / 164, of 2 x (2048 x 5504)
+  // 62 / 68, of 40 x (1408 x 5632) 482 / 511.
+  // The tiles past the last whole 256 are one contiguous run per XCD in either order: dealt out singly, no two workgroups
+  // of an XCD shared an operand there (X X^T of 6 x (1024 x 8192), 216 tiles, 100 us instead of 50; of 12 x (1536 x 6144) 180
+  // instead of 141; B X of 32 x (4096 x 14336) 11208 instead of 11064).
+  const int64_t p_mb = ((int64_t)p.M * p.K * 2) >> 20;
+  if (bm != 256) p.xcd_interleave = 0;
+  else p.xcd_interleave = p_mb >= 16 && (p.q_kmajor || p.K >= 3584) ? 1 : 0;
 }
 
 // Workgroup barrier preceded by the counter waits the software pipeline needs: every LDS read
