@@ -15,7 +15,7 @@ DION_BF16 = 0
 DION_F32 = 1
 DION_NS_GRAM = 1
 DION_NS_STATIC_SCRATCH_BYTES = 64 << 20
-ABI_VERSION = 12  # dion_abi_version() of the library these signatures describe
+ABI_VERSION = 13  # dion_abi_version() of the library these signatures describe
 
 _u64p = ctypes.POINTER(ctypes.c_uint64)
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -86,6 +86,8 @@ SIGNATURES = {
                                               c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p]),
     "dion_dion2_gather_prepared": (c_int, [_u64p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float,
                                            c_void_p, c_void_p, c_void_p]),
+    "dion_dion2_gather_padded": (c_int, [_u64p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float, c_void_p,
+                                         c_void_p, c_int, c_int, c_void_p]),
     "dion_dion2_post": (c_int, [_u64p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_float, c_void_p]),
     "dion_dion2_index_map": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p]),

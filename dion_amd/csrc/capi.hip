@@ -37,7 +37,7 @@ static inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 static inline bool aligned16(uint64_t p) { return (p & 15) == 0; }
 
 extern "C" const char* dion_last_error(void) { return g_err; }
-extern "C" int dion_abi_version(void) { return 12; }
+extern "C" int dion_abi_version(void) { return 13; }
 
 // ---------------------------------------------------------------------------------------------
 // Kernel-level GEMMs
@@ -1577,6 +1577,35 @@ extern "C" int dion_dion2_gather_prepared(const uint64_t* M_ptrs, int m_dtype, i
                                          (bf16_t*)U_sel + mat0 * sel_numel, sumsq + mat0 * blocks, vec4,
                                          (hipStream_t)stream),
             "dion_dion2_gather_prepared");
+  }
+  return DION_OK;
+}
+
+extern "C" int dion_dion2_gather_padded(const uint64_t* M_ptrs, int m_dtype, int n, int mats_per_ptr, int rows, int cols,
+                                        const int32_t* idx, int k, float ef_decay, void* U, float* sumsq, int mp, int np,
+                                        void* stream) {
+  const char* who = "dion_dion2_gather_padded";
+  if (int rc = check_state_dtype(who, "m_dtype", m_dtype)) return rc;
+  if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0 || k < 0 || k > rows) return fail(DION_E_INVALID, "%s: bad size", who);
+  if (n == 0 || rows == 0 || cols == 0 || k == 0) return DION_OK;
+  if (!M_ptrs || !idx || !U || !sumsq) return fail(DION_E_INVALID, "%s: null argument", who);
+  const int lo = k < cols ? k : cols, hi = k < cols ? cols : k;
+  if (mp % 64 || np % 64 || mp < lo || np < hi || mp / 64 > 65535)
+    return fail(DION_E_INVALID, "%s: %d x %d blocks padded to %d x %d", who, k, cols, mp, np);
+  if (!aligned16((uint64_t)(uintptr_t)U)) return fail(DION_E_INVALID, "%s: U is not 16-byte aligned", who);
+  const int chunk = ptr_chunk(mats_per_ptr);
+  if (chunk == 0) return fail(DION_E_INVALID, "%s: more than 65535 matrices behind one pointer", who);
+  const bool aligned = table_aligned(M_ptrs, n);
+  const int64_t blocks = (int64_t)(mp / 64) * (np / 64);
+  for (int i0 = 0; i0 < n; i0 += chunk) {
+    const int c = (n - i0) < chunk ? (n - i0) : chunk;
+    PtrTab m;
+    fill_tab(m, M_ptrs + i0, c);
+    const int64_t mat0 = (int64_t)i0 * mats_per_ptr;
+    HIP_TRY(launch_dion2_gather_padded(m, dt(m_dtype), c * mats_per_ptr, mats_per_ptr, rows, cols, idx + mat0 * k, k,
+                                       ef_decay, (bf16_t*)U + mat0 * mp * np, mp, np, sumsq + mat0 * blocks, aligned,
+                                       (hipStream_t)stream),
+            who);
   }
   return DION_OK;
 }

@@ -86,6 +86,11 @@ hipError_t launch_dion2_gather(const PtrTab& M, int m_dtype, int n_mat, int mats
 hipError_t launch_dion2_gather_prepared(const PtrTab& M, int m_dtype, int n_mat, int mats_per_ptr, int rows,
                                         int cols, int select_rows, const int32_t* idx, int k, float ef_decay,
                                         bf16_t* U, float* sumsq, bool vec4, hipStream_t st);
+// Selected rows that do not fill whole tiles: X [n_mat][mp][np] zero outside the block, short side along rows, a
+// partial sum per 64 x 64 tile.
+hipError_t launch_dion2_gather_padded(const PtrTab& M, int m_dtype, int n_mat, int mats_per_ptr, int rows, int cols,
+                                      const int32_t* idx, int k, float ef_decay, bf16_t* X, int mp, int np, float* sumsq,
+                                      bool aligned, hipStream_t st);
 hipError_t launch_dion2_post(const PtrTab& X, int x_dtype, int n_mat, int mats_per_ptr, int rows, int cols,
                              int select_rows, const void* U, int u_dtype, int k, const int32_t* map,
                              const float* row_scale, const float* lr_dev, const float* adj_lr_dev,

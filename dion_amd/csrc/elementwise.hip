@@ -413,7 +413,8 @@ __global__ __launch_bounds__(256) void muon_pre_transposed_kernel(PtrTab G, PtrT
 // and its transpose give the same bits.
 // Bound: HBM.  12 x (2730 x 1000) fp32, momentum update included: 95 us beside another stream's GEMMs, where the update
 // (76), the norm's pass over its result (14) and the scaled copy (30) took 120; 4 x (2730 x 1000) fp32 copied: 15.0 us
-// where copy and norm took 23.4.
+// where copy and norm took 23.4.  Selected rows gathered here instead of copied a second time: NorDion2 on 12 layers of 1600,
+// a step, 4100 -> 3960 us (bf16 state 3571 -> 3400).
 // ------------------------------------------------------------------------------------------
 template <typename T, int V>
 static __device__ __forceinline__ void load_group(const T* p, int64_t i, float* v) {
@@ -444,9 +445,11 @@ struct PadCopyOp {
   __device__ __forceinline__ At at(int mat, int mats, int64_t mat_elems) const { return {in + (int64_t)mat * mat_elems}; }
   struct Raw { float v[8]; };
   template <int V>
-  static __device__ __forceinline__ void load(const At& a, int64_t i, Raw& r) { load_group<T, V>(a.p, i, r.v); }
+  static __device__ __forceinline__ void load(const At& a, int row, int c, int C, Raw& r) {
+    load_group<T, V>(a.p, (int64_t)row * C + c, r.v);
+  }
   template <int V>
-  __device__ __forceinline__ void finish(const At&, int64_t, Raw& r, float* u) const {
+  __device__ __forceinline__ void finish(const At&, int, int, int, Raw& r, float* u) const {
 #pragma unroll
     for (int e = 0; e < V; ++e) u[e] = r.v[e];
   }
@@ -465,18 +468,47 @@ struct PadPreOp {
   }
   struct Raw { float g[8], m[8]; };
   template <int V>
-  static __device__ __forceinline__ void load(const At& a, int64_t i, Raw& r) {
-    load_group<GT, V>(a.g, i, r.g);
-    load_group<MT, V>(a.m, i, r.m);
+  static __device__ __forceinline__ void load(const At& a, int row, int c, int C, Raw& r) {
+    load_group<GT, V>(a.g, (int64_t)row * C + c, r.g);
+    load_group<MT, V>(a.m, (int64_t)row * C + c, r.m);
   }
   template <int V>
-  __device__ __forceinline__ void finish(const At& a, int64_t i, Raw& r, float* u) const {
+  __device__ __forceinline__ void finish(const At& a, int row, int c, int C, Raw& r, float* u) const {
 #pragma unroll
     for (int e = 0; e < V; ++e) {
       r.m[e] = __fadd_rn(__fmul_rn(r.m[e], mu), r.g[e]);
       u[e] = nesterov ? __fadd_rn(__fmul_rn(r.m[e], mu), r.g[e]) : r.m[e];
     }
-    store_group<MT, V>(a.m, i, r.m);
+    store_group<MT, V>(a.m, (int64_t)row * C + c, r.m);
+  }
+};
+// the selected rows of dion2_gather_kernel, which decay where they lie.  (Columns are not taken: a tile's ends fall inside lines
+// that two workgroups then write, and a step of 12 layers of 1600 took 3250 us instead of 3220.)
+template <typename MT>
+struct PadGatherRowsOp {
+  PtrTab M;
+  const int32_t* idx;
+  int rows, cols, k;
+  float ef_decay;
+  struct At { MT* m; const int32_t* id; };
+  __device__ __forceinline__ At at(int mat, int mats, int64_t) const {
+    const int p = mat / mats;
+    return {(MT*)M.p[p] + (int64_t)(mat - p * mats) * rows * cols, idx + (int64_t)mat * k};
+  }
+  struct Raw { float v[8]; int64_t at; };
+  template <int V>
+  static __device__ __forceinline__ void load(const At& a, int row, int c, int C, Raw& r) {
+    r.at = (int64_t)a.id[row] * C + c;
+    load_group<MT, V>(a.m, r.at, r.v);
+  }
+  template <int V>
+  __device__ __forceinline__ void finish(const At& a, int, int, int, Raw& r, float* u) const {
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      u[e] = r.v[e];
+      r.v[e] = __fmul_rn(r.v[e], ef_decay);
+    }
+    store_group<MT, V>(a.m, r.at, r.v);
   }
 };
 
@@ -496,7 +528,7 @@ __global__ __launch_bounds__(256) void pad_tile_kernel(const Op op, int mats, in
 #pragma unroll
   for (int ps = 0; ps < NP; ++ps) {
     const int r = r0 + rr + ps * RPP;
-    if (r < R && c < C) op.template load<V>(at, (int64_t)r * C + c, raw[ps]);
+    if (r < R && c < C) op.template load<V>(at, r, c, C, raw[ps]);
   }
 #pragma unroll
   for (int ps = 0; ps < NP; ++ps) {
@@ -504,7 +536,7 @@ __global__ __launch_bounds__(256) void pad_tile_kernel(const Op op, int mats, in
     float u[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) u[e] = 0.f;
-    if (r < R && c < C) op.template finish<V>(at, (int64_t)r * C + c, raw[ps], u);
+    if (r < R && c < C) op.template finish<V>(at, r, c, C, raw[ps], u);
     store_group<bf16_t, V>(&tile[i][0], grp * V, u);
   }
   __syncthreads();
@@ -575,6 +607,16 @@ hipError_t launch_muon_pre_padded(const PtrTab& G, int g_dtype, const PtrTab& M,
                         : muon_pre_padded<bf16_t, float>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st);
   return m_dtype == 0 ? muon_pre_padded<float, bf16_t>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st)
                       : muon_pre_padded<float, float>(G, M, X, sumsq, n, mats, rows, cols, mp, np, mu, nesterov, aligned, st);
+}
+
+hipError_t launch_dion2_gather_padded(const PtrTab& M, int m_dtype, int n_mat, int mats_per_ptr, int rows, int cols,
+                                      const int32_t* idx, int k, float ef_decay, bf16_t* X, int mp, int np, float* sumsq,
+                                      bool aligned, hipStream_t st) {
+  if (m_dtype == 0)
+    return launch_pad_tile(PadGatherRowsOp<bf16_t>{M, idx, rows, cols, k, ef_decay}, n_mat, mats_per_ptr, k, cols, aligned, X,
+                           mp, np, sumsq, st);
+  return launch_pad_tile(PadGatherRowsOp<float>{M, idx, rows, cols, k, ef_decay}, n_mat, mats_per_ptr, k, cols, aligned, X, mp,
+                         np, sumsq, st);
 }
 
 // Workgroups for the tile-per-workgroup kernels: one per 512 chunks, at most 2^20.

@@ -554,7 +554,8 @@ def _late_add_pays(m_dtype: int, elements: int) -> bool:
     return m_dtype == DION_F32 and elements >= 1 << 23
 
 
-def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_decay: float, prepared: bool = False):
+def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_decay: float, prepared: bool = False,
+                 extents: Optional[Tuple[int, int]] = None):
     """``M += G``; pick the ``k`` slices of largest L1 norm along ``select_dim`` of every matrix; return
     (U_sel bf16 arena, idx int32 [n_mat, k] ascending, map int32 [n_mat, dim]) and decay the selected
     slices of ``M`` by ``ef_decay``.  Mirrors ``dion2_pre_orthogonalize`` (dion/dion2.py:439-547).
@@ -562,9 +563,12 @@ def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_d
     ``prepared=True`` (only where ``dion2_prepared_blocks`` is not 0): the selected blocks are written as a
     prepared orthogonalization input -- ``U_sel [n_mat, min, max]`` with the short side of the block along rows
     (a tall block transposed) -- and a fourth result ``sumsq [n_mat, blocks]`` holds partial sums of their
-    squares."""
+    squares.  ``extents`` (``ns_padded_extents`` of the blocks of selected rows): they are written in that padded form
+    instead, also with ``sumsq``."""
     if select_dim not in (-2, -1):
         raise ValueError(f"select_dim must be -2 or -1, got {select_dim}")
+    if extents is not None and select_dim != -2:
+        raise ValueError("selected columns are not gathered into the padded form")
     n = len(G)
     assert n == len(M) and n > 0
     shape = M[0].shape
@@ -580,7 +584,7 @@ def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_d
     idx = torch.empty(n_mat, k, dtype=torch.int32, device=dev)
     imap = torch.empty(n_mat, dim, dtype=torch.int32, device=dev)
     sel_shape = (n, *shape[:-2], k, cols) if select_dim == -2 else (n, *shape[:-2], rows, k)
-    U = torch.empty(sel_shape, dtype=torch.bfloat16, device=dev)
+    U = torch.empty(sel_shape if extents is None else (n_mat, *extents), dtype=torch.bfloat16, device=dev)
     lib = _lib.load()
     st = _stream_handle(dev)
     sbytes = lib.dion_dion2_accumulate_scratch_bytes(n_mat, rows, cols, select_dim)
@@ -599,6 +603,12 @@ def dion2_select(G: List[Tensor], M: List[Tensor], k: int, select_dim: int, ef_d
               "dion2_accumulate")
     check(lib.dion_dion2_topk(norms.data_ptr(), n_mat, dim, k, idx.data_ptr(), imap.data_ptr(), st),
           "dion2_topk")
+    if extents is not None:
+        sumsq = torch.empty(n_mat, (extents[0] // 64) * (extents[1] // 64), dtype=torch.float32, device=dev)
+        check(lib.dion_dion2_gather_padded(mp, mcode, n, mats_per_ptr, rows, cols, idx.data_ptr(), k,
+                                           float(ef_decay), U.data_ptr(), sumsq.data_ptr(), *extents, st),
+              "dion2_gather_padded")
+        return U, idx, imap, sumsq
     if prepared:
         blocks = dion2_prepared_blocks(rows, cols, select_dim, k)
         if blocks == 0:

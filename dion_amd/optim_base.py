@@ -375,17 +375,19 @@ class OrthoOptimizer(Optimizer):
     # parameters' layout, normalised and transposed by passes of the orthogonalization call)
     prepared_input = True
 
-    def _takes_prepared(self, n_mat: int, rows: int, cols: int, select_dim: int, k: int, flat3d: bool,
-                        M: List[Tensor]) -> bool:
+    def _selection_form(self, n_mat: int, rows: int, cols: int, select_dim: int, k: int, flat3d: bool,
+                        M: List[Tensor]) -> Tuple[bool, Optional[Tuple[int, int]]]:
         """Dion2 / NorDion2: whether the ``k`` slices selected along ``select_dim`` of ``n_mat`` matrices of
-        ``rows x cols`` go to a built-in orthogonalization as the gather kernel writes them."""
+        ``rows x cols`` go to a built-in orthogonalization as the gather kernel writes them, and the extents of the
+        padded form it writes where rows are selected and do not fill whole tiles."""
         if not self.prepared_input or flat3d or self._custom_ns:
-            return False
-        if ops.dion2_prepared_blocks(rows, cols, select_dim, k) == 0:
-            return False
+            return False, None
         sr, sc = (k, cols) if select_dim == -2 else (rows, k)
-        return ns.accepts_prepared(self._newton_schulz_func, n_mat, sr, sc) and \
-            all(m.data_ptr() % 16 == 0 for m in M)
+        if ops.dion2_prepared_blocks(rows, cols, select_dim, k) and \
+                ns.accepts_prepared(self._newton_schulz_func, n_mat, sr, sc) and all(m.data_ptr() % 16 == 0 for m in M):
+            return True, None
+        extents = ns.padded_extents(self._newton_schulz_func, n_mat, sr, sc) if select_dim == -2 else None
+        return extents is not None, extents
 
     def _orthogonalize_update(self, U: Tensor, epsilon: float, X: List[Tensor], lr: Tensor, adj_ratio: float,
                               weight_decay, cautious_wd: bool) -> bool:

@@ -341,14 +341,17 @@ class Dion2(OrthoOptimizer):
 
         eps = float(group["epsilon"])
         sel_rows, sel_cols = (k, cols) if select_dim == -2 else (rows, k)
-        if self._takes_prepared(n * mats, rows, cols, select_dim, k, flatten and len(shape) >= 3, M):
+        handed_over, extents = self._selection_form(n * mats, rows, cols, select_dim, k, flatten and len(shape) >= 3, M)
+        if handed_over:
             # the gather writes the selected blocks the way the iteration carries them, with the partial sums
             # of their Frobenius norms (no norm / scale / transpose pass inside the orthogonalization call)
-            U_sel, _idx, imap, sumsq = ops.dion2_select(G, M, k, select_dim, group["ef_decay"], prepared=True)
+            U_sel, _idx, imap, sumsq = ops.dion2_select(G, M, k, select_dim, group["ef_decay"], prepared=extents is None,
+                                                        extents=extents)
             yield
             _note_stream(U_sel)
             _note_stream(sumsq)
-            O = ns.orthogonalize_prepared(self._newton_schulz_func, U_sel, sumsq, sel_rows, sel_cols, eps)
+            O = ns.orthogonalize_prepared(self._newton_schulz_func, U_sel, sumsq, sel_rows, sel_cols, eps,
+                                          padded=extents is not None)
             del U_sel, sumsq
             yield
             _note_stream(O)
@@ -469,12 +472,15 @@ class NorDion2(OrthoOptimizer):
         # error-feedback decay of the selected rows is the momentum factor (dion/nordion2.py:352-359)
         eps = float(group["epsilon"])
         flat3d = flatten and len(shape) >= 3
-        if self._takes_prepared(n * mats, rows, cols, select_dim, k, flat3d, M):
-            U_sel, idx, imap, sumsq = ops.dion2_select(G, M, k, select_dim, group["mu"], prepared=True)
+        handed_over, extents = self._selection_form(n * mats, rows, cols, select_dim, k, flat3d, M)
+        if handed_over:
+            U_sel, idx, imap, sumsq = ops.dion2_select(G, M, k, select_dim, group["mu"], prepared=extents is None,
+                                                       extents=extents)
             yield
             _note_stream(U_sel)
             _note_stream(sumsq)
-            O = ns.orthogonalize_prepared(self._newton_schulz_func, U_sel, sumsq, k, cols, eps)
+            O = ns.orthogonalize_prepared(self._newton_schulz_func, U_sel, sumsq, k, cols, eps,
+                                          padded=extents is not None)
             del sumsq
         else:
             U_sel, idx, imap = ops.dion2_select(G, M, k, select_dim, group["mu"])

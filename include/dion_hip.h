@@ -338,6 +338,12 @@ int dion_dion2_gather_sumsq_blocks(int rows, int cols, int select_dim, int k);
 int dion_dion2_gather_prepared(const uint64_t* M_ptrs, int m_dtype, int n, int mats_per_ptr, int rows, int cols,
                                int select_dim, const int32_t* idx, int k, float ef_decay, void* U_sel,
                                float* sumsq, void* stream);
+/* The same for selected rows that do not fill whole tiles, in the form dion_ns_orthogonalize_padded takes: U bf16
+ * [n * mats_per_ptr][mp][np] (dion_ns_padded_extents of the block), zero outside the block, short side along rows, and
+ * sumsq [n * mats_per_ptr][(mp / 64) * (np / 64)]. */
+int dion_dion2_gather_padded(const uint64_t* M_ptrs, int m_dtype, int n, int mats_per_ptr, int rows, int cols,
+                             const int32_t* idx, int k, float ef_decay, void* U, float* sumsq, int mp, int np,
+                             void* stream);
 
 /* The tall form (select_dim -1, rows > k) with M += G in the gather: dion_dion2_column_norms gives the norms of
  * dion_dion2_accumulate, bit for bit, without writing M, and dion_dion2_add_gather_columns then adds G, writes U_sel
