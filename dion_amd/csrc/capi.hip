@@ -200,7 +200,8 @@ NsPlan make_plan(int batch, int rows, int cols, int flags) {
   pl.gram = (flags & DION_NS_GRAM) && gram_pays(pl.m, pl.n);
   const int g = gemm_pad_granule(pl.m, pl.n, batch);
   pl.mp = round_up(pl.m, g);
-  pl.np = round_up(pl.n, g);
+  // (matrices of whole tiles stay as they are: they are read where they lie)
+  pl.np = pl.mp == pl.m && pl.n % g == 0 ? pl.n : gemm_pad_long(pl.mp, pl.n, batch, g);
   const int64_t numel = (int64_t)rows * cols;
   int64_t nb = numel / (256 * 32);
   if (nb < 1) nb = 1;

@@ -268,5 +268,7 @@ hipError_t launch_gemm_nt_post(const GemmParams& p, const FusedPost& post, int x
 // Tile edge (128 or 256) launch_gemm_nt would use for a problem whose padded short/long
 // dims are given; workspaces are padded to this.
 int gemm_pad_granule(int m, int n, int batch);
+// ... and the padded long side n of matrices whose short side is padded to mp.
+int gemm_pad_long(int mp, int n, int batch, int granule);
 
 }  // namespace dion

@@ -1765,6 +1765,19 @@ int gemm_pad_granule(int m, int n, int batch) {
   return padded_ops(256) >= 1.22 * padded_ops(128) ? 128 : 256;
 }
 
+int gemm_pad_long(int mp, int n, int batch, int granule) {
+  // The long side of a matrix that is padded to 128: to 256 where B X then offers more than a round and a half of the CUs
+  // (384 tiles) on 256-wide tiles.  128-wide ones take twice the operand bytes there: B X of 24 x (512 x 8064) 167 us where
+  // 24 x (512 x 8192) takes 118.  NS5, us a call padded to 128 / 256: 24 x (512 x 8056) 1245 / 1064, 6 x (1280 x 3448) 725 / 658, 30 x
+  // (512 x 1656) 415 / 380, 12 x (1024 x 3448) 857 / 799, 24 x (512 x 2168) 374 / 352, 12 x (768 x 2936) 468 / 446, 9 x (1024 x
+  // 2680) 559 / 545, 48 x (512 x 2168) 706 / 700, 6 x (1536 x 4216) 1032 / 1029; at 384 tiles 24 x (500 x 1920) 325 / 328, 16 x
+  // (768 x 1912) 458 / 450, fewer 24 x (512 x 1400) 286 / 291, and where B has one row of tiles 60 x (256 x 2168) 331 / 344.  A Muon
+  // step of 10 layers of 1530 x 4100 7051 / 6510, NorMuon, 8 of 1280 x 3400, 3448 / 3292, 24 of 512 x 2168 1327 / 1313.
+  const int np = (n + granule - 1) / granule * granule;
+  const bool fits = mp % 256 == 0 && mp >= 512 && np % 256 == 128;
+  return fits && (int64_t)(mp / 256) * ((np + 128) / 256) * batch > 384 ? np + 128 : np;
+}
+
 // Which kernel a product runs on, by the number of tiles it offers the 256 CUs.  Figures: us per launch on one box, a launch
 // repeated on the same operands unless it says otherwise.  In a call, behind the launch that wrote an operand, a launch
 // of few tiles takes up to 3 us more (X X^T of one 768 x 3072 13.0, B X 10.1).
