@@ -226,12 +226,12 @@ __device__ __forceinline__ int div_known(int x, int d, uint32_t inv, int& rem) {
 template <int BM, int BN, bool TRI>
 __device__ __forceinline__ void tile_of(const GemmParams& p, int pid, int total, int& b, int& ti, int& tj) {
   const int tilesM = p.M / BM, tilesN = p.N / BN;
-  int lt;
-  if (p.xcd_interleave && pid < (total & ~255)) {
+  int base = 0, lt;
+  if constexpr (BM == 256) base = p.xcd_interleave ? total & ~255 : 0;  // (the only tiles that are interleaved)
+  if (BM == 256 && pid < base) {
     const int j = pid & 255;
     lt = (pid & ~255) + (j & 7) * 32 + (j >> 3);
   } else {
-    const int base = p.xcd_interleave ? total & ~255 : 0;
     const int xcd = pid & 7, loc = (pid - base) >> 3;
     const int q = (total - base) >> 3, r = total & 7;
     lt = base + xcd * q + (xcd < r ? xcd : r) + loc;
