@@ -48,8 +48,11 @@ def _as_matrices(tensors: List[Tensor], mats: int, rows: int, cols: int) -> List
 
 
 def _row_blocks(tensors: List[Tensor], blocks) -> List[Tensor]:
-    """The row blocks ``(rows of each, first rows)`` of every 2D tensor."""
+    """The row blocks ``(rows of each, first rows)`` of every 2D tensor.  (A block of one row is contiguous whatever the
+    tensor is: what the kernels refuse of the whole is refused here, before anything is updated.)"""
     rows, first = blocks
+    if not all(t.is_contiguous() for t in tensors):
+        raise ValueError("split_sizes: tensors must be contiguous")
     return [t[at:at + rows] for at in first for t in tensors]
 
 
