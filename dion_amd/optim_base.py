@@ -18,12 +18,6 @@ from . import newton_schulz as ns
 from . import ops, scalar_opts
 
 
-# Row blocks of equal height, updated as matrices of their own: (rows of a block, first rows of the blocks).
-RowBlocks = Tuple[int, List[int]]
-# What is updated together: param group, its parameters of one shape, None or the row blocks of each.
-ShapeGroup = Tuple[dict, List[Tensor], Optional[RowBlocks]]
-
-
 class LiveScalars:
     """Hyper-parameters the kernels read from device memory instead of taking by value.
 
@@ -263,7 +257,7 @@ class OrthoOptimizer(Optimizer):
             else:
                 raise ValueError(f"Unknown algorithm: {algo}")
 
-        work: List[ShapeGroup] = []
+        work: List[Tuple[dict, List[Tensor]]] = []
         for group in ortho:
             assert all(p.ndim >= 2 for p in group["params"]), (
                 f"{type(self).__name__} optimizer only supports matrix parameters."
@@ -275,7 +269,7 @@ class OrthoOptimizer(Optimizer):
             for p in with_grad:
                 buckets[(p.shape, p.dtype)].append(p)
             for params in buckets.values():
-                work.extend(self._shape_groups(group, params))
+                work.append((group, params))
         self._run_shape_groups(work)
 
         for group in lion:
@@ -284,17 +278,14 @@ class OrthoOptimizer(Optimizer):
             scalar_opts.adamw_step(self, group)
         return loss
 
-    def _shape_groups(self, group: dict, params: List[Tensor]) -> List[ShapeGroup]:
-        """What is updated together of parameters of one shape: whole parameters, or equal row blocks of them."""
-        return [(group, params, None)]
-
-    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks: Optional[RowBlocks]):
+    def _shape_group_phases(self, group: dict, params: List[Tensor]):
         """Generator over the three phases of one shape group's update: memory-bound preparation,
-        ``yield``, orthogonalization (GEMM-bound), ``yield``, memory-bound update."""
+        ``yield``, orthogonalization (GEMM-bound), ``yield``, memory-bound update.  They run on one stream, where missing
+        state of the parameters may therefore be made: a parameter is in one shape group, whatever it is cut into."""
         raise NotImplementedError
 
-    def _update_shape_group(self, work: ShapeGroup) -> None:
-        for _ in self._shape_group_phases(*work):
+    def _update_shape_group(self, group: dict, params: List[Tensor]) -> None:
+        for _ in self._shape_group_phases(group, params):
             pass
 
     # Shape groups are independent.  Groups whose kernels are a few rounds of workgroups or less (GPT-small:
@@ -307,13 +298,10 @@ class OrthoOptimizer(Optimizer):
     _N_SIDE_STREAMS = 2
 
     @staticmethod
-    def _group_flop(work: ShapeGroup) -> float:
-        _group, params, blocks = work
+    def _group_flop(params: List[Tensor]) -> float:
         r, c = params[0].shape[-2], params[0].shape[-1]
-        mats = len(params) * (params[0].numel() // (r * c))
-        if blocks is not None:
-            r, mats = blocks[0], mats * len(blocks[1])
         m, n = min(r, c), max(r, c)
+        mats = len(params) * (params[0].numel() // (r * c))
         return mats * 5.0 * (4.0 * m * m * n + 2.0 * m ** 3)
 
     # One pool per device for the whole process, shared by every optimizer instance: the runtime maps streams
@@ -330,36 +318,36 @@ class OrthoOptimizer(Optimizer):
             OrthoOptimizer._side_pools[key] = pool
         return pool
 
-    def _run_shape_groups(self, work: List[ShapeGroup]) -> None:
+    def _run_shape_groups(self, work: List[Tuple[dict, List[Tensor]]]) -> None:
         if not work:
             return
-        on_gpu = all(params[0].is_cuda for _g, params, _b in work)
+        on_gpu = all(params[0].is_cuda for _g, params in work)
         if not on_gpu:
-            for w in work:
-                self._update_shape_group(w)
+            for group, params in work:
+                self._update_shape_group(group, params)
             return
-        small = [w for w in work if self._group_flop(w) < self._MEDIUM_GROUP_FLOP]
-        big = [w for w in work if self._group_flop(w) >= self._MEDIUM_GROUP_FLOP]
+        small = [w for w in work if self._group_flop(w[1]) < self._MEDIUM_GROUP_FLOP]
+        big = [w for w in work if self._group_flop(w[1]) >= self._MEDIUM_GROUP_FLOP]
         # (Running the memory-bound phases of neighbouring large groups under these GEMMs on a
         # second stream was measured: no gain -- the chip is power-limited, not idle.)
-        for w in big:
-            self._update_shape_group(w)
+        for group, params in big:
+            self._update_shape_group(group, params)
         if len(small) < 2:
-            for w in small:
-                self._update_shape_group(w)
+            for group, params in small:
+                self._update_shape_group(group, params)
             return
         device = small[0][1][0].device
         pool = self._side_pool(device)
         main = torch.cuda.current_stream(device)
         fork = main.record_event()
         used = []
-        for i, w in enumerate(small):
+        for i, (group, params) in enumerate(small):
             side = pool[i % len(pool)]
             if side not in used:
                 side.wait_event(fork)
                 used.append(side)
             with torch.cuda.stream(side):
-                self._update_shape_group(w)
+                self._update_shape_group(group, params)
         for side in used:
             main.wait_stream(side)
 

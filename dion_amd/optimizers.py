@@ -73,37 +73,25 @@ class _MomentumOrtho(OrthoOptimizer):
     # Muon only: run orthogonalization and update as one library call (False: the two-call sequence)
     fused_update = True
 
-    def _shape_groups(self, group: dict, params: List[Tensor]):
-        """``split_sizes``: row blocks are matrices of their own (dion/megabatch_base.py:911-949), each with the lr ratio
-        of its own shape (:952-981), and a block of a contiguous parameter is contiguous: equal blocks are a shape
-        group like any other.  (A caller's orthogonalization gets them stacked, as the reference stacks them.)"""
-        split_sizes = self._resolve_split_sizes(group)
-        if split_sizes is None or self._custom_ns:
-            return [(group, params, None)]
-        self._validate_split_shape(split_sizes, params[0].shape)
-        first = {}
-        row = 0
-        for rows in split_sizes:
-            first.setdefault(rows, []).append(row)
-            row += rows
-        return [(group, params, (rows, at)) for rows, at in first.items()]
+    def _shape_group_phases(self, group: dict, params: List[Tensor]):
+        """Generator: [momentum / cast] yield [orthogonalization GEMMs] yield [normalise / update], once, or for the row
+        blocks of each height one after another.
 
-    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks):
-        """Generator: [momentum / cast] yield [orthogonalization GEMMs] yield [normalise / update]."""
+        ``split_sizes``: row blocks are matrices of their own (dion/megabatch_base.py:911-949), each with the lr ratio of
+        its own shape (:952-981), and a block of a contiguous parameter is contiguous: they are updated where they lie.
+        (A caller's orthogonalization gets them stacked, as the reference stacks them.)  Blocks of several heights stay on
+        one stream: they share gradients, and state that may have to be made first."""
         num_heads = self._resolve_num_heads(group)
-        split_sizes = self._resolve_split_sizes(group) if blocks is None else None
-        shape = params[0].shape if blocks is None else (blocks[0], params[0].shape[1])
-        flatten = group["flatten"]
-        split_scales = None
+        split_sizes = self._resolve_split_sizes(group)
+        shape = params[0].shape
         if split_sizes is not None:
             self._validate_split_shape(split_sizes, shape)
-            split_scales = split_lr_scales(split_sizes, shape, group["adjust_lr"])
         if num_heads is not None:
             mats, rows, cols = self._head_geometry(num_heads, shape)
             ratio_shape = (mats, rows, cols)  # the per-head 3D view decides the lr adjustment
         else:
             rows, cols = shape[-2], shape[-1]
-            mats = 1 if blocks is not None else params[0].numel() // (rows * cols)
+            mats = params[0].numel() // (rows * cols)
             ratio_shape = shape
         _require_state_dtype(params, type(self).__name__)
         X = [p.data for p in params]
@@ -111,9 +99,23 @@ class _MomentumOrtho(OrthoOptimizer):
         states = [self._get_or_initialize_state(p, self._algo_name) for p in params]
         M = [s["momentum"] for s in states]
         V = [s["variance_neuron"] for s in states] if self._normalize else None
-        if blocks is not None:
-            X, G, M = (_row_blocks(t, blocks) for t in (X, G, M))
-            V = V and _row_blocks(V, blocks)
+        if split_sizes is None or self._custom_ns:
+            yield from self._matrix_phases(group, X, G, M, V, shape, mats, rows, cols, ratio_shape, split_sizes)
+            return
+        first, at = {}, 0
+        for rows in split_sizes:
+            first.setdefault(rows, []).append(at)
+            at += rows
+        for rows, at in first.items():
+            Xb, Gb, Mb = (_row_blocks(t, (rows, at)) for t in (X, G, M))
+            Vb = V and _row_blocks(V, (rows, at))
+            yield from self._matrix_phases(group, Xb, Gb, Mb, Vb, (rows, cols), 1, rows, cols, (rows, cols), None)
+
+    def _matrix_phases(self, group: dict, X, G, M, V, shape, mats: int, rows: int, cols: int, ratio_shape, split_sizes):
+        """The phases for tensors of ``shape``, each ``mats`` matrices of ``rows x cols``.  ``split_sizes``: row blocks that
+        are stacked for a caller's orthogonalization."""
+        flatten = group["flatten"]
+        split_scales = None if split_sizes is None else split_lr_scales(split_sizes, shape, group["adjust_lr"])
         n = len(X)
         eps = float(group["epsilon"])
 
@@ -289,7 +291,7 @@ class Dion2(OrthoOptimizer):
         self.verbose = verbose
         self._triton_post_ortho = bool(triton_post_ortho)
 
-    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks):
+    def _shape_group_phases(self, group: dict, params: List[Tensor]):
         """Generator: [accumulate / select / gather] yield [orthogonalization] yield [update]."""
         num_heads = self._resolve_num_heads(group)
         if group.get("split_sizes") is not None:
@@ -426,7 +428,7 @@ class NorDion2(OrthoOptimizer):
             state["variance_neuron"] = torch.zeros_like(param[..., 0:1])
         return state
 
-    def _shape_group_phases(self, group: dict, params: List[Tensor], blocks):
+    def _shape_group_phases(self, group: dict, params: List[Tensor]):
         """Generator: [accumulate / select rows / gather] yield [orthogonalization] yield
         [normalise selected rows / update]."""
         num_heads = self._resolve_num_heads(group)
