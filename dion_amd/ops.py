@@ -356,7 +356,48 @@ def ns_orthogonalize_update_prepared(U: Tensor, sumsq: Tensor, rows: int, cols: 
 # ---------------------------------------------------------------------------------------------
 # optimizer-step kernels on lists of same-shape parameters
 # ---------------------------------------------------------------------------------------------
+class RowBlocks:
+    """Equal row blocks of contiguous 2D tensors of one shape, as the list of tensors that the functions below take: ``rows``
+    rows from row ``first[0]`` of every tensor, then from ``first[1]`` of every tensor, and so on.  Addresses are all that
+    these functions need of a block, and a view of each would cost more host time than the step of a small model takes
+    (32 x (4096 x 1024), 64 rows a block: 7.9 ms a step instead of 1.3)."""
+
+    __slots__ = ("tensors", "rows", "first")
+
+    def __init__(self, tensors: List[Tensor], rows: int, first: List[int]):
+        # (a block of one row is contiguous whatever the tensor is: what the kernels refuse of the whole is refused here)
+        if not all(t.is_contiguous() for t in tensors):
+            raise ValueError("row blocks: tensors must be contiguous")
+        self.tensors, self.rows, self.first = tensors, rows, first
+
+    def __len__(self) -> int:
+        return len(self.tensors) * len(self.first)
+
+    def __getitem__(self, i: int) -> Tensor:
+        which, tensor = divmod(i, len(self.tensors))
+        at = self.first[which]
+        return self.tensors[tensor][at:at + self.rows]
+
+    def offsets(self) -> List[int]:
+        """First byte of each block of a tensor."""
+        row_bytes = self.tensors[0].shape[1] * self.tensors[0].element_size()
+        return [at * row_bytes for at in self.first]
+
+
+def aligned16(ts) -> bool:
+    """Whether every tensor (or row block) of a list starts on a 16-byte boundary."""
+    if type(ts) is RowBlocks:
+        return all(at % 16 == 0 for at in ts.offsets()) and aligned16(ts.tensors)
+    return all(t.data_ptr() % 16 == 0 for t in ts)
+
+
 def _list_ptrs(ts: List[Tensor], name: str, dtype=None, numel=None):
+    if type(ts) is RowBlocks:
+        shape = ts.tensors[0].shape
+        if numel is not None and numel != ts.rows * shape[1]:
+            raise ValueError(f"{name}: all tensors of a shape group must have {numel} elements")
+        whole = _list_ptrs(ts.tensors, name, dtype, shape.numel())
+        return ptr_table([p + at for at in ts.offsets() for p in whole])
     # A step passes a few hundred tensors through here: the checks are spelled out instead of called.
     ptrs = []
     for t in ts:

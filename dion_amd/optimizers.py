@@ -47,13 +47,35 @@ def _as_matrices(tensors: List[Tensor], mats: int, rows: int, cols: int) -> List
     return [t.view(mats, rows, cols) for t in tensors]
 
 
-def _row_blocks(tensors: List[Tensor], blocks) -> List[Tensor]:
-    """The row blocks ``(rows of each, first rows)`` of every 2D tensor.  (A block of one row is contiguous whatever the
-    tensor is: what the kernels refuse of the whole is refused here, before anything is updated.)"""
-    rows, first = blocks
-    if not all(t.is_contiguous() for t in tensors):
-        raise ValueError("split_sizes: tensors must be contiguous")
-    return [t[at:at + rows] for at in first for t in tensors]
+def _row_blocks(tensors: List[Tensor], blocks) -> ops.RowBlocks:
+    """The row blocks ``(rows of each, first rows)`` of every 2D tensor; refused before anything is updated where the
+    tensors are not contiguous."""
+    return ops.RowBlocks(tensors, *blocks)
+
+
+# Matrices of one height that are updated where they lie, in one call each for momentum, orthogonalization and update; more of
+# them are stacked (one call takes 65535 matrices and about 9000 addresses).
+_MOST_ROW_BLOCKS = 32768
+_MOST_ROW_BLOCK_ADDRESSES = 4096
+
+
+def _equal_blocks(split_sizes) -> List[Tuple[int, int, List[int]]]:
+    """``(rows, mats, first rows)`` for each height among the row blocks: ``mats`` neighbours of ``rows`` rows start at each
+    of the first rows.  Neighbours are the matrices of one address, as heads are; ``mats`` is what divides every run of them."""
+    runs = {}  # height -> [first row, blocks] of every run
+    at = 0
+    for rows in split_sizes:
+        of_height = runs.setdefault(rows, [])
+        if of_height and of_height[-1][0] + of_height[-1][1] * rows == at:
+            of_height[-1][1] += 1
+        else:
+            of_height.append([at, 1])
+        at += rows
+    out = []
+    for rows, of_height in runs.items():
+        mats = math.gcd(*(count for _at, count in of_height))
+        out.append((rows, mats, [at + i * rows for at, count in of_height for i in range(0, count, mats)]))
+    return out
 
 
 def _require_state_dtype(params: List[Tensor], who: str) -> None:
@@ -79,8 +101,9 @@ class _MomentumOrtho(OrthoOptimizer):
 
         ``split_sizes``: row blocks are matrices of their own (dion/megabatch_base.py:911-949), each with the lr ratio of
         its own shape (:952-981), and a block of a contiguous parameter is contiguous: they are updated where they lie.
-        (A caller's orthogonalization gets them stacked, as the reference stacks them.)  Blocks of several heights stay on
-        one stream: they share gradients, and state that may have to be made first."""
+        (A caller's orthogonalization gets them stacked, as the reference stacks them, and so do the operators here more
+        blocks than one call takes.)  Blocks of several heights stay on one stream: they share gradients, and state that
+        may have to be made first."""
         num_heads = self._resolve_num_heads(group)
         split_sizes = self._resolve_split_sizes(group)
         shape = params[0].shape
@@ -99,21 +122,20 @@ class _MomentumOrtho(OrthoOptimizer):
         states = [self._get_or_initialize_state(p, self._algo_name) for p in params]
         M = [s["momentum"] for s in states]
         V = [s["variance_neuron"] for s in states] if self._normalize else None
-        if split_sizes is None or self._custom_ns:
+        blocks = [] if split_sizes is None or self._custom_ns else _equal_blocks(split_sizes)
+        n = len(params)
+        if not blocks or any(n * mats * len(at) > _MOST_ROW_BLOCKS or n * len(at) > _MOST_ROW_BLOCK_ADDRESSES
+                             for _rows, mats, at in blocks):
             yield from self._matrix_phases(group, X, G, M, V, shape, mats, rows, cols, ratio_shape, split_sizes)
             return
-        first, at = {}, 0
-        for rows in split_sizes:
-            first.setdefault(rows, []).append(at)
-            at += rows
-        for rows, at in first.items():
-            Xb, Gb, Mb = (_row_blocks(t, (rows, at)) for t in (X, G, M))
-            Vb = V and _row_blocks(V, (rows, at))
-            yield from self._matrix_phases(group, Xb, Gb, Mb, Vb, (rows, cols), 1, rows, cols, (rows, cols), None)
+        for rows, mats, at in blocks:
+            Xb, Gb, Mb = (_row_blocks(t, (mats * rows, at)) for t in (X, G, M))
+            Vb = V and _row_blocks(V, (mats * rows, at))
+            yield from self._matrix_phases(group, Xb, Gb, Mb, Vb, (mats * rows, cols), mats, rows, cols, (rows, cols), None)
 
     def _matrix_phases(self, group: dict, X, G, M, V, shape, mats: int, rows: int, cols: int, ratio_shape, split_sizes):
         """The phases for tensors of ``shape``, each ``mats`` matrices of ``rows x cols``.  ``split_sizes``: row blocks that
-        are stacked for a caller's orthogonalization."""
+        are stacked for the orthogonalization."""
         flatten = group["flatten"]
         split_scales = None if split_sizes is None else split_lr_scales(split_sizes, shape, group["adjust_lr"])
         n = len(X)
@@ -127,7 +149,7 @@ class _MomentumOrtho(OrthoOptimizer):
         # The others are written into the zero-padded form the iteration carries, by the same pass.
         handed_over = self.prepared_input and split_sizes is None and not flat3d and not self._custom_ns
         prepared = (handed_over and ns.accepts_prepared(self._newton_schulz_func, n * mats, rows, cols)
-                    and all(t.data_ptr() % 16 == 0 for t in G + M))
+                    and ops.aligned16(G) and ops.aligned16(M))
         extents = ns.padded_extents(self._newton_schulz_func, n * mats, rows, cols) if handed_over else None
         if prepared or extents is not None:
             padded = extents is not None
