@@ -15,7 +15,7 @@ DION_BF16 = 0
 DION_F32 = 1
 DION_NS_GRAM = 1
 DION_NS_STATIC_SCRATCH_BYTES = 64 << 20
-ABI_VERSION = 13  # dion_abi_version() of the library these signatures describe
+ABI_VERSION = 14  # dion_abi_version() of the library these signatures describe
 
 _u64p = ctypes.POINTER(ctypes.c_uint64)
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -71,6 +71,8 @@ SIGNATURES = {
                                c_float, c_void_p, c_float, c_int, c_void_p]),
     "dion_normuon_stats": (c_int, [c_void_p, _u64p, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p,
                                    c_void_p]),
+    "dion_normuon_stats_scaled": (c_int, [c_void_p, _u64p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p,
+                                          c_void_p]),
     "dion_normuon_stats_selected": (c_int, [c_void_p, _u64p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                             c_float, c_void_p, c_void_p]),
     "dion_dion2_accumulate_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),

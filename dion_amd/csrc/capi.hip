@@ -37,7 +37,7 @@ static inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 static inline bool aligned16(uint64_t p) { return (p & 15) == 0; }
 
 extern "C" const char* dion_last_error(void) { return g_err; }
-extern "C" int dion_abi_version(void) { return 13; }
+extern "C" int dion_abi_version(void) { return 14; }
 
 // ---------------------------------------------------------------------------------------------
 // Kernel-level GEMMs
@@ -1365,7 +1365,7 @@ extern "C" int dion_scale_rows(const void* U, const float* scale, void* out, int
 
 static int normuon_stats_impl(const char* who, const void* U, const uint64_t* V_ptrs, int v_dtype, int n,
                               int mats_per_ptr, int rows, int cols, const int32_t* row_idx, int v_rows,
-                              float beta2, float* row_scale, void* stream) {
+                              float beta2, float* row_scale, void* stream, float u_scale = 1.0f) {
   if (int rc = check_state_dtype(who, "v_dtype", v_dtype)) return rc;
   if (n < 0 || mats_per_ptr <= 0 || rows < 0 || cols < 0 || v_rows < rows)
     return fail(DION_E_INVALID, "%s: bad size", who);
@@ -1381,7 +1381,7 @@ static int normuon_stats_impl(const char* who, const void* U, const uint64_t* V_
     const int64_t mat0 = (int64_t)i0 * mats_per_ptr;
     HIP_TRY(launch_normuon_stats((const bf16_t*)U + mat0 * rows * cols, v, dt(v_dtype), c * mats_per_ptr,
                                  mats_per_ptr, rows, cols, row_idx ? row_idx + mat0 * rows : nullptr,
-                                 v_rows, w, row_scale + mat0 * rows, (hipStream_t)stream),
+                                 v_rows, w, u_scale * u_scale, row_scale + mat0 * rows, (hipStream_t)stream),
             who);
   }
   return DION_OK;
@@ -1392,6 +1392,12 @@ extern "C" int dion_normuon_stats(const void* U, const uint64_t* V_ptrs, int v_d
                                   void* stream) {
   return normuon_stats_impl("dion_normuon_stats", U, V_ptrs, v_dtype, n, mats_per_ptr, rows, cols, nullptr, rows,
                             beta2, row_scale, stream);
+}
+
+extern "C" int dion_normuon_stats_scaled(const void* U, const uint64_t* V_ptrs, int v_dtype, int n, int mats_per_ptr,
+                                         int rows, int cols, float u_scale, float beta2, float* row_scale, void* stream) {
+  return normuon_stats_impl("dion_normuon_stats_scaled", U, V_ptrs, v_dtype, n, mats_per_ptr, rows, cols, nullptr, rows,
+                            beta2, row_scale, stream, u_scale);
 }
 
 extern "C" int dion_normuon_stats_selected(const void* U, const uint64_t* V_ptrs, int v_dtype, int n,

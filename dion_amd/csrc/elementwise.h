@@ -61,7 +61,7 @@ hipError_t launch_muon_post(const PtrTab& X, int x_dtype, const void* U, int u_d
 hipError_t launch_scale_rows(const bf16_t* U, const float* scale, void* out, int out_dtype, int64_t n_rows,
                              int cols, hipStream_t st);
 hipError_t launch_normuon_stats(const bf16_t* U, const PtrTab& V, int v_dtype, int n_mat, int mats_per_ptr,
-                                int rows, int cols, const int32_t* row_idx, int v_rows, float w,
+                                int rows, int cols, const int32_t* row_idx, int v_rows, float w, float u_sq,
                                 float* row_scale, hipStream_t st);
 hipError_t launch_dion2_accumulate(const PtrTab& G, int g_dtype, const PtrTab& M, int m_dtype, int n_mat,
                                    int mats_per_ptr, int rows, int cols, int select_rows,

@@ -795,12 +795,13 @@ hipError_t launch_scale_rows(const bf16_t* U, const float* scale, void* out, int
 // of selected rows only (NorDion2, dion/nordion2.py:430-447).  A negative row_idx entry marks a row
 // that is not part of the update (an all-zero row of a masked full-size tensor,
 // dion/nordion2.py:485-497): its second moment is left alone and its scale is 0.
-// Pass 1: one wavefront per row.  V <- lerp(V, mean(u^2), w);  tmp[row] = sum(u^2).
+// Pass 1: one wavefront per row.  V <- lerp(V, mean(u^2), w);  tmp[row] = sum(u^2).  u_sq is the square of a factor that the
+// rows count with (1: as they lie).
 template <typename VT>
 __global__ __launch_bounds__(256) void normuon_rows_kernel(const bf16_t* __restrict__ U, PtrTab V,
                                                            int mats_per_ptr, int rows, int cols,
                                                            const int32_t* __restrict__ row_idx,
-                                                           int v_rows, float w,
+                                                           int v_rows, float w, float u_sq,
                                                            float* __restrict__ rowsq) {
   const int mat = blockIdx.y;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -825,7 +826,7 @@ __global__ __launch_bounds__(256) void normuon_rows_kernel(const bf16_t* __restr
       s += v * v;
     }
   }
-  s = wave_sum(s);
+  s = wave_sum(s) * u_sq;
   if (lane == 0) {
     const int vr = row_idx ? row_idx[(int64_t)mat * rows + row] : row;
     if (vr >= 0) {
@@ -868,18 +869,18 @@ __global__ __launch_bounds__(1024) void normuon_scale_kernel(PtrTab V, int mats_
 }
 
 hipError_t launch_normuon_stats(const bf16_t* U, const PtrTab& V, int v_dtype, int n_mat, int mats_per_ptr,
-                                int rows, int cols, const int32_t* row_idx, int v_rows, float w,
+                                int rows, int cols, const int32_t* row_idx, int v_rows, float w, float u_sq,
                                 float* row_scale, hipStream_t st) {
   // U / row_scale / row_idx are offset to the first matrix by the caller; V is the table chunk
   // covering them.
   if (v_dtype == 0) {
     hipLaunchKernelGGL(normuon_rows_kernel<bf16_t>, dim3((rows + 3) / 4, n_mat), dim3(256), 0, st, U, V,
-                       mats_per_ptr, rows, cols, row_idx, v_rows, w, row_scale);
+                       mats_per_ptr, rows, cols, row_idx, v_rows, w, u_sq, row_scale);
     hipLaunchKernelGGL(normuon_scale_kernel<bf16_t>, dim3(n_mat), dim3(1024), 0, st, V, mats_per_ptr, rows,
                        row_idx, v_rows, row_scale);
   } else {
     hipLaunchKernelGGL(normuon_rows_kernel<float>, dim3((rows + 3) / 4, n_mat), dim3(256), 0, st, U, V,
-                       mats_per_ptr, rows, cols, row_idx, v_rows, w, row_scale);
+                       mats_per_ptr, rows, cols, row_idx, v_rows, w, u_sq, row_scale);
     hipLaunchKernelGGL(normuon_scale_kernel<float>, dim3(n_mat), dim3(1024), 0, st, V, mats_per_ptr, rows,
                        row_idx, v_rows, row_scale);
   }

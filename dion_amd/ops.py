@@ -540,10 +540,11 @@ def scale_rows(U: Tensor, scale: Tensor, dtype: torch.dtype) -> Tensor:
     return out
 
 
-def normuon_stats(U: Tensor, V: List[Tensor], beta2: float) -> Tensor:
+def normuon_stats(U: Tensor, V: List[Tensor], beta2: float, u_scale: float = 1.0) -> Tensor:
     """Updates every ``V[i]`` (``[..., rows, 1]``, fp32 or bf16) in place from the orthogonalized arena
     ``U [N, ..., rows, cols]`` and returns the per-row scales ``[n_mat, rows]`` that turn ``U`` into the
-    NorMuon-normalised update.  Mirrors ``normuon_normalization_stacked`` (dion/normuon.py:345-399)."""
+    NorMuon-normalised update.  Mirrors ``normuon_normalization_stacked`` (dion/normuon.py:345-399).  ``u_scale``: the
+    statistics of ``u_scale * U`` (the scales still apply to ``U``, times that factor)."""
     n = len(V)
     assert n > 0 and U.shape[0] == n
     _check_bf16(U, "U")
@@ -553,8 +554,10 @@ def normuon_stats(U: Tensor, V: List[Tensor], beta2: float) -> Tensor:
     vp, vcode = _state_ptrs(V, "V", mats_per_ptr * rows)
     scale = torch.empty(n_mat, rows, dtype=torch.float32, device=U.device)
     lib = _lib.load()
-    check(lib.dion_normuon_stats(U.data_ptr(), vp, vcode, n, mats_per_ptr, rows, cols, float(beta2),
-                                 scale.data_ptr(), _stream_handle(U.device)), "normuon_stats")
+    args = (U.data_ptr(), vp, vcode, n, mats_per_ptr, rows, cols)
+    tail = (float(beta2), scale.data_ptr(), _stream_handle(U.device))
+    check(lib.dion_normuon_stats(*args, *tail) if u_scale == 1.0 else
+          lib.dion_normuon_stats_scaled(*args, float(u_scale), *tail), "normuon_stats")
     return scale
 
 

@@ -131,11 +131,15 @@ class _MomentumOrtho(OrthoOptimizer):
         for rows, mats, at in blocks:
             Xb, Gb, Mb = (_row_blocks(t, (mats * rows, at)) for t in (X, G, M))
             Vb = V and _row_blocks(V, (mats * rows, at))
-            yield from self._matrix_phases(group, Xb, Gb, Mb, Vb, (mats * rows, cols), mats, rows, cols, (rows, cols), None)
+            scales = split_lr_scales((rows,), shape, group["adjust_lr"])
+            yield from self._matrix_phases(group, Xb, Gb, Mb, Vb, (mats * rows, cols), mats, rows, cols, (rows, cols), None,
+                                           1.0 if scales is None else scales[0])
 
-    def _matrix_phases(self, group: dict, X, G, M, V, shape, mats: int, rows: int, cols: int, ratio_shape, split_sizes):
+    def _matrix_phases(self, group: dict, X, G, M, V, shape, mats: int, rows: int, cols: int, ratio_shape, split_sizes,
+                       block_scale: float = 1.0):
         """The phases for tensors of ``shape``, each ``mats`` matrices of ``rows x cols``.  ``split_sizes``: row blocks that
-        are stacked for the orthogonalization."""
+        are stacked for the orthogonalization; ``block_scale``: what row blocks updated where they lie would be rescaled by
+        there, before the second moments are taken (the state is the same whichever way a step goes)."""
         flatten = group["flatten"]
         split_scales = None if split_sizes is None else split_lr_scales(split_sizes, shape, group["adjust_lr"])
         n = len(X)
@@ -169,7 +173,7 @@ class _MomentumOrtho(OrthoOptimizer):
             del U, sumsq
             yield
             _note_stream(O)
-            self._normalize_and_update(group, X, V, O, n, mats, rows, cols, ratio, None)
+            self._normalize_and_update(group, X, V, O, n, mats, rows, cols, ratio, None, block_scale)
             return
 
         U = ops.muon_pre(G, M, group["mu"], group["nesterov"])  # [n, *shape] bf16
@@ -195,9 +199,9 @@ class _MomentumOrtho(OrthoOptimizer):
         del U
         yield
         _note_stream(O)
-        self._normalize_and_update(group, X, V, O, n, mats, rows, cols, ratio, split_sizes)
+        self._normalize_and_update(group, X, V, O, n, mats, rows, cols, ratio, split_sizes, block_scale)
 
-    def _normalize_and_update(self, group, X, V, O, n, mats, rows, cols, ratio, split_sizes) -> None:
+    def _normalize_and_update(self, group, X, V, O, n, mats, rows, cols, ratio, split_sizes, block_scale) -> None:
         """NorMuon's neuron-wise normalisation (when this class normalises) and the update pass."""
         row_scale = None
         if self._normalize:
@@ -212,7 +216,7 @@ class _MomentumOrtho(OrthoOptimizer):
                     off += sz
                 row_scale = torch.cat(scales, dim=1).contiguous()
             else:
-                row_scale = ops.normuon_stats(O3, V, group["muon_beta2"])
+                row_scale = ops.normuon_stats(O3, V, group["muon_beta2"], block_scale)
         ops.muon_post(X, O.view(n, -1), group["lr"], ratio, group["weight_decay"],
                       group["cautious_wd"], row_scale=row_scale)
 

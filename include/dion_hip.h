@@ -281,6 +281,11 @@ int dion_scale_rows(const void* U, const float* scale, void* out, int out_dtype,
  * dion/normuon.py:320. */
 int dion_normuon_stats(const void* U, const uint64_t* V_ptrs, int v_dtype, int n, int mats_per_ptr,
                        int rows, int cols, float beta2, float* row_scale, void* stream);
+/* The same for matrices that count u_scale times what U holds: row blocks under split_sizes, whose second moments are those
+ * of the rescaled block (dion/megabatch_base.py:940-949, dion/normuon.py:359-369), from the block as it was
+ * orthogonalized. */
+int dion_normuon_stats_scaled(const void* U, const uint64_t* V_ptrs, int v_dtype, int n, int mats_per_ptr,
+                              int rows, int cols, float u_scale, float beta2, float* row_scale, void* stream);
 
 /* NorMuon statistics for an update made of k selected rows per matrix (NorDion2): U [n_mat, k,
  * cols] bf16, row_idx [n_mat, k] int32 gives the row of the parameter each update row belongs to

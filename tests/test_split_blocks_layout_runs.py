@@ -43,7 +43,7 @@ def test_addresses_a_step_hands_over(cls, split, calls, monkeypatch):
     opt = cls([{"params": params, "split_sizes": split}])
     seen = []
 
-    def phases(group, X, G, M, V, shape, mats, rows, cols, ratio_shape, split_sizes):
+    def phases(group, X, G, M, V, shape, mats, rows, cols, ratio_shape, split_sizes, block_scale=1.0):
         seen.append((len(X), mats, rows))
         assert len(G) == len(M) == len(X) and (V is None or len(V) == len(X)) and cols == 4
         assert (split_sizes is not None) == (len(split) > 4096) and tuple(ratio_shape) == (rows, cols)
