@@ -181,6 +181,12 @@ namespace {
 struct NsPlan {
   int m, n, mp, np, tall, nblk;
   bool gram;  // the Gram-matrix recurrence is used (requested and worth it for this aspect ratio)
+  // Whole 128-wide tiles that 256 would pad.  Their matrices are copied as a padded one is, and like it scaled in the copy where
+  // the squared norm is outside what the folded factor carries (a prepared one where it lies): which granule is faster
+  // does not decide what magnitudes an input may have.  us a call, copied / read where it lies: wide bf16 48 x (640 x 2560)
+  // 1309 / 1256, 30 x (896 x 3584) 1843 / 1807 (Gram form 1308 / 1260), 16 x (1408 x 1408) 1029 / 1035; fp32 and tall ones,
+  // whose norm was a pass over the copy, 30 x (896 x 3584) 1870 / 1943, 48 x (2560 x 640) 1297 / 1292.
+  bool ranged;
   size_t x_bytes, a_bytes, partial_bytes, inv_bytes, total;
 };
 
@@ -202,6 +208,7 @@ NsPlan make_plan(int batch, int rows, int cols, int flags) {
   pl.mp = round_up(pl.m, g);
   // (matrices of whole tiles stay as they are: they are read where they lie)
   pl.np = pl.mp == pl.m && pl.n % g == 0 ? pl.n : gemm_pad_long(pl.mp, pl.n, batch, g);
+  pl.ranged = pl.mp == pl.m && pl.np == pl.n && (pl.m % 256 || pl.n % 256) && gemm_pad_is_chosen(pl.m, batch);
   const int64_t numel = (int64_t)rows * cols;
   int64_t nb = numel / (256 * 32);
   if (nb < 1) nb = 1;
@@ -454,16 +461,17 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
   // GEMMs where it lies, any other is copied (rounded to bf16, transposed if tall) value for value, and the
   // normalisation rides on the first two GEMMs as for a prepared input -- one pass over a wide bf16 input instead
   // of two, and the same arithmetic whichever way (orientation, fp32 or bf16) a matrix is handed over.
-  const bool self_prep = !sumsq && aligned16((uint64_t)(uintptr_t)in) &&
+  const bool ranged = padded || (n_iters > 0 && pl.ranged);
+  const bool self_prep = !sumsq && !ranged && aligned16((uint64_t)(uintptr_t)in) &&
                          ns_takes_prepared(batch, rows, cols, flags, n_iters);
   // (not when `out` overlaps `in`: the copy is then what keeps a caller's in-place call working)
   const bool aliased = out && overlap(call.in_lo, call.in_hi - call.in_lo, call.out_lo, call.out_hi - call.out_lo);
   const bool in_place = self_prep && !pl.tall && in_dtype == DION_BF16 && !aliased;
   const bool copy_first = self_prep && pl.tall;
-  // A matrix that needs padding is copied, rounded to bf16 and unscaled, into its padded form; the copy delivers the
-  // partial sums of the norm, so it is the only pass over the input.  The partials (one per 64 x 64 tile) lie in the
+  // A matrix that needs padding, or whose range the copy keeps, is copied, rounded to bf16 and unscaled, into its padded
+  // form; the copy delivers the partial sums of the norm, so it is the only pass over the input.  The partials (one per 64 x 64 tile) lie in the
   // third X buffer, which only a call without iterations uses otherwise.
-  const bool pad_copy = padded && !sumsq;
+  const bool pad_copy = ranged && !sumsq;
   auto plan_norm = [&]() {
     if (sumsq || pad_copy) {
       NsStep s = blank_step(NsStep::kNormFinalize, "frobenius norm");
@@ -473,7 +481,7 @@ int ns_build(const void* in, int in_dtype, void* out, int batch, int rows, int c
       s.partial = sumsq ? const_cast<float*>(sumsq) : (float*)Xt;
       s.nblk = sumsq ? sumsq_blocks : (mp / 64) * (np / 64);
       s.inv = inv;
-      if (padded) {  // (a copy in either case: the caller's tensors themselves are never scaled)
+      if (ranged) {  // (a copy in either case: the caller's tensors themselves are never scaled)
         s.same = sumsq ? (bf16_t*)const_cast<void*>(in) : X[0];
         s.Rp = mp;
         s.Cp = np;
@@ -1063,7 +1071,7 @@ extern "C" int dion_ns_accepts_prepared(int batch, int rows, int cols, int flags
   return ns_accepts_prepared(batch, rows, cols, flags, n_iters) ? 1 : 0;
 }
 
-extern "C" int dion_ns_orthogonalize_prepared(const void* in, const float* sumsq, int sumsq_blocks, void* out,
+extern "C" int dion_ns_orthogonalize_prepared(void* in, const float* sumsq, int sumsq_blocks, void* out,
                                               int batch, int rows, int cols, const float* coeffs, int n_iters,
                                               float norm_scale, float eps, int flags, int gram_reset,
                                               void* workspace, size_t workspace_bytes, void* stream) {
@@ -1095,7 +1103,7 @@ static int update_prepared(const char* who, bool in_padded, const void* in, cons
                 workspace, workspace_bytes, stream, &ps, sumsq, sumsq_blocks, in_padded);
 }
 
-extern "C" int dion_ns_orthogonalize_update_prepared(const void* in, const float* sumsq, int sumsq_blocks,
+extern "C" int dion_ns_orthogonalize_update_prepared(void* in, const float* sumsq, int sumsq_blocks,
                                                      const uint64_t* X_ptrs, int x_dtype, int n_ptrs,
                                                      int mats_per_ptr, int rows, int cols, const float* coeffs,
                                                      int n_iters, float norm_scale, float eps, int flags,

@@ -268,6 +268,8 @@ hipError_t launch_gemm_nt_post(const GemmParams& p, const FusedPost& post, int x
 // Tile edge (128 or 256) launch_gemm_nt would use for a problem whose padded short/long
 // dims are given; workspaces are padded to this.
 int gemm_pad_granule(int m, int n, int batch);
+// Whether the symmetric products of the batch offer 256-wide tiles a full round of the CUs, so that 128 is a choice there.
+bool gemm_pad_is_chosen(int m, int batch);
 // ... and the padded long side n of matrices whose short side is padded to mp.
 int gemm_pad_long(int mp, int n, int batch, int granule);
 

@@ -1746,6 +1746,11 @@ static hipError_t launch_k64(const GemmParams& p, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
+bool gemm_pad_is_chosen(int m, int batch) {
+  const int64_t m256 = ((int64_t)m + 255) / 256;
+  return m256 * (m256 + 1) / 2 * batch >= 256;
+}
+
 int gemm_pad_granule(int m, int n, int batch) {
   // To 256 once whole 256-wide tiles make more than one round of the CUs for the symmetric products, so that every product may
   // use them -- unless the padding to 128 leaves 18 % of the operations out: 256-wide tiles take up to 13 % less time for the same
@@ -1755,9 +1760,7 @@ int gemm_pad_granule(int m, int n, int batch) {
   // (1.245); but 12 x (1920 x 1920) 1880 / 1936 (1.21), 40 x (1408 x 5632) 7970 / 8150 (1.20), 20 x (1664 x 6656) 6396 / 6702
   // (1.17), 24 x (1920 x 7680) 11020 / 11777 (1.14), 3 x (4224 x 4224) 4150 / 4618 (1.09).  Between 1.1 and 1.2 rounds of the CUs
   // decide some square ones the other way: 10 x (2176 x 2176) 2371 / 2195 (1.19), 8 x (2432 x 2432) 2569 / 2328 (1.17).
-  const int64_t m256 = (m + 255) / 256;
-  const int64_t syrk_tiles = m256 * (m256 + 1) / 2 * batch;
-  if (syrk_tiles < 256) return 128;
+  if (!gemm_pad_is_chosen(m, batch)) return 128;
   auto padded_ops = [&](int64_t g) {
     const int64_t mp = (m + g - 1) / g, np = (n + g - 1) / g;  // (in tiles: no overflow)
     return (double)(g * mp) * (double)(g * mp) * (double)(g * (3 * np + mp));

@@ -158,17 +158,19 @@ int dion_ns_orthogonalize_update(const void* in, int in_dtype, const uint64_t* X
  * plain calls give every matrix to one workgroup; DION_E_INVALID otherwise (use dion_ns_orthogonalize).  Such a batch
  * of whole-tile matrices with more than 64 rows or columns on the short side (16 and more matrices of 128 x up to 1024) is
  * taken all the same: it runs the GEMMs, slower than the plain call.
+ * Where rows or cols is an odd multiple of 128 (and the batch large enough for 256-wide tiles, which would pad it) a matrix
+ * whose squared norm lies outside 2^-80 ... 2^80 is scaled in place before the iteration.
  * Results may differ from dion_ns_orthogonalize in the last bf16 bit (the norm is summed in another order; where that
  * call runs the small-matrix kernel, every sum is).
  * ------------------------------------------------------------------------------------------ */
 int dion_ns_accepts_prepared(int batch, int rows, int cols, int flags, int n_iters);
-int dion_ns_orthogonalize_prepared(const void* in, const float* sumsq, int sumsq_blocks, void* out, int batch,
+int dion_ns_orthogonalize_prepared(void* in, const float* sumsq, int sumsq_blocks, void* out, int batch,
                                    int rows, int cols, const float* coeffs, int n_iters, float norm_scale,
                                    float eps, int flags, int gram_reset, void* workspace,
                                    size_t workspace_bytes, void* stream);
 /* dion_ns_orthogonalize_update on a prepared input (the update always rides on the last GEMM:
  * every shape that takes a prepared input fuses).  Workspace from dion_ns_update_workspace_bytes. */
-int dion_ns_orthogonalize_update_prepared(const void* in, const float* sumsq, int sumsq_blocks,
+int dion_ns_orthogonalize_update_prepared(void* in, const float* sumsq, int sumsq_blocks,
                                           const uint64_t* X_ptrs, int x_dtype, int n_ptrs, int mats_per_ptr,
                                           int rows, int cols, const float* coeffs, int n_iters,
                                           float norm_scale, float eps, int flags, int gram_reset,
