@@ -4,7 +4,6 @@ import pytest
 import torch
 
 import dion
-from dion_amd import newton_schulz as ns
 from dion_amd import ops
 
 pytestmark = pytest.mark.gpu
@@ -55,10 +54,20 @@ def test_select_into_the_padded_form(rows, cols, k, offset, mdtype):
     assert sumsq.shape == tiles.shape and bool(((sumsq.double() - tiles).abs() <= 32 * 2.0 ** -24 * tiles).all())
 
 
-@pytest.mark.parametrize("cls", [dion.Dion2, dion.NorDion2])
-@pytest.mark.parametrize("shape", [(600, 900), (900, 600), (2304, 768), (768, 1000), (1100, 1100)])
-def test_step_is_the_unprepared_one(cls, shape):
-    assert ns.padded_extents(ns.polar_express, 3, 150, 900) is not None
+# (Dion2 selects rows of matrices that are no taller than wide, NorDion2 always; the last block is a tall one, 600 x 300)
+@pytest.mark.parametrize("cls,shape", [
+    (dion.Dion2, (600, 900)), (dion.Dion2, (768, 1000)), (dion.Dion2, (1100, 1100)),
+    (dion.NorDion2, (600, 900)), (dion.NorDion2, (900, 600)), (dion.NorDion2, (2304, 768)), (dion.NorDion2, (768, 1000)),
+    (dion.NorDion2, (1100, 1100)), (dion.NorDion2, (2400, 300)),
+])
+def test_step_is_the_unprepared_one(cls, shape, monkeypatch):
+    select, forms = ops.dion2_select, []
+
+    def seen(*args, **kw):
+        forms.append(kw.get("extents"))
+        return select(*args, **kw)
+
+    monkeypatch.setattr(ops, "dion2_select", seen)
     got = []
     for handed_over in (True, False):
         params = [torch.nn.Parameter(_rand(shape, i)) for i in range(3)]
@@ -69,4 +78,5 @@ def test_step_is_the_unprepared_one(cls, shape):
                 p.grad = _rand(shape, 50 + 10 * step + i)
             opt.step()
         got.append([p.data for p in params] + [opt.state[p]["momentum"] for p in params])
+    assert all(forms[:2]) and forms[2:] == [None, None]  # the padded gather in both steps of the first run, in none of the second
     assert all(torch.equal(a, b) for a, b in zip(*got))
