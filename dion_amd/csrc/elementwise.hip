@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void muon_pre_transposed_kernel(PtrTab G, PtrT
 // Bound: HBM.  12 x (2730 x 1000) fp32, momentum update included: 95 us beside another stream's GEMMs, where the update
 // (76), the norm's pass over its result (14) and the scaled copy (30) took 120; 4 x (2730 x 1000) fp32 copied: 15.0 us
 // where copy and norm took 23.4.  Selected rows gathered here instead of copied a second time: NorDion2 on 12 layers of 1600,
-// a step, 4100 -> 3960 us (bf16 state 3571 -> 3400).
+// a step, 4130 -> 3935 us (bf16 state 3594 -> 3372).
 // ------------------------------------------------------------------------------------------
 template <typename T, int V>
 static __device__ __forceinline__ void load_group(const T* p, int64_t i, float* v) {

@@ -298,8 +298,8 @@ static void set_tile_order(GemmParams& p, int bm, int bn) {
   // 128-wide tiles are two to a CU, 64 of them side by side on an XCD: X X^T of 8 x (1024 x 14336) 132 / 164, of 2 x (2048 x 5504)
   // 62 / 68, of 40 x (1408 x 5632) 482 / 511.
   // The tiles past the last whole 256 are one contiguous run per XCD in either order: dealt out singly, no two workgroups
-  // of an XCD shared an operand there (X X^T of 6 x (1024 x 8192), 216 tiles, 100 us instead of 50; of 12 x (1536 x 6144) 180
-  // instead of 141; B X of 32 x (4096 x 14336) 11208 instead of 11064).
+  // of an XCD shared an operand there (repeated on one operand, X X^T of 6 x (1024 x 8192), 216 tiles, 101 us instead of 53, of
+  // 12 x (1536 x 6144) 180 instead of 141; B X of 32 x (4096 x 14336) 11208 instead of 11064).
   const int64_t p_mb = ((int64_t)p.M * p.K * 2) >> 20;
   if (bm != 256) p.xcd_interleave = 0;
   else p.xcd_interleave = p_mb >= 16 && (p.q_kmajor || p.K >= 3584) ? 1 : 0;
@@ -1760,6 +1760,9 @@ int gemm_pad_granule(int m, int n, int batch) {
   // (1.245); but 12 x (1920 x 1920) 1880 / 1936 (1.21), 40 x (1408 x 5632) 7970 / 8150 (1.20), 20 x (1664 x 6656) 6396 / 6702
   // (1.17), 24 x (1920 x 7680) 11020 / 11777 (1.14), 3 x (4224 x 4224) 4150 / 4618 (1.09).  Between 1.1 and 1.2 rounds of the CUs
   // decide some square ones the other way: 10 x (2176 x 2176) 2371 / 2195 (1.19), 8 x (2432 x 2432) 2569 / 2328 (1.17).
+  // The Gram form, whose products are others, loses nowhere: padded to 256 / by this rule 100 x (384 x 1536) 819 / 552, 90 x (300 x
+  // 1000) 636 / 426, 48 x (640 x 2560) 1090 / 860, 30 x (896 x 3584) 1543 / 1229, 50 x (1152 x 4608) 4716 / 4322; the same extents for
+  // 40 x (1408 x 5632) 6067 / 6066.
   if (!gemm_pad_is_chosen(m, batch)) return 128;
   auto padded_ops = [&](int64_t g) {
     const int64_t mp = (m + g - 1) / g, np = (n + g - 1) / g;  // (in tiles: no overflow)
@@ -1776,6 +1779,7 @@ int gemm_pad_long(int mp, int n, int batch, int granule) {
   // 2680) 559 / 545, 48 x (512 x 2168) 706 / 700, 6 x (1536 x 4216) 1032 / 1029; at 384 tiles 24 x (500 x 1920) 325 / 328, 16 x
   // (768 x 1912) 458 / 450, fewer 24 x (512 x 1400) 286 / 291, and where B has one row of tiles 60 x (256 x 2168) 331 / 344.  A Muon
   // step of 10 layers of 1530 x 4100 7051 / 6510, NorMuon, 8 of 1280 x 3400, 3448 / 3292, 24 of 512 x 2168 1327 / 1313.
+  // Gram form 24 x (512 x 8056) 674 / 600, 12 x (1024 x 3448) 660 / 628, 48 x (512 x 2168) 538 / 527, 24 x (512 x 2168) 283 / 279.
   const int np = (n + granule - 1) / granule * granule;
   const bool fits = mp % 256 == 0 && mp >= 512 && np % 256 == 128;
   return fits && (int64_t)(mp / 256) * ((np + 128) / 256) * batch > 384 ? np + 128 : np;
