@@ -1760,6 +1760,7 @@ int gemm_pad_granule(int m, int n, int batch) {
   // (1.245); but 12 x (1920 x 1920) 1880 / 1936 (1.21), 40 x (1408 x 5632) 7970 / 8150 (1.20), 20 x (1664 x 6656) 6396 / 6702
   // (1.17), 24 x (1920 x 7680) 11020 / 11777 (1.14), 3 x (4224 x 4224) 4150 / 4618 (1.09).  Between 1.1 and 1.2 rounds of the CUs
   // decide some square ones the other way: 10 x (2176 x 2176) 2371 / 2195 (1.19), 8 x (2432 x 2432) 2569 / 2328 (1.17).
+  // (Taken with whole 128-wide tiles read where they lie; a plain call copies them, 1-4 % more of a wide bf16 one: NsPlan::ranged.)
   // The Gram form, whose products are others, loses nowhere: padded to 256 / by this rule 100 x (384 x 1536) 819 / 552, 90 x (300 x
   // 1000) 636 / 426, 48 x (640 x 2560) 1090 / 860, 30 x (896 x 3584) 1543 / 1229, 50 x (1152 x 4608) 4716 / 4322; the same extents for
   // 40 x (1408 x 5632) 6067 / 6066.
