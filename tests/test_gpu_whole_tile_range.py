@@ -62,3 +62,32 @@ def test_norms_past_fp32_and_values_that_are_not_finite(shape):
         assert bool(O[1].isnan().all())
         assert torch.equal(O[2:], want[2:])
     assert float(G[0, 0, 0]) == 2.0 ** 64  # a plain call leaves its input alone
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("gram", [False, True])
+def test_launches_stay_in_their_buffers(shape, gram):
+    """Every launch of plain, updating, in-place and prepared calls inside the call's buffers; in a short workspace, not."""
+    from dion_amd import _lib
+
+    lib, (b, r, c), flags = _lib.load(), shape, _lib.DION_NS_GRAM if gram else 0
+    for in_dtype in (_lib.DION_BF16, _lib.DION_F32):
+        for update in (0, 1):
+            assert lib.dion_ns_plan_audit(b, r, c, in_dtype, 5, flags, 2, update, _lib.DION_F32, 3, 0) > 0
+    assert lib.dion_ns_plan_audit_prepared(b, r, c, 5, flags, 2, 1, _lib.DION_F32, 3, 0) > 0
+    assert lib.dion_ns_plan_audit_overlap(b, r, c, _lib.DION_BF16, 5, flags, 2, 0) > 0
+    assert lib.dion_ns_plan_audit(b, r, c, _lib.DION_BF16, 5, flags, 2, 0, _lib.DION_F32, 1, 1 << 20) < 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", SHAPES[:2])
+def test_update_on_the_last_product(shape, x_dtype):
+    """One call against orthogonalization and update, bit for bit."""
+    b, r, c = shape
+    G, lr = _rand(shape, 3), torch.tensor(0.02, device=DEV)
+    X1 = [_rand((3, r, c), 10 + i, x_dtype) for i in range(b // 3)]
+    X2 = [x.clone() for x in X1]
+    ns.orthogonalize_update(ns.polar_express, G, 1e-6, X1, lr, 0.7, 0.1, True)
+    ops.muon_post(X2, ns.polar_express(G, 1e-6).view(b // 3, -1), lr, 0.7, 0.1, True)
+    assert all(torch.equal(x, y) for x, y in zip(X1, X2))
